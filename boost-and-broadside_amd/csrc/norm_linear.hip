@@ -1,6 +1,6 @@
 // RMSNorm + Linear as ONE kernel on the matrix cores (gfx950), optionally over gathered rows.
 //
-//   n   = x[row] * rsqrt(mean(x[row]^2) + eps) * w_norm               x fp32, 128 channels
+//   n   = x[row] * rsqrt(mean(x[row]^2) + eps) * w_norm               x fp32 or bf16, 128 channels
 //   out = bf16(n W^T + bias)                                          W (N, 128) bf16, N % 64 == 0
 // Reference: `self.kv_bullet(self.norm_bullet(bullets))` (models/yemong/attention.py:150-151),
 // `self.qkv(self.norm1(x))` (:94-96,132) and the temporal block's `linear1(norm1(x))`
@@ -20,6 +20,11 @@
 // consecutive features (16-byte stores, the two lanes of a row side by side):
 //   [fb][ks][l][e] = W[32fb + 16((r/8)/2) + 8((r/4)%2) + 4((r/8)%2) + r%4][ch(ks, l/32, e)],  r = l%32
 // Weights stream through LDS in chunks of 64 features (16 KB), double-buffered.
+//
+// bf16 rows (what an encoder under bf16 autocast hands over) are 256 bytes: one pass brings them in whole, and the
+// staging area holds them as they are.  The kernel is bound by its bytes, so they are read in the type they have and only
+// where a bullet is in flight; the library's norm and projection over every slot that they went through before took 1.6 of
+// the 2.23 ms of a rollout step of 7808 environments x 80 slots (now 0.86 ms).
 
 #include "common.h"
 
@@ -32,9 +37,12 @@ constexpr int kNlChunkFeatures = 64;
 constexpr int kNlChunkHalfs = kNlChunkFeatures * kNlD;                 // 8192 bf16 = 16 KB
 constexpr int kNlPrefetch = kNlChunkHalfs / 8 / kNlThreads;           // 16-byte pieces per thread per chunk
 constexpr int kNlHalfPitch = 64 + 4;                                   // floats per staged half row (bank spread)
+constexpr int kNlRowPitch = kNlD + 8;                                  // halfs per staged bf16 row
+static_assert(kNlRowPitch * 2 <= kNlHalfPitch * 4, "a staged bf16 row fits the slice's row pitch");
 
+template <typename XT>
 __global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
-    const float *__restrict__ x, int64_t x_stride, const int32_t *__restrict__ row_index,
+    const XT *__restrict__ x, int64_t x_stride, const int32_t *__restrict__ row_index,
     const int32_t *__restrict__ n_rows, const float *__restrict__ norm_w, float eps,
     const uint16_t *__restrict__ wpack, const float *__restrict__ bias, uint16_t *__restrict__ out, int64_t R, int N,
     uint16_t *__restrict__ n_out = nullptr)
@@ -86,38 +94,60 @@ __global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
     // channels arrive (the row never sits in registers as fp32), same relative rounding.
     bf16x8 nb[8];
     float ss = 0.0f;
-    // both passes' rows are requested before the first one is staged: one round trip to memory instead of two
-    f32x4 xv[2][8];
+    auto operand = [&](int ks, const float (&t)[8]) {  // k-slots of contraction step ks: channels 16 ks + ...
+        const f32x4 wl = *reinterpret_cast<const f32x4 *>(norm_w + 16 * ks + 4 * half);
+        const f32x4 wh = *reinterpret_cast<const f32x4 *>(norm_w + 16 * ks + 8 + 4 * half);
+        const float wv[8] = {wl.x, wl.y, wl.z, wl.w, wh.x, wh.y, wh.z, wh.w};
 #pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            xv[pass][j] = __builtin_nontemporal_load(
-                reinterpret_cast<const f32x4 *>(x + src_row[j] * x_stride + 64 * pass + io_col));
-    }
-#pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            *reinterpret_cast<f32x4 *>(stage + (4 * j + io_row) * kNlHalfPitch + io_col) = xv[pass][j];
-        __syncthreads();
-#pragma unroll
-        for (int k4 = 0; k4 < 4; ++k4) {  // contraction step ks = 4 pass + k4: channels 16 ks + ...
-            const int ks = 4 * pass + k4;
-            const float *sp = stage + m * kNlHalfPitch + 16 * k4 + 4 * half;
-            const f32x4 lo = *reinterpret_cast<const f32x4 *>(sp);
-            const f32x4 hi = *reinterpret_cast<const f32x4 *>(sp + 8);
-            const f32x4 wl = *reinterpret_cast<const f32x4 *>(norm_w + 16 * ks + 4 * half);
-            const f32x4 wh = *reinterpret_cast<const f32x4 *>(norm_w + 16 * ks + 8 + 4 * half);
-            const float t[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-            const float wv[8] = {wl.x, wl.y, wl.z, wl.w, wh.x, wh.y, wh.z, wh.w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                nb[ks][e] = (__bf16)(t[e] * wv[e]);
-                ss = fmaf(t[e], t[e], ss);
-            }
+        for (int e = 0; e < 8; ++e) {
+            nb[ks][e] = (__bf16)(t[e] * wv[e]);
+            ss = fmaf(t[e], t[e], ss);
         }
-        __syncthreads();
+    };
+    if constexpr (is_bf16<XT>::value) {
+        uint16_t *stage_x = reinterpret_cast<uint16_t *>(stage);  // 32 x 136 halfs fill the slice's 32 x 68 floats
+        u32x4 xv[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            xv[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + src_row[j] * x_stride + 2 * io_col));
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            *reinterpret_cast<u32x4 *>(stage_x + (4 * j + io_row) * kNlRowPitch + 2 * io_col) = xv[j];
+        wave_lds_handover();
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+            const uint16_t *sp = stage_x + m * kNlRowPitch + 16 * ks + 4 * half;
+            const Row4 lo = load4<false>(sp), hi = load4<false>(sp + 8);
+            const float t[8] = {lo.v[0], lo.v[1], lo.v[2], lo.v[3], hi.v[0], hi.v[1], hi.v[2], hi.v[3]};
+            operand(ks, t);
+        }
+        __syncthreads();  // the slices are read out before the weights move in
+    } else {
+        // both passes' rows are requested before the first one is staged: one round trip to memory instead of two
+        f32x4 xv[2][8];
+#pragma unroll
+        for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                xv[pass][j] = __builtin_nontemporal_load(
+                    reinterpret_cast<const f32x4 *>(x + src_row[j] * x_stride + 64 * pass + io_col));
+        }
+#pragma unroll
+        for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                *reinterpret_cast<f32x4 *>(stage + (4 * j + io_row) * kNlHalfPitch + io_col) = xv[pass][j];
+            __syncthreads();
+#pragma unroll
+            for (int k4 = 0; k4 < 4; ++k4) {
+                const float *sp = stage + m * kNlHalfPitch + 16 * k4 + 4 * half;
+                const f32x4 lo = *reinterpret_cast<const f32x4 *>(sp);
+                const f32x4 hi = *reinterpret_cast<const f32x4 *>(sp + 8);
+                const float t[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                operand(4 * pass + k4, t);
+            }
+            __syncthreads();
+        }
     }
     ss += __shfl_xor(ss, 32);
     const float rstd = rsqrtf(ss * (1.0f / kNlD) + eps);
@@ -126,15 +156,13 @@ __global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
         // The update keeps the normalised rows for the weight gradient: the operand this kernel multiplies is
         // rstd * bf16(x * w_norm); its bfloat16 rounding leaves as whole 256-byte rows through this wave's slice
         // of the staging area (32 rows x 136 halfs fit in the 32 x 68 floats of the slice).
-        constexpr int kNPitch = kNlD + 8;
-        static_assert(kNPitch * 2 <= kNlHalfPitch * 4, "a staged bf16 row fits the slice's row pitch");
         uint16_t *stage_n = reinterpret_cast<uint16_t *>(stage);
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
             float t[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) t[e] = (float)nb[ks][e] * rstd;
-            uint16_t *sp = stage_n + m * kNPitch + 16 * ks + 4 * half;
+            uint16_t *sp = stage_n + m * kNlRowPitch + 16 * ks + 4 * half;
             *reinterpret_cast<u32x2 *>(sp) = u32x2{pack_bf16x2(t[0], t[1]), pack_bf16x2(t[2], t[3])};
             *reinterpret_cast<u32x2 *>(sp + 8) = u32x2{pack_bf16x2(t[4], t[5]), pack_bf16x2(t[6], t[7])};
         }
@@ -143,7 +171,7 @@ __global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int64_t r = row0 + 4 * j + a_row;
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(stage_n + (4 * j + a_row) * kNPitch + a_col);
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(stage_n + (4 * j + a_row) * kNlRowPitch + a_col);
             if (r < rows) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(n_out + r * kNlD + a_col));
         }
         __syncthreads();  // the slices are read out before the weights move in
@@ -232,26 +260,47 @@ __global__ __launch_bounds__(64) void mask_fill_kernel(const uint8_t *__restrict
 
 }  // namespace bnb
 
-extern "C" int bnb_norm_linear_fwd(const float *x, int64_t x_row_stride, const int32_t *row_index,
-                                   const int32_t *n_rows, const float *norm_weight, float eps,
-                                   const void *weight_packed, const float *bias, void *out, int64_t R, int D, int N,
-                                   void *stream)
+namespace bnb {
+
+template <typename XT>
+static int launch_norm_linear(const XT *x, int64_t x_row_stride, const int32_t *row_index, const int32_t *n_rows,
+                              const float *norm_weight, float eps, const void *weight_packed, const float *bias, void *out,
+                              int64_t R, int D, int N, void *stream)
 {
-    using namespace bnb;
     if (R < 0 || x_row_stride < D || N < 1) return BNB_ERR_BAD_SHAPE;
     if (D != kNlD || N % kNlChunkFeatures != 0) return BNB_ERR_UNSUPPORTED;
     if (R == 0) return 0;
     if (!x || !norm_weight || !weight_packed || !out) return BNB_ERR_NULL_POINTER;
     if (!aligned16(x) || !aligned16(out) || !aligned16(norm_weight) || !aligned16(weight_packed) ||
-        (bias && !aligned16(bias)) || (x_row_stride % 4) != 0)
+        (bias && !aligned16(bias)) || (x_row_stride * sizeof(XT)) % 16 != 0)
         return BNB_ERR_MISALIGNED;
     if ((reinterpret_cast<uintptr_t>(row_index) | reinterpret_cast<uintptr_t>(n_rows)) & 3u) return BNB_ERR_MISALIGNED;
     const int64_t blocks = (R + kNlWaves * 32 - 1) / (kNlWaves * 32);
     if (blocks > 0x7fffffffLL) return BNB_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(norm_linear_kernel, dim3((unsigned)blocks), dim3(kNlThreads), 0, (hipStream_t)stream, x,
+    hipLaunchKernelGGL(norm_linear_kernel<XT>, dim3((unsigned)blocks), dim3(kNlThreads), 0, (hipStream_t)stream, x,
                        x_row_stride, row_index, n_rows, norm_weight, eps, (const uint16_t *)weight_packed, bias,
-                       (uint16_t *)out, R, N);
+                       (uint16_t *)out, R, N, (uint16_t *)nullptr);
     return (int)hipGetLastError();
+}
+
+}  // namespace bnb
+
+extern "C" int bnb_norm_linear_fwd(const float *x, int64_t x_row_stride, const int32_t *row_index,
+                                   const int32_t *n_rows, const float *norm_weight, float eps,
+                                   const void *weight_packed, const float *bias, void *out, int64_t R, int D, int N,
+                                   void *stream)
+{
+    return bnb::launch_norm_linear(x, x_row_stride, row_index, n_rows, norm_weight, eps, weight_packed, bias, out, R, D, N,
+                                   stream);
+}
+
+extern "C" int bnb_norm_linear_bf16_fwd(const void *x, int64_t x_row_stride, const int32_t *row_index,
+                                        const int32_t *n_rows, const float *norm_weight, float eps,
+                                        const void *weight_packed, const float *bias, void *out, int64_t R, int D, int N,
+                                        void *stream)
+{
+    return bnb::launch_norm_linear((const uint16_t *)x, x_row_stride, row_index, n_rows, norm_weight, eps, weight_packed,
+                                   bias, out, R, D, N, stream);
 }
 
 extern "C" int bnb_norm_linear_train_fwd(const float *x, int64_t x_row_stride, const float *norm_weight, float eps,
@@ -268,7 +317,7 @@ extern "C" int bnb_norm_linear_train_fwd(const float *x, int64_t x_row_stride, c
         return BNB_ERR_MISALIGNED;
     const int64_t blocks = (R + kNlWaves * 32 - 1) / (kNlWaves * 32);
     if (blocks > 0x7fffffffLL) return BNB_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(norm_linear_kernel, dim3((unsigned)blocks), dim3(kNlThreads), 0, (hipStream_t)stream, x,
+    hipLaunchKernelGGL(norm_linear_kernel<float>, dim3((unsigned)blocks), dim3(kNlThreads), 0, (hipStream_t)stream, x,
                        x_row_stride, (const int32_t *)nullptr, (const int32_t *)nullptr, norm_weight, eps,
                        (const uint16_t *)weight_packed, (const float *)nullptr, (uint16_t *)out, R, N, (uint16_t *)n_out);
     return (int)hipGetLastError();

@@ -2591,14 +2591,14 @@ def norm_linear(
 ) -> torch.Tensor:
     """``linear(rmsnorm(x) * norm_weight)`` in one matrix-core kernel with bfloat16 projection.
 
-    x (..., 128) float32 with contiguous rows; ``weight_packed`` from ``pack_linear_weights``
+    x (..., 128) float32 or bfloat16 with contiguous rows; ``weight_packed`` from ``pack_linear_weights``
     (N features).  With ``rows`` only the listed rows of the flattened x are projected, into
     the leading ``rows.total`` rows of a (capacity, N) result in list order; the remaining
     rows of the result are left unwritten.  Returns bfloat16 (..., N), or (capacity, N) with ``rows``.
     """
     D = x.shape[-1]
-    if not (x.is_cuda and x.dtype == torch.float32 and D == FFN_WIDTH):
-        raise RuntimeError("norm_linear covers float32 (..., 128) inputs on the GPU")
+    if not (x.is_cuda and x.dtype in _DTYPE_CODE and D == FFN_WIDTH):
+        raise RuntimeError("norm_linear covers float32 and bfloat16 (..., 128) inputs on the GPU")
     if torch.is_grad_enabled() and x.requires_grad:
         raise RuntimeError("norm_linear is forward-only; call it under torch.no_grad()")
     if weight_packed.dtype != torch.bfloat16 or weight_packed.dim() != 4 or not weight_packed.is_contiguous():
@@ -2622,7 +2622,8 @@ def norm_linear(
     norm_weight = norm_weight.detach().contiguous()
     if R:
         with _on_device(x.device):
-            rc = _native.load().bnb_norm_linear_fwd(
+            lib = _native.load()
+            rc = (lib.bnb_norm_linear_fwd if x.dtype == torch.float32 else lib.bnb_norm_linear_bf16_fwd)(
                 x2.data_ptr(), x2.stride(0), None if rows is None else rows.index.data_ptr(),
                 None if rows is None else rows.total.data_ptr(), norm_weight.data_ptr(),
                 float(_F32_EPS if eps is None else eps), weight_packed.data_ptr(), bias_ptr, out.data_ptr(), R, D, N,

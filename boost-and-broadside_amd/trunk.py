@@ -707,10 +707,10 @@ class TransformerBlock(_WeightCaches, nn.Module):
 
     def _compact_read_ok(self, qkv, bullets) -> bool:
         """Whether the bullet read can run on the compacted list (bf16 projections, width 128,
-        heads of 32, at most 160 entity tokens, float32 bullet tokens on the GPU)."""
+        heads of 32, at most 160 entity tokens, float32 or bfloat16 bullet tokens on the GPU)."""
         return (
             qkv.dtype == torch.bfloat16 and self.d_model == ops.FFN_WIDTH and self.head_dim == 32 and qkv.shape[1] <= 160
-            and bullets.is_cuda and bullets.dtype == torch.float32 and self.kv_bullet.bias is None
+            and bullets.is_cuda and bullets.dtype in (torch.float32, torch.bfloat16) and self.kv_bullet.bias is None
             # the compacted [K | V] rows are addressed with 32-bit element offsets over the full slot capacity
             and bullets.shape[0] * bullets.shape[1] * 2 * self.d_model < 2 ** 32
         )
@@ -1587,7 +1587,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
         bullet_rows = bullet_mask
         if (
             bullets is not None and bullet_mask is not None and self.config.reads_bullets and bullets.is_cuda
-            and bullets.dtype == torch.float32 and _projection_dtype() == torch.bfloat16 and D == ops.FFN_WIDTH
+            and bullets.dtype in (torch.float32, torch.bfloat16) and _projection_dtype() == torch.bfloat16 and D == ops.FFN_WIDTH
             and D // self.config.n_heads == 32 and NM <= 160
         ):
             bullet_rows = ops.CompactRows(bullet_mask)

@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define BNB_ABI_VERSION 28
+#define BNB_ABI_VERSION 29
 
 /* element types of activation buffers */
 #define BNB_F32 0
@@ -699,6 +699,13 @@ int bnb_norm_linear_fwd(const float *x, int64_t x_row_stride, const int32_t *row
                         const int32_t *n_rows, const float *norm_weight, float eps,
                         const void *weight_packed, const float *bias, void *out,
                         int64_t R, int D, int N, void *stream);
+
+/* bnb_norm_linear_fwd over bf16 rows x (row stride in elements, a multiple of 8): the tokens an encoder emits under bf16
+ * autocast (models/yemong/encoder.py:82-101), read in the type they have. */
+int bnb_norm_linear_bf16_fwd(const void *x, int64_t x_row_stride, const int32_t *row_index,
+                             const int32_t *n_rows, const float *norm_weight, float eps,
+                             const void *weight_packed, const float *bias, void *out,
+                             int64_t R, int D, int N, void *stream);
 
 /*
  * bnb_norm_linear_fwd for the PPO update (train/rl/ppo.py:1417-1425 re-evaluates the rollout in grad mode): the same

@@ -1470,6 +1470,22 @@ def test_compact_rows_and_gathered_projection(B, n, p):
         assert max_rel(out[:total].float().cpu(), want) <= BF16_TOL
 
 
+@pytest.mark.parametrize("R", [1, 31, 129, 1000])
+@pytest.mark.parametrize("listed", [False, True])
+def test_norm_linear_over_bfloat16_rows_gives_the_bits_of_the_widened_rows(R, listed):
+    """bfloat16 rows are exact in float32 and the operand and sums are formed in the same order: no tolerance."""
+    g = torch.Generator().manual_seed(R)
+    D, N = 128, 512
+    wide = torch.randn(R, 2 * D, generator=g).bfloat16().to(DEV)
+    x = wide[:, D:]  # rows of a wider tensor
+    nw = (1.0 + 0.1 * torch.randn(D, generator=g)).to(DEV)
+    pk = ops.pack_linear_weights((torch.randn(N, D, generator=g) / D ** 0.5).to(DEV))
+    rows = ops.CompactRows((torch.rand(1, R, generator=g) < 0.4).to(DEV)) if listed else None
+    total = rows.total_host() if listed else R
+    got, want = ops.norm_linear(x, nw, pk, rows=rows)[:total], ops.norm_linear(x.float(), nw, pk, rows=rows)[:total]
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("B,NQ,NK,p", [(4, 12, 80, 0.5), (3, 84, 800, 0.3), (3, 156, 1520, 0.1), (2, 33, 3000, 0.6), (5, 20, 190, 0.0),
                                        (3, 131, 900, 0.4), (4, 160, 1520, 0.02)])
 def test_sdpa_cross_over_compacted_rows_equals_the_masked_form(B, NQ, NK, p):

@@ -1265,6 +1265,26 @@ def test_bfloat16_tokens_under_autocast_run_on_the_kernels_and_match_the_oracle(
     assert xs.grad.dtype == torch.bfloat16 and torch.isfinite(xs.grad).all() and xs.grad.abs().max() > 0
 
 
+@pytest.mark.parametrize("readers", [1, 2])
+def test_bfloat16_bullets_are_read_on_the_kernels_and_give_the_widened_bullets_result(readers):
+    """Bullet tokens of a bfloat16 encoder: no library dispatch, and the same values as the same bullets in float32."""
+    from boost_and_broadside_amd import trunk as trunk_module
+
+    D, H, B, N, M = 128, 4, 9, 5, 3
+    torch.manual_seed(51)
+    trunk = bnb.YemongTrunk(_cfg(D, H, readers, 2, 1, bullets=1)).eval().to(DEV)
+    g = torch.Generator().manual_seed(52)
+    x = torch.randn(B, N + M, D, generator=g).bfloat16().to(DEV)
+    bul = torch.randn(B, 10 * N, D, generator=g).bfloat16().to(DEV)
+    bm = (torch.rand(B, 10 * N, generator=g) < 0.3).to(DEV)
+    alive = (torch.rand(B, N + M, generator=g) < 0.8).to(DEV)
+    hidden = trunk.initial_hidden(B, N, DEV)
+    with torch.autocast("cuda", dtype=torch.bfloat16), trunk_module.forbid_library_dispatch():
+        out, state = trunk(x, alive, hidden, bul, bm)
+        want, want_state = trunk(x, alive, hidden, bul.float(), bm)
+    assert torch.equal(out, want) and torch.equal(state, want_state)
+
+
 def test_team_pooling_takes_a_bfloat16_stream_under_autocast_on_the_kernels():
     from boost_and_broadside_amd import trunk as trunk_module
 

@@ -42,6 +42,7 @@
 
 #include "common.h"
 #include "ffn_math.h"
+#include "ffn_small.h"
 
 namespace bnb {
 
@@ -581,6 +582,10 @@ extern "C" int bnb_ffn_fused_proj_next_fwd(const float *x, int64_t x_row_stride,
     NextHead next;
     next.norm_weight = next_norm_weight, next.eps = next_eps, next.packed = next_packed, next.out = next_out, next.features = next_features;
     hipStream_t s = (hipStream_t)stream;
+    if (R <= ffn_small_rows_limit())
+        return launch_ffn_small({x, x_row_stride, (const uint16_t *)rows_a, rows_a_stride, (const uint16_t *)rows_b, rows_b_stride,
+                                 (const uint16_t *)proj_packed, norm_weight, eps, (const uint16_t *)weights_packed, out, R,
+                                 next_norm_weight, next_eps, (const uint16_t *)next_packed, (uint16_t *)next_out, next_features, nullptr, nullptr}, s);
     if (rows_b)
         return launch_ffn<kDeltaGate, false, true>(x, x_row_stride, rows_a, rows_b, proj_packed, norm_weight, eps, weights_packed,
                                                    out, R, rows_a_stride, rows_b_stride, s, nullptr, nullptr, next);
@@ -601,6 +606,10 @@ extern "C" int bnb_ffn_fused_proj_train_fwd(const float *x, int64_t x_row_stride
     if (rows_a_stride < kFfnD) return BNB_ERR_BAD_SHAPE;
     if (!aligned16(rows_a) || rows_a_stride % 8 != 0 || !aligned16(proj_packed) || !aligned16(s_out) || !aligned16(n_out))
         return BNB_ERR_MISALIGNED;
+    if (R <= ffn_small_rows_limit())  // the same rule as for inference: both forms of one call give the same bits
+        return launch_ffn_small({x, x_row_stride, (const uint16_t *)rows_a, rows_a_stride, nullptr, kFfnD,
+                                 (const uint16_t *)proj_packed, norm_weight, eps, (const uint16_t *)weights_packed, out, R,
+                                 nullptr, 0.0f, nullptr, nullptr, 0, s_out, (uint16_t *)n_out}, (hipStream_t)stream);
     return launch_ffn<kDeltaProj, true>(x, x_row_stride, rows_a, nullptr, proj_packed, norm_weight, eps, weights_packed, out,
                                         R, rows_a_stride, kFfnD, (hipStream_t)stream, s_out, (uint16_t *)n_out);
 }
@@ -622,6 +631,10 @@ extern "C" int bnb_ffn_fused_proj_fwd(const float *x, int64_t x_row_stride, cons
         (rows_b && (!aligned16(rows_b) || rows_b_stride % 8 != 0)))
         return BNB_ERR_MISALIGNED;
     hipStream_t s = (hipStream_t)stream;
+    if (R <= ffn_small_rows_limit())
+        return launch_ffn_small({x, x_row_stride, (const uint16_t *)rows_a, rows_a_stride, (const uint16_t *)rows_b, rows_b_stride,
+                                 (const uint16_t *)proj_packed, norm_weight, eps, (const uint16_t *)weights_packed, out, R,
+                                 nullptr, 0.0f, nullptr, nullptr, 0, nullptr, nullptr}, s);
     if (rows_b)
         return launch_ffn<kDeltaGate>(x, x_row_stride, rows_a, rows_b, proj_packed, norm_weight, eps, weights_packed,
                                       out, R, rows_a_stride, rows_b_stride, s);

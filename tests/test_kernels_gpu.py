@@ -1570,6 +1570,29 @@ def test_ffn_fused_with_the_next_sublayers_head_matches_oracle(R, N, gated):
     assert max_rel(head.float().cpu(), alone.float().cpu()) <= BF16_TOL
 
 
+@pytest.mark.parametrize("R", [1, 31, 32, 33, 8193, 16384, 16385])
+@pytest.mark.parametrize("gated", [False, True])
+def test_ffn_fused_at_the_edges_of_the_few_row_form(R, gated):
+    """Tiles of 32 rows and the row count at which the launch changes kernels.  The same call with its rows inside a larger
+    batch (beyond the limit) goes through the wide kernel: only the order of the float32 sums over hidden units differs, and
+    the head's bfloat16 rounding of rows that differ that little."""
+    x, _, nw, p = _ffn_case(R + 3, R)
+    g = torch.Generator().manual_seed(R)
+    D, N, pad = 128, 384, 16500
+    pk = ops.pack_ffn_weights(p["f.gate_proj.weight"].to(DEV), p["f.up_proj.weight"].to(DEV), p["f.down_proj.weight"].to(DEV))
+    wp = ops.pack_proj_weights((torch.randn(D, D, generator=g) / D ** 0.5).to(DEV))
+    head = (torch.ones(D, device=DEV), None, ops.pack_head_weights((torch.randn(N, D, generator=g) / D ** 0.5).to(DEV)), N)
+    rows = [torch.randn(R, D, generator=g).bfloat16().to(DEV) for _ in range(2 if gated else 1)]
+    big = [torch.cat([t, torch.zeros(pad, D, dtype=t.dtype, device=DEV)]) for t in (x.to(DEV), *rows)]
+    out, h = ops.ffn_fused(x.to(DEV), None, nw.to(DEV), pk, proj=(*rows, wp), next_head=head)
+    want, want_h = ops.ffn_fused(big[0], None, nw.to(DEV), pk, proj=(*big[1:], wp), next_head=head)
+    # 512 products added in another order: 512 * 2^-24 of the sum of their magnitudes at most, far less on average
+    assert max_rel(out.cpu(), want[:R].cpu()) <= 1e-5
+    assert max_rel(h.float().cpu(), want_h[:R].float().cpu()) <= 2 ** -7  # one bfloat16 step of the largest value
+    if R > 16384:
+        assert torch.equal(out, want[:R])
+
+
 def test_next_head_one_hot_weights_hit_the_documented_positions():
     D, N, R = 128, 384, 70
     x, _, nw, p = _ffn_case(11, R)

@@ -2494,6 +2494,9 @@ def pack_linear_weights(weight: torch.Tensor) -> torch.Tensor:
     return weight.detach().to(torch.bfloat16)[rows, cols].contiguous()
 
 
+_MASK_ROWS_MAX = 65536  # rows up to which the list kernel sums the counts before it itself (its cost grows with their square)
+
+
 class CompactRows:
     """The set entries of a (B, n) bool mask as a device-side list: ``index`` (capacity B*n,
     int32 flat positions b*n + j, ascending, the first ``offsets[B]`` valid) and ``offsets``
@@ -2524,16 +2527,24 @@ class CompactRows:
         self._host = None if total is None else (int(total), int(max_count))
         self._hinted = total is not None
         self.shared_kv = None  # set by the trunk: {id(layer): [K | V] rows of the listed entries}, one projection pass for all readers
-        counts = torch.empty(B, dtype=torch.int32, device=mask.device)
-        self.offsets = torch.zeros(B + 1, dtype=torch.int32, device=mask.device)
-        self.index = torch.empty(max(B * n, 1), dtype=torch.int32, device=mask.device)
         if B and n:
+            counts = torch.empty(B, dtype=torch.int32, device=mask.device)
+            self.offsets = torch.empty(B + 1, dtype=torch.int32, device=mask.device)
+            self.index = torch.empty(B * n, dtype=torch.int32, device=mask.device)
             lib = _native.load()
             with _on_device(mask.device):
-                _native.check(lib.bnb_mask_count(mask.data_ptr(), counts.data_ptr(), B, n, _stream()), "bnb_mask_count")
-                torch.cumsum(counts, dim=0, dtype=torch.int32, out=self.offsets[1:])
-                _native.check(lib.bnb_mask_fill(mask.data_ptr(), self.offsets.data_ptr(), self.index.data_ptr(), B, n,
-                                                _stream()), "bnb_mask_fill")
+                if B <= _MASK_ROWS_MAX:
+                    _native.check(lib.bnb_mask_rows(mask.data_ptr(), counts.data_ptr(), self.offsets.data_ptr(), self.index.data_ptr(),
+                                                    B, n, _stream()), "bnb_mask_rows")
+                else:
+                    _native.check(lib.bnb_mask_count(mask.data_ptr(), counts.data_ptr(), B, n, _stream()), "bnb_mask_count")
+                    self.offsets[:1].zero_()
+                    torch.cumsum(counts, dim=0, dtype=torch.int32, out=self.offsets[1:])
+                    _native.check(lib.bnb_mask_fill(mask.data_ptr(), self.offsets.data_ptr(), self.index.data_ptr(), B, n,
+                                                    _stream()), "bnb_mask_fill")
+        else:
+            self.offsets = torch.zeros(B + 1, dtype=torch.int32, device=mask.device)
+            self.index = torch.empty(1, dtype=torch.int32, device=mask.device)
 
         if self._hinted and os.environ.get("BNB_CHECK_HINTS") == "1":
             self.check_hints()

@@ -756,6 +756,10 @@ int bnb_linear_f32_fwd(const float *x, int64_t x_row_stride, const float *x2, in
 int bnb_mask_count(const uint8_t *mask, int32_t *counts, int B, int n, void *stream);
 int bnb_mask_fill(const uint8_t *mask, const int32_t *offsets, int32_t *index, int B, int n, void *stream);
 
+/* Both at once, the offsets formed on the way (two launches): counts (B) is scratch, offsets (B + 1) and index as above;
+ * B >= 1.  The offsets cost B^2 / 128 reads of counts, so beyond some 65536 rows a scan of the caller's is the better way. */
+int bnb_mask_rows(const uint8_t *mask, int32_t *counts, int32_t *offsets, int32_t *index, int B, int n, void *stream);
+
 /*
  * Residual add + RMSNorm + gated MLP + residual add in one matrix-core kernel (bf16 compute):
  *     s = x + delta;  n = rmsnorm(s) * norm_weight;  out = s + Wd (gelu(Wg n) * (Wu n))

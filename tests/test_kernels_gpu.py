@@ -1470,6 +1470,29 @@ def test_compact_rows_and_gathered_projection(B, n, p):
         assert max_rel(out[:total].float().cpu(), want) <= BF16_TOL
 
 
+@pytest.mark.parametrize("B,n", [(15, 4), (16, 7), (17, 256), (1000, 20), (5000, 257), (8192, 8), (8193, 8), (8256, 8), (65536, 3),
+                                 (65537, 3)])
+def test_compact_rows_across_the_list_kernels_groups(B, n):
+    """Groups of 16 and 64 rows, byte and dword rows, a mask that starts off a dword boundary, and the scan beyond 65536 rows."""
+    g = torch.Generator().manual_seed(B + n)
+    flat = torch.rand(B * n + 1, generator=g) < 0.3
+    mask = flat[1:].view(B, n)
+    rows = ops.CompactRows(flat.to(DEV)[1:].view(B, n))
+    offs = torch.cat([torch.zeros(1, dtype=torch.long), mask.sum(1).cumsum(0)])
+    assert torch.equal(rows.offsets.cpu().long(), offs)
+    assert torch.equal(rows.index[:int(offs[-1])].cpu().long(), mask.flatten().nonzero().flatten())
+
+
+@pytest.mark.parametrize("R,N", [(40, 384), (20000, 384), (24576, 512), (24577, 512), (33000, 640)])
+def test_norm_linear_feature_groups_give_the_same_bits(R, N):
+    """Few rows: the features are dealt to work-groups of their own; a row's result does not depend on it."""
+    g = torch.Generator().manual_seed(N)
+    x, nw = torch.randn(R, 128, generator=g).to(DEV), torch.ones(128, device=DEV)
+    pk = ops.pack_linear_weights((torch.randn(N, 128, generator=g) / 128 ** 0.5).to(DEV))
+    big = torch.cat([x, torch.zeros(110000, 128, device=DEV)])
+    assert torch.equal(ops.norm_linear(x, nw, pk), ops.norm_linear(big, nw, pk)[:R])
+
+
 @pytest.mark.parametrize("R", [1, 31, 129, 1000])
 @pytest.mark.parametrize("listed", [False, True])
 def test_norm_linear_over_bfloat16_rows_gives_the_bits_of_the_widened_rows(R, listed):

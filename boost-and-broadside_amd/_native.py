@@ -76,6 +76,7 @@ SIGNATURES = {
     "bnb_norm_linear_bf16_fwd": (_i, [_vp, _i64, _vp, _vp, _vp, _f, _vp, _vp, _vp, _i64, _i, _i, _vp]),
     "bnb_norm_linear_train_fwd": (_i, [_vp, _i64, _vp, _f, _vp, _vp, _vp, _i64, _i, _i, _vp]),
     "bnb_linear_f32_fwd": (_i, [_vp, _i64, _vp, _i64, _vp, _f, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _i, _i, _i, _vp]),
+    "bnb_linear_f32_split_fwd": (_i, [_vp, _i64, _vp, _i64, _vp, _f, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _i, _i, _i, _vp]),
     "bnb_mask_count": (_i, [_vp, _vp, _i, _i, _vp]),
     "bnb_mask_fill": (_i, [_vp, _vp, _vp, _i, _i, _vp]),
     "bnb_mask_rows": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp]),

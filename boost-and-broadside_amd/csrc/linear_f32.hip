@@ -21,6 +21,7 @@
 // steps are one 16-byte load of a 1 KB contiguous wave read, straight from L2, a few loads ahead.
 
 #include "common.h"
+#include "linear_split.h"
 
 namespace bnb {
 
@@ -202,12 +203,13 @@ static int launch_linear_f32(const float *x, int64_t x_stride, const float *x2, 
 
 }  // namespace bnb
 
-extern "C" int bnb_linear_f32_fwd(const float *x, int64_t x_row_stride, const float *x2, int64_t x2_row_stride,
-                                  const float *norm_weight, float eps, const float *weight_packed, const float *bias,
-                                  const float *resid, int64_t resid_row_stride, float *out, int64_t out_row_stride, int64_t R,
-                                  int K, int N, int gate, void *stream)
+namespace bnb {
+
+// 0 = nothing to do, 1 = go on, anything else an error
+static int linear_f32_checks(const float *x, int64_t x_row_stride, const float *x2, int64_t x2_row_stride, const float *norm_weight,
+                             const void *weight_packed, const float *bias, const float *resid, int64_t resid_row_stride,
+                             const float *out, int64_t out_row_stride, int64_t R, int K, int N, int gate)
 {
-    using namespace bnb;
     if (R < 0 || K < 1 || N < 1) return BNB_ERR_BAD_SHAPE;
     if (K % 128 != 0 || N % 32 != 0 || (gate && N % 64 != 0)) return BNB_ERR_UNSUPPORTED;
     if (norm_weight != nullptr && (K != 128 || x2 != nullptr)) return BNB_ERR_UNSUPPORTED;
@@ -220,6 +222,20 @@ extern "C" int bnb_linear_f32_fwd(const float *x, int64_t x_row_stride, const fl
     if (!aligned16(x) || !aligned16(weight_packed) || x_row_stride % 4 != 0 || (x2 && (!aligned16(x2) || x2_row_stride % 4 != 0)) ||
         (norm_weight && !aligned16(norm_weight)))
         return BNB_ERR_MISALIGNED;
+    return 1;
+}
+
+}  // namespace bnb
+
+extern "C" int bnb_linear_f32_fwd(const float *x, int64_t x_row_stride, const float *x2, int64_t x2_row_stride,
+                                  const float *norm_weight, float eps, const float *weight_packed, const float *bias,
+                                  const float *resid, int64_t resid_row_stride, float *out, int64_t out_row_stride, int64_t R,
+                                  int K, int N, int gate, void *stream)
+{
+    using namespace bnb;
+    const int rc = linear_f32_checks(x, x_row_stride, x2, x2_row_stride, norm_weight, weight_packed, bias, resid, resid_row_stride, out,
+                                     out_row_stride, R, K, N, gate);
+    if (rc != 1) return rc;
     hipStream_t s = (hipStream_t)stream;
     if (norm_weight != nullptr) {
         if (gate)
@@ -236,4 +252,17 @@ extern "C" int bnb_linear_f32_fwd(const float *x, int64_t x_row_stride, const fl
                                                      resid_row_stride, out, out_row_stride, R, K, N, s);
     return launch_linear_f32<false, false, false>(x, x_row_stride, nullptr, 0, nullptr, eps, weight_packed, bias, resid,
                                                   resid_row_stride, out, out_row_stride, R, K, N, s);
+}
+
+extern "C" int bnb_linear_f32_split_fwd(const float *x, int64_t x_row_stride, const float *x2, int64_t x2_row_stride,
+                                        const float *norm_weight, float eps, const void *weight_packed, const float *bias,
+                                        const float *resid, int64_t resid_row_stride, float *out, int64_t out_row_stride, int64_t R,
+                                        int K, int N, int gate, void *stream)
+{
+    using namespace bnb;
+    const int rc = linear_f32_checks(x, x_row_stride, x2, x2_row_stride, norm_weight, weight_packed, bias, resid, resid_row_stride, out,
+                                     out_row_stride, R, K, N, gate);
+    if (rc != 1) return rc;
+    return launch_linear_split({x, x_row_stride, x2, x2_row_stride, norm_weight, eps, (const uint16_t *)weight_packed, bias, resid,
+                                resid_row_stride, out, out_row_stride, R, K, N / 32}, gate != 0, (hipStream_t)stream);
 }

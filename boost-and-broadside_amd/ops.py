@@ -2397,10 +2397,10 @@ def ffn_fused(
 
 
 def pack_linear_f32(weight: torch.Tensor, up_weight: torch.Tensor | None = None) -> torch.Tensor:
-    """A float32 Linear weight (N, K), N % 32 == 0, K % 128 == 0, as the operand stream of ``linear_f32``:
-    ``[fb][s4][l][e] = W[32 fb + l%32][(l/32) K/2 + 4 s4 + e]`` (a lane's four next contraction steps are one
-    16-byte piece of a 1 KB contiguous wave read).  With ``up_weight`` (same shape) the two matrices are
-    interleaved in blocks of 32 rows, ``[gate block u, up block u]``, for the gated form."""
+    """A float32 Linear weight (N, K), N % 32 == 0, K % 128 == 0, as the operand stream of ``linear_f32``: three bf16
+    pieces whose sum is the weight, ``[fb][K/128][ks][piece][l][e] = piece of W[32 fb + l%32][128 t + 16 ks + 8 (e/4) +
+    4 (l/32) + e%4]`` (every matrix-core operand is one contiguous 1 KB run).  With ``up_weight`` (same shape) the two
+    matrices are interleaved in blocks of 32 rows, ``[gate block u, up block u]``, for the gated form."""
     w = weight.detach().float()
     N, K = w.shape
     if N % 32 or K % 128 or (up_weight is not None and up_weight.shape != weight.shape):
@@ -2409,12 +2409,12 @@ def pack_linear_f32(weight: torch.Tensor, up_weight: torch.Tensor | None = None)
         u = up_weight.detach().float()
         w = torch.stack([w.view(N // 32, 32, K), u.view(N // 32, 32, K)], dim=1).reshape(2 * N, K)
         N = 2 * N
-    dev = w.device
-    lane = torch.arange(64, device=dev)
-    rows = (32 * torch.arange(N // 32, device=dev)[:, None, None, None] + (lane % 32)[None, None, :, None]).expand(-1, K // 8, -1, 4)
-    cols = ((lane // 32)[None, None, :, None] * (K // 2) + 4 * torch.arange(K // 8, device=dev)[None, :, None, None]
-            + torch.arange(4, device=dev)[None, None, None, :]).expand(N // 32, -1, -1, -1)
-    return w[rows, cols].contiguous()
+    # [fb][m][t][ks][e / 4][half][e % 4] -> [fb][t][ks][half][m][e / 4][e % 4]
+    w = w.view(N // 32, 32, K // 128, 8, 2, 2, 4).permute(0, 2, 3, 5, 1, 4, 6).reshape(N // 32, K // 128, 8, 1, 64, 8)
+    h = w.bfloat16()
+    rest = (w - h).nan_to_num_(0.0, 0.0, 0.0)  # an infinite weight is its first piece
+    m = rest.bfloat16()
+    return torch.cat([h, m, (rest - m).bfloat16()], dim=3)
 
 
 def linear_f32_supported(x: torch.Tensor, n_features: int) -> bool:
@@ -2426,7 +2426,7 @@ def linear_f32_supported(x: torch.Tensor, n_features: int) -> bool:
 def linear_f32(x: torch.Tensor, weight_packed: torch.Tensor, *, bias: torch.Tensor | None = None,
                norm_weight: torch.Tensor | None = None, eps: float | None = None, gelu_times: torch.Tensor | None = None,
                gate: bool = False, resid: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
-    """A float32 Linear with its neighbours folded in, one kernel on the fp32 matrix cores.
+    """A float32 Linear with its neighbours folded in, one kernel on the matrix cores.
 
     ``out = A W^T + bias (+ resid)`` with ``A = x``, or ``rmsnorm(x) * norm_weight`` (K = 128), or
     ``gelu(x) * gelu_times``; with ``gate`` the packed weight holds gate and up projections
@@ -2434,10 +2434,12 @@ def linear_f32(x: torch.Tensor, weight_packed: torch.Tensor, *, bias: torch.Tens
     unit-stride channels and evenly spaced rows; ``resid`` / ``out`` (..., N_out) float32 contiguous."""
     K = x.shape[-1]
     _need_device(x, "x")
-    if x.dtype != torch.float32 or weight_packed.dtype != torch.float32:
-        raise TypeError("linear_f32 takes float32 rows and a float32 packed weight")
+    if x.dtype != torch.float32 or weight_packed.dtype not in (torch.float32, torch.bfloat16):
+        raise TypeError("linear_f32 takes float32 rows and a packed float32 weight")
+    # three bf16 pieces, or whole float32 values in the order of the fp32 matrix cores (see bnb_amd.h)
+    pieces = weight_packed.dtype == torch.bfloat16
     n_blocks = weight_packed.shape[0]
-    if weight_packed.dim() != 4 or weight_packed.shape[1:] != (K // 8, 64, 4) or not weight_packed.is_contiguous():
+    if weight_packed.shape != ((n_blocks, K // 128, 8, 3, 64, 8) if pieces else (n_blocks, K // 8, 64, 4)) or not weight_packed.is_contiguous():
         raise ValueError("weight_packed must come from pack_linear_f32 for this contraction width")
     N = 32 * n_blocks
     n_out = N // 2 if gate else N
@@ -2463,7 +2465,8 @@ def linear_f32(x: torch.Tensor, weight_packed: torch.Tensor, *, bias: torch.Tens
     if R == 0:
         return out
     with _on_device(x.device):
-        rc = _native.load().bnb_linear_f32_fwd(
+        lib = _native.load()
+        rc = (lib.bnb_linear_f32_split_fwd if pieces else lib.bnb_linear_f32_fwd)(
             x2.data_ptr(), x2.stride(0) if R > 1 else K, None if y2 is None else y2.data_ptr(),
             0 if y2 is None else (y2.stride(0) if R > 1 else K), None if norm_weight is None else norm_weight.detach().contiguous().data_ptr(),
             float(_F32_EPS if eps is None else eps), weight_packed.data_ptr(), None if bias is None else bias.detach().contiguous().data_ptr(),

@@ -747,6 +747,18 @@ int bnb_linear_f32_fwd(const float *x, int64_t x_row_stride, const float *x2, in
                        int K, int N, int gate, void *stream);
 
 /*
+ * The same, with W as three bf16 pieces and the products on the bf16 matrix cores (closer to float64 than the form
+ * above, and faster at every size): weight_packed is [fb][K/128][ks][piece][l][e], fb < N/32, ks < 8, piece < 3, l < 64,
+ * e < 8, the piece-th bf16 piece (h = bf16(w), m = bf16(w - h), l = bf16(w - h - m)) of
+ * W[32 fb + l%32][128 t + 16 ks + 8 (e/4) + 4 (l/32) + e%4] (with gate: blocks 2u, 2u+1 = rows 32u.. of gate_proj, of
+ * up_proj).  Arguments, requirements and error codes are otherwise those of bnb_linear_f32_fwd.
+ */
+int bnb_linear_f32_split_fwd(const float *x, int64_t x_row_stride, const float *x2, int64_t x2_row_stride,
+                             const float *norm_weight, float eps, const void *weight_packed, const float *bias,
+                             const float *resid, int64_t resid_row_stride, float *out, int64_t out_row_stride, int64_t R,
+                             int K, int N, int gate, void *stream);
+
+/*
  * Compact list of the set entries of a byte mask (B, n), e.g. the bullets in flight of
  * models/yemong/policy.py:222-228: bnb_mask_count writes the number of set bytes per row;
  * the caller turns the counts into exclusive offsets (B+1, last = total); bnb_mask_fill writes

@@ -2884,6 +2884,36 @@ def test_linear_f32_reads_column_blocks_in_place_and_writes_into_the_residual():
         ops.pack_linear_f32(torch.zeros(48, 128))
 
 
+@pytest.mark.parametrize("R,K,N,gate", [(1, 512, 96, False), (33, 1024, 128, False), (10241, 512, 96, False), (10300, 512, 128, False),
+                                        (40, 256, 64, False), (161, 256, 64, True), (127, 128, 32, False), (129, 128, 2048, False)])
+@pytest.mark.parametrize("form", ["plain", "times"])
+def test_linear_f32_forms_and_values_beyond_the_pieces_range(R, K, N, gate, form):
+    # every form of the launch (K split over waves, pairs and single blocks, gate), and rows whose values three bf16 pieces
+    # cannot carry: infinities and the top of the float32 range come out as float32 products give them
+    if gate and form == "times":
+        return
+    g = torch.Generator().manual_seed(R + K + N)
+    x, w, up = torch.randn(R, K, generator=g), torch.randn(N, K, generator=g) / K ** 0.5, torch.randn(N, K, generator=g) / K ** 0.5
+    packed = ops.pack_linear_f32(w.to(DEV), up.to(DEV) if gate else None)
+    times = torch.rand(R, K, generator=g) + 0.5 if form == "times" else None
+    kw = dict(gate=True) if gate else {}
+    if times is not None:
+        kw["gelu_times"] = times.to(DEV)
+    a = x.double() if times is None else _gelu64(x.double()) * times.double()
+    ref = _gelu64(a @ w.double().t()) * (a @ up.double().t()) if gate else a @ w.double().t()
+    got = ops.linear_f32(x.to(DEV), packed, **kw).cpu()
+    assert max_rel(got.double(), ref) <= F32_TOL
+    if not gate and times is None:
+        row = R // 2
+        wp = w.abs() + 0.25
+        packed = ops.pack_linear_f32(wp.to(DEV))
+        x[row, 3], x[row, K - 1] = 1.0, float("inf")
+        assert torch.isposinf(ops.linear_f32(x.to(DEV), packed).cpu()[row]).all()
+        x[row] = 0.0
+        x[row, K - 2] = -3.4e38
+        torch.testing.assert_close(ops.linear_f32(x.to(DEV), packed).cpu()[row], -3.4e38 * wp[:, K - 2], rtol=2e-7, atol=0.0)
+
+
 # ------------------------------------------------------------------ norm + projection of the update (forward kernel writes n)
 
 

@@ -253,3 +253,81 @@ extern "C" int bnb_gelu_mul_bwd(const void *a, int a_dtype, int64_t a_row_stride
     }
 #undef BNB_GMB
 }
+
+namespace bnb {
+
+// The bullets in flight as rows of their own, and back.  The update reads the listed 128-wide token rows in every
+// bullet-reading sublayer; gathered once (widened to float32) they are also where those sublayers' gradients meet, and one
+// pass then writes the gradient of ALL slots, zeros included.  Bound by memory: 32768 environments x 80 float32 slots, a
+// quarter live, 155 us in (0.7 GB) and 300 us out (1.7 GB).
+template <typename T>
+__global__ __launch_bounds__(256) void rows_gather_kernel(const T *__restrict__ src, const int32_t *__restrict__ index,
+                                                          const int32_t *__restrict__ total, float *__restrict__ out, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);  // a half-wave per row
+    if (i >= n) return;
+    const int col = (threadIdx.x & 31) * 4;
+    Row4 v = {{0.0f, 0.0f, 0.0f, 0.0f}};
+    if (i < *total) v = load4<true>(src + (int64_t)index[i] * 128 + col);
+    store4<false>(out + i * 128 + col, v);
+}
+
+// One work-group per row of the mask: the slots' positions in the list through LDS, then whole rows in order
+template <typename T>
+__global__ __launch_bounds__(256) void rows_scatter_kernel(const float *__restrict__ rows, const int32_t *__restrict__ index,
+                                                           const int32_t *__restrict__ offsets, T *__restrict__ out, int n, int64_t rows_held)
+{
+    extern __shared__ int32_t s_pos[];
+    const int64_t b = blockIdx.x;
+    for (int j = threadIdx.x; j < n; j += 256) s_pos[j] = -1;
+    __syncthreads();
+    const int first = offsets[b], end = offsets[b + 1];
+    for (int i = first + (int)threadIdx.x; i < end; i += 256)
+        if (i < rows_held) s_pos[(int)(index[i] - b * n)] = i;
+    __syncthreads();
+    const int col = (threadIdx.x & 31) * 4;
+    for (int j = threadIdx.x >> 5; j < n; j += 8) {
+        const int i = s_pos[j];
+        Row4 v = {{0.0f, 0.0f, 0.0f, 0.0f}};
+        if (i >= 0) v = load4<true>(rows + (int64_t)i * 128 + col);
+        store4<true>(out + (b * n + j) * 128 + col, v);
+    }
+}
+
+}  // namespace bnb
+
+extern "C" int bnb_rows_gather(const void *src, int src_dtype, const int32_t *index, const int32_t *total, float *out, int64_t n,
+                               int D, void *stream)
+{
+    using namespace bnb;
+    if (n < 0) return BNB_ERR_BAD_SHAPE;
+    if (D != 128 || (n + 7) / 8 > 0x7fffffffLL) return BNB_ERR_UNSUPPORTED;
+    if (src_dtype != BNB_F32 && src_dtype != BNB_BF16) return BNB_ERR_BAD_DTYPE;
+    if (n == 0) return 0;
+    if (!src || !index || !total || !out) return BNB_ERR_NULL_POINTER;
+    if (!aligned16(src) || !aligned16(out)) return BNB_ERR_MISALIGNED;
+    const dim3 grid((unsigned)((n + 7) / 8));
+    if (src_dtype == BNB_F32)
+        hipLaunchKernelGGL((rows_gather_kernel<float>), grid, dim3(256), 0, (hipStream_t)stream, (const float *)src, index, total, out, n);
+    else
+        hipLaunchKernelGGL((rows_gather_kernel<uint16_t>), grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t *)src, index, total, out, n);
+    return (int)hipGetLastError();
+}
+
+extern "C" int bnb_rows_scatter(const float *rows, int64_t rows_held, const int32_t *index, const int32_t *offsets, void *out,
+                                int out_dtype, int B, int n, int D, void *stream)
+{
+    using namespace bnb;
+    if (B < 0 || n < 0 || rows_held < 0) return BNB_ERR_BAD_SHAPE;
+    if (D != 128 || n > 8192) return BNB_ERR_UNSUPPORTED;
+    if (out_dtype != BNB_F32 && out_dtype != BNB_BF16) return BNB_ERR_BAD_DTYPE;
+    if (B == 0 || n == 0) return 0;
+    if ((!rows && rows_held) || !index || !offsets || !out) return BNB_ERR_NULL_POINTER;
+    if (!aligned16(rows) || !aligned16(out)) return BNB_ERR_MISALIGNED;
+    const size_t lds = (size_t)n * 4;
+    if (out_dtype == BNB_F32)
+        hipLaunchKernelGGL((rows_scatter_kernel<float>), dim3((unsigned)B), dim3(256), lds, (hipStream_t)stream, rows, index, offsets, (float *)out, n, rows_held);
+    else
+        hipLaunchKernelGGL((rows_scatter_kernel<uint16_t>), dim3((unsigned)B), dim3(256), lds, (hipStream_t)stream, rows, index, offsets, (uint16_t *)out, n, rows_held);
+    return (int)hipGetLastError();
+}

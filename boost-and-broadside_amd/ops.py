@@ -2529,6 +2529,7 @@ class CompactRows:
             raise ValueError("give both total and max_count, or neither")
         self._host = None if total is None else (int(total), int(max_count))
         self._hinted = total is not None
+        self.live_rows = None  # set by the trunk: the listed token rows, gathered once for all readers of an update
         self.shared_kv = None  # set by the trunk: {id(layer): [K | V] rows of the listed entries}, one projection pass for all readers
         if B and n:
             counts = torch.empty(B, dtype=torch.int32, device=mask.device)
@@ -2592,6 +2593,57 @@ class CompactRows:
     def max_count_host(self) -> int:
         """Largest number of entries in one row of the mask, as a Python int (same copy, cached)."""
         return self._host_counts()[1]
+
+
+class _RowsGather(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, rows):
+        D = x.shape[-1]
+        x2 = x.reshape(-1, D)
+        if not x2.is_contiguous() or x2.data_ptr() % 16:
+            x2 = x2.clone(memory_format=torch.contiguous_format)
+        n = rows.total_host()
+        out = torch.empty((n, D), dtype=torch.float32, device=x.device)
+        if n:
+            with _on_device(x.device):
+                rc = _native.load().bnb_rows_gather(x2.data_ptr(), _DTYPE_CODE[x.dtype], rows.index.data_ptr(),
+                                                    rows.offsets[-1:].data_ptr(), out.data_ptr(), n, D, _stream())
+            _native.check(rc, "bnb_rows_gather")
+        # the list's tensors are saved, not the list: what the caller hangs on it later stays out of the graph
+        ctx.save_for_backward(rows.index, rows.offsets)
+        ctx.mask_shape, ctx.x_shape, ctx.x_dtype = rows.shape, x.shape, x.dtype
+        return out
+
+    @staticmethod
+    @_outside_autocast
+    def backward(ctx, dout):
+        index, offsets = ctx.saved_tensors
+        B, n = ctx.mask_shape
+        D = ctx.x_shape[-1]
+        dout = dout.float().contiguous()
+        dx = torch.empty(ctx.x_shape, dtype=ctx.x_dtype, device=dout.device)
+        if dx.numel():
+            with _on_device(dout.device):
+                rc = _native.load().bnb_rows_scatter(dout.data_ptr(), dout.shape[0], index.data_ptr(), offsets.data_ptr(), dx.data_ptr(),
+                                                     _DTYPE_CODE[ctx.x_dtype], B, n, D, _stream())
+            _native.check(rc, "bnb_rows_scatter")
+        return dx, None
+
+
+def rows_gather_supported(x: torch.Tensor, rows: CompactRows) -> bool:
+    """Whether ``rows_gather`` covers this: float32 or bfloat16 (..., 128) tokens on the list's device, one row per mask
+    entry, at most 8192 entries per mask row."""
+    B, n = rows.shape
+    return (x.is_cuda and x.device == rows.index.device and x.dtype in _DTYPE_CODE and x.shape[-1] == FFN_WIDTH
+            and x.numel() == B * n * FFN_WIDTH and n <= 8192)
+
+
+def rows_gather(x: torch.Tensor, rows: CompactRows) -> torch.Tensor:
+    """The listed rows of x (..., 128), in list order, as float32 (total, 128).  Differentiable: the backward writes the
+    gradient of all of x, zeros for the rows not listed, in one pass (rounded once to x's dtype)."""
+    if not rows_gather_supported(x, rows):
+        raise RuntimeError("rows_gather covers float32 and bfloat16 (..., 128) tokens on the GPU, one row per mask entry")
+    return _RowsGather.apply(x, rows)
 
 
 def norm_linear(

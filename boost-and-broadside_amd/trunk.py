@@ -42,6 +42,7 @@ from __future__ import annotations
 
 import collections
 import contextlib
+import copy
 import warnings
 from dataclasses import dataclass
 
@@ -738,8 +739,14 @@ class TransformerBlock(_WeightCaches, nn.Module):
             total = rows.total_host()
             if total == 0:
                 return torch.zeros_like(qkv[..., :D])
-            live = bullets.reshape(B * NB, D).index_select(0, rows.index[:total].long())
-            kv_rows = _project(self.kv_bullet, _train_norm(self.norm_bullet, live)[1])
+            shared = rows.live_rows  # one gather for all readers (YemongTrunk.sequence), or this reader's own
+            live = shared.rows if shared is not None else bullets.reshape(B * NB, D).index_select(0, rows.index[:total].long())
+            if _norm_linear_train_ok(live, _projection_dtype(), self.norm_bullet, self.kv_bullet):
+                live, kv_rows, _ = _norm_linear_train(live, self.norm_bullet, self.kv_bullet)
+                if shared is not None and shared.chained:
+                    shared.rows = live  # the next reader's gradient reaches the rows inside this reader's norm backward
+            else:
+                kv_rows = _project(self.kv_bullet, _train_norm(self.norm_bullet, live)[1])
             if kv_rows.dtype == torch.bfloat16:
                 return ops.sdpa_cross_rows_train(qkv, kv_rows, rows, self.n_heads)
         kv = _project(self.kv_bullet, _train_norm(self.norm_bullet, bullets)[1])
@@ -1458,6 +1465,16 @@ def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
     return a0 < b1 and b0 < a1
 
 
+class _LiveRows:
+    """The gathered rows of the bullets in flight; ``chained``: each reader hands them on to the next (not across
+    recomputed blocks, whose readers all start from the gathered rows themselves)."""
+
+    __slots__ = ("rows", "chained")
+
+    def __init__(self, rows: torch.Tensor, chained: bool) -> None:
+        self.rows, self.chained = rows, chained
+
+
 class YemongTrunk(_WeightCaches, nn.Module):
     """The recurrent trunk: ``forward(tokens, alive_mask, recurrent_state) -> (hidden, new_state)``.
 
@@ -1508,6 +1525,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
         if (bullets is not None and isinstance(bullet_mask, torch.Tensor) and bullet_mask.is_cuda
                 and bullet_mask.dtype == torch.bool and bullet_mask.dim() == 2):
             bullet_mask = ops.CompactRows(bullet_mask)  # one list of the bullets in flight for every bullet-reading layer
+        bullet_mask = self._with_live_rows(bullets, bullet_mask, NM, chained=not grad_checkpoint)
         h_all = initial_hidden[:, :, :D]
         cb_all = initial_hidden[:, :, D:].reshape(n_layers, rows, CONV_KERNEL - 1, D)
         slot = 0
@@ -1523,6 +1541,23 @@ class YemongTrunk(_WeightCaches, nn.Module):
             else:
                 x = run(x)
         return x
+
+    def _with_live_rows(self, bullets, rows, num_tokens, *, chained):
+        """The list ``rows`` (a ``CompactRows``) with the listed bullets' rows gathered once for every reading sublayer
+        of an update under bfloat16 autocast, or ``rows`` itself where that does not apply.  The gradients of all readers
+        meet on the gathered rows, a fraction of the slots, instead of as full-size tensors.  The caller's own list
+        is left as it is."""
+        readers = [layer for block in self.yemong_layers for layer in block.spatial if layer.reads_bullets]
+        if not (
+            _TRAIN_KERNELS and torch.is_grad_enabled() and bullets is not None and isinstance(rows, ops.CompactRows) and readers
+            and _projection_dtype() == torch.bfloat16 and num_tokens <= 160 and rows.shape[1] <= 2048
+            and bullets.dim() == 3 and tuple(bullets.shape[:2]) == rows.shape and ops.rows_gather_supported(bullets, rows)
+            and all(l.head_dim == 32 and l.kv_bullet.bias is None for l in readers) and rows.total_host()
+        ):
+            return rows
+        own = copy.copy(rows)
+        own.live_rows = _LiveRows(ops.rows_gather(bullets, rows), chained)
+        return own
 
     def _bullet_kv_of_all_layers(self, bullets, rows):
         """``{id(layer): [K | V] rows}`` of every bullet-reading sublayer of the step from ONE pass over the bullets in

@@ -773,6 +773,16 @@ int bnb_mask_fill(const uint8_t *mask, const int32_t *offsets, int32_t *index, i
 int bnb_mask_rows(const uint8_t *mask, int32_t *counts, int32_t *offsets, int32_t *index, int B, int n, void *stream);
 
 /*
+ * The listed rows of a (B * n, 128) tensor (fp32 or bf16, src_dtype) as n_rows contiguous fp32 rows, out[i] = src[index[i]]
+ * (zeros from *total on), and the way back for a gradient: out (B * n, 128) in out_dtype gets row i of `rows` at
+ * index[i] and zeros everywhere else (entries from rows_held on are left out).  n <= 8192 slots per mask row for the latter.
+ */
+int bnb_rows_gather(const void *src, int src_dtype, const int32_t *index, const int32_t *total, float *out, int64_t n_rows,
+                    int D, void *stream);
+int bnb_rows_scatter(const float *rows, int64_t rows_held, const int32_t *index, const int32_t *offsets, void *out,
+                     int out_dtype, int B, int n, int D, void *stream);
+
+/*
  * Residual add + RMSNorm + gated MLP + residual add in one matrix-core kernel (bf16 compute):
  *     s = x + delta;  n = rmsnorm(s) * norm_weight;  out = s + Wd (gelu(Wg n) * (Wu n))
  * Replaces `x = x + <attention output>` and `x + self.ffn(self.norm2(x))` of

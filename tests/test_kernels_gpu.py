@@ -2884,6 +2884,26 @@ def test_linear_f32_reads_column_blocks_in_place_and_writes_into_the_residual():
         ops.pack_linear_f32(torch.zeros(48, 128))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,n,p", [(1, 1, 1.0), (5, 7, 0.3), (300, 80, 0.25), (3, 2048, 0.9), (9, 1520, 0.02)])
+def test_rows_gather_and_its_gradient_are_the_indexed_selection(dtype, B, n, p):
+    g = torch.Generator().manual_seed(B * n)
+    mask = torch.rand(B, n, generator=g) < p
+    mask[0, -1] = True
+    if B > 3:
+        mask[2] = False
+    rows = ops.CompactRows(mask.to(DEV))
+    # a view that starts in the middle of a 16-byte piece, as a slice of a larger buffer may
+    x = torch.randn(B * n * 128 + 2, generator=g).to(dtype).to(DEV)[2:].view(B, n, 128).requires_grad_()
+    got = ops.rows_gather(x, rows)
+    assert got.dtype == torch.float32 and torch.equal(got, x.detach()[mask.to(DEV)].float())
+    d = torch.randn(got.shape, generator=g).to(DEV)
+    got.backward(d)
+    want = torch.zeros(B, n, 128, device=DEV)
+    want[mask.to(DEV)] = d
+    assert x.grad.dtype == dtype and torch.equal(x.grad, want.to(dtype))
+
+
 @pytest.mark.parametrize("R,K,N,gate", [(1, 512, 96, False), (33, 1024, 128, False), (10241, 512, 96, False), (10300, 512, 128, False),
                                         (40, 256, 64, False), (161, 256, 64, True), (127, 128, 32, False), (129, 128, 2048, False)])
 @pytest.mark.parametrize("form", ["plain", "times"])

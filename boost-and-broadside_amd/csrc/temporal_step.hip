@@ -263,6 +263,169 @@ __global__ __launch_bounds__(kTsMaxWaves * kWave) __attribute__((amdgpu_waves_pe
     }
 }
 
+// Few rows: the kernel above spends its time on serial latencies (64 KB of weights into LDS, then per half of the channels a
+// chain of loads, products, exchange, recurrence), 13 us for anything that fits one round.  Here a work-group of four waves
+// owns 32 rows: every load of the step (rows, state, and the wave's sixteen 1 KB weight operands, L2 to registers) is
+// requested up front, a wave runs conv and recurrence for eight of the rows and the gate products of a quarter of the
+// features for all 32, and two barriers exchange v and the gates.  Rounding points and order of the arithmetic are those of
+// the kernel above (which products the compiler fuses may differ: the last bit of v).
+constexpr int kTsSmallGatePitch = 2 * kTsD + 8;
+// us, form above -> this one: 128 rows 11.6 -> 7.1, 4096 rows 14.0 -> 8.7, 8192 rows (one work-group per CU) 16.0 -> 11.2,
+// 16384 rows 20.4 -> 20.8, 32768 rows 29.8 -> 38.9.  Of the 128 rows' 7.1 us most is launch, one round trip to memory and the
+// way of 7 KB of code into the instruction cache: with sixteen log-sigmoids inlined per lane (22 KB) it was 10.8 us.
+constexpr int64_t kTsSmallRows = 8192;
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void temporal_step_small_kernel(
+    const uint16_t *__restrict__ b1, int64_t b1_group_stride, int64_t b1_row_stride, const float *conv_in,
+    int64_t conv_in_stride, float *conv_out, int64_t conv_out_stride, const float *h_in, int64_t h_in_stride,
+    float *h_out, int64_t h_out_stride, const float *__restrict__ conv_weight, const float *__restrict__ conv_bias,
+    const uint16_t *__restrict__ gate_weight_packed, const float *__restrict__ gate_bias,
+    const float *__restrict__ log_lambda, float c, uint16_t *__restrict__ y, int64_t y_group_stride,
+    int64_t y_row_stride, const uint8_t *__restrict__ reset, int rows_per_env, int64_t R)
+{
+    __shared__ __align__(16) uint16_t s_v[kTsRows * kTsPitch];
+    __shared__ __align__(16) uint16_t s_g[kTsRows * kTsSmallGatePitch];  // [row][half of the channels][gate][64]
+    __shared__ float s_l2sig[kTsD];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = lane >> 3, c4 = (lane & 7) * 4;  // row mapping, as above
+    const int m = lane & 31, half = lane >> 5;       // matrix-core mapping
+    auto ch = [&](int e) { return c4 + (e & 3) + 32 * (e >> 2); };
+    auto ld8 = [&](auto *half_base) -> Row8 {
+        const Row4 a = load4<false>(half_base + c4), b = load4<false>(half_base + c4 + 32);
+        return Row8{{a.v[0], a.v[1], a.v[2], a.v[3], b.v[0], b.v[1], b.v[2], b.v[3]}};
+    };
+    auto st8 = [&](auto *half_base, const Row8 &r) {
+        store4<false>(half_base + c4, Row4{{r.v[0], r.v[1], r.v[2], r.v[3]}});
+        store4<false>(half_base + c4 + 32, Row4{{r.v[4], r.v[5], r.v[6], r.v[7]}});
+    };
+
+    const float lam = log_lambda[threadIdx.x & (kTsD - 1)];
+    // ---- requests: this lane's row, then the weights of the wave's feature blocks (gate wave % 2 of half wave / 2) ----
+    const int64_t r = (int64_t)blockIdx.x * kTsRows + 8 * wave + sub;
+    const bool valid = r < R;
+    const int64_t row = valid ? r : R - 1;  // rows past the end repeat the last row and store nothing
+    const int64_t env = (int64_t)((uint32_t)row / (uint32_t)rows_per_env);
+    const int64_t in_env = row - env * rows_per_env;
+    Row8 cur[2], p0[2], p1[2], p2[2], hv[2];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+        const int d0 = 64 * hf;
+        cur[hf] = ld8(b1 + (b1_group_stride != 0 ? env * b1_group_stride + in_env * b1_row_stride : row * b1_row_stride) + d0);
+        const float *pin = conv_in + row * conv_in_stride + d0;
+        p0[hf] = ld8(pin);
+        p1[hf] = ld8(pin + kTsD);
+        p2[hf] = ld8(pin + 2 * kTsD);
+        hv[hf] = ld8(h_in + row * h_in_stride + d0);
+    }
+    // an absent input's load goes to some other readable byte: a branch around it would wait for it on the spot
+    const uint32_t flag = reset != nullptr ? 0xffu : 0u;
+    const uint32_t reset_byte = *(reset != nullptr ? reset + env : reinterpret_cast<const uint8_t *>(conv_weight));
+    const float *cbp = conv_bias != nullptr ? conv_bias : conv_weight;
+    f32x4 cw[2][8];
+    float cb[2][8], gb[2][16];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            cw[hf][e] = *reinterpret_cast<const f32x4 *>(conv_weight + (64 * hf + ch(e)) * 4);
+            cb[hf][e] = cbp[64 * hf + ch(e)];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int g = 0; g < 16; ++g) gb[j][g] = gate_bias[(wave & 1) * kTsD + 64 * (wave >> 1) + 32 * j + 16 * half + g];
+    }
+    u32x4 wreg[2][8];
+    {
+        const uint16_t *wp = gate_weight_packed + ((int64_t)(wave * 2) * 8 * 64 + lane) * 8;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (int ks = 0; ks < 8; ++ks) wreg[j][ks] = *reinterpret_cast<const u32x4 *>(wp + (j * 8 + ks) * 512);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // one channel per thread, while the rows are on their way: sixteen per lane would be a third of the kernel's code, and
+    // at these sizes its way into the instruction cache is part of the time
+    s_l2sig[threadIdx.x & (kTsD - 1)] = log2_sigmoid(lam);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- conv taps, buffer shift; bf16(v) into LDS ----
+    const bool zero = (reset_byte & flag) != 0;
+    float v[2][8];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+        const int d0 = 64 * hf;
+        if (zero) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) p0[hf].v[e] = p1[hf].v[e] = p2[hf].v[e] = hv[hf].v[e] = 0.0f;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const f32x4 w = cw[hf][e];
+            float acc = p0[hf].v[e] * w.x;
+            acc = fmaf(p1[hf].v[e], w.y, acc);
+            acc = fmaf(p2[hf].v[e], w.z, acc);
+            acc = fmaf(cur[hf].v[e], w.w, acc);
+            v[hf][e] = acc + (conv_bias != nullptr ? cb[hf][e] : 0.0f);
+        }
+        if (valid) {
+            float *pout = conv_out + row * conv_out_stride + d0;
+            st8(pout, p1[hf]);
+            st8(pout + kTsD, p2[hf]);
+            st8(pout + 2 * kTsD, cur[hf]);
+        }
+        uint16_t *tp = s_v + (8 * wave + sub) * kTsPitch + d0 + c4;
+        *reinterpret_cast<u32x2 *>(tp) = u32x2{pack_bf16x2(v[hf][0], v[hf][1]), pack_bf16x2(v[hf][2], v[hf][3])};
+        *reinterpret_cast<u32x2 *>(tp + 32) = u32x2{pack_bf16x2(v[hf][4], v[hf][5]), pack_bf16x2(v[hf][6], v[hf][7])};
+    }
+    __syncthreads();
+
+    // ---- the wave's gate products for all 32 rows ----
+    {
+        const int hf = wave >> 1, gate = wave & 1;
+        f32x16 acc[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (int g = 0; g < 16; ++g) acc[j][g] = round_to_bf16(gb[j][g]);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+            const bf16x8 vb = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(s_v + m * kTsPitch + 16 * ks + 8 * half));
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wreg[j][ks]), vb, acc[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            uint16_t *gp = s_g + m * kTsSmallGatePitch + 128 * hf + 64 * gate + 32 * j + 16 * half;
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+                *reinterpret_cast<u32x4 *>(gp + 8 * g) =
+                    u32x4{pack_bf16x2(acc[j][8 * g + 0], acc[j][8 * g + 1]), pack_bf16x2(acc[j][8 * g + 2], acc[j][8 * g + 3]),
+                          pack_bf16x2(acc[j][8 * g + 4], acc[j][8 * g + 5]), pack_bf16x2(acc[j][8 * g + 6], acc[j][8 * g + 7])};
+        }
+    }
+    __syncthreads();
+
+    // ---- recurrence on the row mapping ----
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+        const uint16_t *gp = s_g + (8 * wave + sub) * kTsSmallGatePitch + 128 * hf;
+        const Row8 ga = ld8(gp), gx = ld8(gp + 64);
+        Row8 out;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) out.v[e] = rglru_element<true, false>(v[hf][e], ga.v[e], gx.v[e], s_l2sig[64 * hf + ch(e)], c, hv[hf].v[e]);
+        if (valid) {
+            st8(h_out + row * h_out_stride + 64 * hf, out);
+            st8(y + (y_group_stride != 0 ? env * y_group_stride + in_env * y_row_stride : row * y_row_stride) + 64 * hf, out);
+        }
+    }
+}
+
 static int ts_cu_count()
 {
     // compute units of the current device, looked up once per device
@@ -307,6 +470,14 @@ extern "C" int bnb_temporal_step_fwd(const void *b1, int64_t b1_group_stride, in
         (b1_group_stride % 8) != 0 || (y_group_stride % 8) != 0 || (y_row_stride % 8) != 0 || (conv_in_row_stride % 4) != 0 ||
         (conv_out_row_stride % 4) != 0 || (h_in_row_stride % 4) != 0 || (h_out_row_stride % 4) != 0)
         return BNB_ERR_MISALIGNED;
+    if (R <= kTsSmallRows) {
+        hipLaunchKernelGGL(temporal_step_small_kernel, dim3((unsigned)((R + kTsRows - 1) / kTsRows)), dim3(256), 0, (hipStream_t)stream,
+                           (const uint16_t *)b1, b1_group_stride, b1_row_stride, conv_in, conv_in_row_stride, conv_out,
+                           conv_out_row_stride, h_in, h_in_row_stride, h_out, h_out_row_stride, conv_weight, conv_bias,
+                           (const uint16_t *)gate_weight_packed, gate_bias, log_lambda, c, (uint16_t *)y, y_group_stride,
+                           y_row_stride, reset, rows_per_env, R);
+        return (int)hipGetLastError();
+    }
     // One work-group per CU at most (LDS), 8 waves each, every wave at least 8 rows.
     const int cus = ts_cu_count();
     const int waves = kTsMaxWaves;

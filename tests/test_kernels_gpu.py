@@ -1351,6 +1351,25 @@ def test_temporal_step_matches_oracle_and_the_three_kernel_composition(R, with_r
     assert max_rel(h_c.cpu(), h_true) <= BF16_TOL
 
 
+@pytest.mark.parametrize("R", [1, 7, 33, 200, 8191, 8192])
+@pytest.mark.parametrize("with_reset,with_bias", [(False, True), (True, False)])
+def test_temporal_step_for_few_rows_agrees_with_the_large_form(R, with_reset, with_bias):
+    t = _temporal_inputs(3, 8200)
+    d = {k: v.to(DEV) for k, v in t.items()}
+    reset = (torch.rand(8200, generator=torch.Generator().manual_seed(R)) < 0.3).to(DEV) if with_reset else None
+    pk, gb, cb = ops.pack_gate_weights(d["wa"], d["wx"]), torch.cat([d["ba"], d["bx"]]), d["cb"] if with_bias else None
+    many = ops.temporal_step(d["b1"], d["buf"], d["h"], d["cw"], cb, pk, gb, d["lam"], 8.0, reset=reset)
+    few = ops.temporal_step(d["b1"][:R], d["buf"][:R], d["h"][:R], d["cw"], cb, pk, gb, d["lam"], 8.0,
+                            reset=None if reset is None else reset[:R])
+    (y, h, buf), (y_m, h_m, buf_m) = few, many
+    assert torch.equal(buf, buf_m[:R]) and torch.equal(y, h.to(torch.bfloat16))
+    # same rounding points; the conv's fused products may differ in the last fp32 bit, which now and then moves a
+    # pre-activation by one bf16 ulp (2^-8 of it, and the state moves by less than that)
+    assert max_rel(h, h_m[:R]) <= 8e-3
+    off = ((h - h_m[:R]).abs() > 1e-5 * h_m[:R].abs().clamp_min(1e-2)).float().mean().item()
+    assert off <= max(1e-3, 2 / h.numel()), off
+
+
 def test_temporal_step_every_gate_weight_reaches_its_channel():
     # one-hot gate weights: channel j of gate g sees exactly conv-output channel perm[j]; any
     # slip in the operand packing or in the channel order of the exchange shows as a mismatch

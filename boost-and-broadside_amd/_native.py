@@ -80,6 +80,7 @@ SIGNATURES = {
     "bnb_mask_count": (_i, [_vp, _vp, _i, _i, _vp]),
     "bnb_mask_fill": (_i, [_vp, _vp, _vp, _i, _i, _vp]),
     "bnb_mask_rows": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp]),
+    "bnb_stage_inputs": (_i, [_i, _vp, _vp, _vp, _vp, _vp]),
     "bnb_rows_gather": (_i, [_vp, _i, _vp, _vp, _vp, _i64, _i, _vp]),
     "bnb_rows_scatter": (_i, [_vp, _i64, _vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "bnb_ffn_fused_fwd": (_i, [_vp, _i64, _vp, _i, _vp, _f, _vp, _vp, _i64, _i, _i, _vp]),

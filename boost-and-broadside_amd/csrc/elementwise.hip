@@ -331,3 +331,67 @@ extern "C" int bnb_rows_scatter(const float *rows, int64_t rows_held, const int3
         hipLaunchKernelGGL((rows_scatter_kernel<uint16_t>), dim3((unsigned)B), dim3(256), lds, (hipStream_t)stream, rows, index, offsets, (uint16_t *)out, n, rows_held);
     return (int)hipGetLastError();
 }
+
+namespace bnb {
+
+// Up to kStageMax inputs of a captured step into its static buffers in one launch: plain copies, and bf16 -> fp32 for tokens
+// that the step carries in float32.  At the sizes a step is captured for, a copy's time is its launch.
+constexpr int kStageMax = 8;
+struct StageArgs {
+    const unsigned char *src[kStageMax];
+    unsigned char *dst[kStageMax];
+    int64_t pieces[kStageMax];   // 16-byte pieces of the source
+    int32_t tail[kStageMax];     // bytes behind them
+    int32_t first[kStageMax + 1];  // first work-group of each input
+    int32_t widen;               // bit i: input i is bf16, its destination fp32
+};
+
+__global__ __launch_bounds__(256) void stage_inputs_kernel(StageArgs a)
+{
+    int i = 0;
+#pragma unroll
+    for (int k = 1; k < kStageMax; ++k) i += (int)blockIdx.x >= a.first[k] ? 1 : 0;
+    const int64_t step = (int64_t)(a.first[i + 1] - a.first[i]) * 256;
+    const int64_t t0 = ((int64_t)blockIdx.x - a.first[i]) * 256 + threadIdx.x;
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(a.src[i]);
+    if (a.widen >> i & 1) {
+        float *dst = reinterpret_cast<float *>(a.dst[i]);
+        for (int64_t t = t0; t < a.pieces[i]; t += step) store8(dst + 8 * t, load8(reinterpret_cast<const uint16_t *>(src + t)));
+        if (t0 * 2 < a.tail[i])
+            dst[8 * a.pieces[i] + t0] = bf16_bits_to_f32(reinterpret_cast<const uint16_t *>(src + a.pieces[i])[t0]);
+    } else {
+        u32x4 *dst = reinterpret_cast<u32x4 *>(a.dst[i]);
+        for (int64_t t = t0; t < a.pieces[i]; t += step) dst[t] = src[t];
+        if (t0 < a.tail[i]) a.dst[i][16 * a.pieces[i] + t0] = a.src[i][16 * a.pieces[i] + t0];
+    }
+}
+
+}  // namespace bnb
+
+extern "C" int bnb_stage_inputs(int count, const void *const *src, void *const *dst, const int64_t *src_bytes, const int32_t *widen,
+                                void *stream)
+{
+    using namespace bnb;
+    if (count < 0 || count > kStageMax) return BNB_ERR_BAD_SHAPE;
+    if (count > 0 && (!src || !dst || !src_bytes || !widen)) return BNB_ERR_NULL_POINTER;
+    StageArgs a = {};
+    int32_t groups = 0;
+    int n = 0;
+    for (int i = 0; i < count; ++i) {
+        if (src_bytes[i] < 0 || (widen[i] && src_bytes[i] % 2)) return BNB_ERR_BAD_SHAPE;
+        if (src_bytes[i] == 0) continue;
+        if (!src[i] || !dst[i]) return BNB_ERR_NULL_POINTER;
+        if (!aligned16(src[i]) || !aligned16(dst[i])) return BNB_ERR_MISALIGNED;
+        a.src[n] = (const unsigned char *)src[i], a.dst[n] = (unsigned char *)dst[i];
+        a.pieces[n] = src_bytes[i] / 16, a.tail[n] = (int32_t)(src_bytes[i] % 16);
+        a.widen |= widen[i] ? 1 << n : 0;
+        a.first[n] = groups;
+        const int64_t want = (a.pieces[n] + 255) / 256;
+        groups += (int32_t)(want < 1 ? 1 : want > 2048 ? 2048 : want);
+        ++n;
+    }
+    if (n == 0) return 0;
+    for (int i = n; i <= kStageMax; ++i) a.first[i] = i == n ? groups : 0x7fffffff;
+    hipLaunchKernelGGL(stage_inputs_kernel, dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream, a);
+    return (int)hipGetLastError();
+}

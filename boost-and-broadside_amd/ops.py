@@ -14,6 +14,7 @@ from __future__ import annotations
 import os
 
 import functools
+import ctypes
 import math
 
 import torch
@@ -2593,6 +2594,34 @@ class CompactRows:
     def max_count_host(self) -> int:
         """Largest number of entries in one row of the mask, as a Python int (same copy, cached)."""
         return self._host_counts()[1]
+
+
+_STAGE_MAX = 8
+
+
+def stage_inputs(pairs) -> None:
+    """``dst.copy_(src)`` for every ``(dst, src)`` pair, in one launch for the pairs that are plain copies on one device
+    (same shape, both contiguous and 16-byte aligned, same dtype or bfloat16 into float32); ``copy_`` does the others."""
+    plain = []
+    for dst, src in pairs:
+        if (dst.is_cuda and src.device == dst.device and src.shape == dst.shape and src.is_contiguous() and dst.is_contiguous()
+                and not src.is_conj() and not src.is_neg() and (src.dtype == dst.dtype or (src.dtype == torch.bfloat16 and dst.dtype == torch.float32))
+                and src.data_ptr() % 16 == 0 and dst.data_ptr() % 16 == 0 and len(plain) < _STAGE_MAX
+                and (not plain or plain[0][0].device == dst.device)):
+            plain.append((dst, src))
+        else:
+            dst.copy_(src)
+    if not plain:
+        return
+    n = len(plain)
+    srcs, dsts = (ctypes.c_void_p * n)(), (ctypes.c_void_p * n)()
+    sizes, widen = (ctypes.c_int64 * n)(), (ctypes.c_int32 * n)()
+    for i, (dst, src) in enumerate(plain):
+        srcs[i], dsts[i], sizes[i], widen[i] = src.data_ptr(), dst.data_ptr(), src.numel() * src.element_size(), src.dtype != dst.dtype
+    with _on_device(plain[0][0].device):
+        rc = _native.load().bnb_stage_inputs(n, ctypes.addressof(srcs), ctypes.addressof(dsts), ctypes.addressof(sizes),
+                                             ctypes.addressof(widen), _stream())
+    _native.check(rc, "bnb_stage_inputs")
 
 
 class _RowsGather(torch.autograd.Function):

@@ -773,6 +773,13 @@ int bnb_mask_fill(const uint8_t *mask, const int32_t *offsets, int32_t *index, i
 int bnb_mask_rows(const uint8_t *mask, int32_t *counts, int32_t *offsets, int32_t *index, int B, int n, void *stream);
 
 /*
+ * Up to 8 contiguous inputs into contiguous buffers in one launch: src_bytes[i] bytes each as they are, or with widen[i]
+ * bf16 elements into fp32 ones.  All addresses 16-byte aligned; the arrays are host memory and read before the call returns.
+ */
+int bnb_stage_inputs(int count, const void *const *src, void *const *dst, const int64_t *src_bytes, const int32_t *widen,
+                     void *stream);
+
+/*
  * The listed rows of a (B * n, 128) tensor (fp32 or bf16, src_dtype) as n_rows contiguous fp32 rows, out[i] = src[index[i]]
  * (zeros from *total on), and the way back for a gradient: out (B * n, 128) in out_dtype gets row i of `rows` at
  * index[i] and zeros everywhere else (entries from rows_held on are left out).  n <= 8192 slots per mask row for the latter.

@@ -2903,6 +2903,22 @@ def test_linear_f32_reads_column_blocks_in_place_and_writes_into_the_residual():
         ops.pack_linear_f32(torch.zeros(48, 128))
 
 
+def test_stage_inputs_is_copy_for_every_pair():
+    # whole and ragged lengths, widening, empty inputs, and the pairs that one launch cannot take (strided, other dtype,
+    # misaligned, broadcast, from the host): every destination ends up as copy_ leaves it
+    g = torch.Generator().manual_seed(2)
+    def r(*shape, dtype=torch.float32):
+        return torch.randn(*shape, generator=g).to(dtype).to(DEV)
+    srcs = [r(700, 128, dtype=torch.bfloat16), r(5, 3), (r(16, 12) > 0), (r(7) > 0), r(0, 4), r(3, 7, dtype=torch.bfloat16), r(64, 6).t(),
+            r(9, dtype=torch.float64), r(33)[1:], r(1, 8), r(4).cpu(), r(5), r(600000)]
+    dsts = [torch.full(s.shape if s.shape != (1, 8) else (5, 8), 7, device=DEV,
+                       dtype=torch.bool if s.dtype == torch.bool else torch.float32) for s in srcs]
+    want = [d.clone().copy_(s) for d, s in zip(dsts, srcs)]
+    ops.stage_inputs(list(zip(dsts, srcs)))
+    for d, w in zip(dsts, want):
+        assert torch.equal(d, w)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,n,p", [(1, 1, 1.0), (5, 7, 0.3), (300, 80, 0.25), (3, 2048, 0.9), (9, 1520, 0.02)])
 def test_rows_gather_and_its_gradient_are_the_indexed_selection(dtype, B, n, p):

@@ -1525,7 +1525,8 @@ class YemongTrunk(_WeightCaches, nn.Module):
         if (bullets is not None and isinstance(bullet_mask, torch.Tensor) and bullet_mask.is_cuda
                 and bullet_mask.dtype == torch.bool and bullet_mask.dim() == 2):
             bullet_mask = ops.CompactRows(bullet_mask)  # one list of the bullets in flight for every bullet-reading layer
-        bullet_mask = self._with_live_rows(bullets, bullet_mask, NM, chained=not grad_checkpoint)
+        given_rows = bullet_mask
+        bullet_mask = self._with_live_rows(bullets, given_rows, NM, chained=not grad_checkpoint)
         h_all = initial_hidden[:, :, :D]
         cb_all = initial_hidden[:, :, D:].reshape(n_layers, rows, CONV_KERNEL - 1, D)
         slot = 0
@@ -1540,6 +1541,8 @@ class YemongTrunk(_WeightCaches, nn.Module):
                 x = torch.utils.checkpoint.checkpoint(run, x, use_reentrant=False)
             else:
                 x = run(x)
+        if bullet_mask is not given_rows and not grad_checkpoint:
+            bullet_mask.live_rows = None  # the readers' nodes keep the list: it must not keep the gathered rows alive past the backward
         return x
 
     def _with_live_rows(self, bullets, rows, num_tokens, *, chained):

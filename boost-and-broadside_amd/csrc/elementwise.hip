@@ -259,7 +259,7 @@ namespace bnb {
 // The bullets in flight as rows of their own, and back.  The update reads the listed 128-wide token rows in every
 // bullet-reading sublayer; gathered once (widened to float32) they are also where those sublayers' gradients meet, and one
 // pass then writes the gradient of ALL slots, zeros included.  Bound by memory: 32768 environments x 80 float32 slots, a
-// quarter live, 96 us in (0.7 GB; index_select 155 us) and 300 us out (1.7 GB; fill, index_add and the sum of two readers 920 us).
+// quarter live, 96 us in (0.7 GB; index_select 155 us) and 300 us out (1.7 GB; two readers with fill, index_add and the sum of both 1.8 ms).
 template <typename T>
 __global__ __launch_bounds__(256) void rows_gather_kernel(const T *__restrict__ src, const int32_t *__restrict__ index,
                                                           const int32_t *__restrict__ total, float *__restrict__ out, int64_t n)

@@ -2702,9 +2702,12 @@ def norm_linear(
     if norm_weight.shape != (D,) or norm_weight.dtype != torch.float32:
         raise ValueError(f"norm_weight must be a float32 {(D,)} tensor")
     x2 = x.reshape(-1, D)
+    R = x2.shape[0]
     if x2.stride(-1) != 1:
         x2 = x2.contiguous()
-    R = x2.shape[0]
+    # bfloat16 rows reach the kernel as whole 16-byte pieces: a view that starts or steps off them is copied
+    if x.dtype == torch.bfloat16 and (x2.data_ptr() % 16 or x2.stride(0) % 8 or x2.stride(0) < D):
+        x2 = x2.clone(memory_format=torch.contiguous_format)
     if rows is not None and rows.shape[0] * rows.shape[1] != R:
         raise ValueError("rows was built for a mask of a different size")
     bias_ptr = None

@@ -1285,6 +1285,30 @@ def test_bfloat16_bullets_are_read_on_the_kernels_and_give_the_widened_bullets_r
     assert torch.equal(out, want) and torch.equal(state, want_state)
 
 
+@pytest.mark.parametrize("readers", [1, 2])
+@pytest.mark.parametrize("view", ["offset", "wide", "repeated"])
+def test_bfloat16_bullets_in_views_the_kernel_cannot_address_give_the_copy_s_result(readers, view):
+    """Rows that start off a 16-byte piece, rows a distance apart that is no multiple of it, one row for every slot."""
+    D, H, B, N, M = 128, 4, 3, 5, 3
+    torch.manual_seed(53)
+    trunk = bnb.YemongTrunk(_cfg(D, H, readers, 2, 1, bullets=1)).eval().to(DEV)
+    g = torch.Generator().manual_seed(54)
+    x = torch.randn(B, N + M, D, generator=g).bfloat16().to(DEV)
+    if view == "offset":
+        bul = torch.randn(B * 10 * N * D + 2, generator=g).bfloat16().to(DEV)[2:].view(B, 10 * N, D)
+    elif view == "wide":
+        bul = torch.randn(B, 10 * N, D + 2, generator=g).bfloat16().to(DEV)[..., :D]
+    else:
+        bul = torch.randn(1, 1, D, generator=g).bfloat16().to(DEV).expand(B, 10 * N, D)
+    bm = (torch.rand(B, 10 * N, generator=g) < 0.3).to(DEV)
+    alive = torch.ones(B, N + M, dtype=torch.bool, device=DEV)
+    hidden = trunk.initial_hidden(B, N, DEV)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        got, _ = trunk(x, alive, hidden, bul, bm)
+        want, _ = trunk(x, alive, hidden, torch.empty(bul.shape, dtype=bul.dtype, device=DEV).copy_(bul), bm)
+    assert torch.equal(got, want)
+
+
 def test_team_pooling_takes_a_bfloat16_stream_under_autocast_on_the_kernels():
     from boost_and_broadside_amd import trunk as trunk_module
 

@@ -679,9 +679,9 @@ class TransformerBlock(_WeightCaches, nn.Module):
             merged = self._self_attention_autograd(qkv, alive_mask)
         if self.reads_bullets and bullets is not None:
             rows = bullet_mask if isinstance(bullet_mask, ops.CompactRows) else None
-            if rows is None and bullet_mask is not None and self._compact_read_ok(qkv, bullets):
+            if rows is None and bullet_mask is not None and self._compact_read_ok(qkv, bullets, bullet_mask):
                 rows = ops.CompactRows(bullet_mask)
-            if rows is not None and self._compact_read_ok(qkv, bullets):
+            if rows is not None and self._compact_read_ok(qkv, bullets, bullet_mask):
                 # only the bullets in flight are normalised and projected (one kernel over a
                 # device-side list of them), and the read walks each environment's run of rows
                 kv_rows = rows.shared_kv.get(id(self)) if rows.shared_kv is not None else None
@@ -706,12 +706,23 @@ class TransformerBlock(_WeightCaches, nn.Module):
                 merged = merged + self._bullet_read(qkv, kv, bullet_mask)
         return _project(self.out_proj, merged) if project else merged
 
-    def _compact_read_ok(self, qkv, bullets) -> bool:
+    def _bullet_rows_ok(self, bullets, bullet_mask) -> bool:
+        """Whether the norm + projection kernel reads these bullet tokens: float32, or bfloat16 under a float32 norm weight
+        (a module cast to bfloat16 as a whole has its norm in bfloat16, which the kernel does not take) and a mask that a
+        list can be built from (the library's read takes any dtype)."""
+        if not bullets.is_cuda:
+            return False
+        if bullets.dtype == torch.bfloat16:
+            listed = isinstance(bullet_mask, ops.CompactRows) or bullet_mask.dtype in (torch.bool, torch.uint8)
+            return listed and self.norm_bullet.weight is not None and self.norm_bullet.weight.dtype == torch.float32
+        return bullets.dtype == torch.float32
+
+    def _compact_read_ok(self, qkv, bullets, bullet_mask) -> bool:
         """Whether the bullet read can run on the compacted list (bf16 projections, width 128,
-        heads of 32, at most 160 entity tokens, float32 or bfloat16 bullet tokens on the GPU)."""
+        heads of 32, at most 160 entity tokens, bullet tokens that the projection kernel reads)."""
         return (
             qkv.dtype == torch.bfloat16 and self.d_model == ops.FFN_WIDTH and self.head_dim == 32 and qkv.shape[1] <= 160
-            and bullets.is_cuda and bullets.dtype in (torch.float32, torch.bfloat16) and self.kv_bullet.bias is None
+            and self._bullet_rows_ok(bullets, bullet_mask) and self.kv_bullet.bias is None
             # the compacted [K | V] rows are addressed with 32-bit element offsets over the full slot capacity
             and bullets.shape[0] * bullets.shape[1] * 2 * self.d_model < 2 ** 32
         )
@@ -1624,9 +1635,10 @@ class YemongTrunk(_WeightCaches, nn.Module):
         # the list of bullets in flight is built once and shared by every layer that reads them
         bullet_rows = bullet_mask
         if (
-            bullets is not None and bullet_mask is not None and self.config.reads_bullets and bullets.is_cuda
-            and bullets.dtype in (torch.float32, torch.bfloat16) and _projection_dtype() == torch.bfloat16 and D == ops.FFN_WIDTH
+            bullets is not None and bullet_mask is not None and self.config.reads_bullets
+            and _projection_dtype() == torch.bfloat16 and D == ops.FFN_WIDTH
             and D // self.config.n_heads == 32 and NM <= 160
+            and all(l._bullet_rows_ok(bullets, bullet_mask) for block in self.yemong_layers for l in block.spatial if l.reads_bullets)
         ):
             bullet_rows = ops.CompactRows(bullet_mask)
             bullet_rows.shared_kv = self._bullet_kv_of_all_layers(bullets, bullet_rows)

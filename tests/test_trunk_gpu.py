@@ -1309,6 +1309,41 @@ def test_bfloat16_bullets_in_views_the_kernel_cannot_address_give_the_copy_s_res
     assert torch.equal(got, want)
 
 
+def test_block_cast_to_bfloat16_reads_bullets_under_a_mask():
+    """All weights in bfloat16 and no autocast: the norm's weight is not what the compact kernels take."""
+    D, H, B, N = 128, 4, 5, 12
+    gen = torch.Generator().manual_seed(55)
+    p = block_params(gen, "b.", D, 1, 0)
+    p["b.spatial.0.norm_bullet.weight"] = 1.0 + 0.1 * torch.randn(D, generator=gen)
+    p["b.spatial.0.kv_bullet.weight"] = 0.15 * torch.randn(2 * D, D, generator=gen)
+    p = {k: v.bfloat16().float() for k, v in p.items()}
+    layer = bnb.TransformerBlock(_cfg(D, H), reads_bullets=True).eval()
+    layer.load_state_dict(_strip(p, "b.spatial.0."))
+    layer.to(DEV).bfloat16()
+    x, bul = (torch.randn(B, n, D, generator=gen).bfloat16() for n in (N, 10 * N))
+    alive = torch.rand(B, N, generator=gen) < 0.7
+    alive[:, 0] = True
+    bm = torch.rand(B, 10 * N, generator=gen) < 0.3
+    bm[1] = False
+    with torch.no_grad():
+        got = layer(x.to(DEV), alive.to(DEV), bul.to(DEV), bm.to(DEV))
+    want = torch_ref.spatial_sublayer(p, "b.spatial.0.", x.float(), alive, H, bullets=bul.float(), bullet_mask=bm)
+    assert got.dtype == torch.bfloat16 and max_rel(got.float().cpu(), want) <= BF16_TOL
+
+
+def test_bfloat16_bullets_on_a_long_slot_axis_take_a_float_mask_as_the_library_does():
+    """Beyond 2048 slots the read used to be the library's, which reads a mask of any dtype as 0 and 1."""
+    D, H, B, N, NB = 128, 4, 2, 6, 2100
+    torch.manual_seed(57)
+    layer = bnb.TransformerBlock(_cfg(D, H), reads_bullets=True).eval().to(DEV)
+    g = torch.Generator().manual_seed(58)
+    x, bul = torch.randn(B, N, D, generator=g).to(DEV), torch.randn(B, NB, D, generator=g).bfloat16().to(DEV)
+    bm = (torch.rand(B, NB, generator=g) < 0.3).to(DEV)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        got, want = layer(x, None, bul, bm.float()), layer(x, None, bul, bm)
+    assert max_rel(got.float().cpu(), want.float().cpu()) <= BF16_TOL
+
+
 def test_team_pooling_takes_a_bfloat16_stream_under_autocast_on_the_kernels():
     from boost_and_broadside_amd import trunk as trunk_module
 

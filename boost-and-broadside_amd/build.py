@@ -15,7 +15,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_DIR = os.path.join(PKG_DIR, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libbnb_amd.so")
-SOURCES = ("abi.hip", "conv_step.hip", "elementwise.hip", "ffn_bwd.hip", "ffn_fused.hip", "ffn_small.hip", "linear_f32.hip", "linear_split.hip", "linear_wgrad.hip",
+SOURCES = ("abi.hip", "conv_step.hip", "elementwise.hip", "ffn_bwd.hip", "ffn_fused.hip", "ffn_small.hip", "linear_split.hip", "linear_wgrad.hip",
     "norm_train.hip", "norm_linear.hip", "probe.hip", "rglru_step.hip", "sdpa_bwd.hip", "sdpa_cross_bwd.hip", "sdpa_cross_f32.hip", "sdpa_env.hip", "sdpa_masked.hip", "team_pool.hip", "temporal_seq.hip", "temporal_step.hip")
 
 HIPCC_FLAGS = [

@@ -1,6 +1,4 @@
-// Float32 Linear layers of the trunk with their neighbours folded in, on the bf16 matrix cores (gfx950).
-//
-// The same function as linear_f32.hip,
+// Float32 Linear layers of the trunk with their neighbours folded in, on the bf16 matrix cores (gfx950):
 //
 //     out[r, :] = ( A[r, :] W^T + bias ) (+ resid[r, :])        A = x                     plain
 //                                                                  | rmsnorm(x) * norm_w     NORM
@@ -26,7 +24,6 @@
 // product as everywhere: k-slot e of step ks in a lane of half h is channel 16 ks + 8 (e/4) + 4 h + e%4.
 
 #include "common.h"
-#include "linear_split.h"
 
 namespace bnb {
 
@@ -34,9 +31,24 @@ constexpr int kLsChunkHalfs = 8 * 3 * 512;  // 32 features x 128 channels x 3 pi
 constexpr int kLsWaves = 4;
 constexpr int kLsFewRows = 10240;  // K = 512, N = 128, us of this form and of the other: 2000 rows 9 / 21, 8192 17 / 23, 12288 26 / 24, 27680 50 / 35
 
+struct LinearSplitArgs {
+    const float *x;
+    int64_t x_stride;
+    const float *x2;  // gelu(x) * x2 when given
+    int64_t x2_stride;
+    const float *norm_w;  // rmsnorm(x) * norm_w when given (K == 128)
+    float eps;
+    const uint16_t *w;  // [fb][K/128][ks][piece][lane][8], fb < n_blocks
+    const float *bias, *resid;
+    int64_t resid_stride;
+    float *out;
+    int64_t out_stride, R;
+    int K, n_blocks;
+};
+
 enum { kLsPlain = 0, kLsNorm = 1, kLsMulGelu = 2 };
 
-// erf-GELU as in linear_f32.hip (Abramowitz-Stegun 7.1.26, |error of gelu| <= 5e-7)
+// erf-GELU, Abramowitz-Stegun 7.1.26 (|error of gelu| <= 5e-7)
 __device__ __forceinline__ float gelu_erf_ls(float v)
 {
     const float x = fabsf(v) * 0.70710678118654752f;
@@ -447,11 +459,44 @@ static int launch_pro(const LinearSplitArgs &p, hipStream_t stream)
     return launch_nb<PRO, GATE, NB, false>(p, stream);
 }
 
-int launch_linear_split(const LinearSplitArgs &p, bool gate, hipStream_t stream)
+static int launch_linear_split(const LinearSplitArgs &p, bool gate, hipStream_t stream)
 {
     if (p.norm_w != nullptr) return gate ? launch_pro<kLsNorm, true>(p, stream) : launch_pro<kLsNorm, false>(p, stream);
     if (p.x2 != nullptr) return launch_pro<kLsMulGelu, false>(p, stream);
     return gate ? launch_pro<kLsPlain, true>(p, stream) : launch_pro<kLsPlain, false>(p, stream);
 }
 
+// 0 = nothing to do, 1 = go on, anything else an error
+static int linear_split_checks(const float *x, int64_t x_row_stride, const float *x2, int64_t x2_row_stride, const float *norm_weight,
+                             const void *weight_packed, const float *bias, const float *resid, int64_t resid_row_stride,
+                             const float *out, int64_t out_row_stride, int64_t R, int K, int N, int gate)
+{
+    if (R < 0 || K < 1 || N < 1) return BNB_ERR_BAD_SHAPE;
+    if (K % 128 != 0 || N % 32 != 0 || (gate && N % 64 != 0)) return BNB_ERR_UNSUPPORTED;
+    if (norm_weight != nullptr && (K != 128 || x2 != nullptr)) return BNB_ERR_UNSUPPORTED;
+    if (gate && (bias != nullptr || x2 != nullptr)) return BNB_ERR_UNSUPPORTED;
+    if (R == 0) return 0;
+    if (!x || !weight_packed || !out) return BNB_ERR_NULL_POINTER;
+    const int n_out = gate ? N / 2 : N;
+    if (x_row_stride < K || out_row_stride < n_out || (x2 && x2_row_stride < K) || (resid && resid_row_stride < n_out))
+        return BNB_ERR_BAD_SHAPE;
+    if (!aligned16(x) || !aligned16(weight_packed) || x_row_stride % 4 != 0 || (x2 && (!aligned16(x2) || x2_row_stride % 4 != 0)) ||
+        (norm_weight && !aligned16(norm_weight)))
+        return BNB_ERR_MISALIGNED;
+    return 1;
+}
+
 }  // namespace bnb
+
+extern "C" int bnb_linear_f32_fwd(const float *x, int64_t x_row_stride, const float *x2, int64_t x2_row_stride,
+                                  const float *norm_weight, float eps, const void *weight_packed, const float *bias,
+                                  const float *resid, int64_t resid_row_stride, float *out, int64_t out_row_stride, int64_t R,
+                                  int K, int N, int gate, void *stream)
+{
+    using namespace bnb;
+    const int rc = linear_split_checks(x, x_row_stride, x2, x2_row_stride, norm_weight, weight_packed, bias, resid, resid_row_stride, out,
+                                       out_row_stride, R, K, N, gate);
+    if (rc != 1) return rc;
+    return launch_linear_split({x, x_row_stride, x2, x2_row_stride, norm_weight, eps, (const uint16_t *)weight_packed, bias, resid,
+                                resid_row_stride, out, out_row_stride, R, K, N / 32}, gate != 0, (hipStream_t)stream);
+}

@@ -2437,12 +2437,14 @@ def linear_f32(x: torch.Tensor, weight_packed: torch.Tensor, *, bias: torch.Tens
     _need_device(x, "x")
     if x.dtype != torch.float32 or weight_packed.dtype not in (torch.float32, torch.bfloat16):
         raise TypeError("linear_f32 takes float32 rows and a packed float32 weight")
-    # three bf16 pieces, or whole float32 values in the order of the fp32 matrix cores (see bnb_amd.h)
-    pieces = weight_packed.dtype == torch.bfloat16
     n_blocks = weight_packed.shape[0]
-    if weight_packed.shape != ((n_blocks, K // 128, 8, 3, 64, 8) if pieces else (n_blocks, K // 8, 64, 4)) or not weight_packed.is_contiguous():
+    # a stream kept from before the three pieces: whole float32 values, packed again here on every call
+    whole = weight_packed.dtype == torch.float32
+    if weight_packed.shape != ((n_blocks, K // 8, 64, 4) if whole else (n_blocks, K // 128, 8, 3, 64, 8)) or not weight_packed.is_contiguous():
         raise ValueError("weight_packed must come from pack_linear_f32 for this contraction width")
     N = 32 * n_blocks
+    if whole:  # [fb][s4][l][e] = W[32 fb + l%32][(l/32) K/2 + 4 s4 + e]
+        weight_packed = pack_linear_f32(weight_packed.view(n_blocks, K // 8, 2, 32, 4).permute(0, 3, 2, 1, 4).reshape(N, K))
     n_out = N // 2 if gate else N
     if torch.is_grad_enabled() and x.requires_grad:
         raise RuntimeError("linear_f32 is forward-only; call it under torch.no_grad()")
@@ -2466,8 +2468,7 @@ def linear_f32(x: torch.Tensor, weight_packed: torch.Tensor, *, bias: torch.Tens
     if R == 0:
         return out
     with _on_device(x.device):
-        lib = _native.load()
-        rc = (lib.bnb_linear_f32_split_fwd if pieces else lib.bnb_linear_f32_fwd)(
+        rc = _native.load().bnb_linear_f32_fwd(
             x2.data_ptr(), x2.stride(0) if R > 1 else K, None if y2 is None else y2.data_ptr(),
             0 if y2 is None else (y2.stride(0) if R > 1 else K), None if norm_weight is None else norm_weight.detach().contiguous().data_ptr(),
             float(_F32_EPS if eps is None else eps), weight_packed.data_ptr(), None if bias is None else bias.detach().contiguous().data_ptr(),

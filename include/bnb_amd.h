@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define BNB_ABI_VERSION 29
+#define BNB_ABI_VERSION 30
 
 /* element types of activation buffers */
 #define BNB_F32 0
@@ -720,7 +720,7 @@ int bnb_norm_linear_train_fwd(const float *x, int64_t x_row_stride, const float 
                               const void *weight_packed, void *out, void *n_out, int64_t R, int D, int N, void *stream);
 
 /*
- * A float32 Linear layer with its neighbours folded in, on the fp32 matrix cores (true fp32 products):
+ * A float32 Linear layer with its neighbours folded in, on the bf16 matrix cores (an operand is three bf16 pieces):
  *     out[r] = A[r] W^T + bias (+ resid[r]),   A[r] = x[r]                          (norm_weight, x2 NULL)
  *                                                   | rmsnorm(x[r]) * norm_weight     (norm_weight given; K == 128)
  *                                                   | gelu(x[r]) * x2[r]              (x2 given)
@@ -734,29 +734,19 @@ int bnb_norm_linear_train_fwd(const float *x, int64_t x_row_stride, const float 
  *
  *   x, x2          (R, K) fp32 rows, x_row_stride / x2_row_stride floats apart (multiples of 4, 16-byte aligned)
  *   norm_weight    (128) fp32 or NULL; eps as in nn.RMSNorm
- *   weight_packed  W (N, K) as [fb][s4][l][e] = W[32 fb + l%32][(l/32) K/2 + 4 s4 + e], fb < N/32, s4 < K/8,
- *                  l < 64, e < 4 (with gate: blocks 2u, 2u+1 = rows 32u.. of gate_proj, of up_proj)
+ *   weight_packed  W (N, K) as three bf16 pieces, h = bf16(w), m = bf16(w - h), l = bf16(w - h - m):
+ *                  [fb][K/128][ks][piece][l][e] = piece of W[32 fb + l%32][128 t + 16 ks + 8 (e/4) + 4 (l/32) + e%4],
+ *                  fb < N/32, ks < 8, piece < 3, l < 64, e < 8 (with gate: blocks 2u, 2u+1 = rows 32u.. of gate_proj, of
+ *                  up_proj).  Up to ABI 28 it was the whole float32 values in another order: not to be handed to this one.
  *   bias           (N) fp32 or NULL (not with gate)
  *   resid          optional (R, N_out) fp32 rows added to the result; may equal out
  *   out            (R, N_out) fp32 rows, N_out = N, or N/2 with gate
  * Requirements: K % 128 == 0, N % 32 == 0 (N % 64 with gate); anything else returns BNB_ERR_UNSUPPORTED.
  */
 int bnb_linear_f32_fwd(const float *x, int64_t x_row_stride, const float *x2, int64_t x2_row_stride,
-                       const float *norm_weight, float eps, const float *weight_packed, const float *bias,
+                       const float *norm_weight, float eps, const void *weight_packed, const float *bias,
                        const float *resid, int64_t resid_row_stride, float *out, int64_t out_row_stride, int64_t R,
                        int K, int N, int gate, void *stream);
-
-/*
- * The same, with W as three bf16 pieces and the products on the bf16 matrix cores (closer to float64 than the form
- * above, and faster at every size): weight_packed is [fb][K/128][ks][piece][l][e], fb < N/32, ks < 8, piece < 3, l < 64,
- * e < 8, the piece-th bf16 piece (h = bf16(w), m = bf16(w - h), l = bf16(w - h - m)) of
- * W[32 fb + l%32][128 t + 16 ks + 8 (e/4) + 4 (l/32) + e%4] (with gate: blocks 2u, 2u+1 = rows 32u.. of gate_proj, of
- * up_proj).  Arguments, requirements and error codes are otherwise those of bnb_linear_f32_fwd.
- */
-int bnb_linear_f32_split_fwd(const float *x, int64_t x_row_stride, const float *x2, int64_t x2_row_stride,
-                             const float *norm_weight, float eps, const void *weight_packed, const float *bias,
-                             const float *resid, int64_t resid_row_stride, float *out, int64_t out_row_stride, int64_t R,
-                             int K, int N, int gate, void *stream);
 
 /*
  * Compact list of the set entries of a byte mask (B, n), e.g. the bullets in flight of

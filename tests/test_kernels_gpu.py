@@ -2903,6 +2903,26 @@ def test_linear_f32_reads_column_blocks_in_place_and_writes_into_the_residual():
         ops.pack_linear_f32(torch.zeros(48, 128))
 
 
+@pytest.mark.parametrize("R,K,N", [(70, 128, 96), (300, 512, 128)])
+def test_linear_f32_entry_takes_the_stream_that_pack_linear_f32_makes(R, K, N):
+    """Through the C entry point, as a ctypes caller would; and a stream kept from before the pieces (whole float32 values,
+    ``[fb][s4][l][e] = W[32 fb + l%32][(l/32) K/2 + 4 s4 + e]``) through the Python one."""
+    from boost_and_broadside_amd import _native
+
+    g = torch.Generator().manual_seed(R)
+    x, w = torch.randn(R, K, generator=g), torch.randn(N, K, generator=g) / K ** 0.5
+    ref = x.double() @ w.double().t()
+    xd, pk, out = x.to(DEV), ops.pack_linear_f32(w.to(DEV)), torch.empty(R, N, device=DEV)
+    rc = _native.load().bnb_linear_f32_fwd(xd.data_ptr(), K, None, 0, None, 0.0, pk.data_ptr(), None, None, 0, out.data_ptr(), N, R,
+                                           K, N, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and max_rel(out.cpu().double(), ref) <= F32_TOL
+    whole = torch.empty(N // 32, K // 8, 64, 4)
+    for lane in range(64):
+        cols = (lane // 32) * (K // 2) + torch.arange(K // 2)
+        whole[:, :, lane] = w[lane % 32::32][:, cols].reshape(N // 32, K // 8, 4)
+    assert torch.equal(ops.linear_f32(xd, whole.to(DEV)), out)
+
+
 def test_stage_inputs_is_copy_for_every_pair():
     # whole and ragged lengths, widening, empty inputs, and the pairs that one launch cannot take (strided, other dtype,
     # misaligned, broadcast, from the host): every destination ends up as copy_ leaves it

@@ -6,16 +6,21 @@
 //     GATE: W = [gate rows ; up rows] interleaved by blocks of 32, out[r, u] = gelu(g[r, u]) * up[r, u]
 //
 // (models/yemong/attention.py:21-37,60-74; models/yemong/griffin.py:165-167,238-247 run without autocast,
-// evaluation/agents.py:214-219), but a float32 operand enters as three bf16 pieces, v = h + m + l, each the
-// rounded rest of the ones before: 27 bits, so nothing of a float32 is lost.  Of the nine piece products the
-// three below 2^-26 of the whole (m l, l m, l l) are left out, a quarter of a float32 rounding; the other six
-// run on v_mfma_f32_32x32x16_bf16, which does in 32 cycles what v_mfma_f32_32x32x2_f32 needs 512 for: 192 cycles
-// per 32 x 32 x 16 block instead of 512.  The leading products have an accumulator of their own, so the sum of
-// K products is rounded K/16 times at full size and not K/2 times: the relative 2-norm error of a launch against
-// float64 is 0.5e-7 .. 1.8e-7, on the fp32 matrix cores 1.2e-7 .. 3.4e-7.
+// evaluation/agents.py:214-219), but a float32 operand enters as three bf16 pieces, v = h + m / 128 + l / 128^2, each
+// the rounded rest of the ones before.  The rests are carried larger because bf16 ends where float32 does: unscaled, the
+// last piece of a value below 8e-34 would have no exponent left.  So a value is carried exactly from 4.7e-38 on, and
+// within 3e-7 down to the smallest normal one.  Of the nine piece products the three below 2^-25 of the whole (m l, l m,
+// l l) are left out, half a float32 rounding at most; the other six run on v_mfma_f32_32x32x16_bf16, which does in 32
+// cycles what v_mfma_f32_32x32x2_f32 needs 512 for: 192 cycles per 32 x 32 x 16 block instead of 512.  The products of
+// each size have an accumulator of their own, so the sum of K products is rounded K/16 times at full size and not K/2
+// times: the relative 2-norm error of a launch against float64 is 0.5e-7 .. 1.8e-7 (fp32 matrix cores 1.2e-7 .. 3.4e-7),
+// at 1e-36 times the usual size as well (unscaled pieces: 4e-5 with tiny rows, 6e-4 with tiny weights).
+// What the pieces cannot carry (infinities, a row value above 3.39e38, products beyond the range) shows as a result that is
+// not finite, and such a result is formed once more from whole values in float32.
 //
-// Time, fp32 matrix cores -> here: 12288 rows norm + 384 features 33 -> 17 us, norm + 2 x 512 + gate 53 -> 29 us,
-// 512 -> 128 32 -> 24 us; 65760 rows 108 -> 52, 219 -> 108, 118 -> 82 us.  Matrix cores busy about 45 % of the
+// Time, fp32 matrix cores -> here: 12288 rows norm + 384 features 33 -> 17 us, norm + 2 x 512 + gate 53 -> 30 us,
+// 512 -> 128 32 -> 26 us; 65760 rows 108 -> 59, 219 -> 120, 118 -> 84 us (with unscaled pieces on the same boxes 52, 113 and
+// 78 us: two more multiplications per value of a row and two more per result).  Matrix cores busy about 45 % of the
 // large launches' time; the rest is the split of the rows, the gate and the row loads (64-byte pieces a row apart).
 //
 // A wave owns 32 rows, four waves share a stream of 32-feature x 128-channel weight chunks (24 KB with the
@@ -63,6 +68,8 @@ __device__ __forceinline__ float gelu_erf_ls(float v)
     return fmaf(fabsf(hv), erf_abs, hv);
 }
 
+constexpr float kLsScale = 128.0f;  // each rest is carried this much larger: it keeps a bf16 exponent down to the smallest values
+
 // eight float32 -> three bf16 operands
 __device__ __forceinline__ void split8(const float (&v)[8], bf16x8 &h, bf16x8 &m, bf16x8 &l)
 {
@@ -71,9 +78,9 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8 &h, bf16x8 &m
     for (int q = 0; q < 4; ++q) {
         const float a = v[2 * q], b = v[2 * q + 1];
         hw[q] = pack_bf16x2(a, b);
-        const float ra = a - __uint_as_float(hw[q] << 16), rb = b - __uint_as_float(hw[q] & 0xffff0000u);
+        const float ra = (a - __uint_as_float(hw[q] << 16)) * kLsScale, rb = (b - __uint_as_float(hw[q] & 0xffff0000u)) * kLsScale;
         mw[q] = pack_bf16x2(ra, rb);
-        lw[q] = pack_bf16x2(ra - __uint_as_float(mw[q] << 16), rb - __uint_as_float(mw[q] & 0xffff0000u));
+        lw[q] = pack_bf16x2((ra - __uint_as_float(mw[q] << 16)) * kLsScale, (rb - __uint_as_float(mw[q] & 0xffff0000u)) * kLsScale);
     }
     h = __builtin_bit_cast(bf16x8, hw), m = __builtin_bit_cast(bf16x8, mw), l = __builtin_bit_cast(bf16x8, lw);
 }
@@ -93,9 +100,8 @@ __device__ __forceinline__ void load_rows(const LinearSplitArgs &p, int64_t row,
 // ... through the prologue and into pieces
 template <int PRO>
 __device__ __forceinline__ void form_operand(const LinearSplitArgs &p, int64_t row, int t, int half, float (&a)[8][8],
-                                         bf16x8 (&ah)[8], bf16x8 (&am)[8], bf16x8 (&al)[8], bool &wide)
+                                         bf16x8 (&ah)[8], bf16x8 (&am)[8], bf16x8 (&al)[8], float &rstd)
 {
-    float rstd = 0.0f;
     const float *nw = nullptr;
     if (PRO == kLsNorm) {
         float ss = 0.0f;
@@ -119,15 +125,6 @@ __device__ __forceinline__ void form_operand(const LinearSplitArgs &p, int64_t r
                 a[ks][e] = gelu_erf_ls(a[ks][e]) * lo[e], a[ks][4 + e] = gelu_erf_ls(a[ks][4 + e]) * hi[e];
         }
     }
-    if (PRO != kLsNorm) {  // a row with such a value has no finite norm in float32 either
-        float top = 0.0f;
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(a[ks][e]));
-        }
-        wide = wide || __any(top > 1e38f);
-    }
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
         if (PRO == kLsNorm) {
@@ -140,32 +137,74 @@ __device__ __forceinline__ void form_operand(const LinearSplitArgs &p, int64_t r
     }
 }
 
+__device__ __forceinline__ bool not_finite(float v) { return __builtin_amdgcn_classf(v, 0x207); }  // NaNs and infinities
+
+// Operand value k of row r in float32
+template <int PRO>
+__device__ __forceinline__ float operand_f32(const LinearSplitArgs &p, int64_t r, int k, float rstd)
+{
+    float av = p.x[r * p.x_stride + k];
+    if (PRO == kLsNorm) av = av * rstd * p.norm_w[k];
+    if (PRO == kLsMulGelu) av = gelu_erf_ls(av) * p.x2[r * p.x2_stride + k];
+    return av;
+}
+
 // One element in float32, from whole values: row r, feature m of block `block`
 template <int PRO>
-__device__ __forceinline__ float dot_f32(const LinearSplitArgs &p, int64_t r, int block, int m)
+__device__ __forceinline__ float dot_f32(const LinearSplitArgs &p, int64_t r, int block, int m, float rstd)
 {
     float sum = 0.0f;
 #pragma unroll 1
     for (int k = 0; k < p.K; ++k) {
-        float av = p.x[r * p.x_stride + k];
-        if (PRO == kLsMulGelu) av = gelu_erf_ls(av) * p.x2[r * p.x2_stride + k];
         const uint16_t *wp = p.w + ((int64_t)block * (p.K >> 7) + (k >> 7)) * kLsChunkHalfs + ((k & 127) >> 4) * 1536 +
                              (((k >> 2) & 1) * 32 + m) * 8 + ((k >> 3) & 1) * 4 + (k & 3);
-        sum = fmaf(av, (bf16_bits_to_f32(wp[0]) + bf16_bits_to_f32(wp[512])) + bf16_bits_to_f32(wp[1024]), sum);
+        const float wm = bf16_bits_to_f32(wp[512]);  // infinite for an infinite weight, whose last piece then says nothing
+        const float wv = fmaf(fmaf(bf16_bits_to_f32(wp[1024]), 1.0f / kLsScale, wm), 1.0f / kLsScale, bf16_bits_to_f32(wp[0]));
+        sum = fmaf(operand_f32<PRO>(p, r, k, rstd), not_finite(wm) ? wm : wv, sum);
     }
     return sum;
 }
 
-// one contraction step: the six piece products, the leading one into an accumulator of its own
-__device__ __forceinline__ void products(bf16x8 ah, bf16x8 am, bf16x8 al, const u32x4 (&w)[3], f32x16 &big, f32x16 &small)
+// A result that is not finite is formed once more in float32, from whole values: an infinite or nearly infinite operand, or a
+// product beyond the range, meets the other pieces as inf - inf or inf * 0, where float32 products have a value.  Only a row
+// that holds a NaN is left alone.  Called by whole half-waves (row r, lane m: its 32 channels in turn).
+template <int PRO>
+__device__ __forceinline__ bool row_has_nan(const LinearSplitArgs &p, int64_t r, int m, float rstd)
+{
+    bool nan = false;
+#pragma unroll 1
+    for (int k = m; k < p.K; k += 32) {
+        const float av = operand_f32<PRO>(p, r, k, rstd);
+        nan = nan || av != av;
+    }
+    return (uint32_t)(__ballot(nan) >> (threadIdx.x & 32)) != 0;
+}
+
+// The sums of a block by size: products of two leading pieces, of a leading and a second piece (1 / kLsScale of their value),
+// and the rest (1 / kLsScale^2).
+struct Sums {
+    f32x16 big, mid, small;
+    __device__ __forceinline__ void clear()
+    {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) big[v] = mid[v] = small[v] = 0.0f;
+    }
+    __device__ __forceinline__ float total(int v) const
+    {
+        return fmaf(fmaf(small[v], 1.0f / kLsScale, mid[v]), 1.0f / kLsScale, big[v]);
+    }
+};
+
+// one contraction step: the six piece products
+__device__ __forceinline__ void products(bf16x8 ah, bf16x8 am, bf16x8 al, const u32x4 (&w)[3], Sums &s)
 {
     const bf16x8 wh = __builtin_bit_cast(bf16x8, w[0]), wm = __builtin_bit_cast(bf16x8, w[1]), wl = __builtin_bit_cast(bf16x8, w[2]);
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, wh, small, 0, 0, 0);
-    big = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, wh, big, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, wm, small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, wl, small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, wh, small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, wm, small, 0, 0, 0);
+    s.small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, wh, s.small, 0, 0, 0);
+    s.mid = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, wh, s.mid, 0, 0, 0);
+    s.big = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, wh, s.big, 0, 0, 0);
+    s.small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, wm, s.small, 0, 0, 0);
+    s.mid = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, wm, s.mid, 0, 0, 0);
+    s.small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, wl, s.small, 0, 0, 0);
 }
 
 template <int N>
@@ -199,6 +238,7 @@ __global__ __launch_bounds__(kLsWaves * 64) __attribute__((amdgpu_waves_per_eu(2
     constexpr int OUT_BLOCKS = GATE ? 1 : NB, kStores = 16 * OUT_BLOCKS;
     // every row of this wave exists: exactly kStores stores a group, at 32-bit offsets
     const bool full = row0 + 32 <= p.R && p.out_stride < (1 << 24) && p.resid_stride < (1 << 24);
+    bool counted = full;  // the last group's results left as kStores stores
     constexpr int kDma = kLsChunkHalfs / 512 / kLsWaves;  // 1 KB pieces per wave and chunk: 6
     // the chunk that is requested next: block b of group g, slab t
     int rg = g0, rt = 0, rb = 0, rbuf = 0;
@@ -223,11 +263,11 @@ __global__ __launch_bounds__(kLsWaves * 64) __attribute__((amdgpu_waves_per_eu(2
     request();
 
     bf16x8 ah[8], am[8], al[8];
-    bool wide = false;  // some value of this wave's rows is beyond what the pieces carry (infinite, or about to round to it)
+    float rstd = 0.0f;
     auto load_slab = [&](int t) {
         float a[8][8];
         load_rows(p, row, t, half, a);
-        form_operand<PRO>(p, row, t, half, a, ah, am, al, wide);
+        form_operand<PRO>(p, row, t, half, a, ah, am, al, rstd);
     };
     load_slab(0);
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's parts of the first two chunks are in LDS
@@ -235,17 +275,14 @@ __global__ __launch_bounds__(kLsWaves * 64) __attribute__((amdgpu_waves_per_eu(2
 
     int buf = 0;
     for (int g = g0; g < g1; ++g) {
-        f32x16 big[NB], small[NB];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) big[b][v] = small[b][v] = 0.0f;
-        }
+        f32x16 big[NB];
         for (int t = 0; t < slabs; ++t) {
             if (LONG && (t > 0 || g > g0)) load_slab(t);
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 const bool more = request();  // two chunks ahead, into the buffer of the chunk before this one
+                Sums sums;  // of this chunk alone: its three accumulators give way to one
+                sums.clear();
                 const uint16_t *wb = s_w[buf] + lane * 8;
                 u32x4 w[2][3];
 #pragma unroll
@@ -257,13 +294,15 @@ __global__ __launch_bounds__(kLsWaves * 64) __attribute__((amdgpu_waves_per_eu(2
                         for (int q = 0; q < 3; ++q) w[(ks + 1) & 1][q] = *reinterpret_cast<const u32x4 *>(wb + ((ks + 1) * 3 + q) * 512);
                     }
                     __builtin_amdgcn_sched_barrier(0);  // the next step's operands are requested before this step's products
-                    products(ah[ks], am[ks], al[ks], w[ks & 1], big[b], small[b]);
+                    products(ah[ks], am[ks], al[ks], w[ks & 1], sums);
                 }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) big[b][v] = LONG && t > 0 ? big[b][v] + sums.total(v) : sums.total(v);
                 buf = buf == 2 ? 0 : buf + 1;
                 // This wave's part of the next chunk has landed once nothing older than the request above and, behind a
                 // group's end, than its kStores result stores (issued between the two requests) is outstanding: the
                 // counter runs in issue order.  A result store has a whole chunk's time to be acknowledged this way.
-                if (!full) {
+                if (!counted) {
                     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): such a wave leaves stores out
                 } else if (t == 0 && b == 0 && g > g0) {
                     if (more) wait_vmcnt<kStores + kDma>();
@@ -277,29 +316,27 @@ __global__ __launch_bounds__(kLsWaves * 64) __attribute__((amdgpu_waves_per_eu(2
             }
         }
         // ---- epilogue: the lane holds feature m of each block, rows 8 i + 4 half + j ----
+        float zero = 0.0f;  // a NaN once some result is not finite
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) big[b][v] += small[b][v];
+            for (int v = 0; v < 16; ++v) zero = fmaf(big[b][v], 0.0f, zero);
         }
-        if (PRO != kLsNorm && wide) {
-            // the pieces of an infinite or nearly infinite value would meet as inf - inf: these products in float32
+        const bool any_off = __any(zero != zero);
+        uint32_t off[OUT_BLOCKS] = {};  // bit v: result v is not finite
+        if (any_off) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-#pragma unroll 1
-                for (int v = 0; v < 16; ++v) {
-                    const int64_t rr = row0 + 8 * (v >> 2) + 4 * half + (v & 3);
-                    const float sum = dot_f32<PRO>(p, rr < p.R ? rr : p.R - 1, g * NB + b, m);
+            for (int b = 0; b < OUT_BLOCKS; ++b) {
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) big[b][i] = i == v ? sum : big[b][i];
-                }
+                for (int v = 0; v < 16; ++v) off[b] |= not_finite(big[b][v]) || (GATE && not_finite(big[NB - 1][v])) ? 1u << v : 0u;
             }
         }
+        counted = full && !any_off;
 #pragma unroll
         for (int b = 0; b < OUT_BLOCKS; ++b) {
             const int feat = (g * OUT_BLOCKS + b) * 32 + m;
             const float bv = p.bias != nullptr ? p.bias[feat] : 0.0f;
-            if (full) {
+            if (counted) {
                 // 32-bit lane offsets, formed here and not kept across the chunk loop (the empty asm hides that they do not change)
                 uint32_t o_off = 4u * half * (uint32_t)p.out_stride + m, r_off = 4u * half * (uint32_t)p.resid_stride + m;
                 asm volatile("" : "+v"(o_off), "+v"(r_off));
@@ -326,15 +363,41 @@ __global__ __launch_bounds__(kLsWaves * 64) __attribute__((amdgpu_waves_per_eu(2
                     for (int v = 0; v < 16; ++v) leave(v, 0.0f);
                 }
             } else {
+                int rr0 = 4 * half;
+                asm volatile("" : "+v"(rr0));  // sixteen row addresses are not kept across the chunk loop for this path either
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
-                    const int64_t r = row0 + 8 * (v >> 2) + 4 * half + (v & 3);
+                    const int64_t r = row0 + 8 * (v >> 2) + rr0 + (v & 3);
                     float o = big[b][v] + bv;
                     if (GATE) o = gelu_erf_ls(o) * big[NB - 1][v];
                     if (p.resid != nullptr && r < p.R) o += p.resid[r * p.resid_stride + feat];
-                    if (r < p.R) p.out[r * p.out_stride + feat] = o;
+                    if (r < p.R && !(off[b] >> v & 1u)) p.out[r * p.out_stride + feat] = o;
                 }
             }
+        }
+        if (any_off) {
+#pragma unroll
+            for (int b = 0; b < OUT_BLOCKS; ++b) {
+                const int feat = (g * OUT_BLOCKS + b) * 32 + m;
+                const float bv = p.bias != nullptr ? p.bias[feat] : 0.0f;
+#pragma unroll 1
+                for (int v = 0; v < 16; ++v) {
+                    if (!__any(off[b] >> v & 1u)) continue;
+                    const int rr = 8 * (v >> 2) + 4 * half + (v & 3);
+                    const int64_t r = row0 + rr < p.R ? row0 + rr : p.R - 1;
+                    const float rs = __shfl(rstd, rr);
+                    const bool nan = row_has_nan<PRO>(p, r, m, rs);
+                    if (!(off[b] >> v & 1u) || row0 + rr >= p.R) continue;
+                    float o = __builtin_nanf("");
+                    if (!nan) {
+                        o = dot_f32<PRO>(p, r, g * NB + b, m, rs) + bv;
+                        if (GATE) o = gelu_erf_ls(o) * dot_f32<PRO>(p, r, g * NB + NB - 1, m, rs);
+                    }
+                    if (p.resid != nullptr) o += p.resid[r * p.resid_stride + feat];
+                    p.out[r * p.out_stride + feat] = o;
+                }
+            }
+            __builtin_amdgcn_s_waitcnt(0x0f70);  // nothing of this path is left for the chunk loop to wait for
         }
     }
 }
@@ -352,21 +415,18 @@ __global__ __launch_bounds__(kLsWaves * 64) __attribute__((amdgpu_waves_per_eu(2
     const int64_t row0 = (int64_t)(blockIdx.x / groups) * 32;
     const int64_t row = row0 + m < p.R ? row0 + m : p.R - 1;
     const int slabs = p.K >> 7;
-    f32x16 big[NB], small[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) big[b][v] = small[b][v] = 0.0f;
-    }
-    bool wide = false;
+    f32x16 big[NB];
+    float rstd = 0.0f;
     for (int t = wave; t < slabs; t += kLsWaves) {
         float a[8][8];
         load_rows(p, row, t, half, a);
         bf16x8 ah[8], am[8], al[8];
-        form_operand<PRO>(p, row, t, half, a, ah, am, al, wide);
+        form_operand<PRO>(p, row, t, half, a, ah, am, al, rstd);
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const uint16_t *wb = p.w + ((int64_t)(g * NB + b) * slabs + t) * kLsChunkHalfs + lane * 8;
+            Sums sums;
+            sums.clear();
             u32x4 w[4][3];  // three steps ahead
 #pragma unroll
             for (int ks = 0; ks < 3; ++ks) {
@@ -380,17 +440,18 @@ __global__ __launch_bounds__(kLsWaves * 64) __attribute__((amdgpu_waves_per_eu(2
                     for (int q = 0; q < 3; ++q) w[(ks + 3) & 3][q] = *reinterpret_cast<const u32x4 *>(wb + ((ks + 3) * 3 + q) * 512);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                products(ah[ks], am[ks], al[ks], w[ks & 3], big[b], small[b]);
+                products(ah[ks], am[ks], al[ks], w[ks & 3], sums);
             }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) big[b][v] = t >= kLsWaves ? big[b][v] + sums.total(v) : sums.total(v);
         }
     }
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) s_part[wave][b * 16 + v][lane] = big[b][v] + small[b][v];
+        for (int v = 0; v < 16; ++v) s_part[wave][b * 16 + v][lane] = big[b][v];
     }
-    const bool any_wide = PRO != kLsNorm && __syncthreads_or(wide);
-    if (PRO == kLsNorm) __syncthreads();
+    __syncthreads();
     // each wave adds up and writes four of a lane's sixteen rows: 8 wave + 4 half + 0..3
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -399,11 +460,12 @@ __global__ __launch_bounds__(kLsWaves * 64) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int64_t r = row0 + 8 * wave + 4 * half + j;
-            if (r >= p.R) continue;
             float o = 0.0f;
 #pragma unroll
             for (int q = 0; q < kLsWaves; ++q) o += s_part[q][b * 16 + 4 * wave + j][lane];
-            if (any_wide) o = dot_f32<PRO>(p, r, g * NB + b, m);
+            if (__any(not_finite(o)) && !row_has_nan<PRO>(p, r < p.R ? r : p.R - 1, m, 0.0f) && not_finite(o))
+                o = dot_f32<PRO>(p, r < p.R ? r : p.R - 1, g * NB + b, m, 0.0f);
+            if (r >= p.R) continue;
             o += bv;
             if (p.resid != nullptr) o += p.resid[r * p.resid_stride + feat];
             p.out[r * p.out_stride + feat] = o;

@@ -2399,8 +2399,8 @@ def ffn_fused(
 
 def pack_linear_f32(weight: torch.Tensor, up_weight: torch.Tensor | None = None) -> torch.Tensor:
     """A float32 Linear weight (N, K), N % 32 == 0, K % 128 == 0, as the operand stream of ``linear_f32``: three bf16
-    pieces whose sum is the weight, ``[fb][K/128][ks][piece][l][e] = piece of W[32 fb + l%32][128 t + 16 ks + 8 (e/4) +
-    4 (l/32) + e%4]`` (every matrix-core operand is one contiguous 1 KB run).  With ``up_weight`` (same shape) the two
+    pieces with ``h + m / 128 + l / 128^2`` = the weight, ``[fb][K/128][ks][piece][l][e] = piece of W[32 fb + l%32][128 t +
+    16 ks + 8 (e/4) + 4 (l/32) + e%4]`` (every matrix-core operand is one contiguous 1 KB run).  With ``up_weight`` (same shape) the two
     matrices are interleaved in blocks of 32 rows, ``[gate block u, up block u]``, for the gated form."""
     w = weight.detach().float()
     N, K = w.shape
@@ -2412,10 +2412,12 @@ def pack_linear_f32(weight: torch.Tensor, up_weight: torch.Tensor | None = None)
         N = 2 * N
     # [fb][m][t][ks][e / 4][half][e % 4] -> [fb][t][ks][half][m][e / 4][e % 4]
     w = w.view(N // 32, 32, K // 128, 8, 2, 2, 4).permute(0, 2, 3, 5, 1, 4, 6).reshape(N // 32, K // 128, 8, 1, 64, 8)
-    h = w.bfloat16()
-    rest = (w - h).nan_to_num_(0.0, 0.0, 0.0)  # an infinite weight is its first piece
+    # the rests are carried 128 and 128^2 times as large, so that they keep a bf16 exponent down to the smallest normal weights
+    top = torch.finfo(torch.bfloat16).max  # what lies above is carried by the second piece, an infinite weight too
+    h = w.clamp(-top, top).bfloat16()
+    rest = (w - h).mul_(128.0)
     m = rest.bfloat16()
-    return torch.cat([h, m, (rest - m).bfloat16()], dim=3)
+    return torch.cat([h, m, (rest - m).mul_(128.0).bfloat16()], dim=3)
 
 
 def linear_f32_supported(x: torch.Tensor, n_features: int) -> bool:

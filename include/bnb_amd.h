@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define BNB_ABI_VERSION 30
+#define BNB_ABI_VERSION 31
 
 /* element types of activation buffers */
 #define BNB_F32 0
@@ -734,10 +734,12 @@ int bnb_norm_linear_train_fwd(const float *x, int64_t x_row_stride, const float 
  *
  *   x, x2          (R, K) fp32 rows, x_row_stride / x2_row_stride floats apart (multiples of 4, 16-byte aligned)
  *   norm_weight    (128) fp32 or NULL; eps as in nn.RMSNorm
- *   weight_packed  W (N, K) as three bf16 pieces, h = bf16(w), m = bf16(w - h), l = bf16(w - h - m):
+ *   weight_packed  W (N, K) as three bf16 pieces, w = h + m / 128 + l / 128^2: h = bf16(w), at most the largest finite
+ *                  bf16 in size; m = bf16(128 (w - h)), infinite for an infinite w; l = bf16(128 (128 (w - h) - m)):
  *                  [fb][K/128][ks][piece][l][e] = piece of W[32 fb + l%32][128 t + 16 ks + 8 (e/4) + 4 (l/32) + e%4],
  *                  fb < N/32, ks < 8, piece < 3, l < 64, e < 8 (with gate: blocks 2u, 2u+1 = rows 32u.. of gate_proj, of
- *                  up_proj).  Up to ABI 28 it was the whole float32 values in another order: not to be handed to this one.
+ *                  up_proj).  Up to ABI 28 it was the whole float32 values in another order, in ABI 29 and 30 the
+ *                  pieces were not scaled: neither is to be handed to this one.
  *   bias           (N) fp32 or NULL (not with gate)
  *   resid          optional (R, N_out) fp32 rows added to the result; may equal out
  *   out            (R, N_out) fp32 rows, N_out = N, or N/2 with gate

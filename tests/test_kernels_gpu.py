@@ -2903,6 +2903,96 @@ def test_linear_f32_reads_column_blocks_in_place_and_writes_into_the_residual():
         ops.pack_linear_f32(torch.zeros(48, 128))
 
 
+_F32_RANGE_FORMS = [(300, 128, 96, "plain"), (70, 128, 64, "norm"), (300, 128, 96, "times"), (130, 128, 64, "gate"),
+                    (130, 128, 64, "norm_gate"), (90, 512, 128, "plain"), (10300, 512, 128, "plain"), (40, 256, 64, "plain")]
+
+
+def _linear_f32_in_float64(x, w, form, times, norm_w, up):
+    a = x.double()
+    if form.startswith("norm"):
+        a = a * torch.rsqrt(a.pow(2).mean(-1, keepdim=True) + float(torch.finfo(torch.float32).eps)) * norm_w.double()
+    if form == "times":
+        a = _gelu64(a) * times.double()
+    out = a @ w.double().t()
+    return _gelu64(out) * (a @ up.double().t()) if form.endswith("gate") else out
+
+
+def _linear_f32_case(R, K, N, form):
+    g = torch.Generator().manual_seed(R + K + len(form))
+    x, w, up = torch.randn(R, K, generator=g), torch.randn(N, K, generator=g) / K ** 0.5, torch.randn(N, K, generator=g) / K ** 0.5
+    return x, w, up, torch.rand(R, K, generator=g) + 0.5, 1.0 + 0.1 * torch.randn(K, generator=g)
+
+
+def _run_linear_f32(x, w, form, times, norm_w, up):
+    kw = {"gelu_times": times.to(DEV)} if form == "times" else {"norm_weight": norm_w.to(DEV)} if form.startswith("norm") else {}
+    gate = form.endswith("gate")
+    return ops.linear_f32(x.to(DEV), ops.pack_linear_f32(w.to(DEV), up.to(DEV) if gate else None), gate=gate, **kw).cpu()
+
+
+@pytest.mark.parametrize("R,K,N,form", _F32_RANGE_FORMS)
+def test_linear_f32_weights_and_products_beyond_the_pieces_range(R, K, N, form):
+    """Infinite weights, finite ones that round to a bfloat16 infinity, products beyond the float32 range and a NaN: what
+    float32 products give, and nothing else than the results they belong to is touched."""
+    x, w, up, times, norm_w = _linear_f32_case(R, K, N, form)
+    x = x.abs().bfloat16().float() + 0.5  # the rows' second and third pieces are often exactly zero
+    up = up.abs() + 0.1
+    clean = _run_linear_f32(x, w, form, times, norm_w, up)
+    w[3, 5], w[7, K - 1] = float("inf"), -float("inf")
+    w[9] = 0.0
+    w[9, 77] = 3.4028e38 / 64  # finite, with a middle piece
+    w[10] = 0.0
+    w[10, 30] = 3.4028e38
+    if form == "plain":  # a small operand, or the product leaves the float32 range
+        x[:, 30] = 0.25
+    bad = R // 2
+    x[bad, 1] = float("nan")
+    got, want = _run_linear_f32(x, w, form, times, norm_w, up), _linear_f32_in_float64(x, w, form, times, norm_w, up).float()
+    assert got[bad].isnan().all()
+    ok = torch.arange(R) != bad
+    assert torch.equal(got[ok].isposinf(), want[ok].isposinf()) and torch.equal(got[ok].isneginf(), want[ok].isneginf())
+    assert torch.equal(got[ok].isnan(), want[ok].isnan())
+    for f in (9, 10):
+        fin = ok & want[:, f].isfinite()
+        torch.testing.assert_close(got[fin, f], want[fin, f], rtol=3e-6, atol=0.0)  # one product (and the norm or gelu of it)
+    if form != "plain":
+        rest = torch.ones(N, dtype=torch.bool)
+        rest[[3, 7, 9, 10]] = False
+        assert torch.equal(got[ok][:, rest], clean[ok][:, rest])
+    if form == "plain":  # 2^140 in one product: an infinity, not the difference of two
+        x[bad, 1] = 1.0
+        x[:, 2], w[4, 2], w[5, 2] = 1.1 * 2.0 ** 70, 1.3 * 2.0 ** 70, -1.3 * 2.0 ** 70
+        got = _run_linear_f32(x, w, form, times, norm_w, up)
+        assert got[:, 4].isposinf().all() and got[:, 5].isneginf().all()
+
+
+@pytest.mark.parametrize("R,K,N,form", _F32_RANGE_FORMS)
+@pytest.mark.parametrize("which", ["rows", "weights"])
+@pytest.mark.parametrize("scale", [1e-30, 1e-34, 1e-36])
+def test_linear_f32_keeps_float32_precision_for_tiny_values(R, K, N, form, which, scale):
+    """Down to values a few times the smallest normal one.  Relative 2-norm error: each of a result's K/16 partial sums is
+    rounded once to 2^-24 of itself, so K/16 2^-24 at the very most (1.9e-6 for 512 channels), and a tenth of it at random."""
+    x, w, up, times, norm_w = _linear_f32_case(R, K, N, form)
+    if form == "times":
+        x = x + 3.0  # gelu(x) is of x's size; its own argument is not scaled
+    if which == "weights":
+        if form.endswith("gate"):
+            up, w = up * scale, w * 1e6  # gelu(g) of a tiny g halves it once more
+        else:
+            w = w * scale
+    elif form == "times":
+        times = times * scale
+    elif form.startswith("norm"):
+        norm_w = norm_w * scale
+    else:
+        x = x * scale
+    if form.endswith("gate") and which == "rows":
+        w, up = w / scale, up * 1e2  # the gate's own product is of ordinary size
+    got, want = _run_linear_f32(x, w, form, times, norm_w, up).double(), _linear_f32_in_float64(x, w, form, times, norm_w, up)
+    assert want.abs().max() > 1e-37
+    rel = ((got - want).norm() / want.norm()).item()
+    assert rel <= 1e-6, rel
+
+
 @pytest.mark.parametrize("R,K,N", [(70, 128, 96), (300, 512, 128)])
 def test_linear_f32_entry_takes_the_stream_that_pack_linear_f32_makes(R, K, N):
     """Through the C entry point, as a ctypes caller would; and a stream kept from before the pieces (whole float32 values,

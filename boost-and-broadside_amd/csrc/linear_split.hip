@@ -9,8 +9,8 @@
 // evaluation/agents.py:214-219), but a float32 operand enters as three bf16 pieces, v = h + m / 128 + l / 128^2, each
 // the rounded rest of the ones before.  The rests are carried larger because bf16 ends where float32 does: unscaled, the
 // last piece of a value below 8e-34 would have no exponent left.  So a value is carried exactly from 4.7e-38 on, and
-// within 3e-7 down to the smallest normal one.  Of the nine piece products the three below 2^-25 of the whole (m l, l m,
-// l l) are left out, half a float32 rounding at most; the other six run on v_mfma_f32_32x32x16_bf16, which does in 32
+// within 3e-7 down to the smallest normal one.  Of the nine piece products the three of at most 2^-25 of the whole, half a
+// float32 rounding each (m l, l m, l l), are left out; the other six run on v_mfma_f32_32x32x16_bf16, which does in 32
 // cycles what v_mfma_f32_32x32x2_f32 needs 512 for: 192 cycles per 32 x 32 x 16 block instead of 512.  The products of
 // each size have an accumulator of their own, so the sum of K products is rounded K/16 times at full size and not K/2
 // times: the relative 2-norm error of a launch against float64 is 0.5e-7 .. 1.8e-7 (fp32 matrix cores 1.2e-7 .. 3.4e-7),

@@ -42,8 +42,11 @@ constexpr int kNlHalfPitch = 64 + 4;                                   // floats
 constexpr int kNlRowPitch = kNlD + 8;                                  // halfs per staged bf16 row
 static_assert(kNlRowPitch * 2 <= kNlHalfPitch * 4, "a staged bf16 row fits the slice's row pitch");
 
-template <typename XT>
-__global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
+// KEEP: n leaves as well (n_out, the update's form; float32 rows, no list, no bias).  Held to the registers of three work-groups
+// per CU, as many as the other forms have.  The row waits in float32 for its factor, which costs 1 to 5 us a launch beside
+// rounding the bf16 operand once more: 93,696 rows x 384 features 28.8 -> 29.9 us, 393,216 rows 122 -> 128 us.
+template <typename XT, bool KEEP>
+__global__ __launch_bounds__(kNlThreads, KEEP ? 3 : 1) void norm_linear_kernel(
     const XT *__restrict__ x, int64_t x_stride, const int32_t *__restrict__ row_index,
     const int32_t *__restrict__ n_rows, const float *__restrict__ norm_w, float eps,
     const uint16_t *__restrict__ wpack, const float *__restrict__ bias, uint16_t *__restrict__ out, int64_t R, int N,
@@ -56,7 +59,7 @@ __global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
     float *s_stage = reinterpret_cast<float *>(s_raw);
     uint16_t *s_w = reinterpret_cast<uint16_t *>(s_raw);
 
-    const int64_t rows = n_rows != nullptr ? (int64_t)*n_rows : R;
+    const int64_t rows = !KEEP && n_rows != nullptr ? (int64_t)*n_rows : R;
     const int64_t block_row0 = (int64_t)blockIdx.x * (kNlWaves * 32);
     if (block_row0 >= rows) return;  // whole work-group past the end of the (device-side) row count
 
@@ -78,7 +81,7 @@ __global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
         for (int q = 0; q < kNlPrefetch; ++q) dst[tid + q * kNlThreads] = pre[q];
     };
     const int c0 = blockIdx.y * chunks_per_group, c_end = c0 + chunks_per_group;  // the launcher divides the chunks evenly
-    fetch(c0);
+    if (!KEEP) fetch(c0);
 
     // ---- rows in: a quarter-wave per 256-byte half row, two passes over the channels ----
     const int64_t row0 = block_row0 + wave * 32;
@@ -90,14 +93,23 @@ __global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
     for (int j = 0; j < 8; ++j) {
         int64_t r = row0 + 4 * j + io_row;
         r = r < rows ? r : rows - 1;
-        src_row[j] = row_index != nullptr ? (int64_t)row_index[r] : r;
+        src_row[j] = !KEEP && row_index != nullptr ? (int64_t)row_index[r] : r;
     }
     // The per-row factor rsqrt(mean(x^2) + eps) is a scalar of the output row, so it is applied
     // to the products instead of the operand: the operand is bf16(x * w_norm), formed as the
     // channels arrive (the row never sits in registers as fp32), same relative rounding.
     bf16x8 nb[8];
     float ss = 0.0f;
+    [[maybe_unused]] float kept[8][8];  // KEEP: the row itself, until its factor is known
     auto operand = [&](int ks, const float (&t)[8]) {  // k-slots of contraction step ks: channels 16 ks + ...
+        if constexpr (KEEP) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                kept[ks][e] = t[e];
+                ss = fmaf(t[e], t[e], ss);
+            }
+            return;
+        }
         const f32x4 wl = *reinterpret_cast<const f32x4 *>(norm_w + 16 * ks + 4 * half);
         const f32x4 wh = *reinterpret_cast<const f32x4 *>(norm_w + 16 * ks + 8 + 4 * half);
         const float wv[8] = {wl.x, wl.y, wl.z, wl.w, wh.x, wh.y, wh.z, wh.w};
@@ -155,27 +167,37 @@ __global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
     ss += __shfl_xor(ss, 32);
     const float rstd = rsqrtf(ss * (1.0f / kNlD) + eps);
 
-    if (n_out != nullptr && blockIdx.y == 0) {
-        // The update keeps the normalised rows for the weight gradient: the operand this kernel multiplies is
-        // rstd * bf16(x * w_norm); its bfloat16 rounding leaves as whole 256-byte rows through this wave's slice
-        // of the staging area (32 rows x 136 halfs fit in the 32 x 68 floats of the slice).
+    if constexpr (KEEP) {
+        // The update keeps the normalised rows for the weight gradient, rounded once from float32 (the operand is bf16 before its
+        // factor and would be rounded a second time).  They leave as whole 256-byte rows through this wave's slice of the
+        // staging area (32 rows x 136 halfs fit in the 32 x 68 floats of the slice).
         uint16_t *stage_n = reinterpret_cast<uint16_t *>(stage);
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
+            const f32x4 wl = *reinterpret_cast<const f32x4 *>(norm_w + 16 * ks + 4 * half);
+            const f32x4 wh = *reinterpret_cast<const f32x4 *>(norm_w + 16 * ks + 8 + 4 * half);
+            const float wv[8] = {wl.x, wl.y, wl.z, wl.w, wh.x, wh.y, wh.z, wh.w};
             float t[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) t[e] = (float)nb[ks][e] * rstd;
+            for (int e = 0; e < 8; ++e) {
+                nb[ks][e] = (__bf16)(kept[ks][e] * wv[e]);
+                t[e] = (kept[ks][e] * rstd) * wv[e];
+            }
             uint16_t *sp = stage_n + m * kNlRowPitch + 16 * ks + 4 * half;
             *reinterpret_cast<u32x2 *>(sp) = u32x2{pack_bf16x2(t[0], t[1]), pack_bf16x2(t[2], t[3])};
             *reinterpret_cast<u32x2 *>(sp + 8) = u32x2{pack_bf16x2(t[4], t[5]), pack_bf16x2(t[6], t[7])};
+            if (ks & 1) __builtin_amdgcn_sched_barrier(0);  // the norm's weights in four portions beside the kept row
         }
+        fetch(c0);  // now that the row has left its registers
         wave_lds_handover();
-        const int a_row = lane >> 4, a_col = (lane & 15) * 8;
+        if (blockIdx.y == 0) {
+            const int a_row = lane >> 4, a_col = (lane & 15) * 8;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int64_t r = row0 + 4 * j + a_row;
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(stage_n + (4 * j + a_row) * kNlRowPitch + a_col);
-            if (r < rows) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(n_out + r * kNlD + a_col));
+            for (int j = 0; j < 8; ++j) {
+                const int64_t r = row0 + 4 * j + a_row;
+                const u32x4 v = *reinterpret_cast<const u32x4 *>(stage_n + (4 * j + a_row) * kNlRowPitch + a_col);
+                if (r < rows) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(n_out + r * kNlD + a_col));
+            }
         }
         __syncthreads();  // the slices are read out before the weights move in
     }
@@ -207,7 +229,7 @@ __global__ __launch_bounds__(kNlThreads) void norm_linear_kernel(
                     float r[8];
 #pragma unroll
                     for (int e = 0; e < 8; ++e) r[e] = z[8 * run + e] * rstd;
-                    if (bias != nullptr) {
+                    if (!KEEP && bias != nullptr) {
                         const f32x4 bl = *reinterpret_cast<const f32x4 *>(bias + f0 + 16 * run);
                         const f32x4 bh = *reinterpret_cast<const f32x4 *>(bias + f0 + 16 * run + 4);
                         r[0] += bl.x; r[1] += bl.y; r[2] += bl.z; r[3] += bl.w;
@@ -360,7 +382,7 @@ static int launch_norm_linear(const XT *x, int64_t x_row_stride, const int32_t *
     const int64_t blocks = (R + kNlWaves * 32 - 1) / (kNlWaves * 32);
     if (blocks > 0x7fffffffLL) return BNB_ERR_UNSUPPORTED;
     const int groups = nl_feature_groups(blocks, N, n_rows != nullptr);
-    hipLaunchKernelGGL(norm_linear_kernel<XT>, dim3((unsigned)blocks, groups), dim3(kNlThreads), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL((norm_linear_kernel<XT, false>), dim3((unsigned)blocks, groups), dim3(kNlThreads), 0, (hipStream_t)stream,
                        x, x_row_stride, row_index, n_rows, norm_weight, eps, (const uint16_t *)weight_packed, bias,
                        (uint16_t *)out, R, N, N / kNlChunkFeatures / groups, (uint16_t *)nullptr);
     return (int)hipGetLastError();
@@ -401,7 +423,7 @@ extern "C" int bnb_norm_linear_train_fwd(const float *x, int64_t x_row_stride, c
     const int64_t blocks = (R + kNlWaves * 32 - 1) / (kNlWaves * 32);
     if (blocks > 0x7fffffffLL) return BNB_ERR_UNSUPPORTED;
     const int groups = nl_feature_groups(blocks, N, false);
-    hipLaunchKernelGGL(norm_linear_kernel<float>, dim3((unsigned)blocks, groups), dim3(kNlThreads), 0, (hipStream_t)stream, x,
+    hipLaunchKernelGGL((norm_linear_kernel<float, true>), dim3((unsigned)blocks, groups), dim3(kNlThreads), 0, (hipStream_t)stream, x,
                        x_row_stride, (const int32_t *)nullptr, (const int32_t *)nullptr, norm_weight, eps,
                        (const uint16_t *)weight_packed, (const float *)nullptr, (uint16_t *)out, R, N,
                        N / kNlChunkFeatures / groups, (uint16_t *)n_out);

@@ -3113,6 +3113,22 @@ def test_norm_linear_train_forward_and_gradients_match_autograd_of_the_oracle(R,
     assert max_rel(nwd.grad.cpu(), nwr.grad.float()) <= BF16_TOL
 
 
+@pytest.mark.parametrize("R,N", [(33, 128), (5000, 256), (30000, 512)])
+def test_norm_linear_train_rounds_the_normalised_rows_once(R, N):
+    """n is bf16(rmsnorm(x) * w) of the float32 value: half a bfloat16 step (2^-9 of the power of two below it) and what the
+    float32 arithmetic before it is off by, 8 of its roundings.  With feature groups and without."""
+    g = torch.Generator().manual_seed(R)
+    D = 128
+    x, nw = 2.0 * torch.randn(R, D, generator=g), 1.0 + 0.1 * torch.randn(D, generator=g)
+    W = torch.randn(N, D, generator=g) / D ** 0.5
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        n = ops.norm_linear_train(x.to(DEV).requires_grad_(), nw.to(DEV), W.to(DEV).requires_grad_())[2].detach().cpu().double()
+    eps = float(torch.finfo(torch.float32).eps)
+    want = x.double() * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + eps) * nw.double()
+    step = torch.exp2(torch.frexp(want)[1].double() - 8)  # of a value in [2^(e-1), 2^e): 2^(e-8)
+    assert ((n - want).abs() <= 0.5 * step + 8 * 2.0 ** -24 * want.abs()).all()
+
+
 def test_norm_linear_train_refuses_what_the_kernel_does_not_cover():
     from boost_and_broadside_amd import _native
 

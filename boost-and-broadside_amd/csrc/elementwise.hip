@@ -391,6 +391,15 @@ extern "C" int bnb_stage_inputs(int count, const void *const *src, void *const *
         ++n;
     }
     if (n == 0) return 0;
+    // all pairs are copied side by side: no destination may hold what another pair, or its own, still reads or writes
+    for (int d = 0; d < n; ++d) {
+        const int64_t held = (a.pieces[d] * 16 + a.tail[d]) * (a.widen >> d & 1 ? 2 : 1);
+        for (int i = 0; i < n; ++i) {
+            const int64_t bytes = a.pieces[i] * 16 + a.tail[i];
+            if (a.src[i] < a.dst[d] + held && a.dst[d] < a.src[i] + bytes) return BNB_ERR_UNSUPPORTED;
+            if (i != d && a.dst[i] < a.dst[d] + held && a.dst[d] < a.dst[i] + bytes * (a.widen >> i & 1 ? 2 : 1)) return BNB_ERR_UNSUPPORTED;
+        }
+    }
     for (int i = n; i <= kStageMax; ++i) a.first[i] = i == n ? groups : 0x7fffffff;
     hipLaunchKernelGGL(stage_inputs_kernel, dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream, a);
     return (int)hipGetLastError();

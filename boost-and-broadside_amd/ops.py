@@ -2603,28 +2603,45 @@ _STAGE_MAX = 8
 
 
 def stage_inputs(pairs) -> None:
-    """``dst.copy_(src)`` for every ``(dst, src)`` pair, in one launch for the pairs that are plain copies on one device
-    (same shape, both contiguous and 16-byte aligned, same dtype or bfloat16 into float32); ``copy_`` does the others."""
-    plain = []
+    """``dst.copy_(src)`` for every ``(dst, src)`` pair in turn (a bool ``src``: ``dst.fill_(src)``).
+
+    The pairs that are plain copies on one device (same shape, both contiguous and 16-byte aligned, same dtype or bfloat16
+    into float32) go in one launch, ``copy_`` does the others.  Where a source lies in the memory of one of the
+    destinations, or two destinations share memory, the order matters and all are copied one after the other."""
+    pairs = list(pairs)
+    plain, others = [], []
     for dst, src in pairs:
-        if (dst.is_cuda and src.device == dst.device and src.shape == dst.shape and src.is_contiguous() and dst.is_contiguous()
-                and not src.is_conj() and not src.is_neg() and (src.dtype == dst.dtype or (src.dtype == torch.bfloat16 and dst.dtype == torch.float32))
+        if (isinstance(src, torch.Tensor) and dst.is_cuda and src.device == dst.device and src.shape == dst.shape
+                and src.is_contiguous() and dst.is_contiguous() and not src.is_conj() and not src.is_neg()
+                and (src.dtype == dst.dtype or (src.dtype == torch.bfloat16 and dst.dtype == torch.float32))
                 and src.data_ptr() % 16 == 0 and dst.data_ptr() % 16 == 0 and len(plain) < _STAGE_MAX
                 and (not plain or plain[0][0].device == dst.device)):
             plain.append((dst, src))
         else:
+            others.append((dst, src))
+    apart = True
+    if plain and others:
+        held = {dst.untyped_storage().data_ptr() for dst, _ in pairs}
+        apart = len(held) == len(pairs) and not any(
+            isinstance(src, torch.Tensor) and src.untyped_storage().data_ptr() in held for _, src in pairs)
+    if plain and apart:
+        n = len(plain)
+        srcs, dsts = (ctypes.c_void_p * n)(), (ctypes.c_void_p * n)()
+        sizes, widen = (ctypes.c_int64 * n)(), (ctypes.c_int32 * n)()
+        for i, (dst, src) in enumerate(plain):
+            srcs[i], dsts[i], sizes[i], widen[i] = src.data_ptr(), dst.data_ptr(), src.numel() * src.element_size(), src.dtype != dst.dtype
+        with _on_device(plain[0][0].device):
+            rc = _native.load().bnb_stage_inputs(n, ctypes.addressof(srcs), ctypes.addressof(dsts), ctypes.addressof(sizes),
+                                                 ctypes.addressof(widen), _stream())
+        if rc == _native.ERR_UNSUPPORTED:  # the memory of one pair reaches into another's
+            apart = False
+        else:
+            _native.check(rc, "bnb_stage_inputs")
+    for dst, src in others if apart else pairs:
+        if isinstance(src, bool):
+            dst.fill_(src)
+        else:
             dst.copy_(src)
-    if not plain:
-        return
-    n = len(plain)
-    srcs, dsts = (ctypes.c_void_p * n)(), (ctypes.c_void_p * n)()
-    sizes, widen = (ctypes.c_int64 * n)(), (ctypes.c_int32 * n)()
-    for i, (dst, src) in enumerate(plain):
-        srcs[i], dsts[i], sizes[i], widen[i] = src.data_ptr(), dst.data_ptr(), src.numel() * src.element_size(), src.dtype != dst.dtype
-    with _on_device(plain[0][0].device):
-        rc = _native.load().bnb_stage_inputs(n, ctypes.addressof(srcs), ctypes.addressof(dsts), ctypes.addressof(sizes),
-                                             ctypes.addressof(widen), _stream())
-    _native.check(rc, "bnb_stage_inputs")
 
 
 class _RowsGather(torch.autograd.Function):

@@ -1790,16 +1790,10 @@ class GraphedTrunk:
             raise ValueError("this capture reads bullets: pass bullets (and bullet_mask) at every step")
         inputs = [(self.tokens, tokens), (self.alive, alive_mask)]
         if self.reset is not None:
-            if reset_mask is None:
-                self.reset.fill_(False)
-            else:
-                inputs.append((self.reset, reset_mask))
+            inputs.append((self.reset, False if reset_mask is None else reset_mask))
         if self.bullets is not None:
             inputs.append((self.bullets, bullets))
-            if bullet_mask is None:
-                self.bullet_mask.fill_(True)
-            else:
-                inputs.append((self.bullet_mask, bullet_mask))
+            inputs.append((self.bullet_mask, True if bullet_mask is None else bullet_mask))
         ops.stage_inputs([(dst, src) for dst, src in inputs if src is not dst])
         self._follow_weights()
         self.graphs[self.cur].replay()

@@ -767,6 +767,7 @@ int bnb_mask_rows(const uint8_t *mask, int32_t *counts, int32_t *offsets, int32_
 /*
  * Up to 8 contiguous inputs into contiguous buffers in one launch: src_bytes[i] bytes each as they are, or with widen[i]
  * bf16 elements into fp32 ones.  All addresses 16-byte aligned; the arrays are host memory and read before the call returns.
+ * The inputs are copied side by side: BNB_ERR_UNSUPPORTED where a buffer overlaps an input or another buffer.
  */
 int bnb_stage_inputs(int count, const void *const *src, void *const *dst, const int64_t *src_bytes, const int32_t *widen,
                      void *stream);

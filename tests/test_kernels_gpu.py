@@ -3029,6 +3029,19 @@ def test_stage_inputs_is_copy_for_every_pair():
         assert torch.equal(d, w)
 
 
+def test_stage_inputs_keeps_the_order_where_a_source_lies_in_a_destination():
+    g = torch.Generator().manual_seed(4)
+    a, b, c = (torch.zeros(600, 64, device=DEV) for _ in range(3))
+    flag, mask = torch.ones(64, dtype=torch.bool, device=DEV), torch.zeros(64, dtype=torch.bool, device=DEV)
+    new = torch.randn(600, 64, generator=g).to(DEV)
+    # a strided read of a buffer filled just before, a plain one of that, a fill and a read of what it filled
+    ops.stage_inputs([(a, new), (b, a.view(64, 600).t()), (c, b.view(600, 64)), (flag, False), (mask, flag[:64])])
+    assert torch.equal(a, new) and torch.equal(b, new.view(64, 600).t()) and torch.equal(c, b) and not mask.any()
+    mask.fill_(True)
+    ops.stage_inputs([(mask, flag), (flag, True)])  # the read comes first
+    assert not mask.any() and flag.all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,n,p", [(1, 1, 1.0), (5, 7, 0.3), (300, 80, 0.25), (3, 2048, 0.9), (9, 1520, 0.02)])
 def test_rows_gather_and_its_gradient_are_the_indexed_selection(dtype, B, n, p):

@@ -2670,6 +2670,8 @@ class _RowsGather(torch.autograd.Function):
         B, n = ctx.mask_shape
         D = ctx.x_shape[-1]
         dout = dout.float().contiguous()
+        if dout.data_ptr() % 16:
+            dout = dout.clone()
         dx = torch.empty(ctx.x_shape, dtype=ctx.x_dtype, device=dout.device)
         if dx.numel():
             with _on_device(dout.device):

@@ -3062,6 +3062,17 @@ def test_rows_gather_and_its_gradient_are_the_indexed_selection(dtype, B, n, p):
     assert x.grad.dtype == dtype and torch.equal(x.grad, want.to(dtype))
 
 
+def test_rows_gather_takes_a_gradient_that_starts_off_a_16_byte_piece():
+    mask = (torch.arange(60) % 3 == 0).view(3, 20).to(DEV)
+    rows = ops.CompactRows(mask)
+    x = torch.randn(3, 20, 128, generator=torch.Generator().manual_seed(1)).to(DEV).requires_grad_()
+    d = torch.randn(20 * 128 + 1, generator=torch.Generator().manual_seed(2)).to(DEV)[1:].view(20, 128)
+    ops.rows_gather(x, rows).backward(d)
+    want = torch.zeros_like(x)
+    want[mask] = d
+    assert torch.equal(x.grad, want)
+
+
 @pytest.mark.parametrize("R,K,N,gate", [(1, 512, 96, False), (33, 1024, 128, False), (10241, 512, 96, False), (10300, 512, 128, False),
                                         (40, 256, 64, False), (161, 256, 64, True), (127, 128, 32, False), (129, 128, 2048, False)])
 @pytest.mark.parametrize("form", ["plain", "times"])

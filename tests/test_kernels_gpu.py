@@ -1219,7 +1219,7 @@ def test_ffn_tail_train_matches_the_inference_kernel_and_autograd_of_the_oracle(
         assert max_rel(w_.grad.cpu(), wd[k].grad.float()) <= BF16_TOL, k
 
 
-@pytest.mark.parametrize("R", [1, 300, 5000])
+@pytest.mark.parametrize("R", [1, 300, 5000, 16400])  # the last on the wide kernel, the others on the one for few rows
 def test_ffn_tail_train_with_the_output_projection_inside_matches_autograd_of_the_oracle(R):
     x, _, nw, p = _ffn_case(R + 17, R)
     g = torch.Generator().manual_seed(R + 2)
@@ -1370,10 +1370,11 @@ def test_temporal_step_for_few_rows_agrees_with_the_large_form(R, with_reset, wi
     assert off <= max(1e-3, 2 / h.numel()), off
 
 
-def test_temporal_step_every_gate_weight_reaches_its_channel():
+@pytest.mark.parametrize("R", [64, 8200])  # the form for few rows, the large one
+def test_temporal_step_every_gate_weight_reaches_its_channel(R):
     # one-hot gate weights: channel j of gate g sees exactly conv-output channel perm[j]; any
     # slip in the operand packing or in the channel order of the exchange shows as a mismatch
-    R, D = 64, 128
+    D = 128
     t = _temporal_inputs(5, R)
     g = torch.Generator().manual_seed(6)
     pa, px = torch.randperm(D, generator=g), torch.randperm(D, generator=g)
@@ -1390,7 +1391,7 @@ def test_temporal_step_every_gate_weight_reaches_its_channel():
     assert torch.allclose(h_new.cpu(), h_true, rtol=3e-2, atol=3e-2)
 
 
-@pytest.mark.parametrize("B,n,NM", [(3, 8, 12), (5, 19, 23), (600, 8, 12), (7, 152, 160)])
+@pytest.mark.parametrize("B,n,NM", [(3, 8, 12), (5, 19, 23), (600, 8, 12), (7, 152, 160), (1100, 8, 12), (60, 152, 160)])
 def test_temporal_step_reads_and_writes_ship_rows_inside_wider_tensors(B, n, NM):
     D, R = 128, B * n
     t = _temporal_inputs(B + NM, R)
@@ -1556,7 +1557,7 @@ def test_sdpa_cross_over_compacted_rows_equals_the_masked_form(B, NQ, NK, p):
         assert torch.equal(got, ops.sdpa_cross(qkv, kv, mask, H, accum=merged.clone()))
 
 
-@pytest.mark.parametrize("R", [1, 130, 5000])
+@pytest.mark.parametrize("R", [1, 130, 5000, 16400])  # the last on the wide kernel
 @pytest.mark.parametrize("gated", [False, True])
 def test_ffn_fused_with_folded_projection_matches_oracle(R, gated):
     x, _, nw, p = _ffn_case(R + 7, R)
@@ -1584,7 +1585,7 @@ def test_ffn_fused_with_folded_projection_matches_oracle(R, gated):
 
 
 @pytest.mark.parametrize("R,N", [(1, 128), (37, 384), (128, 256), (130, 384), (5000, 256), (4096, 384), (700, 192), (3000, 320),
-                                 (260, 640)])
+                                 (260, 640), (16400, 384), (16517, 640)])  # the last two on the wide kernel
 @pytest.mark.parametrize("gated", [False, True])
 def test_ffn_fused_with_the_next_sublayers_head_matches_oracle(R, N, gated):
     # the same launch goes on to rmsnorm(out) * w2 -> bf16 -> @ Wh^T, the projection the next sublayer starts with
@@ -1635,8 +1636,9 @@ def test_ffn_fused_at_the_edges_of_the_few_row_form(R, gated):
         assert torch.equal(out, want[:R])
 
 
-def test_next_head_one_hot_weights_hit_the_documented_positions():
-    D, N, R = 128, 384, 70
+@pytest.mark.parametrize("R", [70, 16400])  # the kernel for few rows, the wide one
+def test_next_head_one_hot_weights_hit_the_documented_positions(R):
+    D, N = 128, 384
     x, _, nw, p = _ffn_case(11, R)
     g = torch.Generator().manual_seed(5)
     rows_a = torch.randn(R, D, generator=g).bfloat16().to(DEV)
@@ -1683,9 +1685,10 @@ def test_next_head_refuses_what_the_kernel_does_not_cover():
     assert lib.bnb_ffn_fused_proj_next_fwd(*args(256, 128)) == 0
 
 
-def test_column_block_operands_are_read_in_place():
+@pytest.mark.parametrize("B", [6, 1400])  # tails of 72 and 16,800 rows: the kernel for few rows, the wide one
+def test_column_block_operands_are_read_in_place(B):
     # [linear1 | linear2] outputs side by side: the conv reads the left block, the tail's gate the right one
-    B, n, NM, D = 6, 8, 12, 128
+    n, NM, D = 8, 12, 128
     g = torch.Generator().manual_seed(4)
     both = torch.randn(B, NM, 2 * D, generator=g).bfloat16().to(DEV)
     b1, gate = both[..., :D], both[..., D:]
@@ -1705,10 +1708,11 @@ def test_column_block_operands_are_read_in_place():
     assert torch.equal(in_place, copied)
 
 
-def test_three_column_blocks_share_one_projection_output():
+@pytest.mark.parametrize("B", [7, 1400])  # 56 and 11,200 ship rows, tails of 84 and 16,800: both kernels of each
+def test_three_column_blocks_share_one_projection_output(B):
     # [linear1 | linear2 | recurrence output] in one (B, NM, 3D) tensor: the fused state kernel
     # writes the ship rows of the third block, the tail reads its gate and y operands in place
-    B, n, NM, D = 7, 8, 12, 128
+    n, NM, D = 8, 12, 128
     t = {k: v.to(DEV) for k, v in _temporal_inputs(9, B * n).items()}
     g = torch.Generator().manual_seed(5)
     wide = torch.randn(B, NM, 3 * D, generator=g).bfloat16().to(DEV)

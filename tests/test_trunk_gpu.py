@@ -923,6 +923,74 @@ def test_trunk_sequence_with_bullets_shares_one_list_and_matches_the_block_loop(
     assert torch.isfinite(xin.grad).all() and all(q.grad is not None and torch.isfinite(q.grad).all() for q in trunk.parameters())
 
 
+def _sequence_with_bullets(B, T, p_live, seed=61, D=128, N=8, M=4):
+    torch.manual_seed(seed)
+    trunk = bnb.YemongTrunk(_cfg(D, 4, 2, 2, 1, bullets=1)).to(DEV)
+    with torch.no_grad():
+        for block in trunk.yemong_layers:
+            block.spatial[0].norm_bullet.weight.uniform_(0.7, 1.3)
+    g = torch.Generator().manual_seed(seed + 1)
+    alive = (torch.rand(T, B, N + M, generator=g) < 0.85)
+    alive[..., 0] = True
+    mask = torch.rand(T * B, N * 10, generator=g) < p_live
+    mask[3] = False
+    return trunk, dict(
+        x=torch.randn(T, B, N + M, D, generator=g).to(DEV), alive=alive.to(DEV), bullets=torch.randn(T * B, N * 10, D, generator=g).to(DEV),
+        mask=mask.to(DEV), done=(torch.rand(T, B, generator=g) < 0.15).to(DEV), up=torch.randn(T, B, N + M, D, generator=g).to(DEV),
+        hidden=0.3 * torch.randn(2, B * N, 4 * D, generator=g).to(DEV), n_rec=N)
+
+
+def _sequence_grads(trunk, c, bullets, run):
+    trunk.zero_grad(set_to_none=True)
+    x, bul = c["x"].clone().requires_grad_(), bullets.clone().requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        out = run(x, bul)
+    (out.float() * c["up"]).sum().backward()
+    return {"out": out.detach(), "x": x.grad, "bullets": bul.grad, **{n: q.grad.clone() for n, q in trunk.named_parameters()}}
+
+
+@pytest.mark.parametrize("checkpoint", [False, True])
+@pytest.mark.parametrize("B,T,p_live", [(10, 6, 0.3), (40, 12, 0.3)])  # some 1,400 live bullets, some 11,500: below and above 8192
+def test_trunk_sequence_gives_every_readers_bullet_gradient_once(B, T, p_live, checkpoint):
+    """Two readers on rows gathered once, handed on from one to the other (or taken by both in recomputed blocks), against the
+    same two readers selecting their rows themselves.  The kernels behind are the same: only the order in which the readers'
+    float32 gradients of a row are added differs."""
+    trunk, c = _sequence_with_bullets(B, T, p_live)
+    n_live = int(c["mask"].sum())
+    assert (n_live >= 8192) == (B == 40)
+
+    def own(x, bul):
+        for i, block in enumerate(trunk.yemong_layers):
+            h = c["hidden"][i:i + 1]
+            x = block.sequence(x, c["alive"], h[:, :, :128], h[:, :, 128:].reshape(1, -1, 3, 128), c["done"], c["n_rec"], bul, c["mask"])[0]
+        return x
+
+    got = _sequence_grads(trunk, c, c["bullets"], lambda x, bul: trunk.sequence(
+        x, c["alive"], c["hidden"], c["done"], bul, c["mask"], grad_checkpoint=checkpoint))
+    want = _sequence_grads(trunk, c, c["bullets"], own)
+    assert got["bullets"][~c["mask"]].abs().max() == 0 and torch.equal(got["out"], want["out"])
+    for name, w in want.items():
+        assert w.abs().max() > 0, name
+        assert max_rel(got[name].cpu(), w.cpu()) <= 1e-6, name  # two additions in another order: 2 * 2^-24 of the largest
+    with_one = _sequence_grads(trunk, c, c["bullets"], lambda x, bul: trunk.sequence(
+        x, c["alive"], c["hidden"], c["done"], bul, bnb.ops.CompactRows(c["mask"]), grad_checkpoint=checkpoint))
+    assert all(torch.equal(with_one[k], got[k]) for k in got)  # the caller's own list
+
+
+@pytest.mark.parametrize("checkpoint", [False, True])
+@pytest.mark.parametrize("B,T,p_live", [(10, 6, 0.3), (40, 12, 0.3)])
+def test_trunk_sequence_bfloat16_bullets_get_the_float32_gradient_rounded_once(B, T, p_live, checkpoint):
+    trunk, c = _sequence_with_bullets(B, T, p_live, seed=71)
+    b16 = c["bullets"].bfloat16()
+
+    def run(x, bul):
+        return trunk.sequence(x, c["alive"], c["hidden"], c["done"], bul, c["mask"], grad_checkpoint=checkpoint)
+
+    got, want = _sequence_grads(trunk, c, b16, run), _sequence_grads(trunk, c, b16.float(), run)
+    assert got["bullets"].dtype == torch.bfloat16 and torch.equal(got["bullets"], want["bullets"].bfloat16())
+    assert all(torch.equal(got[k], want[k]) for k in got if k != "bullets")
+
+
 # ------------------------------------------------------------------ weights that change after the first forward
 
 

@@ -266,10 +266,10 @@ __global__ __launch_bounds__(kFsThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     }
 }
 
-// A work-group takes a CU's LDS, so 32 rows for each of the 256 CUs are one round (13.5 us against the wide kernel's 28.2 us
+// A work-group takes a CU's LDS, so 32 rows for each of 256 CUs are one round (13.5 us against the wide kernel's 28.2 us
 // at 8192 rows) and two rounds still win (24.4 us against 30.2 us at 16384 rows); a third would not (the wide kernel takes
 // 31.5 us at 24576 rows).
-int64_t ffn_small_rows_limit() { return 16384; }
+int64_t ffn_small_rows_limit() { return (int64_t)64 * cu_count(); }
 
 int launch_ffn_small(const FfnSmallArgs &a, hipStream_t s)
 {

@@ -34,7 +34,9 @@ namespace bnb {
 
 constexpr int kLsChunkHalfs = 8 * 3 * 512;  // 32 features x 128 channels x 3 pieces
 constexpr int kLsWaves = 4;
-constexpr int kLsFewRows = 10240;  // K = 512, N = 128, us of this form and of the other: 2000 rows 9 / 21, 8192 17 / 23, 12288 26 / 24, 27680 50 / 35
+// Rows per CU up to which a contraction of 512 or more is split over waves.  The one such layer of the trunk is 512 -> 128, us of this
+// form and of the other on 256 CUs: 2000 rows 9 / 21, 8192 17 / 23, 12288 26 / 25, 27680 50 / 35; other N were not measured.
+constexpr int kLsFewRowsPerCu = 40;
 
 struct LinearSplitArgs {
     const float *x;
@@ -477,7 +479,7 @@ template <int PRO, bool GATE, int NB, bool LONG>
 static int launch_nb(const LinearSplitArgs &p, hipStream_t stream)
 {
     const int64_t tiles = (p.R + 32 * kLsWaves - 1) / (32 * kLsWaves);
-    const int groups = p.n_blocks / NB, slabs = p.K / 128;
+    const int groups = p.n_blocks / NB, slabs = p.K / 128, cus = cu_count();
     // Feature blocks per work-group: the split whose slowest CU has the least to do.  A work-group's time in chunks:
     // its products, and the load + split of its rows (about 1.5 chunks a slab); two work-groups share a CU, and an odd
     // one left over runs at 0.65 of a pair's time.
@@ -485,7 +487,7 @@ static int launch_nb(const LinearSplitArgs &p, hipStream_t stream)
     double best_t = 0.0;
     for (int per = groups; per >= 1; --per) {
         const int splits = (groups + per - 1) / per;
-        const int64_t n = (tiles * splits + 255) / 256;
+        const int64_t n = (tiles * splits + cus - 1) / cus;
         const double unit = slabs == 1 ? 1.5 + per * NB : per * slabs * (1.5 + NB);
         const double t = unit * ((double)(n / 2) + (n & 1 ? 0.65 : 0.0));
         if (per == groups || t < best_t) best = per, best_t = t;
@@ -504,7 +506,7 @@ static int launch_pro(const LinearSplitArgs &p, hipStream_t stream)
     if constexpr (PRO != kLsNorm) {
         if (p.K > 128) {
             if constexpr (!GATE) {
-                if (p.K >= 512 && p.R <= kLsFewRows) {
+                if (p.K >= 512 && p.R <= (int64_t)kLsFewRowsPerCu * cu_count()) {
                     const int64_t tiles = (p.R + 31) / 32;
                     if (p.n_blocks % 2 == 0)
                         hipLaunchKernelGGL((linear_split_k_kernel<PRO, 2>), dim3((unsigned)(tiles * (p.n_blocks / 2))), dim3(256), 0, stream, p, p.n_blocks / 2);

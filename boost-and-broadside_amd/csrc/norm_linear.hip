@@ -360,7 +360,7 @@ namespace bnb {
 static int nl_feature_groups(int64_t row_groups, int N, bool listed)
 {
     const int chunks = N / kNlChunkFeatures;
-    const int64_t room = (listed ? 4 : 1) * 3 * 256;
+    const int64_t room = (listed ? 4 : 1) * 3 * (int64_t)cu_count();
     for (int g = chunks; g > 1; --g)
         if (chunks % g == 0 && row_groups * g <= room) return g;
     return 1;

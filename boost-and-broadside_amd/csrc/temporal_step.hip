@@ -273,7 +273,7 @@ constexpr int kTsSmallGatePitch = 2 * kTsD + 8;
 // us, form above -> this one: 128 rows 11.6 -> 7.1, 4096 rows 14.0 -> 8.7, 8192 rows (one work-group per CU) 16.0 -> 11.2,
 // 16384 rows 20.4 -> 20.8, 32768 rows 29.8 -> 38.9.  Of the 128 rows' 7.1 us most is launch, one round trip to memory and the
 // way of 7 KB of code into the instruction cache: with sixteen log-sigmoids inlined per lane (22 KB) it was 10.8 us.
-constexpr int64_t kTsSmallRows = 8192;
+constexpr int kTsSmallRowsPerCu = kTsRows;  // one work-group per CU
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void temporal_step_small_kernel(
     const uint16_t *__restrict__ b1, int64_t b1_group_stride, int64_t b1_row_stride, const float *conv_in,
@@ -426,20 +426,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     }
 }
 
-static int ts_cu_count()
-{
-    // compute units of the current device, looked up once per device
-    static int cached[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cached[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
-}
-
 }  // namespace bnb
 
 extern "C" int bnb_temporal_step_fwd(const void *b1, int64_t b1_group_stride, int64_t b1_row_stride,
@@ -470,7 +456,7 @@ extern "C" int bnb_temporal_step_fwd(const void *b1, int64_t b1_group_stride, in
         (b1_group_stride % 8) != 0 || (y_group_stride % 8) != 0 || (y_row_stride % 8) != 0 || (conv_in_row_stride % 4) != 0 ||
         (conv_out_row_stride % 4) != 0 || (h_in_row_stride % 4) != 0 || (h_out_row_stride % 4) != 0)
         return BNB_ERR_MISALIGNED;
-    if (R <= kTsSmallRows) {
+    if (R <= (int64_t)kTsSmallRowsPerCu * cu_count()) {
         hipLaunchKernelGGL(temporal_step_small_kernel, dim3((unsigned)((R + kTsRows - 1) / kTsRows)), dim3(256), 0, (hipStream_t)stream,
                            (const uint16_t *)b1, b1_group_stride, b1_row_stride, conv_in, conv_in_row_stride, conv_out,
                            conv_out_row_stride, h_in, h_in_row_stride, h_out, h_out_row_stride, conv_weight, conv_bias,
@@ -479,7 +465,7 @@ extern "C" int bnb_temporal_step_fwd(const void *b1, int64_t b1_group_stride, in
         return (int)hipGetLastError();
     }
     // One work-group per CU at most (LDS), 8 waves each, every wave at least 8 rows.
-    const int cus = ts_cu_count();
+    const int cus = cu_count();
     const int waves = kTsMaxWaves;
     int64_t blocks = (R + (int64_t)waves * 8 - 1) / ((int64_t)waves * 8);
     if (blocks > cus) blocks = cus;

@@ -20,7 +20,7 @@
 //
 // Time, fp32 matrix cores -> here: 12288 rows norm + 384 features 33 -> 17 us, norm + 2 x 512 + gate 53 -> 30 us,
 // 512 -> 128 32 -> 26 us; 65760 rows 108 -> 59, 219 -> 120, 118 -> 84 us (with unscaled pieces on the same boxes 52, 113 and
-// 78 us: two more multiplications per value of a row and two more per result).  Matrix cores busy about 45 % of the
+// 78 us: two more multiplications per value of a row and two more per result).  Matrix cores busy 33 to 50 % of the
 // large launches' time; the rest is the split of the rows, the gate and the row loads (64-byte pieces a row apart).
 //
 // A wave owns 32 rows, four waves share a stream of 32-feature x 128-channel weight chunks (24 KB with the

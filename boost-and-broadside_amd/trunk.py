@@ -630,7 +630,7 @@ class TransformerBlock(_WeightCaches, nn.Module):
                 attn = self._attn(None, alive_mask, bullets, bullet_mask, qkv=qkv)
         elif (_f32_fused_ok(x, act, self.qkv, self.out_proj) and self.qkv.bias is None and self.out_proj.bias is None
               and self.norm1.weight is not None):
-            # float32 (evaluation without autocast): every Linear on the fp32 matrix cores with its norm, gate and
+            # float32 (evaluation without autocast): every Linear as one kernel (operands in bf16 pieces) with its norm, gate and
             # residual folded in: norm1 + qkv, attention, out_proj + residual, norm2 + gate/up + gelu gate, down + residual
             qkv = ops.linear_f32(x, _packed_f32(self.qkv, "_bnb_f32_pack", self.qkv.weight), norm_weight=self.norm1.weight,
                                  eps=self.norm1.eps)
@@ -831,7 +831,7 @@ class RGLRU(_WeightCaches, nn.Module):
         act = _projection_dtype()
         wa, wx, ba, bx = self.linear_a.weight, self.linear_x.weight, self.linear_a.bias, self.linear_x.bias
         if _f32_fused_ok(x, act, self.linear_a, self.linear_x) and x.dim() == 2 and ba is not None and bx is not None:
-            # float32: both gate projections and their biases as one kernel on the fp32 matrix cores
+            # float32: both gate projections and their biases as one kernel
             pk = _cached_cast(self, "_bnb_f32_gates", (wa, wx), torch.float32,
                               lambda: ops.pack_linear_f32(torch.cat([wa.detach(), wx.detach()], dim=0)))
             bias = _cached_cast(self, "_bnb_f32_gate_bias", (ba, bx), torch.float32,
@@ -1843,8 +1843,10 @@ class EagerTrunkStepper:
         return out, new_state
 
 
-# tokens per step below which a captured step beats plain launches (measured on MI355X with the default trunk of
-# 2 blocks x (2 attention + 1 temporal sublayer)): the launches of a step take the host ~0.4 ms
+# tokens per step below which a captured step beats plain launches, with the default trunk of 2 blocks x (2 attention +
+# 1 temporal sublayer) and bullets: the launches of a step take the host ~0.6 ms (float32 0.78 ms), a captured step copies its inputs.
+# us a step, captured / plain.  float32: 7,920 tokens 558 / 778, 9,960 705 / 775, 10,240 (160 a battle) 815 / 801, 12,288 750 / 775,
+# 16,320 866 / 832.  bfloat16: 40,000 479 .. 558 / 590, 50,400 539 / 590, 64,000 735 / 674, 93,696 924 / 860.
 GRAPH_BELOW_TOKENS = {torch.float32: 10_000, torch.bfloat16: 40_000}
 
 

@@ -2810,3 +2810,72 @@ def sdpa_cross_rows(
             )
     _native.check(rc, "bnb_sdpa_cross_ranges_fwd")
     return out
+
+
+TRUNK_TOKENS = 32  # tokens of an environment that trunk_step covers
+_TRUNK_SLOTS = 2048  # bullet slots of the environments that share a work-group
+_FLAGS = (torch.bool, torch.uint8)
+
+
+def trunk_step_supported(B: int, NM: int, n_rec: int, D: int, n_heads: int, n_layers: int, slots: int) -> bool:
+    """Whether ``trunk_step`` covers these sizes (``slots``: bullet slots of an environment, 0 without a read)."""
+    return (D == FFN_WIDTH and n_heads == 4 and 1 <= n_rec <= NM <= TRUNK_TOKENS and 1 <= n_layers <= _native.TRUNK_MAX_LAYERS
+            and B > 0 and (TRUNK_TOKENS // NM) * slots <= _TRUNK_SLOTS)
+
+
+def trunk_step_pays(B: int, NM: int, device) -> bool:
+    """Whether the whole step as one kernel is faster than the separate kernels.
+
+    One round of work-groups over the chip (32 rows each, whole environments) takes about 64 us with the default trunk, the
+    separate kernels about 100 us and 9 us for every thousand rows.  us, one kernel / separate: 16 environments of 12 tokens
+    65 / 121, 512 of 8 70 / 146, 1024 of 12 (2 rounds) 133 / 233, 512 of 23 (2) 136 / 243, 1280 of 23 (5) 313 / 375, 3072 of 12
+    (6) 387 / 458, 6144 of 8 (6) 444 / 571, 7808 of 12 (16) 1000 / 882."""
+    groups = -(-B // (TRUNK_TOKENS // NM))
+    rounds = -(-groups // torch.cuda.get_device_properties(device).multi_processor_count)
+    return rounds == 1 or 64 * rounds <= 100 + 0.009 * B * NM
+
+
+def trunk_table(layers):
+    """The layers of ``trunk_step`` as the native call takes them: dicts with the fields of ``bnb_trunk_layer``
+    (include/bnb_amd.h), tensors where it has pointers.  The tensors have to outlive the table's use."""
+    table = (_native.TrunkLayer * len(layers))()
+    for entry, given in zip(table, layers):
+        for name, value in given.items():
+            setattr(entry, name, value.data_ptr() if isinstance(value, torch.Tensor) else value)
+    return table
+
+
+def trunk_step(table, x, n_rec, alive, state_in, state_out, *, reset=None, bullets=None, in_flight=None, bullet_eps=0.0, out=None,
+               out_dtype=torch.float32):
+    """One timestep of every sublayer of the trunk as one kernel (small fleets, bfloat16 autocast flow).
+
+    table: ``trunk_table``.  x (B, NM, 128) float32 or bfloat16; alive (B, NM) and in_flight (B, NB) bool or uint8 or None;
+    reset (B,) or None; bullets (B, NB, 128) float32 or bfloat16 or None; state_in / state_out (slots, B * n_rec, 512)
+    float32.  All contiguous, rows and state 16-byte aligned.  Writes ``state_out``, returns (B, NM, 128): ``out`` or a new
+    tensor in ``out_dtype``."""
+    B, NM, D = x.shape
+    NB = 0 if bullets is None else bullets.shape[1]
+    _need_device(x, "x")
+    if not trunk_step_supported(B, NM, n_rec, D, 4, len(table), NB):
+        raise RuntimeError("trunk_step covers up to 32 tokens an environment, width 128 and 4 heads")
+    if out is None:
+        out = torch.empty((B, NM, D), dtype=out_dtype, device=x.device)
+    slots = state_in.shape[0]
+    rows, floats = (torch.float32, torch.bfloat16), (torch.float32,)
+    for name, t, shape, dtypes in (("x", x, (B, NM, D), rows), ("out", out, (B, NM, D), rows), ("alive", alive, (B, NM), _FLAGS),
+                                   ("reset", reset, (B,), _FLAGS), ("bullets", bullets, (B, NB, D), rows),
+                                   ("in_flight", in_flight, (B, NB), _FLAGS), ("state_in", state_in, (slots, B * n_rec, 4 * D), floats),
+                                   ("state_out", state_out, (slots, B * n_rec, 4 * D), floats)):
+        if t is not None and (t.shape != shape or t.dtype not in dtypes or not t.is_contiguous() or t.device != x.device):
+            raise ValueError(f"{name} must be a contiguous {shape} tensor of {dtypes} on {x.device}")
+    if sum(entry.temporal for entry in table) > slots:
+        raise ValueError("more recurrent sublayers than slots of the state")
+    ptr = [None if t is None else t.data_ptr() for t in (alive, reset, bullets, in_flight)]
+    with _on_device(x.device):
+        rc = _native.load().bnb_trunk_step_fwd(
+            ctypes.addressof(table), len(table), x.data_ptr(), _DTYPE_CODE[x.dtype], out.data_ptr(), _DTYPE_CODE[out.dtype],
+            ptr[0], ptr[1], ptr[2], 0 if bullets is None else _DTYPE_CODE[bullets.dtype], ptr[3], float(bullet_eps), NB,
+            state_in.data_ptr(), state_out.data_ptr(), B, NM, n_rec, D, 4, FFN_HIDDEN, _stream(),
+        )
+    _native.check(rc, "bnb_trunk_step_fwd")
+    return out

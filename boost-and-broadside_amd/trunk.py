@@ -43,7 +43,9 @@ from __future__ import annotations
 import collections
 import contextlib
 import copy
+import math
 import warnings
+import weakref
 from dataclasses import dataclass
 
 import torch
@@ -164,6 +166,7 @@ def forbid_library_dispatch():
 
 
 _CACHE_PREFIX = "_bnb_"
+_FLAGS = (torch.bool, torch.uint8)
 
 
 class _DerivedWeight:
@@ -1486,6 +1489,24 @@ class _LiveRows:
         self.rows, self.chained = rows, chained
 
 
+class _SteppedShape:
+    """Held by every stepper of one shape over one trunk."""
+
+    __slots__ = ("__weakref__",)
+
+
+_STEPPED = weakref.WeakKeyDictionary()  # trunk -> {(environments, tokens, recurrent tokens, bullet slots): _SteppedShape} of its steppers
+
+
+def _stepped_shapes(trunk):
+    return _STEPPED.get(trunk, ())
+
+
+def _register_shape(trunk, *shape) -> _SteppedShape:
+    shapes = _STEPPED.setdefault(trunk, weakref.WeakValueDictionary())
+    return shapes.setdefault(shape, _SteppedShape())
+
+
 class YemongTrunk(_WeightCaches, nn.Module):
     """The recurrent trunk: ``forward(tokens, alive_mask, recurrent_state) -> (hidden, new_state)``.
 
@@ -1573,6 +1594,117 @@ class YemongTrunk(_WeightCaches, nn.Module):
         own.live_rows = _LiveRows(ops.rows_gather(bullets, rows), chained)
         return own
 
+    def _folded_bullet_pack(self, readers):
+        """The ``kv_bullet`` weights of all reading sublayers side by side, each with its ``norm_bullet`` weight folded in."""
+        ws = tuple(t for l in readers for t in (l.kv_bullet.weight, l.norm_bullet.weight))
+
+        def folded():
+            with torch.autocast("cuda", enabled=False):
+                return ops.pack_linear_weights(torch.cat(
+                    [l.kv_bullet.weight.detach().float() * l.norm_bullet.weight.detach().float()[None, :] for l in readers], dim=0))
+
+        return _cached_cast(self, "_bnb_bullet_kv_pack", ws, torch.bfloat16, folded)
+
+    def _whole_step_layers(self, B, NM, n_rec, slots, device):
+        """``(layers of ops.trunk_table, eps of the bullet norm)`` where the whole step runs as one kernel for B environments of
+        NM tokens, n_rec of them recurrent, with ``slots`` bullet slots (0: no read): small fleets under bfloat16 autocast,
+        every layer in its standard form.  Else None."""
+        blocks = list(self.yemong_layers)
+        readers = [l for block in blocks for l in block.spatial if l.reads_bullets] if slots else []
+        n_layers = sum(len(block.spatial) + len(block.temporal) for block in blocks)
+        if not (
+            _HEAD_FUSION and device.type == "cuda" and _projection_dtype() == torch.bfloat16
+            and ops.trunk_step_supported(B, NM, n_rec, self.config.d_model, self.config.n_heads, n_layers, slots if readers else 0)
+            and ops.trunk_step_pays(B, NM, device)
+        ):
+            return None
+
+        def vector(t):
+            return t is not None and t.dtype == torch.float32 and t.is_contiguous()
+
+        def plain(layer, mlp, *linears):
+            return (not layer._forward_hooks and not layer._forward_pre_hooks and vector(layer.norm1.weight) and vector(layer.norm2.weight)
+                    and all(l.bias is None for l in (*linears, mlp.gate_proj, mlp.up_proj, mlp.down_proj))
+                    and tuple(mlp.gate_proj.weight.shape) == (ops.FFN_HIDDEN, ops.FFN_WIDTH))
+
+        def eps(norm):
+            return ops._F32_EPS if norm.eps is None else norm.eps
+
+        def shared(layer, mlp, out):
+            w = out.weight
+            return {"proj": _cached_cast(out, "_bnb_proj_pack", (w,), torch.bfloat16, lambda: ops.pack_proj_weights(w)),
+                    "ffn": mlp.packed_weights(), "norm1": layer.norm1.weight, "norm2": layer.norm2.weight, "eps1": eps(layer.norm1),
+                    "eps2": eps(layer.norm2)}
+
+        if any(l.kv_bullet.bias is not None or not vector(l.norm_bullet.weight) or l.norm_bullet.eps != readers[0].norm_bullet.eps
+               for l in readers):
+            return None
+        kv = self._folded_bullet_pack(readers) if readers else None
+        table, slot, reader = [], 0, 0
+        for block in blocks:
+            for l in block.spatial:
+                if not (type(l) is TransformerBlock and plain(l, l.ffn, l.qkv, l.out_proj)):
+                    return None
+                w = l.qkv.weight
+                entry = shared(l, l.ffn, l.out_proj)
+                entry["head"] = _cached_cast(l.qkv, "_bnb_head_pack", (w,), torch.bfloat16, lambda w=w: ops.pack_head_weights(w))
+                if kv is not None and l.reads_bullets:
+                    entry["kv"] = kv[8 * reader]  # four blocks of 32 features of K, four of V
+                    reader += 1
+                table.append(entry)
+            for j, l in enumerate(block.temporal):
+                rg = l.rg_lru
+                fold, ws = l._head_weights(NM, n_rec, block.field_sub[j] if NM > n_rec else None)
+                if not (type(l) is GriffinTemporalBlock and plain(l, l.gated_mlp, l.linear1, l.linear2, l.linear_out)
+                        and rg.linear_a.bias is not None and rg.linear_x.bias is not None and fold == (NM > n_rec)
+                        and vector(l.conv.weight) and (l.conv.bias is None or vector(l.conv.bias)) and rg.log_lambda.dtype == torch.float32):
+                    return None
+                gw, gb = (rg.linear_a.weight, rg.linear_x.weight), (rg.linear_a.bias, rg.linear_x.bias)
+                entry = shared(l, l.gated_mlp, l.linear_out)
+                entry.update({
+                    "head": _cached_cast(l, "_bnb_l12f_head_pack" if fold else "_bnb_l12_head_pack", ws, torch.bfloat16,
+                                         lambda l=l, ws=ws: ops.pack_head_weights(l._head_matrix(ws))),
+                    "conv_weight": l.conv.weight, "conv_bias": l.conv.bias,
+                    "gates": _cached_cast(rg, "_bnb_gate_pack", gw, torch.bfloat16, lambda gw=gw: ops.pack_gate_weights(*gw)),
+                    "gate_bias": _cached_cast(rg, "_bnb_gate_bias", gb, torch.float32,
+                                              lambda gb=gb: torch.cat([gb[0], gb[1]], dim=0).detach().float()),
+                    "log2_sigmoid": _cached_cast(rg, "_bnb_log2_sigmoid", (rg.log_lambda,), torch.float32,
+                                                 lambda rg=rg: torch.log1p(torch.exp(-rg.log_lambda.detach())) * -math.log2(math.e)),
+                    "c": float(rg.c), "state_slot": slot, "temporal": 1, "head_blocks": 4 * len(ws)})
+                slot += 1
+                table.append(entry)
+        return table, (eps(readers[0].norm_bullet) if readers else 0.0)
+
+    def _whole_step(self, x, alive, state_in, state_out, n_rec, reset, bullets, in_flight):
+        """The step as one kernel where a stepper for this shape exists and that applies, else None.
+
+        A direct call lays the kernel's table out anew each time, so it is left to shapes that a program is known to step again
+        and again: those of the steppers alive, whose results a direct call then also repeats bit for bit."""
+        B, NM, D = x.shape
+        slots = bullets.shape[1] if bullets is not None and self.config.reads_bullets and bullets.dim() == 3 else 0
+        if (B, NM, n_rec, slots) not in _stepped_shapes(self):
+            return None
+
+        def given(t, shape, dtypes):
+            return t is None or (isinstance(t, torch.Tensor) and tuple(t.shape) == shape and t.dtype in dtypes and t.device == x.device)
+
+        def whole(t):  # in place where t is dense and on a 16-byte piece
+            if t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0):
+                return t
+            return t.clone(memory_format=torch.contiguous_format)
+
+        rows, flags = (torch.float32, torch.bfloat16), (torch.bool, torch.uint8)
+        if not (given(x, (B, NM, D), rows) and given(alive, (B, NM), flags) and given(reset, (B,), flags)
+                and all(t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (state_in, state_out))
+                and (not slots or (given(bullets, (B, slots, D), rows) and given(in_flight, (B, slots), flags)))):
+            return None
+        found = self._whole_step_layers(B, NM, n_rec, slots, x.device)
+        if found is None:
+            return None
+        return ops.trunk_step(ops.trunk_table(found[0]), whole(x), n_rec, whole(alive), state_in, state_out, reset=whole(reset),
+                              bullets=whole(bullets) if slots else None, in_flight=whole(in_flight) if slots else None,
+                              bullet_eps=found[1], out_dtype=x.dtype)
+
     def _bullet_kv_of_all_layers(self, bullets, rows):
         """``{id(layer): [K | V] rows}`` of every bullet-reading sublayer of the step from ONE pass over the bullets in
         flight, or None when there are fewer than two such sublayers (or their norms differ in eps).
@@ -1591,14 +1723,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
         # a layer's column block is addressed with 32-bit element offsets over the full slot capacity
         if bullets.shape[0] * bullets.shape[1] * 2 * D * len(readers) >= 2 ** 32:
             return None
-        ws = tuple(t for l in readers for t in (l.kv_bullet.weight, l.norm_bullet.weight))
-
-        def folded():
-            with torch.autocast("cuda", enabled=False):
-                return ops.pack_linear_weights(torch.cat(
-                    [l.kv_bullet.weight.detach().float() * l.norm_bullet.weight.detach().float()[None, :] for l in readers], dim=0))
-
-        pk = _cached_cast(self, "_bnb_bullet_kv_pack", ws, torch.bfloat16, folded)
+        pk = self._folded_bullet_pack(readers)
         ones = _cached_cast(self, "_bnb_unit_norm", (readers[0].norm_bullet.weight,), torch.float32,
                             lambda: torch.ones(D, dtype=torch.float32, device=bullets.device))
         kv = ops.norm_linear(bullets, ones, pk, eps=readers[0].norm_bullet.eps, rows=rows)  # (capacity, 2 D x layers)
@@ -1632,6 +1757,9 @@ class YemongTrunk(_WeightCaches, nn.Module):
             raise ValueError("out_state must be a float32 tensor shaped like recurrent_state that shares no memory with it")
         if reset_mask is not None:
             reset_mask = reset_mask.contiguous()
+        fused = self._whole_step(tokens, alive_mask, recurrent_state, out_state, n_rec, reset_mask, bullets, bullet_mask)
+        if fused is not None:
+            return fused, out_state
         # the list of bullets in flight is built once and shared by every layer that reads them
         bullet_rows = bullet_mask
         if (
@@ -1690,6 +1818,8 @@ class GraphedTrunk:
     the inputs into static buffers, replays one graph and returns the static output and state tensors.
     The packed state lives in two buffers that alternate as input and output, hence two
     graphs.  Outputs are overwritten by the next ``step``; clone what must outlive it.
+    Where the whole step is one kernel (small fleets under bfloat16 autocast) there is nothing to capture: ``step`` launches
+    it on the caller's tensors, copying only what the kernel cannot read as it is.
 
     Weights: the captured kernels read the parameters themselves (norm weights, float32 GEMM operands)
     and the derived copies the layers cache (bfloat16 casts, concatenations, operand packings) at the
@@ -1723,6 +1853,14 @@ class GraphedTrunk:
         self.states = [trunk.initial_hidden(num_envs, num_recurrent, dev) for _ in range(2)]
         self.cur = 0  # index of the buffer holding the current state
         self.graphs, self.outputs = [], []
+        self._sizes = (num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
+        self._shape = _register_shape(trunk, *self._sizes)
+        self._whole = self._whole_step_table()
+        if self._whole is not None:
+            # one launch is all there is: it reads the caller's tensors, and there is nothing to capture
+            self.outputs = [torch.empty_like(self.tokens) for _ in range(2)]
+            self._keep_weights()
+            return
         side = torch.cuda.Stream(device=dev)
         side.wait_stream(torch.cuda.current_stream(dev))
         with torch.cuda.stream(side):
@@ -1739,11 +1877,47 @@ class GraphedTrunk:
             self.outputs.append(out)
         for s in self.states:
             s.zero_()
-        # the derived weights the captured kernels read: held here so their memory outlives any cache
+        self._keep_weights()
+
+    def _keep_weights(self) -> None:
+        # the derived weights the kernels read: held here so their memory outlives any cache
         # invalidation on the module, and rebuilt in place when their sources change
-        self._derived = derived_weights(trunk)
-        self._params = list(trunk.parameters())
+        self._derived = derived_weights(self.trunk)
+        self._params = list(self.trunk.parameters())
         self._stamp = _weights_stamp(self._params)
+
+    def _whole_step_table(self):
+        """``(table, eps of the bullet norm)`` of the step as one kernel, or None where that does not apply."""
+        with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None), torch.no_grad():
+            found = self.trunk._whole_step_layers(*self._sizes, self.tokens.device)
+        return None if found is None else (ops.trunk_table(found[0]), found[1])
+
+    def _step_whole(self, inputs):
+        """The step as one kernel: an input that is as the kernel reads it is read in place, any other is copied first."""
+        if self._follow_weights():
+            # assigning ``.data`` moves a parameter: its address is looked up anew
+            whole = self._whole_step_table()
+            if whole is None:
+                raise RuntimeError("the trunk's layers have changed their form: make a new stepper")
+            self._whole = whole
+            self._derived = derived_weights(self.trunk)
+        table, bullet_eps = self._whole
+        ready = {}
+        for name, held, given in inputs:
+            if given is held or (given is None and name in ("reset", "bullets", "in_flight")):
+                ready[name] = given
+                continue
+            rows = held.dtype == torch.float32 or name == "bullets"
+            if (isinstance(given, torch.Tensor) and given.shape == held.shape and given.device == held.device and given.is_contiguous()
+                    and (given.dtype in (torch.float32, torch.bfloat16) and given.data_ptr() % 16 == 0 if rows else given.dtype in _FLAGS)
+                    and not given.is_neg()):
+                ready[name] = given
+            else:
+                held.copy_(given)
+                ready[name] = held
+        return ops.trunk_step(table, ready["x"], self._sizes[2], ready["alive"], self.states[self.cur], self.states[1 - self.cur],
+                              reset=ready["reset"], bullets=ready["bullets"], in_flight=ready["in_flight"], bullet_eps=bullet_eps,
+                              out=self.outputs[self.cur])
 
     def refresh_weights(self) -> None:
         """Rebuild every derived weight copy the graphs read from the current parameters, in place."""
@@ -1751,13 +1925,15 @@ class GraphedTrunk:
             entry.refresh()
         self._stamp = _weights_stamp(self._params)
 
-    def _follow_weights(self) -> None:
+    def _follow_weights(self) -> bool:
         stamp = _weights_stamp(self._params)
-        if stamp != self._stamp:
-            for entry in self._derived:
-                if entry.key != _cache_key(entry.tensors, entry.dtype):
-                    entry.refresh()
-            self._stamp = stamp
+        if stamp == self._stamp:
+            return False
+        for entry in self._derived:
+            if entry.key != _cache_key(entry.tensors, entry.dtype):
+                entry.refresh()
+        self._stamp = stamp
+        return True
 
     def _run(self, src: int) -> torch.Tensor:
         with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None):
@@ -1788,6 +1964,11 @@ class GraphedTrunk:
             raise ValueError("this capture was made without bullet inputs")
         if self.bullets is not None and bullets is None:
             raise ValueError("this capture reads bullets: pass bullets (and bullet_mask) at every step")
+        if self._whole is not None:
+            out = self._step_whole((("x", self.tokens, tokens), ("alive", self.alive, alive_mask), ("reset", self.reset, reset_mask),
+                                    ("bullets", self.bullets, bullets), ("in_flight", self.bullet_mask, bullet_mask)))
+            self.cur = 1 - self.cur
+            return out, self.states[self.cur]
         inputs = [(self.tokens, tokens), (self.alive, alive_mask)]
         if self.reset is not None:
             inputs.append((self.reset, False if reset_mask is None else reset_mask))
@@ -1817,6 +1998,7 @@ class EagerTrunkStepper:
         if num_bullet_slots and not trunk.config.reads_bullets:
             raise ValueError("this trunk has no bullet-reading sublayer")
         self.reads_bullets = bool(num_bullet_slots)
+        self._shape = _register_shape(trunk, num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
         self.states = [trunk.initial_hidden(num_envs, num_recurrent, dev) for _ in range(2)]
         self.cur = 0
 

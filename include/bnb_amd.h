@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define BNB_ABI_VERSION 31
+#define BNB_ABI_VERSION 32
 
 /* element types of activation buffers */
 #define BNB_F32 0
@@ -945,6 +945,46 @@ int bnb_copy_bytes(const void *src, void *dst, int64_t bytes, void *stream);
  */
 int bnb_issue_probe(int valu_per_mfma, int with_mfma, int with_transcendentals, int waves_per_simd, int iters,
                     float *sink, void *stream);
+
+/*
+ * One timestep of the whole trunk for small fleets (at most 32 tokens an environment) under bfloat16 autocast:
+ * every sublayer of every block (models/yemong/griffin.py:376-417) in one launch, the residual stream in registers.
+ * The weights are the operand streams of the separate entry points, all 16-byte aligned:
+ */
+#define BNB_TRUNK_MAX_LAYERS 24
+typedef struct bnb_trunk_layer {
+    const void *head;          /* attention: qkv (384 features), temporal: [linear1 | linear2 (| field_sub linear1)]; as next_packed of bnb_ffn_fused_proj_next_fwd */
+    const float *norm1;        /* (128) fp32 */
+    const void *kv;            /* attention sublayer that reads bullets: [K | V] projection (256 features, same order) with the bullet
+                                  norm's weight folded into its columns; NULL: none */
+    const void *proj;          /* out_proj / linear_out, as weights_packed of bnb_ffn_fused_proj_fwd's projection */
+    const float *norm2;
+    const void *ffn;           /* as weights_packed of bnb_ffn_fused_fwd */
+    const float *conv_weight;  /* temporal sublayers: (128, 4) fp32 */
+    const float *conv_bias;    /* (128) or NULL */
+    const void *gates;         /* as gate_weight_packed of bnb_temporal_step_fwd */
+    const float *gate_bias;    /* (256) fp32 */
+    const float *log2_sigmoid; /* (128) fp32: log2 sigmoid(log_lambda) */
+    int64_t state_slot;        /* index of this sublayer's rows in the packed state */
+    float eps1, eps2, c;
+    int32_t temporal;
+    int32_t head_blocks;       /* temporal: blocks of 32 features, 12 with the field projection (n_rec < NM), else 8 */
+} bnb_trunk_layer;
+
+/*
+ *   layers     host array of n_layers entries (copied at the call), at most BNB_TRUNK_MAX_LAYERS
+ *   x, out     (B, NM, 128) contiguous, fp32 or bf16 each; the first n_rec tokens of an environment are recurrent
+ *   alive      (B, NM) uint8 or NULL; an environment without a live token attends to all its tokens alike
+ *   reset      (B) uint8 or NULL: environments whose state reads as zero
+ *   bullets    (B, NB, 128) contiguous, fp32 or bf16, or NULL; in_flight (B, NB) uint8 or NULL (all); an environment
+ *              without a bullet in flight reads zero.  (32 / NM) * NB <= 2048
+ *   state_in, state_out  (slots, B * n_rec, 512) fp32 rows [h | p0 | p1 | p2], contiguous, not overlapping
+ * D == 128, H == 4, hidden == 512, 1 <= n_rec <= NM <= 32, else BNB_ERR_UNSUPPORTED.
+ */
+int bnb_trunk_step_fwd(const bnb_trunk_layer *layers, int n_layers, const void *x, int x_dtype, void *out, int out_dtype,
+                       const uint8_t *alive, const uint8_t *reset, const void *bullets, int bullets_dtype,
+                       const uint8_t *in_flight, float bullet_eps, int NB, const float *state_in, float *state_out,
+                       int B, int NM, int n_rec, int D, int H, int hidden, void *stream);
 
 #ifdef __cplusplus
 }

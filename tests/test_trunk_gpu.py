@@ -1794,3 +1794,72 @@ def test_bullet_reading_layers_share_one_projection_pass_over_the_live_bullets(m
     ref2, ref_state2 = torch_ref.trunk_step(p2, 2, 2, 1, H, x, alive, torch.zeros(2, B * N, 4 * D), bullets=bul, bullet_mask=bm)
     assert max_rel(out2.cpu(), ref2) <= BF16_TOL and max_rel(state2.cpu(), ref_state2) <= BF16_TOL
     assert max_rel(ref2, ref_out) > 10 * BF16_TOL  # the update did change the result
+
+
+@pytest.mark.parametrize("B,N,M,K,dtype,blocks,spatial,temporal", [
+    (16, 8, 4, 10, torch.float32, 2, 2, 1),  # two environments a work-group
+    (5, 8, 4, 10, torch.bfloat16, 2, 2, 1),  # the last work-group half empty
+    (3, 1, 0, 3, torch.float32, 2, 2, 1),  # 32 environments a work-group, three there; one token an environment
+    (70, 1, 1, 0, torch.float32, 1, 1, 2),  # no bullets; the first token recurrent, the other not
+    (2, 28, 4, 10, torch.float32, 1, 1, 1),  # a full tile
+    (300, 15, 2, 4, torch.bfloat16, 1, 2, 1),  # 17 of 32 rows, more than one round
+    (2, 32, 0, 64, torch.float32, 2, 1, 1),  # 2048 slots: bullets in several pieces
+    (4, 16, 0, 11, torch.float32, 3, 0, 1),  # recurrent sublayers only
+    (4, 13, 3, 11, torch.float32, 2, 1, 0),  # attention sublayers only
+])
+def test_small_fleets_step_as_one_kernel_matches_the_oracle(B, N, M, K, dtype, blocks, spatial, temporal):
+    D, H = 128, 4
+    gen = torch.Generator().manual_seed(B * 100 + N)
+    p = trunk_params(7 * B + N, D, blocks, spatial, temporal)
+    reads = K > 0 and spatial > 0
+    for i in range(blocks):
+        for j in range(temporal):
+            p[f"yemong_layers.{i}.field_sub.{j}.weight"] = torch.eye(D) + 0.05 * torch.randn(D, D, generator=gen)
+        if reads:
+            p[f"yemong_layers.{i}.spatial.0.norm_bullet.weight"] = 1.0 + 0.1 * torch.randn(D, generator=gen)
+            p[f"yemong_layers.{i}.spatial.0.kv_bullet.weight"] = 0.1 * torch.randn(2 * D, D, generator=gen)
+    trunk = bnb.YemongTrunk(_cfg(D, H, blocks, spatial, temporal, bullets=int(reads))).eval()
+    trunk.load_state_dict(p)
+    trunk.to(DEV)
+    slots = N * K if reads else None
+    stepper = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, num_bullet_slots=slots, bullet_dtype=dtype)
+    assert stepper._whole is not None
+    L = blocks * temporal
+    hidden = 0.5 * torch.randn(L, B * N, 4 * D, generator=gen)
+    stepper.load_state(hidden.to(DEV))
+    for t in range(2):
+        x = torch.randn(B, N + M, D, generator=gen).to(dtype)
+        alive = torch.rand(B, N + M, generator=gen) < 0.6
+        alive[0] = False  # nobody alive: everyone with the same weight
+        reset = torch.rand(B, generator=gen) < 0.3
+        bul = mask = None
+        if reads:
+            bul = torch.randn(B, slots, D, generator=gen).to(dtype)
+            mask = torch.rand(B, slots, generator=gen) < (0.9 if K > 32 else 0.3)
+            mask[-1] = False
+        dev = [None if v is None else v.to(DEV) for v in (x, alive, reset, bul, mask)]
+        out, state = stepper.step(*dev)
+        kw = {"bullets": bul.float(), "bullet_mask": mask} if reads else {}
+        ref_out, hidden = torch_ref.trunk_step(p, blocks, spatial, temporal, H, x.float(), alive, torch_ref.reset_hidden(hidden, reset, N), **kw)
+        assert out.dtype == torch.float32 and max_rel(out.cpu(), ref_out) <= BF16_TOL, t
+        if L:
+            assert max_rel(state.cpu(), hidden) <= BF16_TOL, t
+            hidden = state.cpu()
+
+    # what a diverged environment holds stays its own: its neighbours in the tile get the same bits
+    if B > 1:
+        stepper.load_state(hidden.to(DEV))
+        clean = [v.clone() for v in stepper.step(*dev)]
+        sick = [None if v is None else v.clone() for v in dev]
+        sick[0][1, 0] = float("nan")
+        sick[1][1, 0] = True
+        if reads:
+            sick[3][1, 0, 5] = float("inf")
+            sick[4][1, 0] = True
+        stepper.load_state(hidden.to(DEV))
+        out, state = stepper.step(*sick)
+        others = [e for e in range(B) if e != 1]
+        assert torch.isnan(out[1]).any()
+        assert torch.equal(out[others], clean[0][others])
+        if L:
+            assert torch.equal(state.view(L, B, -1)[:, others], clean[1].view(L, B, -1)[:, others])

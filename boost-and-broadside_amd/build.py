@@ -42,7 +42,8 @@ EXTRA_FLAGS = {
     "ffn_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "linear_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ffn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
-    "trunk_step.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    # (here also an exact register count while scheduling: nothing may spill, a reload would wait for every operand under way)
+    "trunk_step.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-use-amdgpu-trackers=1"],
 }
 
 

@@ -2823,16 +2823,19 @@ def trunk_step_supported(B: int, NM: int, n_rec: int, D: int, n_heads: int, n_la
             and B > 0 and (TRUNK_TOKENS // NM) * slots <= _TRUNK_SLOTS)
 
 
-def trunk_step_pays(B: int, NM: int, device) -> bool:
+def trunk_step_pays(B: int, NM: int, reads: bool, device) -> bool:
     """Whether the whole step as one kernel is faster than the separate kernels.
 
-    One round of work-groups over the chip (32 rows each, whole environments) takes about 64 us with the default trunk, the
-    separate kernels about 100 us and 9 us for every thousand rows.  us, one kernel / separate: 16 environments of 12 tokens
-    65 / 121, 512 of 8 70 / 146, 1024 of 12 (2 rounds) 133 / 233, 512 of 23 (2) 136 / 243, 1280 of 23 (5) 313 / 375, 3072 of 12
-    (6) 387 / 458, 6144 of 8 (6) 444 / 571, 7808 of 12 (16) 1000 / 882."""
+    Up to one work-group of 32 rows (whole environments) a CU it takes about 65 us with the default trunk, behind that 15 us and
+    0.2 us a work-group of 256 CUs; the separate kernels about 95 us and 8.2 us for every thousand rows.  Without bullets 0.175 us
+    and 6.4 us.  us, one kernel / separate: 16 environments of 12 tokens 64 / 121,
+    512 of 8 71 / 146, 1024 of 12 (512 work-groups) 112 / 232, 1024 of 23 (1024) 214 / 343, 4096 of 12 (2048) 428 / 515, 7808 of 12
+    (3904) 798 / 880, 4096 of 23 (4096) 849 / 919, 8192 of 20 (8192, 20 of 32 rows filled) 1525 / 1347; without bullets 4955 of 9 (1652)
+    319 / 490, 5579 of 11 (2790) 499 / 490."""
     groups = -(-B // (TRUNK_TOKENS // NM))
-    rounds = -(-groups // torch.cuda.get_device_properties(device).multi_processor_count)
-    return rounds == 1 or 64 * rounds <= 100 + 0.009 * B * NM
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    a_group, a_row = (0.2, 0.0082) if reads else (0.175, 0.0064)
+    return groups <= cus or 15 + a_group * groups * 256 / cus <= 95 + a_row * B * NM
 
 
 def trunk_table(layers):

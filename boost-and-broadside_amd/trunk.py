@@ -1489,6 +1489,27 @@ class _LiveRows:
         self.rows, self.chained = rows, chained
 
 
+class _LayoutWatch:
+    """Whether a module still consists of the same submodules and parameters, unwritten, without forward hooks and with its
+    derived weights valid (``invalidate_weight_caches``).  Keeps those weights alive."""
+
+    def __init__(self, module: nn.Module) -> None:
+        self.children = [(m._modules, name, child) for m in module.modules() for name, child in m._modules.items()]
+        self.params = [(m._parameters, name, p) for m in module.modules() for name, p in m._parameters.items()]
+        self.derived = [(m.__dict__, k, v) for m in module.modules() for k, v in m.__dict__.items()
+                        if k.startswith(_CACHE_PREFIX) and isinstance(v, _DerivedWeight)]
+        self.stamp = self._stamp()
+
+    def _stamp(self) -> int:
+        return _weights_stamp([p for _, _, p in self.params if p is not None])
+
+    def same(self) -> bool:
+        return (all(d.get(name) is child and not child._forward_hooks and not child._forward_pre_hooks for d, name, child in self.children)
+                and all(d.get(name) is p for d, name, p in self.params)
+                and all(d.get(slot) is entry and entry.key is not None for d, slot, entry in self.derived)
+                and self._stamp() == self.stamp)
+
+
 class _SteppedShape:
     """Held by every stepper of one shape over one trunk."""
 
@@ -1615,7 +1636,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
         if not (
             _HEAD_FUSION and device.type == "cuda" and _projection_dtype() == torch.bfloat16
             and ops.trunk_step_supported(B, NM, n_rec, self.config.d_model, self.config.n_heads, n_layers, slots if readers else 0)
-            and ops.trunk_step_pays(B, NM, device)
+            and ops.trunk_step_pays(B, NM, bool(readers), device)
         ):
             return None
 
@@ -1675,11 +1696,12 @@ class YemongTrunk(_WeightCaches, nn.Module):
                 table.append(entry)
         return table, (eps(readers[0].norm_bullet) if readers else 0.0)
 
-    def _whole_step(self, x, alive, state_in, state_out, n_rec, reset, bullets, in_flight):
+    def _whole_step(self, x, alive, state_in, state_out, n_rec, reset, bullets, in_flight, laid_out=None):
         """The step as one kernel where a stepper for this shape exists and that applies, else None.
 
         A direct call lays the kernel's table out anew each time, so it is left to shapes that a program is known to step again
-        and again: those of the steppers alive, whose results a direct call then also repeats bit for bit."""
+        and again: those of the steppers alive, whose results a direct call then also repeats bit for bit.  ``laid_out``: a
+        stepper's own table, ``(ops.trunk_table, eps of the bullet norm)``."""
         B, NM, D = x.shape
         slots = bullets.shape[1] if bullets is not None and self.config.reads_bullets and bullets.dim() == 3 else 0
         if (B, NM, n_rec, slots) not in _stepped_shapes(self):
@@ -1698,12 +1720,14 @@ class YemongTrunk(_WeightCaches, nn.Module):
                 and all(t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (state_in, state_out))
                 and (not slots or (given(bullets, (B, slots, D), rows) and given(in_flight, (B, slots), flags)))):
             return None
-        found = self._whole_step_layers(B, NM, n_rec, slots, x.device)
-        if found is None:
-            return None
-        return ops.trunk_step(ops.trunk_table(found[0]), whole(x), n_rec, whole(alive), state_in, state_out, reset=whole(reset),
+        if laid_out is None:
+            found = self._whole_step_layers(B, NM, n_rec, slots, x.device)
+            if found is None:
+                return None
+            laid_out = (ops.trunk_table(found[0]), found[1])
+        return ops.trunk_step(laid_out[0], whole(x), n_rec, whole(alive), state_in, state_out, reset=whole(reset),
                               bullets=whole(bullets) if slots else None, in_flight=whole(in_flight) if slots else None,
-                              bullet_eps=found[1], out_dtype=x.dtype)
+                              bullet_eps=laid_out[1], out_dtype=x.dtype)
 
     def _bullet_kv_of_all_layers(self, bullets, rows):
         """``{id(layer): [K | V] rows}`` of every bullet-reading sublayer of the step from ONE pass over the bullets in
@@ -1998,7 +2022,9 @@ class EagerTrunkStepper:
         if num_bullet_slots and not trunk.config.reads_bullets:
             raise ValueError("this trunk has no bullet-reading sublayer")
         self.reads_bullets = bool(num_bullet_slots)
-        self._shape = _register_shape(trunk, num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
+        self._sizes = (num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
+        self._shape = _register_shape(trunk, *self._sizes)
+        self._whole = self._whole_watch = None
         self.states = [trunk.initial_hidden(num_envs, num_recurrent, dev) for _ in range(2)]
         self.cur = 0
 
@@ -2019,10 +2045,28 @@ class EagerTrunkStepper:
         if not self.reads_bullets and bullets is not None:
             raise ValueError("this stepper was made without bullet inputs")
         with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None):
-            out, new_state = self.trunk(tokens, alive_mask, self.states[self.cur], bullets, bullet_mask,
-                                        reset_mask=reset_mask, out_state=self.states[1 - self.cur])
+            out = self._step_whole(tokens, alive_mask, reset_mask, bullets, bullet_mask)
+            if out is None:
+                out, _ = self.trunk(tokens, alive_mask, self.states[self.cur], bullets, bullet_mask,
+                                    reset_mask=reset_mask, out_state=self.states[1 - self.cur])
         self.cur = 1 - self.cur
-        return out, new_state
+        return out, self.states[self.cur]
+
+    def _step_whole(self, tokens, alive_mask, reset_mask, bullets, bullet_mask):
+        """The step as one kernel where that applies, with its table kept while the trunk stays as it is; else None."""
+        dev = self.states[0].device
+        if self.autocast_dtype != torch.bfloat16 or not _HEAD_FUSION or self._sizes[1] > ops.TRUNK_TOKENS:
+            return None
+        if self._whole is None or not self._whole_watch.same():
+            found = self.trunk._whole_step_layers(*self._sizes, dev)
+            self._whole = None
+            if found is None:
+                return None
+            self._whole, self._whole_watch = (ops.trunk_table(found[0]), found[1]), _LayoutWatch(self.trunk)
+        if tuple(tokens.shape[:2]) != self._sizes[:2]:
+            return None
+        return self.trunk._whole_step(tokens, alive_mask, self.states[self.cur], self.states[1 - self.cur], self._sizes[2], reset_mask,
+                                      bullets, bullet_mask, laid_out=self._whole)
 
 
 # tokens per step below which a captured step beats plain launches, with the default trunk of 2 blocks x (2 attention +

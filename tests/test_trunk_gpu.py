@@ -1802,7 +1802,9 @@ def test_bullet_reading_layers_share_one_projection_pass_over_the_live_bullets(m
     (3, 1, 0, 3, torch.float32, 2, 2, 1),  # 32 environments a work-group, three there; one token an environment
     (70, 1, 1, 0, torch.float32, 1, 1, 2),  # no bullets; the first token recurrent, the other not
     (2, 28, 4, 10, torch.float32, 1, 1, 1),  # a full tile
-    (300, 15, 2, 4, torch.bfloat16, 1, 2, 1),  # 17 of 32 rows, more than one round
+    (300, 15, 2, 4, torch.bfloat16, 1, 2, 1),  # 17 of 32 rows, more work-groups than CUs
+    (601, 8, 4, 10, torch.float32, 1, 2, 1),  # more work-groups than CUs, two environments each, the last with one
+    (260, 32, 0, 10, torch.bfloat16, 2, 1, 1),  # more work-groups than CUs, bullets in several pieces
     (2, 32, 0, 64, torch.float32, 2, 1, 1),  # 2048 slots: bullets in several pieces
     (4, 16, 0, 11, torch.float32, 3, 0, 1),  # recurrent sublayers only
     (4, 13, 3, 11, torch.float32, 2, 1, 0),  # attention sublayers only
@@ -1863,3 +1865,46 @@ def test_small_fleets_step_as_one_kernel_matches_the_oracle(B, N, M, K, dtype, b
         assert torch.equal(out[others], clean[0][others])
         if L:
             assert torch.equal(state.view(L, B, -1)[:, others], clean[1].view(L, B, -1)[:, others])
+
+
+def test_whole_step_of_an_uncaptured_stepper_follows_weights_hooks_and_invalidated_caches():
+    D, H, B, N, M = 128, 4, 6, 8, 4
+    trunk, _ = _rollout_trunk(161)
+    stepper = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, graph=False)
+    gen = torch.Generator().manual_seed(162)
+    x = torch.randn(B, N + M, D, generator=gen).to(DEV)
+    alive = torch.ones(B, N + M, dtype=torch.bool, device=DEV)
+    state = torch.randn(stepper.state.shape, generator=gen).to(DEV)
+
+    def step():
+        stepper.load_state(state)
+        out = stepper.step(x, alive)[0].clone()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert torch.equal(out, trunk(x, alive, state)[0])
+        return out
+
+    seen = [step()]
+    assert stepper._whole is not None
+    layer = trunk.yemong_layers[0].spatial[0]
+    with torch.no_grad():
+        layer.qkv.weight.mul_(1.5)  # a version counter
+    seen.append(step())
+    layer.norm2.weight.data = 1.5 * layer.norm2.weight.detach()  # another address
+    seen.append(step())
+    layer.out_proj.weight = torch.nn.Parameter(2.0 * layer.out_proj.weight.detach())  # another parameter
+    seen.append(step())
+    alias = layer.ffn.up_proj.weight.detach()
+    step()
+    torch._C.TensorBase.data.__get__(layer.ffn.up_proj.weight).mul_(0.5)  # a write that nothing counts
+    trunk.invalidate_weight_caches()
+    seen.append(step())
+    del alias
+    for a, b in zip(seen, seen[1:]):
+        assert not torch.equal(a, b)
+    calls = []
+    handle = layer.register_forward_hook(lambda *a: calls.append(1))
+    step()
+    assert calls and stepper._whole is None
+    handle.remove()
+    step()
+    assert stepper._whole is not None

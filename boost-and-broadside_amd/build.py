@@ -16,7 +16,7 @@ INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_DIR = os.path.join(PKG_DIR, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libbnb_amd.so")
 SOURCES = ("abi.hip", "conv_step.hip", "elementwise.hip", "ffn_bwd.hip", "ffn_fused.hip", "ffn_small.hip", "linear_split.hip", "linear_wgrad.hip",
-    "norm_train.hip", "norm_linear.hip", "probe.hip", "rglru_step.hip", "sdpa_bwd.hip", "sdpa_cross_bwd.hip", "sdpa_cross_f32.hip", "sdpa_env.hip", "sdpa_masked.hip", "team_pool.hip", "temporal_seq.hip", "temporal_step.hip",
+    "norm_train.hip", "norm_linear.hip", "probe.hip", "rglru_step.hip", "sdpa_bwd.hip", "sdpa_cross_bwd.hip", "sdpa_cross_f32.hip", "sdpa_env.hip", "sdpa_masked.hip", "tail_split.hip", "team_pool.hip", "temporal_seq.hip", "temporal_step.hip",
     "trunk_step.hip")
 
 HIPCC_FLAGS = [
@@ -42,6 +42,7 @@ EXTRA_FLAGS = {
     "ffn_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "linear_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ffn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "tail_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # (here also an exact register count while scheduling: nothing may spill, a reload would wait for every operand under way)
     "trunk_step.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-use-amdgpu-trackers=1"],
 }

@@ -33,6 +33,7 @@
 #include "common.h"
 #include "ffn_math.h"
 #include "rglru_math.h"
+#include "tile_rows.h"
 
 namespace bnb {
 
@@ -79,23 +80,6 @@ struct TrunkStepArgs {
     const float *state_in;
     float *state_out;
 };
-
-// Waits for this wave's LDS traffic only: operands requested from memory stay on their way across the barrier.
-__device__ __forceinline__ void tk_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v)
-{
-    return v + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, false));
-}
-// Sum over the 16 lanes of a row, in all of them.
-__device__ __forceinline__ float sum16(float v)
-{
-    v = dpp_add<0x128>(v);  // row_ror:8, 4, 2, 1
-    v = dpp_add<0x124>(v);
-    v = dpp_add<0x122>(v);
-    return dpp_add<0x121>(v);
-}
 
 __device__ __forceinline__ bf16x8 lds_operand(const uint16_t *p) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(p)); }
 __device__ __forceinline__ bf16x8 mem_operand(const uint16_t *p) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(p)); }
@@ -250,7 +234,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
     int total = 0;
     if (slots > 0) {
         if (tid <= here) s.off[tid] = 0;
-        tk_barrier();
+        lds_barrier();
 #pragma unroll 1
         for (int p0 = 0; p0 < slots; p0 += THREADS) {
             const int p = p0 + tid;
@@ -260,7 +244,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
             if (lane == 0) s.count[wave] = (int)__popcll(vote);
             if (set)
                 for (int e = p / a.NB + 1; e <= here; ++e) atomicAdd(&s.off[e], 1);
-            tk_barrier();
+            lds_barrier();
             int before = 0, all = 0;
 #pragma unroll
             for (int w = 0; w < WAVES; ++w) {
@@ -270,7 +254,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
             }
             if (set) s.list[total + before + (int)__popcll(vote & ((1ull << lane) - 1ull))] = (uint16_t)p;
             total += all;
-            tk_barrier();
+            lds_barrier();
         }
         total = __builtin_amdgcn_readfirstlane(total);
     }
@@ -365,7 +349,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
                 first_q(f), first_kv(f);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            tk_barrier();
+            lds_barrier();
         };
 
         if (!temporal) {
@@ -478,9 +462,9 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
                     }
                 }
                 if (!read || seg + 1 >= segments || (!SPLIT && self)) break;
-                tk_barrier();
+                lds_barrier();
                 stage_bullets(seg + 1);
-                tk_barrier();
+                lds_barrier();
             }
             // merged heads (SPLIT: and the read behind them) as operand rows of the projection
             const float inv = sum == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(sum);
@@ -578,7 +562,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
                 return r < rows && r % NM < n_rec;
             };
             auto state_at = [&](int rp) { return state_row(row + PASS * rp) * (4 * kTkD) + c4; };
-            tk_barrier();
+            lds_barrier();
 
             // ---- conv taps and buffer shift ----
             float v[RP][8];
@@ -616,7 +600,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
                 __builtin_amdgcn_sched_barrier(0);
                 gate_operands();  // here there are registers for them
             }
-            tk_barrier();
+            lds_barrier();
 
             // ---- gate pre-activations ----
             uint16_t *const s_g = reinterpret_cast<uint16_t *>(s.part);
@@ -633,7 +617,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
                 *reinterpret_cast<bf16x8 *>(p) = t[0];
                 *reinterpret_cast<bf16x8 *>(p + 8) = t[1];
             }
-            tk_barrier();
+            lds_barrier();
 
             // ---- recurrence, and gelu(gate) * y as operand rows of the projection ----
             __builtin_amdgcn_sched_barrier(0);
@@ -674,7 +658,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
         wn[1] = *reinterpret_cast<const f32x4 *>(L.norm2 + 64 + c4);
         hidden_operands(0);
         __builtin_amdgcn_sched_barrier(0);
-        tk_barrier();
+        lds_barrier();
         {
             f32x16 z = {0.0f};
             const uint16_t *p = proj_rows + m * kTkPitch + 64 * kh + 8 * half;
@@ -686,10 +670,10 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
             }
             store_part(z);
         }
-        tk_barrier();
+        lds_barrier();
         add_parts();
         norm_rows(L.eps2);
-        tk_barrier();
+        lds_barrier();
 
         // ---- gate / up: the wave's chunks of 32 hidden units; down: a channel block (SPLIT: over half of the hidden units) ----
         const uint16_t *wdp = (const uint16_t *)L.ffn + (int64_t)(8 * kh) * kTkChunkHalfs + 8192 + cb * 1024;
@@ -731,7 +715,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
             *reinterpret_cast<bf16x8 *>(p) = t[0];
             *reinterpret_cast<bf16x8 *>(p + 16) = t[1];
         }
-        tk_barrier();
+        lds_barrier();
         {
             f32x16 z = {0.0f};
             const uint16_t *p = s.h + m * kTkHiddenPitch + 256 * kh + 8 * half;
@@ -748,7 +732,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
             }
             store_part(z);
         }
-        tk_barrier();
+        lds_barrier();
     }
 
     mappings();

@@ -2480,6 +2480,73 @@ def linear_f32(x: torch.Tensor, weight_packed: torch.Tensor, *, bias: torch.Tens
     return out
 
 
+def tail_f32_supported(x: torch.Tensor, rows: torch.Tensor) -> bool:
+    """Whether ``tail_f32`` covers these rows: float32 (..., 128) on the GPU, both of one shape."""
+    return (x.is_cuda and x.dtype == torch.float32 and x.shape[-1] == FFN_WIDTH and rows.dtype == torch.float32
+            and rows.shape == x.shape and rows.device == x.device)
+
+
+def tail_f32(x: torch.Tensor, rows: torch.Tensor, proj_packed: torch.Tensor, norm_weight: torch.Tensor, gate_up_packed: torch.Tensor,
+             down_packed: torch.Tensor, *, eps: float | None = None, gelu_times: torch.Tensor | None = None, next_head: tuple | None = None):
+    """The tail of a sublayer in float32 as one kernel: ``s = x + A Wp^T`` with ``A = rows`` or ``gelu(rows) * gelu_times``, then
+    ``s + down(gelu(gate(n)) * up(n))`` with ``n = rmsnorm(s) * norm_weight``.  Weights from ``pack_linear_f32``: (128, 128),
+    the (gate, up) pair of (512, 128) and (128, 512).
+
+    ``next_head = (norm weight, eps, (packed, ...))``, one or two ``pack_linear_f32`` streams of K = 128: the launch goes on to the
+    next sublayer's norm and projections, and the call returns ``(out, (projection, ...))``."""
+    D = FFN_WIDTH
+    if not tail_f32_supported(x, rows) or (gelu_times is not None and not tail_f32_supported(x, gelu_times)):
+        raise RuntimeError("tail_f32 covers float32 (..., 128) rows on the GPU")
+    if torch.is_grad_enabled() and (x.requires_grad or rows.requires_grad):
+        raise RuntimeError("tail_f32 is forward-only; call it under torch.no_grad()")
+    streams = [(proj_packed, (4, 1, 8, 3, 64, 8)), (gate_up_packed, (32, 1, 8, 3, 64, 8)), (down_packed, (4, 4, 8, 3, 64, 8))]
+    norms = [norm_weight]
+    heads = ()
+    if next_head is not None:
+        norms.append(next_head[0])
+        heads = next_head[2]
+        if len(heads) not in (1, 2):
+            raise ValueError("next_head takes one or two projections")
+        streams += [(w, (w.shape[0], 1, 8, 3, 64, 8)) for w in heads]
+    for w, shape in streams:
+        if w.dtype != torch.bfloat16 or tuple(w.shape) != shape or not w.is_contiguous() or w.device != x.device:
+            raise ValueError(f"expected a contiguous pack_linear_f32 stream of shape {shape}, got {tuple(w.shape)} {w.dtype}")
+    for w in norms:
+        if w.shape != (D,) or w.dtype != torch.float32:
+            raise ValueError("norm weights must be float32 (128,)")
+
+    def flat(t):
+        t = t.reshape(-1, D) if _uniform_rows(t, D) else t.reshape(-1, D).contiguous()
+        return t if t.data_ptr() % 16 == 0 and (t.shape[0] < 2 or t.stride(0) % 4 == 0) else t.clone(memory_format=torch.contiguous_format)
+
+    x2, a2 = flat(x), flat(rows)
+    y2 = None if gelu_times is None else flat(gelu_times)
+    R = x2.shape[0]
+    out = torch.empty((R, D), dtype=torch.float32, device=x.device)
+    made = tuple(torch.empty((R, 32 * w.shape[0]), dtype=torch.float32, device=x.device) for w in heads)
+    norms = [w.detach().contiguous() for w in norms]
+    if R:
+        def pitch(t):
+            return 0 if t is None else t.stride(0) if R > 1 else D
+
+        def ptr(t):
+            return None if t is None else t.data_ptr()
+
+        h1, h2 = (heads + (None, None))[:2]
+        o1, o2 = (made + (None, None))[:2]
+        with _on_device(x.device):
+            rc = _native.load().bnb_tail_f32_fwd(
+                x2.data_ptr(), pitch(x2), a2.data_ptr(), pitch(a2), ptr(y2), pitch(y2), proj_packed.data_ptr(), norms[0].data_ptr(),
+                float(_F32_EPS if eps is None else eps), gate_up_packed.data_ptr(), down_packed.data_ptr(), out.data_ptr(),
+                norms[1].data_ptr() if heads else None, float(_F32_EPS if not heads or next_head[1] is None else next_head[1]), ptr(h1), ptr(o1),
+                0 if h1 is None else 32 * h1.shape[0], ptr(h2), ptr(o2), 0 if h2 is None else 32 * h2.shape[0], R, D, FFN_HIDDEN, _stream())
+        _native.check(rc, "bnb_tail_f32_fwd")
+    out = out.reshape(x.shape)
+    if next_head is None:
+        return out
+    return out, tuple(o.reshape(*x.shape[:-1], o.shape[1]) for o in made)
+
+
 def pack_linear_weights(weight: torch.Tensor) -> torch.Tensor:
     """A Linear weight (N, 128), N a multiple of 64, as the bfloat16 operand stream of
     ``norm_linear``: ``[fb][ks][l][e]`` with the index meaning given in ``include/bnb_amd.h``

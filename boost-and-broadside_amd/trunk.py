@@ -447,6 +447,16 @@ class ModelConfig:
             )
 
 
+@dataclass(frozen=True)
+class _HeadF32:
+    """What a sublayer starts with in float32, for the tail kernel of the one before: its norm and the operand streams of its
+    projections (``ops.tail_f32(next_head=...)``)."""
+
+    norm: torch.Tensor
+    eps: float | None
+    streams: tuple
+
+
 class GatedMLP(_WeightCaches, nn.Module):
     """``down_proj(gelu(gate_proj(x)) * up_proj(x))`` with a 4x hidden width by default."""
 
@@ -518,13 +528,30 @@ class GatedMLP(_WeightCaches, nn.Module):
     def tail_f32(self, x1: torch.Tensor, norm: nn.RMSNorm) -> torch.Tensor | None:
         """``x1 + self(norm(x1))`` in float32 as two kernels (norm + gate/up + gelu gate; down + residual), or None
         when that does not apply (other widths, biases)."""
-        if (self.gate_proj.bias is not None or self.up_proj.bias is not None or self.down_proj.bias is not None
-                or self.gate_proj.out_features % 128 or norm.weight is None
-                or not _f32_fused_ok(x1, torch.float32, self.gate_proj, self.up_proj, self.down_proj)):
+        if not self._f32_tail_ok(x1, norm):
             return None
         gu = _packed_f32(self, "_bnb_f32_gate_up", self.gate_proj.weight, self.up_proj.weight)
         hid = ops.linear_f32(x1, gu, norm_weight=norm.weight, eps=norm.eps, gate=True)
         return ops.linear_f32(hid, _packed_f32(self.down_proj, "_bnb_f32_pack", self.down_proj.weight), resid=x1)
+
+    def _f32_tail_ok(self, x: torch.Tensor, norm: nn.RMSNorm) -> bool:
+        return (self.gate_proj.bias is None and self.up_proj.bias is None and self.down_proj.bias is None
+                and self.gate_proj.out_features % 128 == 0 and norm.weight is not None
+                and _f32_fused_ok(x, torch.float32, self.gate_proj, self.up_proj, self.down_proj))
+
+    def sublayer_tail_f32(self, x, rows, proj_layer: nn.Linear, norm: nn.RMSNorm, *, gelu_times=None, next_head=None):
+        """``s = x + proj_layer(rows)`` (``rows``, or ``gelu(rows) * gelu_times``), then ``s + self(norm(s))`` in float32 as one kernel
+        (hidden width 512), with ``next_head`` (a ``_HeadF32``) the next sublayer's norm and projections too: ``out`` or the pair
+        ``(out, that head)``.  None when that does not apply."""
+        w = proj_layer.weight
+        if (proj_layer.bias is None and tuple(w.shape) == (ops.FFN_WIDTH, ops.FFN_WIDTH) and norm.weight is not None
+                and norm.weight.dtype == torch.float32 and self.gate_proj.out_features == ops.FFN_HIDDEN and self._f32_tail_ok(x, norm)
+                and w.dtype == torch.float32 and ops.tail_f32_supported(x, rows) and (gelu_times is None or ops.tail_f32_supported(x, gelu_times))):
+            return ops.tail_f32(x, rows, _packed_f32(proj_layer, "_bnb_f32_pack", w), norm.weight,
+                                _packed_f32(self, "_bnb_f32_gate_up", self.gate_proj.weight, self.up_proj.weight),
+                                _packed_f32(self.down_proj, "_bnb_f32_pack", self.down_proj.weight), eps=norm.eps, gelu_times=gelu_times,
+                                next_head=None if next_head is None else (next_head.norm, next_head.eps, next_head.streams))
+        return None
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         hidden = self.gate_proj.out_features
@@ -571,7 +598,9 @@ class TransformerBlock(_WeightCaches, nn.Module):
     def head_spec(self, x: torch.Tensor):
         """``(norm weight, eps, packed weight, features)`` of this sublayer's head ``qkv(norm1(x))`` for the tail
         kernel of the sublayer before (``ops.ffn_fused(next_head=...)``), or None when this sublayer would not take
-        the bfloat16 kernel path for rows like ``x``."""
+        the bfloat16 kernel path for rows like ``x``.  In float32 a ``_HeadF32``."""
+        if _HEAD_FUSION and self._f32_ok(x, _projection_dtype()) and self.norm1.weight.dtype == torch.float32:
+            return _HeadF32(self.norm1.weight, self.norm1.eps, (_packed_f32(self.qkv, "_bnb_f32_pack", self.qkv.weight),))
         if not (_HEAD_FUSION and not torch.is_grad_enabled() and _projection_dtype() == torch.bfloat16 and x.is_cuda
                 and x.dtype == torch.float32 and self.d_model == ops.FFN_WIDTH and self.qkv.bias is None
                 and self.norm1.weight is not None and self.norm1.weight.dtype == torch.float32):
@@ -579,6 +608,10 @@ class TransformerBlock(_WeightCaches, nn.Module):
         w = self.qkv.weight
         hp = _cached_cast(self.qkv, "_bnb_head_pack", (w,), torch.bfloat16, lambda: ops.pack_head_weights(w))
         return (self.norm1.weight, self.norm1.eps, hp, 3 * self.d_model)
+
+    def _f32_ok(self, x, act) -> bool:
+        return (_f32_fused_ok(x, act, self.qkv, self.out_proj) and self.qkv.bias is None and self.out_proj.bias is None
+                and self.norm1.weight is not None)
 
     def forward(self, x, alive_mask=None, bullets=None, bullet_mask=None, *, head=None, next_head=None):
         """``head``: this sublayer's ``qkv(norm1(x))`` when the sublayer before has already formed it;
@@ -631,13 +664,18 @@ class TransformerBlock(_WeightCaches, nn.Module):
                 attn = _project(self.out_proj, merged)
             else:
                 attn = self._attn(None, alive_mask, bullets, bullet_mask, qkv=qkv)
-        elif (_f32_fused_ok(x, act, self.qkv, self.out_proj) and self.qkv.bias is None and self.out_proj.bias is None
-              and self.norm1.weight is not None):
-            # float32 (evaluation without autocast): every Linear as one kernel (operands in bf16 pieces) with its norm, gate and
-            # residual folded in: norm1 + qkv, attention, out_proj + residual, norm2 + gate/up + gelu gate, down + residual
-            qkv = ops.linear_f32(x, _packed_f32(self.qkv, "_bnb_f32_pack", self.qkv.weight), norm_weight=self.norm1.weight,
-                                 eps=self.norm1.eps)
+        elif self._f32_ok(x, act):
+            # float32 (evaluation without autocast), operands in bf16 pieces: norm1 + qkv, attention, and one kernel for everything
+            # from out_proj on, the next sublayer's norm1 + projections included
+            if head is not None:
+                qkv, = head  # formed by the tail kernel of the sublayer before
+            else:
+                qkv = ops.linear_f32(x, _packed_f32(self.qkv, "_bnb_f32_pack", self.qkv.weight), norm_weight=self.norm1.weight,
+                                     eps=self.norm1.eps)
             merged = self._attn(None, alive_mask, bullets, bullet_mask, qkv=qkv, project=False)
+            tail = self.ffn.sublayer_tail_f32(x, merged, self.out_proj, self.norm2, next_head=next_head)
+            if tail is not None:
+                return tail
             x1 = ops.linear_f32(merged, _packed_f32(self.out_proj, "_bnb_f32_pack", self.out_proj.weight), resid=x)
             tail = self.ffn.tail_f32(x1, self.norm2)
             if tail is not None:
@@ -1011,7 +1049,10 @@ class GriffinTemporalBlock(_WeightCaches, nn.Module):
             gate_in = _project(self.linear2, normed)
         if (_f32_fused_ok(x, act, self.linear_out) and self.linear_out.bias is None and gate_in.dtype == torch.float32
                 and y.dtype == torch.float32 and y.shape == gate_in.shape):
-            # float32: gelu(linear2) * y, linear_out and the residual in one kernel, then the gated MLP's two
+            # float32: gelu(linear2) * y, linear_out, the residual and the gated MLP in one kernel
+            tail = self.gated_mlp.sublayer_tail_f32(x, gate_in, self.linear_out, self.norm2, gelu_times=y, next_head=next_head)
+            if tail is not None:
+                return tail
             x1 = ops.linear_f32(gate_in, _packed_f32(self.linear_out, "_bnb_f32_pack", self.linear_out.weight), gelu_times=y,
                                 resid=x)
             tail = self.gated_mlp.tail_f32(x1, self.norm2)
@@ -1089,7 +1130,9 @@ class GriffinTemporalBlock(_WeightCaches, nn.Module):
     def head_spec(self, x: torch.Tensor, n_rec: int, field_sub):
         """``(norm weight, eps, packed weight, features)`` of this sublayer's head as ``step_tokens`` forms it, for the
         tail kernel of the sublayer before (``ops.ffn_fused(next_head=...)``), or None when ``step_tokens`` would not
-        take the bfloat16 kernel path for tokens like ``x`` (B, NM, D)."""
+        take the bfloat16 kernel path for tokens like ``x`` (B, NM, D).  In float32 a ``_HeadF32``."""
+        if _HEAD_FUSION and self._f32_ok(x, _projection_dtype()) and self.norm1.weight.dtype == torch.float32:
+            return _HeadF32(self.norm1.weight, self.norm1.eps, self._f32_streams(x.shape[1] > n_rec, field_sub))
         if not (_HEAD_FUSION and not torch.is_grad_enabled() and _projection_dtype() == torch.bfloat16 and x.is_cuda
                 and x.dtype == torch.float32 and x.shape[-1] == ops.FFN_WIDTH and self.linear1.bias is None
                 and self.linear2.bias is None and self.norm1.weight is not None and self.norm1.weight.dtype == torch.float32):
@@ -1098,6 +1141,22 @@ class GriffinTemporalBlock(_WeightCaches, nn.Module):
         hp = _cached_cast(self, "_bnb_l12f_head_pack" if fold else "_bnb_l12_head_pack", ws, torch.bfloat16,
                           lambda: ops.pack_head_weights(self._head_matrix(ws)))
         return (self.norm1.weight, self.norm1.eps, hp, len(ws) * ops.FFN_WIDTH)
+
+    def _f32_ok(self, x, act) -> bool:
+        return (_f32_fused_ok(x, act, self.linear1, self.linear2) and self.linear1.bias is None and self.linear2.bias is None
+                and self.norm1.weight is not None)
+
+    def _f32_streams(self, has_fields, field_sub) -> tuple:
+        """Operand streams of the float32 head: [linear1 | linear2], and with field tokens field_sub(linear1(.)) as one more
+        projection of the same normed rows (field_sub . linear1 folded in float32)."""
+        w12 = (self.linear1.weight, self.linear2.weight)
+        streams = (_cached_cast(self, "_bnb_f32_l12", w12, torch.float32,
+                                lambda: ops.pack_linear_f32(torch.cat([w12[0].detach(), w12[1].detach()], dim=0))),)
+        if has_fields and field_sub is not None and field_sub.bias is None and field_sub.weight.dtype == torch.float32:
+            ws = (field_sub.weight, self.linear1.weight)
+            streams += (_cached_cast(self, "_bnb_f32_fsub", ws, torch.float32,
+                                     lambda: ops.pack_linear_f32(ws[0].detach().float() @ ws[1].detach().float())),)
+        return streams
 
     def step_tokens(self, x, n_rec, state_in, state_out, reset, field_sub, *, head=None, next_head=None):
         """One timestep over all tokens of every environment at once.
@@ -1132,21 +1191,18 @@ class GriffinTemporalBlock(_WeightCaches, nn.Module):
             b1, gate_in = both[..., :D], both[..., D:2 * D]
             if fold:
                 y = both[..., 2 * D:]
-        elif (_f32_fused_ok(x, act, self.linear1, self.linear2) and self.linear1.bias is None and self.linear2.bias is None
-              and self.norm1.weight is not None):
+        elif self._f32_ok(x, act):
             # float32: norm1 and [linear1 | linear2] as one kernel; with field tokens field_sub(linear1(.)) is one more
-            # projection of the same normed rows (field_sub . linear1 folded in float32), written for every token and
-            # then overwritten on the ship rows by the recurrence
-            w12 = (self.linear1.weight, self.linear2.weight)
-            pk = _cached_cast(self, "_bnb_f32_l12", w12, torch.float32,
-                              lambda: ops.pack_linear_f32(torch.cat([w12[0].detach(), w12[1].detach()], dim=0)))
-            both = ops.linear_f32(x, pk, norm_weight=self.norm1.weight, eps=self.norm1.eps)  # (B, NM, 2D)
+            # projection, written for every token and then overwritten on the ship rows by the recurrence
+            if head is not None:
+                made = head  # formed by the tail kernel of the sublayer before
+            else:
+                made = tuple(ops.linear_f32(x, w, norm_weight=self.norm1.weight, eps=self.norm1.eps)
+                             for w in self._f32_streams(NM > n_rec, field_sub))
+            both = made[0]  # (B, NM, 2D)
             b1, gate_in = both[..., :D], both[..., D:]
-            if NM > n_rec and field_sub is not None and field_sub.bias is None and field_sub.weight.dtype == torch.float32:
-                ws = (field_sub.weight, self.linear1.weight)
-                pf = _cached_cast(self, "_bnb_f32_fsub", ws, torch.float32,
-                                  lambda: ops.pack_linear_f32(ws[0].detach().float() @ ws[1].detach().float()))
-                y = ops.linear_f32(x, pf, norm_weight=self.norm1.weight, eps=self.norm1.eps)  # (B, NM, D)
+            if len(made) > 1:
+                y = made[1]  # (B, NM, D)
         else:
             x, normed = self._norm_in(x)
             b1 = _project(self.linear1, normed)

@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define BNB_ABI_VERSION 32
+#define BNB_ABI_VERSION 33
 
 /* element types of activation buffers */
 #define BNB_F32 0
@@ -985,6 +985,25 @@ int bnb_trunk_step_fwd(const bnb_trunk_layer *layers, int n_layers, const void *
                        const uint8_t *alive, const uint8_t *reset, const void *bullets, int bullets_dtype,
                        const uint8_t *in_flight, float bullet_eps, int NB, const float *state_in, float *state_out,
                        int B, int NM, int n_rec, int D, int H, int hidden, void *stream);
+
+/*
+ * The tail of a sublayer in float32, with its output projection and the head of the next sublayer, in one launch
+ * (models/yemong/attention.py:97-98,169; models/yemong/griffin.py:281-287, without autocast):
+ *     s   = x + A Wp^T,  A = a, or gelu(a) * y
+ *     out = s + (gelu(n Wg^T) * (n Wu^T)) Wd^T,  n = rmsnorm(s) * norm_weight
+ *     head1_out = n' W1^T, head2_out = n' W2^T,  n' = rmsnorm(out) * head_norm_weight      (head_norm_weight NULL: no head)
+ *
+ *   x, a, y        (R, 128) fp32 rows, strides multiples of 4; y NULL: plain projection
+ *   *_packed       weights in the piece order of bnb_linear_f32_fwd: proj (128, 128), gate_up interleaved as for its gated
+ *                  form, down (128, 512), heads (features, 128) with features % 32 == 0 (head2_features 0: one head)
+ *   out            (R, 128), head*_out (R, features): fp32 contiguous; none may overlap an input
+ * D == 128, hidden == 512, else BNB_ERR_UNSUPPORTED.
+ */
+int bnb_tail_f32_fwd(const float *x, int64_t x_row_stride, const float *a, int64_t a_row_stride, const float *y,
+                     int64_t y_row_stride, const void *proj_packed, const float *norm_weight, float eps, const void *gate_up_packed,
+                     const void *down_packed, float *out, const float *head_norm_weight, float head_eps, const void *head1_packed,
+                     float *head1_out, int head1_features, const void *head2_packed, float *head2_out, int head2_features,
+                     int64_t R, int D, int hidden, void *stream);
 
 #ifdef __cplusplus
 }

@@ -2907,6 +2907,56 @@ def test_linear_f32_reads_column_blocks_in_place_and_writes_into_the_residual():
         ops.pack_linear_f32(torch.zeros(48, 128))
 
 
+def _tail_f32_in_float64(x, a, y, wp, nw, wg, wu, wd, head_norm, heads):
+    eps = float(torch.finfo(torch.float32).eps)
+    norm = lambda t, w: t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + eps) * w.double()
+    x, a = x.double(), a.double()
+    s = x + (a if y is None else _gelu64(a) * y.double()) @ wp.double().t()
+    n = norm(s, nw)
+    out = s + (_gelu64(n @ wg.double().t()) * (n @ wu.double().t())) @ wd.double().t()
+    return [out] + [norm(out, head_norm) @ w.double().t() for w in heads]
+
+
+@pytest.mark.parametrize("heads", [(), (96,), (256, 128)])
+@pytest.mark.parametrize("R", [1, 31, 33, 64, 8200])
+def test_tail_f32_matches_the_float64_statement(R, heads):
+    """The float32 sublayer tail as one kernel at the edges of its 32-row tiles, rows read in place from wider tensors, with one
+    row of numbers too large for the bf16 pieces, one of tiny numbers, one infinity and one NaN."""
+    g = torch.Generator().manual_seed(R + len(heads))
+    wide = torch.randn(R, 384, generator=g) * (0.3 + 2.0 * torch.rand(R, 1, generator=g))
+    x = torch.randn(R, 128, generator=g)
+    wp, wg, wu, wd = (torch.randn(n, k, generator=g) / k ** 0.5 for n, k in ((128, 128), (512, 128), (512, 128), (128, 512)))
+    hw = [torch.randn(n, 128, generator=g) / 128 ** 0.5 for n in heads]
+    nw, hn = 1.0 + 0.2 * torch.randn(128, generator=g), 1.0 + 0.2 * torch.randn(128, generator=g)
+    if R > 30:  # beside ordinary rows of their tiles
+        wide[3, :256] *= 1e-30
+        x[3] *= 1e-30
+        wide[R - 1, 7], wide[17, 200], x[20, 5] = float("inf"), float("nan"), float("inf")
+        x[9] = 0.0
+        x[9, 4] = 3.4e38  # rounds to a bfloat16 infinity; its norm leaves the float32 range
+    dw = wide.to(DEV)
+    pack = ops.pack_linear_f32
+    ws = (pack(wp.to(DEV)), nw.to(DEV), pack(wg.to(DEV), wu.to(DEV)), pack(wd.to(DEV)))
+    nh = (hn.to(DEV), None, tuple(pack(w.to(DEV)) for w in hw)) if heads else None
+    for times in (False, True):
+        got = ops.tail_f32(x.to(DEV), dw[:, :128], *ws, gelu_times=dw[:, 128:256] if times else None, next_head=nh)
+        got = [t.cpu() for t in ((got[0],) + got[1] if heads else (got,))]
+        want = _tail_f32_in_float64(x, wide[:, :128], wide[:, 128:256] if times else None, wp, nw, wg, wu, wd, hn, hw)
+        s = ops.linear_f32(dw[:, :128], ws[0], gelu_times=dw[:, 128:256] if times else None, resid=x.to(DEV))
+        sep = ops.linear_f32(ops.linear_f32(s, ws[2], norm_weight=ws[1], gate=True), ws[3], resid=s)
+        sep = [sep.cpu()] + [ops.linear_f32(sep, w, norm_weight=nh[0]).cpu() for w in (nh[2] if heads else ())]
+        odd = [r for r in (9, 17, 20, R - 1) if R > 30]
+        plain = torch.ones(R, dtype=torch.bool)
+        plain[odd] = False
+        for k, (t, ref, each) in enumerate(zip(got, want, sep)):
+            assert max_rel(t[plain].double(), ref[plain]) <= F32_TOL, (k, times)
+            for r in odd:  # the float32 range and its special values: as the separate kernels give them
+                assert torch.equal(t[r].isfinite(), each[r].isfinite()) and torch.equal(t[r].isnan(), each[r].isnan()), (k, r, times)
+                fin = each[r].isfinite()
+                # sums of up to 512 terms of order one, twice each in float32: 2 * 512 * 2^-24 = 6e-5 of them
+                torch.testing.assert_close(t[r][fin], each[r][fin], rtol=1e-4, atol=6e-5)
+
+
 _F32_RANGE_FORMS = [(300, 128, 96, "plain"), (70, 128, 64, "norm"), (300, 128, 96, "times"), (130, 128, 64, "gate"),
                     (130, 128, 64, "norm_gate"), (90, 512, 128, "plain"), (10300, 512, 128, "plain"), (40, 256, 64, "plain")]
 

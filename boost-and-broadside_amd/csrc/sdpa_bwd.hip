@@ -255,7 +255,10 @@ constexpr int kMbPitch = kSbDh + 8;  // halfs per token row in LDS (80 bytes: 16
 // values come from a second buffer kv (B, NK, 2*H*32) with its own mask (the bullet read,
 // models/yemong/attention.py:149-166): an environment without a live key contributed exactly nothing
 // in the forward (the reference gates it off), so all its gradients are zero; `out` is that read's own
-// result, before it was added to anything.
+// result, before it was added to anything.  dq_add: dq rows hold the gradient of the queries' other use already (self-attention over
+// the same projection) and this one is added to them in float32, rounded once, in place of a gradient three times as wide that is
+// mostly zeros and a pass that adds it (32,768 environments of 12 tokens, 393,216 x 384 gradients: 260 us of fills, copies and
+// additions a read).
 // PAIR (NB = 1, up to 16 tokens, an even number of heads): two heads of one environment share the tile, as
 // in the forward kernel for small fleets.  Row r of every staged operand is token r % 16 of head
 // 2 * pair + r / 16, and the score blocks between the two heads start at -inf like a dead key, so P and
@@ -264,8 +267,8 @@ template <int NB, bool CROSS, bool PAIR>
 __global__ __launch_bounds__(kWave * NB) __attribute__((amdgpu_waves_per_eu(NB == 1 && !PAIR ? 3 : 4))) void sdpa_bwd_mfma_kernel(
     const uint16_t *__restrict__ q, int64_t q_row_stride, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,
     int64_t kv_row_stride, const uint8_t *__restrict__ alive, const int32_t *__restrict__ ranges, int64_t kv_capacity,
-    const uint16_t *__restrict__ out, const uint16_t *__restrict__ dout, uint16_t *__restrict__ dq_out, int64_t dq_row_stride,
-    uint16_t *__restrict__ dk_out, uint16_t *__restrict__ dv_out, int64_t dkv_row_stride, int B, int NQ, int NK_all, int H,
+    const uint16_t *__restrict__ out, const uint16_t *__restrict__ dout, uint16_t *dq_out, int64_t dq_row_stride,
+    int dq_add, uint16_t *__restrict__ dk_out, uint16_t *__restrict__ dv_out, int64_t dkv_row_stride, int B, int NQ, int NK_all, int H,
     float scale)
 {
     constexpr int CAP = NB * 32;
@@ -405,7 +408,7 @@ __global__ __launch_bounds__(kWave * NB) __attribute__((amdgpu_waves_per_eu(NB =
     if (CROSS && none_live) {
         // the forward gated this environment off: nothing depends on its inputs
         const f32x16 z16 = {0.0f};
-        if (wave < nqb) store_grad(z16, dq_out, dq_row_stride, q_base, own, NQ);
+        if (wave < nqb && !dq_add) store_grad(z16, dq_out, dq_row_stride, q_base, own, NQ);
         if (wave < nkb) {
             store_grad(z16, dk_out, dkv_row_stride, k_base, own, NK);
             store_grad(z16, dv_out, dkv_row_stride, k_base, own, NK);
@@ -474,6 +477,13 @@ __global__ __launch_bounds__(kWave * NB) __attribute__((amdgpu_waves_per_eu(NB =
         const float lse = mc + __builtin_amdgcn_logf(sum);  // log2 of the sum of exp2(z c)
         if (half == 0) s_lse[own] = lse, s_delta[own] = delta;
 
+        // with dq_add: what this lane's row holds, on its way while the gradient is formed
+        u32x2 held[4] = {};
+        if (CROSS && dq_add) {
+            const uint16_t *src = dq_out + (q_base + (own < NQ ? own : NQ - 1)) * dq_row_stride + own_ch + 4 * half;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) held[i] = *reinterpret_cast<const u32x2 *>(src + 8 * i);
+        }
         f32x16 dq = {0.0f};
         for (int kb = 0; kb < nkb; ++kb) {
             const f32x16 z = scores_t(kb);
@@ -490,6 +500,13 @@ __global__ __launch_bounds__(kWave * NB) __attribute__((amdgpu_waves_per_eu(NB =
             for (int vv = 0; vv < 16; ++vv) ds[vv] = __builtin_amdgcn_exp2f(fmaf(z[vv], c, -lse)) * (dp[vv] - delta) * scale;
 #pragma unroll
             for (int t = 0; t < 2; ++t) dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_operand(s_tr[0], kb, t), pack8(ds, t), dq, 0, 0, 0);
+        }
+        if (CROSS) {
+#pragma unroll
+            for (int vv = 0; vv < 16; ++vv) {
+                const uint32_t w = held[vv >> 2][(vv >> 1) & 1];
+                dq[vv] += __uint_as_float((vv & 1) ? w & 0xffff0000u : w << 16);
+            }
         }
         store_grad(dq, dq_out, dq_row_stride, q_base, own, NQ);
     }
@@ -547,14 +564,14 @@ __global__ __launch_bounds__(kWave * NB) __attribute__((amdgpu_waves_per_eu(NB =
 template <int NB, bool CROSS, bool PAIR = false>
 static int launch_sdpa_bwd_mfma(const void *q, int64_t q_row_stride, const void *k, const void *v, int64_t kv_row_stride,
                                 const uint8_t *alive, const int32_t *ranges, int64_t kv_capacity, const void *out, const void *dout,
-                                void *dq, int64_t dq_row_stride, void *dk, void *dv, int64_t dkv_row_stride, int64_t B, int NQ,
+                                void *dq, int64_t dq_row_stride, int dq_add, void *dk, void *dv, int64_t dkv_row_stride, int64_t B, int NQ,
                                 int NK, int H, hipStream_t stream)
 {
     const int64_t groups = (B * (PAIR ? H / 2 : H) + 7) / 8 * 8;  // a multiple of 8: the XCD mapping deals whole rounds
     if (groups > 0x7fffffffLL) return BNB_ERR_UNSUPPORTED;
     hipLaunchKernelGGL((sdpa_bwd_mfma_kernel<NB, CROSS, PAIR>), dim3((unsigned)groups), dim3(kWave * NB), 0, stream, (const uint16_t *)q,
                        q_row_stride, (const uint16_t *)k, (const uint16_t *)v, kv_row_stride, alive, ranges, kv_capacity,
-                       (const uint16_t *)out, (const uint16_t *)dout, (uint16_t *)dq, dq_row_stride, (uint16_t *)dk, (uint16_t *)dv, dkv_row_stride, (int)B,
+                       (const uint16_t *)out, (const uint16_t *)dout, (uint16_t *)dq, dq_row_stride, dq_add, (uint16_t *)dk, (uint16_t *)dv, dkv_row_stride, (int)B,
                        NQ, NK, H, 1.0f / sqrtf((float)kSbDh));
     return (int)hipGetLastError();
 }
@@ -562,16 +579,16 @@ static int launch_sdpa_bwd_mfma(const void *q, int64_t q_row_stride, const void 
 template <bool CROSS>
 static int dispatch_sdpa_bwd_mfma(const void *q, int64_t q_row_stride, const void *k, const void *v, int64_t kv_row_stride,
                                   const uint8_t *alive, const int32_t *ranges, int64_t kv_capacity, const void *out, const void *dout,
-                                  void *dq, int64_t dq_row_stride, void *dk, void *dv, int64_t dkv_row_stride, int64_t B, int NQ,
+                                  void *dq, int64_t dq_row_stride, int dq_add, void *dk, void *dv, int64_t dkv_row_stride, int64_t B, int NQ,
                                   int NK, int H, hipStream_t s)
 {
     const int nb = ((NQ > NK ? NQ : NK) + 31) / 32;
     if (!CROSS && NQ <= 16 && H % 2 == 0)
         return launch_sdpa_bwd_mfma<1, false, true>(q, q_row_stride, k, v, kv_row_stride, alive, ranges, kv_capacity, out, dout, dq,
-                                                    dq_row_stride, dk, dv, dkv_row_stride, B, NQ, NK, H, s);
+                                                    dq_row_stride, dq_add, dk, dv, dkv_row_stride, B, NQ, NK, H, s);
 #define BNB_SBM(NBV) \
     return launch_sdpa_bwd_mfma<NBV, CROSS>(q, q_row_stride, k, v, kv_row_stride, alive, ranges, kv_capacity, out, dout, dq, \
-                                            dq_row_stride, dk, dv, dkv_row_stride, B, NQ, NK, H, s)
+                                            dq_row_stride, dq_add, dk, dv, dkv_row_stride, B, NQ, NK, H, s)
     switch (nb) {
         case 1: BNB_SBM(1);
         case 2: BNB_SBM(2);
@@ -609,7 +626,7 @@ extern "C" int bnb_sdpa_masked_bwd_path(const void *qkv, int64_t qkv_row_stride,
         const int D = H * dh;
         uint16_t *g = (uint16_t *)dqkv;
         return dispatch_sdpa_bwd_mfma<false>(p, qkv_row_stride, p + D, p + 2 * D, qkv_row_stride, alive, nullptr, 0, out, dout, g,
-                                             3 * (int64_t)D, g + D, g + 2 * D, 3 * (int64_t)D, B, NM, NM, H, s);
+                                             3 * (int64_t)D, 0, g + D, g + 2 * D, 3 * (int64_t)D, B, NM, NM, H, s);
     }
     if (!small) return BNB_ERR_UNSUPPORTED;
     if (dtype == BNB_BF16) return launch_sdpa_bwd<uint16_t>(qkv, qkv_row_stride, alive, out, dout, dqkv, B, NM, H, s);
@@ -639,27 +656,27 @@ extern "C" int bnb_sdpa_cross_bwd(const void *q, int64_t q_row_stride, int NQ, c
     if (B > 0x7fffffffLL / H) return BNB_ERR_UNSUPPORTED;
     const uint16_t *kp = (const uint16_t *)kv;
     uint16_t *g = (uint16_t *)dkv;
-    return dispatch_sdpa_bwd_mfma<true>(q, q_row_stride, kp, kp + D, kv_row_stride, key_mask, nullptr, 0, out, dout, dq, D, g, g + D,
+    return dispatch_sdpa_bwd_mfma<true>(q, q_row_stride, kp, kp + D, kv_row_stride, key_mask, nullptr, 0, out, dout, dq, D, 0, g, g + D,
                                         2 * (int64_t)D, B, NQ, NK, H, (hipStream_t)stream);
 }
 
 extern "C" int bnb_sdpa_cross_ranges_bwd(const void *q, int64_t q_row_stride, int NQ, const void *kv_rows, int64_t kv_row_stride,
                                          const int32_t *ranges, int64_t capacity, int max_keys, const void *out, const void *dout,
-                                         void *dq, void *dkv_rows, int64_t B, int H, int dh, int dtype, void *stream)
+                                         void *dq, int64_t dq_row_stride, int dq_add, void *dkv_rows, int64_t B, int H, int dh, int dtype, void *stream)
 {
     using namespace bnb;
     if (B < 0 || NQ < 1 || H < 1 || dh < 1 || capacity < 1 || max_keys < 1) return BNB_ERR_BAD_SHAPE;  // an empty list: nothing to call
     if (dtype != BNB_BF16 || dh != kSbDh || NQ > 160 || max_keys > 160) return BNB_ERR_UNSUPPORTED;
     const int D = H * dh;
-    if (q_row_stride < D || kv_row_stride < 2 * (int64_t)D) return BNB_ERR_BAD_SHAPE;
+    if (q_row_stride < D || kv_row_stride < 2 * (int64_t)D || dq_row_stride < D) return BNB_ERR_BAD_SHAPE;
     if (B == 0) return 0;
     if (!q || !ranges || !out || !dout || !dq || !kv_rows || !dkv_rows) return BNB_ERR_NULL_POINTER;
     if (!aligned16(q) || !aligned16(kv_rows) || !aligned16(out) || !aligned16(dout) || !aligned16(dq) || !aligned16(dkv_rows) ||
-        (q_row_stride % 8) != 0 || (kv_row_stride % 8) != 0)
+        (q_row_stride % 8) != 0 || (dq_row_stride % 8) != 0 || (kv_row_stride % 8) != 0)
         return BNB_ERR_MISALIGNED;
     if (B > 0x7fffffffLL / H) return BNB_ERR_UNSUPPORTED;
     const uint16_t *kp = (const uint16_t *)kv_rows;
     uint16_t *g = (uint16_t *)dkv_rows;
-    return dispatch_sdpa_bwd_mfma<true>(q, q_row_stride, kp, kp + D, kv_row_stride, nullptr, ranges, capacity, out, dout, dq, D, g,
+    return dispatch_sdpa_bwd_mfma<true>(q, q_row_stride, kp, kp + D, kv_row_stride, nullptr, ranges, capacity, out, dout, dq, dq_row_stride, dq_add, g,
                                         g + D, 2 * (int64_t)D, B, NQ, max_keys, H, (hipStream_t)stream);
 }

@@ -84,7 +84,7 @@ template <int NB, bool HAVE_LSE>
 __global__ __launch_bounds__(kWave *NB, NB == 5 ? 5 : 3) void cross_bwd_dq_kernel(
     const uint16_t *__restrict__ q, int64_t q_row_stride, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,
     int64_t kv_row_stride, const int32_t *__restrict__ ranges, const int32_t *__restrict__ row_index, int64_t capacity,
-    const uint16_t *__restrict__ out, const uint16_t *__restrict__ dout, uint16_t *__restrict__ dq_out, float *__restrict__ stats,
+    const uint16_t *__restrict__ out, const uint16_t *__restrict__ dout, uint16_t *dq_out, int64_t dq_row_stride, int dq_add, float *__restrict__ stats,
     const float *__restrict__ lse_in, int B, int NQ, int H, float scale)
 {
     constexpr int CAP = NB * 32;  // keys per tile
@@ -111,13 +111,13 @@ __global__ __launch_bounds__(kWave *NB, NB == 5 ? 5 : 3) void cross_bwd_dq_kerne
     const int nqb = (NQ + 31) >> 5;  // <= NB
     const int own = wave * 32 + m;   // this lane's query
     const int64_t q_base = (int64_t)env * NQ;
-    uint16_t *dq_row = dq_out + (q_base + own) * D + head * kCbDh + 4 * half;
+    uint16_t *dq_row = dq_out + (q_base + own) * dq_row_stride + head * kCbDh + 4 * half;
     float *stat_row = stats + (((int64_t)env * H + head) * NQ + own) * 2;
     if (cnt == 0) {
         // the forward gated this environment off: nothing depends on its queries
         if (own < NQ) {
             const f32x16 z16 = {0.0f};
-            cb_store_row(z16, dq_row);
+            if (!dq_add) cb_store_row(z16, dq_row);
             if (half == 0) stat_row[0] = 0.0f, stat_row[1] = 0.0f;
         }
         return;
@@ -268,7 +268,19 @@ __global__ __launch_bounds__(kWave *NB, NB == 5 ? 5 : 3) void cross_bwd_dq_kerne
     }
 #pragma unroll
     for (int vv = 0; vv < 16; ++vv) dq[vv] *= scale;
-    if (own < NQ) cb_store_row(dq, dq_row);
+    if (own < NQ) {
+        if (dq_add) {  // onto the gradient of the queries' other use
+            u32x2 held[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) held[i] = *reinterpret_cast<const u32x2 *>(dq_row + 8 * i);
+#pragma unroll
+            for (int vv = 0; vv < 16; ++vv) {
+                const uint32_t w = held[vv >> 2][(vv >> 1) & 1];
+                dq[vv] += __uint_as_float((vv & 1) ? w & 0xffff0000u : w << 16);
+            }
+        }
+        cb_store_row(dq, dq_row);
+    }
 }
 
 // Waves: the key blocks are dealt to the waves in turn, so their number is free; never more than four.  A CU places
@@ -406,7 +418,7 @@ __global__ __launch_bounds__(kWave *(NB < 4 ? NB : 4), 3) void cross_bwd_dkv_ker
 
 template <int NB>
 static int launch_cross_stream_bwd(const void *q, int64_t q_row_stride, const void *kv, int64_t kv_row_stride, const int32_t *ranges,
-                                   const int32_t *row_index, int64_t capacity, const void *out, const void *dout, void *dq, void *dkv,
+                                   const int32_t *row_index, int64_t capacity, const void *out, const void *dout, void *dq, int64_t dq_row_stride, int dq_add, void *dkv,
                                    float *stats, const float *lse, int64_t B, int NQ, int H, hipStream_t stream)
 {
     const int64_t groups = (B * H + 7) / 8 * 8;  // a multiple of 8: the XCD mapping deals whole rounds
@@ -418,11 +430,11 @@ static int launch_cross_stream_bwd(const void *q, int64_t q_row_stride, const vo
     if (lse != nullptr)
         hipLaunchKernelGGL((cross_bwd_dq_kernel<NB, true>), dim3((unsigned)groups), dim3(kWave * NB), 0, stream, (const uint16_t *)q,
                            q_row_stride, kp, kp + D, kv_row_stride, ranges, row_index, capacity, (const uint16_t *)out,
-                           (const uint16_t *)dout, (uint16_t *)dq, stats, lse, (int)B, NQ, H, scale);
+                           (const uint16_t *)dout, (uint16_t *)dq, dq_row_stride, dq_add, stats, lse, (int)B, NQ, H, scale);
     else
         hipLaunchKernelGGL((cross_bwd_dq_kernel<NB, false>), dim3((unsigned)groups), dim3(kWave * NB), 0, stream, (const uint16_t *)q,
                            q_row_stride, kp, kp + D, kv_row_stride, ranges, row_index, capacity, (const uint16_t *)out,
-                           (const uint16_t *)dout, (uint16_t *)dq, stats, lse, (int)B, NQ, H, scale);
+                           (const uint16_t *)dout, (uint16_t *)dq, dq_row_stride, dq_add, stats, lse, (int)B, NQ, H, scale);
     int rc = (int)hipGetLastError();
     if (rc != 0) return rc;
     hipLaunchKernelGGL((cross_bwd_dkv_kernel<NB>), dim3((unsigned)groups), dim3(kWave * (NB < 4 ? NB : 4)), 0, stream, (const uint16_t *)q, q_row_stride, kp,
@@ -436,20 +448,20 @@ static int launch_cross_stream_bwd(const void *q, int64_t q_row_stride, const vo
 namespace bnb {
 static int cross_stream_bwd(const void *q, int64_t q_row_stride, int NQ, const void *kv, int64_t kv_row_stride,
                             const int32_t *ranges, const int32_t *row_index, int64_t capacity, const void *out, const void *dout,
-                            void *dq, void *dkv, float *stats, const float *lse, int64_t B, int H, int dh, int dtype, void *stream)
+                            void *dq, int64_t dq_row_stride, int dq_add, void *dkv, float *stats, const float *lse, int64_t B, int H, int dh, int dtype, void *stream)
 {
     if (B < 0 || NQ < 1 || H < 1 || dh < 1 || capacity < 1) return BNB_ERR_BAD_SHAPE;
     if (dtype != BNB_BF16 || dh != kCbDh || NQ > 160) return BNB_ERR_UNSUPPORTED;
     const int D = H * dh;
-    if (q_row_stride < D || kv_row_stride < 2 * (int64_t)D) return BNB_ERR_BAD_SHAPE;
+    if (q_row_stride < D || kv_row_stride < 2 * (int64_t)D || dq_row_stride < D) return BNB_ERR_BAD_SHAPE;
     if (B == 0) return 0;
     if (!q || !kv || !ranges || !out || !dout || !dq || !dkv || !stats) return BNB_ERR_NULL_POINTER;
     if (!aligned16(q) || !aligned16(kv) || !aligned16(out) || !aligned16(dout) || !aligned16(dq) || !aligned16(dkv) ||
-        (q_row_stride % 8) != 0 || (kv_row_stride % 8) != 0)
+        (q_row_stride % 8) != 0 || (kv_row_stride % 8) != 0 || (dq_row_stride % 8) != 0)
         return BNB_ERR_MISALIGNED;
     if (B > 0x7fffffffLL / H) return BNB_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
-#define BNB_CSB(NBV) return launch_cross_stream_bwd<NBV>(q, q_row_stride, kv, kv_row_stride, ranges, row_index, capacity, out, dout, dq, dkv, stats, lse, B, NQ, H, s)
+#define BNB_CSB(NBV) return launch_cross_stream_bwd<NBV>(q, q_row_stride, kv, kv_row_stride, ranges, row_index, capacity, out, dout, dq, dq_row_stride, dq_add, dkv, stats, lse, B, NQ, H, s)
     switch ((NQ + 31) / 32) {
         case 1: BNB_CSB(1);
         case 2: BNB_CSB(2);
@@ -464,20 +476,20 @@ static int cross_stream_bwd(const void *q, int64_t q_row_stride, int NQ, const v
 
 extern "C" int bnb_sdpa_cross_stream_bwd(const void *q, int64_t q_row_stride, int NQ, const void *kv, int64_t kv_row_stride,
                                          const int32_t *ranges, const int32_t *row_index, int64_t capacity, const void *out,
-                                         const void *dout, void *dq, void *dkv, float *stats, int64_t B, int H, int dh, int dtype,
+                                         const void *dout, void *dq, int64_t dq_row_stride, int dq_add, void *dkv, float *stats, int64_t B, int H, int dh, int dtype,
                                          void *stream)
 {
-    return bnb::cross_stream_bwd(q, q_row_stride, NQ, kv, kv_row_stride, ranges, row_index, capacity, out, dout, dq, dkv, stats,
+    return bnb::cross_stream_bwd(q, q_row_stride, NQ, kv, kv_row_stride, ranges, row_index, capacity, out, dout, dq, dq_row_stride, dq_add, dkv, stats,
                                  nullptr, B, H, dh, dtype, stream);
 }
 
 extern "C" int bnb_sdpa_cross_stream_bwd_lse(const void *q, int64_t q_row_stride, int NQ, const void *kv, int64_t kv_row_stride,
                                              const int32_t *ranges, const int32_t *row_index, int64_t capacity, const void *out,
-                                             const void *dout, const float *lse, void *dq, void *dkv, float *stats, int64_t B,
+                                             const void *dout, const float *lse, void *dq, int64_t dq_row_stride, int dq_add, void *dkv, float *stats, int64_t B,
                                              int H, int dh, int dtype, void *stream)
 {
     if (lse == nullptr && B > 0) return BNB_ERR_NULL_POINTER;
     if (reinterpret_cast<uintptr_t>(lse) & 3u) return BNB_ERR_MISALIGNED;
-    return bnb::cross_stream_bwd(q, q_row_stride, NQ, kv, kv_row_stride, ranges, row_index, capacity, out, dout, dq, dkv, stats,
+    return bnb::cross_stream_bwd(q, q_row_stride, NQ, kv, kv_row_stride, ranges, row_index, capacity, out, dout, dq, dq_row_stride, dq_add, dkv, stats,
                                  lse, B, H, dh, dtype, stream);
 }

@@ -301,10 +301,22 @@ def sdpa_cross_train_supported(qkv: torch.Tensor, kv: torch.Tensor, n_heads: int
     return cross_supported(qkv, kv, n_heads) and qkv.dtype == torch.bfloat16 and kv.dim() == 3 and qkv.dim() == 3
 
 
-def sdpa_cross_stream_bwd(qkv, kv, rows: "CompactRows", n_heads, out, dout, *, indexed: bool, lse: torch.Tensor | None = None):
+def _dq_of(qkv: torch.Tensor, dq_into: torch.Tensor | None) -> tuple[torch.Tensor, int]:
+    """Where a read's query gradient goes, and whether it is added there."""
+    B, NQ, D3 = qkv.shape
+    if dq_into is None:
+        return torch.empty((B, NQ, D3 // 3), dtype=torch.bfloat16, device=qkv.device), 0
+    if dq_into.shape != qkv.shape or dq_into.dtype != torch.bfloat16 or not dq_into.is_contiguous() or dq_into.device != qkv.device:
+        raise ValueError("dq_into must be a contiguous bfloat16 tensor of qkv's shape on its device")
+    return dq_into[..., : D3 // 3], 1
+
+
+def sdpa_cross_stream_bwd(qkv, kv, rows: "CompactRows", n_heads, out, dout, *, indexed: bool, lse: torch.Tensor | None = None,
+                          dq_into: torch.Tensor | None = None):
     """Gradients ``(dq (B, NQ, D), dkv)`` of the bullet read for any number of listed keys per environment.
     ``lse`` (B, n_heads, NQ) float32, optional: the log-sum-exp ``sdpa_cross_rows(..., lse=...)`` wrote in the forward
     pass over the same queries and keys; without it the first kernel recomputes it (a second pass over every key).
+    ``dq_into`` (B, NQ, 3D) contiguous, optional: dq is added to its query third, and is that view.
 
     ``indexed=False``: ``kv`` (capacity, 2D) holds ``[K | V]`` of the entries of ``rows`` in list order and
     ``dkv`` has that layout.  ``indexed=True``: ``kv`` is the (B, NK, 2D) buffer the mask of ``rows`` was
@@ -332,9 +344,9 @@ def sdpa_cross_stream_bwd(qkv, kv, rows: "CompactRows", n_heads, out, dout, *, i
     if B and NQ and (qkv.stride(-1) != 1 or (B > 1 and qkv.stride(0) != NQ * qkv.stride(1))):
         qkv = qkv.contiguous()
     out, dout = out.contiguous(), dout.contiguous()
-    dq = torch.empty((B, NQ, D), dtype=torch.bfloat16, device=qkv.device)
+    dq, dq_add = _dq_of(qkv, dq_into)
     if capacity == 0:
-        return dq.zero_(), dkv
+        return dq if dq_add else dq.zero_(), dkv
     if lse is not None and (lse.shape != (B, n_heads, NQ) or lse.dtype != torch.float32 or not lse.is_contiguous()
                             or lse.device != qkv.device):
         raise ValueError(f"lse must be a contiguous float32 {(B, n_heads, NQ)} tensor on the queries' device")
@@ -346,12 +358,12 @@ def sdpa_cross_stream_bwd(qkv, kv, rows: "CompactRows", n_heads, out, dout, *, i
                 rc = lib.bnb_sdpa_cross_stream_bwd(
                     qkv.data_ptr(), qkv.stride(1), NQ, kv.data_ptr(), 2 * D, rows.offsets.data_ptr(),
                     rows.index.data_ptr() if indexed else None, capacity, out.data_ptr(), dout.data_ptr(), dq.data_ptr(),
-                    dkv.data_ptr(), stats.data_ptr(), B, n_heads, D // n_heads, _native.BF16, _stream())
+                    dq.stride(1), dq_add, dkv.data_ptr(), stats.data_ptr(), B, n_heads, D // n_heads, _native.BF16, _stream())
             else:
                 rc = lib.bnb_sdpa_cross_stream_bwd_lse(
                     qkv.data_ptr(), qkv.stride(1), NQ, kv.data_ptr(), 2 * D, rows.offsets.data_ptr(),
                     rows.index.data_ptr() if indexed else None, capacity, out.data_ptr(), dout.data_ptr(), lse.data_ptr(),
-                    dq.data_ptr(), dkv.data_ptr(), stats.data_ptr(), B, n_heads, D // n_heads, _native.BF16, _stream())
+                    dq.data_ptr(), dq.stride(1), dq_add, dkv.data_ptr(), stats.data_ptr(), B, n_heads, D // n_heads, _native.BF16, _stream())
         _native.check(rc, "bnb_sdpa_cross_stream_bwd")
     return dq, dkv
 
@@ -425,10 +437,12 @@ def sdpa_cross_train(qkv: torch.Tensor, kv: torch.Tensor, key_mask: torch.Tensor
         return _SdpaCrossTrain.apply(qkv, kv, key_mask, n_heads)
 
 
-def sdpa_cross_rows_bwd(qkv, kv_rows, rows: "CompactRows", n_heads, out, dout, total: int, lse: torch.Tensor | None = None):
+def sdpa_cross_rows_bwd(qkv, kv_rows, rows: "CompactRows", n_heads, out, dout, total: int, lse: torch.Tensor | None = None,
+                        dq_into: torch.Tensor | None = None):
     """Gradients ``(dq (B, NQ, D), dkv_rows (total, 2D))`` of ``sdpa_cross_rows`` (without accumulator);
     ``total`` = ``rows.total_host()`` rows of ``kv_rows`` are valid.  ``lse``: what the forward wrote with
-    ``sdpa_cross_rows(..., lse=...)``; used when some environment lists more than 160 keys (the streaming kernels)."""
+    ``sdpa_cross_rows(..., lse=...)``; used when some environment lists more than 160 keys (the streaming kernels).
+    ``dq_into`` (B, NQ, 3D) contiguous, optional: dq is added to its query third, and is that view."""
     B, NQ, D3 = qkv.shape
     D = D3 // 3
     for name, t in (("qkv", qkv), ("kv_rows", kv_rows), ("out", out), ("dout", dout)):
@@ -440,20 +454,21 @@ def sdpa_cross_rows_bwd(qkv, kv_rows, rows: "CompactRows", n_heads, out, dout, t
     if rows.shape[0] != B or out.shape != (B, NQ, D) or dout.shape != (B, NQ, D):
         raise ValueError("rows must list the entries of the B environments; out and dout are (B, NQ, D)")
     if rows.max_count_host() > 160:
-        return sdpa_cross_stream_bwd(qkv, kv_rows[:total], rows, n_heads, out, dout, indexed=False, lse=lse)
+        return sdpa_cross_stream_bwd(qkv, kv_rows[:total], rows, n_heads, out, dout, indexed=False, lse=lse, dq_into=dq_into)
     if B and NQ and (qkv.stride(-1) != 1 or (B > 1 and qkv.stride(0) != NQ * qkv.stride(1))):
         qkv = qkv.contiguous()
     out, dout = out.contiguous(), dout.contiguous()
-    dq = torch.empty((B, NQ, D), dtype=torch.bfloat16, device=qkv.device)
+    dq, dq_add = _dq_of(qkv, dq_into)
     dkv = torch.empty((total, 2 * D), dtype=torch.bfloat16, device=qkv.device)
     if total == 0:
-        return dq.zero_(), dkv
+        return dq if dq_add else dq.zero_(), dkv
     if B:
         with _on_device(qkv.device):
             rc = _native.load().bnb_sdpa_cross_ranges_bwd(qkv.data_ptr(), qkv.stride(1), NQ, kv_rows.data_ptr(), kv_rows.stride(0),
                                                           rows.offsets.data_ptr(), total, max(1, rows.max_count_host()), out.data_ptr(),
                                                           dout.data_ptr(),
-                                                          dq.data_ptr(), dkv.data_ptr(), B, n_heads, D // n_heads, _native.BF16, _stream())
+                                                          dq.data_ptr(), dq.stride(1), dq_add, dkv.data_ptr(), B, n_heads, D // n_heads,
+                                                          _native.BF16, _stream())
         _native.check(rc, "bnb_sdpa_cross_ranges_bwd")
     return dq, dkv
 
@@ -492,6 +507,42 @@ def sdpa_cross_rows_train(qkv: torch.Tensor, kv_rows: torch.Tensor, rows: "Compa
         raise ValueError(f"kv_rows must hold the {total} listed rows")
     with torch.autocast("cuda", enabled=False):
         return _SdpaCrossRowsTrain.apply(qkv, kv_rows.contiguous(), rows, n_heads, total)
+
+
+class _SdpaReadTrain(torch.autograd.Function):
+    """``sdpa_masked`` plus ``sdpa_cross_rows`` over the same queries: the backward adds the read's query gradient to the
+    self-attention's inside the kernel."""
+
+    @staticmethod
+    def forward(ctx, qkv, kv_rows, alive, rows, n_heads, total):
+        B, NQ, _ = qkv.shape
+        lse = (torch.empty((B, n_heads, NQ), dtype=torch.float32, device=qkv.device)
+               if B and NQ and rows.max_count_host() > 160 else None)
+        with torch.no_grad():
+            own = sdpa_masked(qkv, alive, n_heads)
+            read = sdpa_cross_rows(qkv, kv_rows, rows, n_heads, total=total, lse=lse)
+        ctx.save_for_backward(qkv, kv_rows, own, read)
+        ctx.alive, ctx.rows, ctx.n_heads, ctx.total, ctx.lse = alive, rows, n_heads, total, lse
+        return own + read
+
+    @staticmethod
+    @_outside_autocast
+    def backward(ctx, dout):
+        qkv, kv_rows, own, read = ctx.saved_tensors
+        dout = dout.to(torch.bfloat16).contiguous()
+        dqkv = sdpa_masked_bwd(qkv, ctx.alive, ctx.n_heads, own, dout)
+        _, dkv = sdpa_cross_rows_bwd(qkv, kv_rows, ctx.rows, ctx.n_heads, read, dout, ctx.total, ctx.lse, dq_into=dqkv)
+        return dqkv, dkv, None, None, None, None
+
+
+def sdpa_read_train(qkv: torch.Tensor, alive: torch.Tensor | None, kv_rows: torch.Tensor, rows: "CompactRows", n_heads: int) -> torch.Tensor:
+    """``sdpa_train(qkv, alive) + sdpa_cross_rows_train(qkv, kv_rows, rows)`` (bfloat16, a non-empty list, where both cover the
+    shapes): the gradient of the queries is summed in float32 and written once."""
+    total = rows.total_host()
+    if kv_rows.shape[0] != total or total == 0:
+        raise ValueError(f"kv_rows must hold the {total} listed rows, at least one")
+    with torch.autocast("cuda", enabled=False):
+        return _SdpaReadTrain.apply(qkv, kv_rows.contiguous(), alive, rows, n_heads, total)
 
 
 def rglru_step(

@@ -699,15 +699,20 @@ class TransformerBlock(_WeightCaches, nn.Module):
         if torch.is_grad_enabled():
             # training: forward and backward kernels for the small token counts of the update,
             # torch's differentiable SDPA for the rest
+            reads = self.reads_bullets and bullets is not None
+            listed = self._listed_bullets_autograd(qkv, bullets, bullet_mask) if reads else None
             if _TRAIN_KERNELS and ops.sdpa_train_supported(qkv, self.n_heads):
+                if listed is not None and listed[0] is not None:  # one backward for both uses of the queries
+                    merged = ops.sdpa_read_train(qkv, alive_mask, *listed, self.n_heads)
+                    return _project(self.out_proj, merged) if project else merged
                 merged = ops.sdpa_train(qkv, alive_mask, self.n_heads)
             else:
                 if _TRAIN_KERNELS and qkv.is_cuda:
                     _note_library("TransformerBlock.self_attention_backward",
                                   f"qkv {tuple(qkv.shape)} {qkv.dtype}, {self.n_heads} heads")
                 merged = self._self_attention_autograd(qkv, alive_mask)
-            if self.reads_bullets and bullets is not None:
-                merged = merged + self._bullet_branch_autograd(qkv, bullets, bullet_mask)
+            if reads:
+                merged = merged + self._bullet_branch_autograd(qkv, bullets, bullet_mask, listed)
             return _project(self.out_proj, merged) if project else merged
         try:
             merged = ops.sdpa_masked(qkv, alive_mask, self.n_heads)  # (B, N, D) head-major
@@ -768,16 +773,16 @@ class TransformerBlock(_WeightCaches, nn.Module):
             and bullets.shape[0] * bullets.shape[1] * 2 * self.d_model < 2 ** 32
         )
 
-    def _bullet_branch_autograd(self, qkv, bullets, bullet_mask):
-        """The bullet read in grad mode, (B, N, D) to be added to the self-attention output.
+    def _listed_bullets_autograd(self, qkv, bullets, bullet_mask):
+        """``(kv_rows, rows)``: the bullets in flight normalised and projected for the read in grad mode, ``(None, rows)`` when there
+        are none, or None when the read runs over every slot.
 
         With a mask, bf16 projections and at most 2048 slots per environment only the bullets in
         flight are normalised and projected: the list of live slots is built on the device, its
         length read back once (torch needs it to size the gathered rows), ``norm_bullet`` and
         ``kv_bullet`` run on the gathered rows and the read and its backward take the compacted
         ``[K | V]`` rows with per-environment ranges (a ``CompactRows`` built with ``total=`` /
-        ``max_count=`` by a caller that knows the counts needs no read-back).  Otherwise every slot is projected and the
-        read is the masked kernel pair, or torch's SDPA for the shapes the kernels do not cover."""
+        ``max_count=`` by a caller that knows the counts needs no read-back)."""
         rows = bullet_mask if isinstance(bullet_mask, ops.CompactRows) else None
         mask = rows.mask if rows is not None else bullet_mask
         B, NB, D = bullets.shape
@@ -790,7 +795,7 @@ class TransformerBlock(_WeightCaches, nn.Module):
                 rows = ops.CompactRows(mask)
             total = rows.total_host()
             if total == 0:
-                return torch.zeros_like(qkv[..., :D])
+                return None, rows
             shared = rows.live_rows  # one gather for all readers (YemongTrunk.sequence), or this reader's own
             live = shared.rows if shared is not None else bullets.reshape(B * NB, D).index_select(0, rows.index[:total].long())
             if _norm_linear_train_ok(live, _projection_dtype(), self.norm_bullet, self.kv_bullet):
@@ -800,7 +805,19 @@ class TransformerBlock(_WeightCaches, nn.Module):
             else:
                 kv_rows = _project(self.kv_bullet, _train_norm(self.norm_bullet, live)[1])
             if kv_rows.dtype == torch.bfloat16:
-                return ops.sdpa_cross_rows_train(qkv, kv_rows, rows, self.n_heads)
+                return kv_rows, rows
+        return None
+
+    def _bullet_branch_autograd(self, qkv, bullets, bullet_mask, listed):
+        """The bullet read in grad mode, (B, N, D) to be added to the self-attention output: over the listed bullets
+        (``_listed_bullets_autograd``), or every slot is projected and the read is the masked kernel pair, or torch's SDPA for
+        the shapes the kernels do not cover."""
+        if listed is not None:
+            kv_rows, rows = listed
+            if kv_rows is None:
+                return torch.zeros_like(qkv[..., :bullets.shape[-1]])
+            return ops.sdpa_cross_rows_train(qkv, kv_rows, rows, self.n_heads)
+        mask = bullet_mask.mask if isinstance(bullet_mask, ops.CompactRows) else bullet_mask
         kv = _project(self.kv_bullet, _train_norm(self.norm_bullet, bullets)[1])
         if _TRAIN_KERNELS and ops.sdpa_cross_train_supported(qkv, kv, self.n_heads):
             return ops.sdpa_cross_train(qkv, kv, mask, self.n_heads)

@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define BNB_ABI_VERSION 33
+#define BNB_ABI_VERSION 34
 
 /* element types of activation buffers */
 #define BNB_F32 0
@@ -359,11 +359,14 @@ int bnb_sdpa_cross_bwd(const void *q, int64_t q_row_stride, int NQ, const void *
  * The same backward over key/value rows compacted beforehand (the counterpart of
  * bnb_sdpa_cross_ranges_fwd): environment b reads rows ranges[b] .. ranges[b+1]-1 of kv_rows
  * (capacity rows of [K | V], all of them live), at most max_keys <= 160 per environment;
- * dkv_rows has kv_rows' layout.  An environment with an empty range gets a zero dq.
+ * dkv_rows has kv_rows' layout.  dq rows are dq_row_stride elements apart (a multiple of 8, at least H * dh);
+ * dq_add 0: they are written, and an environment with an empty range gets zeros; 1: the gradient is added to what
+ * they hold (in float32, rounded once), e.g. the query third that bnb_sdpa_masked_bwd wrote of a (B, NQ, 3D) gradient.
  */
 int bnb_sdpa_cross_ranges_bwd(const void *q, int64_t q_row_stride, int NQ, const void *kv_rows, int64_t kv_row_stride,
                               const int32_t *ranges, int64_t capacity, int max_keys, const void *out, const void *dout,
-                              void *dq, void *dkv_rows, int64_t B, int H, int dh, int dtype, void *stream);
+                              void *dq, int64_t dq_row_stride, int dq_add, void *dkv_rows, int64_t B, int H, int dh, int dtype,
+                              void *stream);
 
 /*
  * The bullet read's backward for ANY number of live keys per environment (bf16, dh = 32, NQ <= 160):
@@ -374,15 +377,14 @@ int bnb_sdpa_cross_ranges_bwd(const void *q, int64_t q_row_stride, int NQ, const
  * bnb_sdpa_cross_ranges_bwd).  row_index != NULL: entry e is row row_index[e] of kv, i.e. the (B, NK, 2D)
  * buffer is read in place through the list of its live slots (bnb_mask_count / bnb_mask_fill); dkv then
  * has that layout too and the rows of slots that are not listed are NOT written (zero them beforehand).
- * out is the read's own result (nothing accumulated), dq (B, NQ, D) contiguous, dkv has kv's row
+ * out is the read's own result (nothing accumulated), dq as for bnb_sdpa_cross_ranges_bwd, dkv has kv's row
  * stride 2D.  stats: workspace of 2 * B * H * NQ floats (per query and head: log2-sum-exp and
- * rowsum(dout * out), written by the first kernel, read by the second).  An environment with an
- * empty range gets a zero dq.
+ * rowsum(dout * out), written by the first kernel, read by the second).
  */
 int bnb_sdpa_cross_stream_bwd(const void *q, int64_t q_row_stride, int NQ, const void *kv, int64_t kv_row_stride,
                               const int32_t *ranges, const int32_t *row_index, int64_t capacity, const void *out,
-                              const void *dout, void *dq, void *dkv, float *stats, int64_t B, int H, int dh, int dtype,
-                              void *stream);
+                              const void *dout, void *dq, int64_t dq_row_stride, int dq_add, void *dkv, float *stats, int64_t B,
+                              int H, int dh, int dtype, void *stream);
 
 /*
  * bnb_sdpa_cross_stream_bwd with the log2-sum-exp of every query taken from the forward pass
@@ -392,8 +394,8 @@ int bnb_sdpa_cross_stream_bwd(const void *q, int64_t q_row_stride, int NQ, const
  */
 int bnb_sdpa_cross_stream_bwd_lse(const void *q, int64_t q_row_stride, int NQ, const void *kv, int64_t kv_row_stride,
                                   const int32_t *ranges, const int32_t *row_index, int64_t capacity, const void *out,
-                                  const void *dout, const float *lse, void *dq, void *dkv, float *stats, int64_t B,
-                                  int H, int dh, int dtype, void *stream);
+                                  const void *dout, const float *lse, void *dq, int64_t dq_row_stride, int dq_add, void *dkv,
+                                  float *stats, int64_t B, int H, int dh, int dtype, void *stream);
 
 /*
  * RMSNorm backward:  y = x * rsqrt(mean(x^2) + eps) * weight

@@ -2518,6 +2518,41 @@ def test_sdpa_cross_train_is_differentiable():
     assert not ops.sdpa_cross_train_supported(qkv.float(), torch.zeros(B, 80, 2 * D, device=DEV), H)
 
 
+@pytest.mark.parametrize("B,NQ,NK,p_live", [(1, 1, 8, 0.5), (37, 12, 40, 0.3), (9, 33, 160, 0.9), (5, 84, 500, 0.8), (3, 160, 300, 0.7), (16, 16, 12, 0.05)])
+def test_self_attention_and_read_share_one_backward(B, NQ, NK, p_live):
+    """``sdpa_read_train`` against the two functions it joins: one partly filled block of queries to five, lists on both sides of the
+    160 keys that the single-tile backward takes, environments without a bullet or a live token."""
+    H, D = 4, 128
+    g = torch.Generator().manual_seed(B * NQ + NK)
+    qkv = torch.randn(B, NQ, 3 * D, generator=g).to(DEV, torch.bfloat16)
+    mask = torch.rand(B, NK, generator=g) < p_live
+    mask[0, 0] = True
+    if B > 2:
+        mask[1] = False
+    alive = torch.rand(B, NQ, generator=g) < 0.8
+    if B > 3:
+        alive[2] = False
+    alive, rows = alive.to(DEV), ops.CompactRows(mask.to(DEV))
+    kv = torch.randn(rows.total_host(), 2 * D, generator=g).to(DEV, torch.bfloat16)
+    up = torch.randn(B, NQ, D, generator=g).to(DEV, torch.bfloat16)
+
+    def grads(fn):
+        q, k = qkv.clone().requires_grad_(), kv.clone().requires_grad_()
+        out = fn(q, k)
+        return (out.detach(),) + torch.autograd.grad(out, (q, k), up)
+
+    out, dqkv, dkv = grads(lambda q, k: ops.sdpa_read_train(q, alive, k, rows, H))
+    out_s, dqkv_s, dkv_s = grads(lambda q, k: ops.sdpa_train(q, alive, H) + ops.sdpa_cross_rows_train(q, k, rows, H))
+    assert torch.equal(out, out_s) and torch.equal(dkv, dkv_s) and torch.equal(dqkv[..., D:], dqkv_s[..., D:])
+    _, own, _ = grads(lambda q, k: ops.sdpa_train(q, alive, H) + 0 * k.sum())
+    _, read, _ = grads(lambda q, k: ops.sdpa_cross_rows_train(q, k, rows, H))
+    a, b = own[..., :D].double(), read[..., :D].double()
+    # b was rounded to bfloat16 (half of 2^-7 of it at most) before this sum, the joined gradient after it
+    assert ((dqkv[..., :D].double() - (a + b)).abs() <= 2.0 ** -8 * (b.abs() + 1.01 * (a + b).abs()) + 1e-30).all()
+    if B > 2:
+        assert torch.equal(dqkv[1, :, :D], own[1, :, :D])  # nothing to read: the self-attention's gradient stays
+
+
 @pytest.mark.parametrize("B,NQ,NK,p_live", [
     (3, 12, 200, 0.5), (4, 23, 480, 0.3), (2, 160, 1520, 0.25), (3, 84, 800, 1.0), (5, 152, 2048, 0.05), (3, 33, 161, 1.0),
     (4, 12, 80, 0.25), (6, 64, 1520, 0.02), (2, 97, 2048, 1.0),

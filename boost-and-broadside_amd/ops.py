@@ -22,13 +22,30 @@ import torch
 from . import _native
 
 _DTYPE_CODE = {torch.float32: _native.F32, torch.bfloat16: _native.BF16}
+class _autocast_off:
+    """``torch.autocast("cuda", enabled=False)`` around calls that state their dtypes themselves: only the flag, and only where
+    autocast is on (the general context costs 5 us a use; a pass of the update enters sixty)."""
+
+    __slots__ = ("was_on",)
+
+    def __enter__(self):
+        self.was_on = torch.is_autocast_enabled("cuda")
+        if self.was_on:
+            torch.set_autocast_enabled("cuda", False)
+
+    def __exit__(self, *exc):
+        if self.was_on:
+            torch.set_autocast_enabled("cuda", True)
+        return False
+
+
 def _outside_autocast(backward):
     """A custom Function's backward inherits the autocast state of the place ``.backward()`` is called
     from; inside it torch GEMMs would return bfloat16 tensors where the kernels are handed float32
     pointers.  Every backward here runs with autocast off and states its dtypes itself."""
     @functools.wraps(backward)
     def wrapped(ctx, *grads):
-        with torch.autocast("cuda", enabled=False):
+        with _autocast_off():
             return backward(ctx, *grads)
     return wrapped
 
@@ -219,7 +236,7 @@ class _SdpaTrain(torch.autograd.Function):
 
 def sdpa_train(qkv: torch.Tensor, alive: torch.Tensor | None, n_heads: int) -> torch.Tensor:
     """Differentiable ``sdpa_masked`` (use where ``sdpa_train_supported`` holds)."""
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _SdpaTrain.apply(qkv, alive, n_heads)
 
 
@@ -433,7 +450,7 @@ class _SdpaCrossTrain(torch.autograd.Function):
 
 def sdpa_cross_train(qkv: torch.Tensor, kv: torch.Tensor, key_mask: torch.Tensor | None, n_heads: int) -> torch.Tensor:
     """Differentiable ``sdpa_cross``: the entity queries' read of a second key/value set, (B, NQ, D)."""
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _SdpaCrossTrain.apply(qkv, kv, key_mask, n_heads)
 
 
@@ -505,7 +522,7 @@ def sdpa_cross_rows_train(qkv: torch.Tensor, kv_rows: torch.Tensor, rows: "Compa
     total = rows.total_host()
     if kv_rows.shape[0] != total:
         raise ValueError(f"kv_rows must hold the {total} listed rows")
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _SdpaCrossRowsTrain.apply(qkv, kv_rows.contiguous(), rows, n_heads, total)
 
 
@@ -541,7 +558,7 @@ def sdpa_read_train(qkv: torch.Tensor, alive: torch.Tensor | None, kv_rows: torc
     total = rows.total_host()
     if kv_rows.shape[0] != total or total == 0:
         raise ValueError(f"kv_rows must hold the {total} listed rows, at least one")
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _SdpaReadTrain.apply(qkv, kv_rows.contiguous(), alive, rows, n_heads, total)
 
 
@@ -764,8 +781,8 @@ def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, out: torch.Tensor | None = N
         raise ValueError("linear_wgrad covers weight shapes whose dimensions are multiples of 128")
     _need_device(dy, "dy")
     _need_device(x, "x")
-    dy2 = dy.reshape(-1, N) if _uniform_rows(dy, N) else dy.reshape(-1, N).contiguous()
-    x2 = x.reshape(-1, K) if _uniform_rows(x, K) else x.reshape(-1, K).contiguous()
+    dy2 = _rows(dy, N)
+    x2 = _rows(x, K)
     R = dy2.shape[0]
     if out is None:
         if accumulate:
@@ -866,7 +883,7 @@ def linear_train(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     """``F.linear(x, weight, bias)`` as bfloat16 autocast computes it, differentiable, with the weight
     gradient accumulated in float32 by ``linear_wgrad`` instead of a library GEMM that contracts
     over the (very long) row axis.  Use where ``linear_wgrad_supported`` holds."""
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _LinearTrain.apply(x, weight, bias)
 
 
@@ -957,7 +974,7 @@ def team_pool(x: torch.Tensor, team_id: torch.Tensor, alive: torch.Tensor, score
                 B, N, int(n_heads), D, _stream(),
             )
             _native.check(rc, "bnb_team_attend_fwd")
-            with torch.autocast("cuda", enabled=False):
+            with _autocast_off():
                 pre = torch.mm(z, folded_projection)
             rc = lib.bnb_team_norm_broadcast_fwd(
                 pre.data_ptr(), norm_weight.detach().contiguous().data_ptr(), float(eps), team_id.data_ptr(),
@@ -1059,7 +1076,7 @@ class _TeamPoolTrain(torch.autograd.Function):
 def team_pool_train(x, team_id, alive, score_vectors, folded_projection, norm_weight, eps, n_heads) -> torch.Tensor:
     """Differentiable ``team_pool`` (the (B, N, 128) broadcast form); ``score_vectors`` and
     ``folded_projection`` from ``team_pool_constants`` so that their gradients reach the parameters."""
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _TeamPoolTrain.apply(x, team_id, alive, score_vectors, folded_projection, norm_weight, eps, n_heads)
 
 
@@ -1396,7 +1413,7 @@ def conv_seq_train(b1, conv_buf, weight, bias, done=None, *, time_major: bool = 
 
     ``also_bf16``: a third result, the bfloat16 rounding of ``v`` written by the same launch (what a bfloat16
     projection of ``v`` would cast for itself); its gradient is added to ``v``'s inside the backward kernel."""
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         v, new_buf, v_lp = _ConvSeqTrain.apply(b1, conv_buf, weight, bias, done, time_major, also_bf16)
     return (v, new_buf, v_lp) if also_bf16 else (v, new_buf)
 
@@ -1627,7 +1644,7 @@ def temporal_mix_train(b1, n, conv_buf, conv_weight, conv_bias, gate_weight, gat
 
     ``gate_weight`` (2D, D) and ``gate_bias`` (2D,) are ``[linear_a | linear_x]``; ``h0`` (B*n, D), ``conv_buf``
     (B*n, 3, D) float32 and ``done`` ((B*n, T) or None) are env-major like the recurrent state."""
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _TemporalMixTrain.apply(b1.contiguous(), int(n), conv_buf, conv_weight, conv_bias, gate_weight, gate_bias, log_lambda,
                                        float(c), h0, done, field_weight)
 
@@ -1704,13 +1721,13 @@ def rmsnorm_bwd(x: torch.Tensor, dy: torch.Tensor, weight: torch.Tensor, *, eps:
         raise TypeError("grad_sum must be float32")
     _need_device(x, "x")
     _need_device(dy, "dy")
-    x2 = x.reshape(-1, D) if _uniform_rows(x, D) else x.reshape(-1, D).contiguous()
-    dy2 = dy.reshape(-1, D) if _uniform_rows(dy, D) else dy.reshape(-1, D).contiguous()
-    gs = None if grad_sum is None else grad_sum.reshape(-1, D).contiguous()
+    x2 = _rows(x, D)
+    dy2 = _rows(dy, D)
+    gs = None if grad_sum is None else grad_sum.contiguous()
     R = x2.shape[0]
-    dx = torch.empty((R, D), dtype=torch.float32, device=x.device)
+    dx = torch.empty(x.shape, dtype=torch.float32, device=x.device)
     dw = torch.empty((D,), dtype=torch.float32, device=x.device)
-    dx_lp = torch.empty((R, D), dtype=torch.bfloat16, device=x.device) if also_bf16 else None
+    dx_lp = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if also_bf16 else None
     lib = _native.load()
     blocks = int(lib.bnb_rmsnorm_bwd_blocks(R, D))
     partials = torch.empty((blocks, D), dtype=torch.float32, device=x.device)
@@ -1721,9 +1738,7 @@ def rmsnorm_bwd(x: torch.Tensor, dy: torch.Tensor, weight: torch.Tensor, *, eps:
                                  dx.data_ptr(), None if dx_lp is None else dx_lp.data_ptr(), partials.data_ptr(), blocks,
                                  dw.data_ptr(), R, D, _stream())
     _native.check(rc, "bnb_rmsnorm_bwd")
-    if also_bf16:
-        return dx.reshape(x.shape), dw, dx_lp.reshape(x.shape)
-    return dx.reshape(x.shape), dw
+    return (dx, dw, dx_lp) if also_bf16 else (dx, dw)
 
 
 def rmsnorm_bwd_static(x: torch.Tensor, dy: torch.Tensor, weight: torch.Tensor, dx: torch.Tensor, dw: torch.Tensor, *,
@@ -1880,7 +1895,7 @@ def norm_linear_train(x: torch.Tensor, norm_weight: torch.Tensor, weight: torch.
     projection of the same normalised rows.  ``packed``: ``pack_linear_weights(weight)``, if the caller caches it."""
     if packed is None:
         packed = pack_linear_weights(weight)
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _NormLinearTrain.apply(x, norm_weight, weight, eps, packed)
 
 
@@ -1895,7 +1910,7 @@ def rmsnorm_train(x: torch.Tensor, weight: torch.Tensor, *, delta: torch.Tensor 
     (an alias, to be used for the residual connection so that its gradient is added inside the backward
     kernel) without ``delta``.  ``normed`` is computed in float32 and rounded once to ``out_dtype`` (what
     ``nn.RMSNorm`` followed by autocast's cast in front of the next Linear gives)."""
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         if delta is None:
             return _RmsNormTrain.apply(x, weight, eps, out_dtype)
         return _AddRmsNormTrain.apply(x, delta, weight, eps, out_dtype)
@@ -2026,7 +2041,7 @@ def gelu_mul_packed_train(gu: torch.Tensor, *, out_dtype: torch.dtype | None = N
     if H2 % 16 or gu.dtype not in (torch.float32, torch.bfloat16):
         raise ValueError("gu must be float32 or bfloat16 with 2H channels, H a multiple of 8")
     _need_device(gu, "gu")
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _GeluMulPackedTrain.apply(gu, gu.dtype if out_dtype is None else out_dtype)
 
 
@@ -2038,7 +2053,7 @@ def gelu_mul_train_supported(a: torch.Tensor, b: torch.Tensor) -> bool:
 
 def gelu_mul_train(a: torch.Tensor, b: torch.Tensor, *, out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """Differentiable ``gelu_mul``."""
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _GeluMulTrain.apply(a, b, out_dtype)
 
 
@@ -2319,9 +2334,16 @@ def ffn_tail_train(x, delta, norm_weight, gate_w, up_w, down_w, *, eps: float | 
     if proj_weight is not None and (delta is None or proj_weight.shape != (FFN_WIDTH, FFN_WIDTH) or proj_packed.dtype != torch.bfloat16
                                     or proj_packed.numel() != FFN_WIDTH * FFN_WIDTH or not proj_packed.is_contiguous()):
         raise ValueError("the folded projection needs its operand rows, a (128, 128) weight and pack_proj_weights' output")
-    with torch.autocast("cuda", enabled=False):
+    with _autocast_off():
         return _FfnTailTrain.apply(x, delta, proj_weight, norm_weight, gate_w, up_w, down_w, _F32_EPS if eps is None else float(eps),
                                    packed_fwd, packed_bwd, proj_packed)
+
+
+def _rows(t: torch.Tensor, D: int) -> torch.Tensor:
+    """``t`` (..., D) as (R, D) rows at one pitch that the kernels read, copied only where it has none."""
+    if not _uniform_rows(t, D):
+        return t.reshape(-1, D).contiguous()
+    return t if t.dim() == 2 else t.view(-1, D)
 
 
 def _uniform_rows(t: torch.Tensor, D: int) -> bool:
@@ -2329,6 +2351,8 @@ def _uniform_rows(t: torch.Tensor, D: int) -> bool:
     column block of a contiguous wider matrix qualifies)."""
     if t.stride(-1) != 1 or t.dim() < 2:
         return False
+    if t.stride(-2) == D and t.shape[-1] == D and t.is_contiguous() and t.numel():
+        return D % 8 == 0 and t.data_ptr() % 16 == 0
     try:
         v = t.view(-1, D)
     except RuntimeError:
@@ -2501,7 +2525,7 @@ def linear_f32(x: torch.Tensor, weight_packed: torch.Tensor, *, bias: torch.Tens
     n_out = N // 2 if gate else N
     if torch.is_grad_enabled() and x.requires_grad:
         raise RuntimeError("linear_f32 is forward-only; call it under torch.no_grad()")
-    x2 = x.reshape(-1, K) if _uniform_rows(x, K) else x.reshape(-1, K).contiguous()
+    x2 = _rows(x, K)
     R = x2.shape[0]
     y2 = None
     if gelu_times is not None:

@@ -36,7 +36,7 @@ __device__ __forceinline__ int wg_slot(int c, int rb) { return c * kWgRows + 8 *
 __global__ __launch_bounds__(kWgThreads) void linear_wgrad_kernel(
     const uint16_t *__restrict__ dy, int64_t dy_stride, const uint16_t *__restrict__ x, int64_t x_stride,
     float *__restrict__ partials, int64_t R, int N, int K, int64_t rows_per_slice, int slices, int64_t dy_tile_stride,
-    int64_t x_tile_stride)
+    int64_t x_tile_stride, int64_t dy_block_stride, int64_t x_block_stride)
 {
     __shared__ __align__(16) uint16_t s_t[2][kWgTile * kWgRows];  // [operand: dy, x][column][row], swizzled
 
@@ -70,8 +70,9 @@ __global__ __launch_bounds__(kWgThreads) void linear_wgrad_kernel(
     const int rg = (tid & 127) >> 4;
     const int cb = tid & 15;
     // the 128 columns of a tile start `tile stride` elements after those of the tile before (128 for plain row-major
-    // operands; R * 128 for operands stored tile by tile)
-    const uint16_t *src = operand ? x + (k0 / kWgTile) * x_tile_stride + 8 * cb : dy + (n0 / kWgTile) * dy_tile_stride + 8 * cb;
+    // operands; R * 128 for operands stored tile by tile), 32 columns within it `block stride` after the 32 before (32 in a row)
+    const uint16_t *src = (operand ? x + (k0 / kWgTile) * x_tile_stride + (cb >> 2) * x_block_stride
+                                   : dy + (n0 / kWgTile) * dy_tile_stride + (cb >> 2) * dy_block_stride) + 8 * (cb & 3);
     const int64_t src_stride = operand ? x_stride : dy_stride;
     uint16_t *dst = s_t[operand];
 
@@ -175,7 +176,7 @@ __device__ __forceinline__ bf16x8 wd_operand(const unsigned char *p)
 __global__ __launch_bounds__(kWgThreads) void linear_wgrad_dma_kernel(
     const uint16_t *__restrict__ dy, int64_t dy_stride, const uint16_t *__restrict__ x, int64_t x_stride,
     float *__restrict__ partials, int64_t R, int N, int K, int64_t rows_per_slice, int slices, int64_t dy_tile_stride,
-    int64_t x_tile_stride)
+    int64_t x_tile_stride, int64_t dy_block_stride, int64_t x_block_stride)
 {
     __shared__ __align__(1024) unsigned char s_st[kWdStages][kWdStageBytes];  // [stage][operand][row][16 slots of 16 B]
 
@@ -208,6 +209,9 @@ __global__ __launch_bounds__(kWgThreads) void linear_wgrad_dma_kernel(
     // the four (clamped to the last row of the matrix), the offset the lane's row within them and its piece.
     const int d_row = lane >> 4;                       // 0..3, also row % 4 (instruction rows start at multiples of 4)
     const int d_piece = (lane & 15) ^ (2 * d_row);
+    // byte offset of the lane's piece within its row: piece / 4 is its block of 32 columns
+    const uint32_t dy_piece = ((uint32_t)(d_piece >> 2) * (uint32_t)dy_block_stride + 8u * (uint32_t)(d_piece & 3)) * 2u;
+    const uint32_t x_piece = ((uint32_t)(d_piece >> 2) * (uint32_t)x_block_stride + 8u * (uint32_t)(d_piece & 3)) * 2u;
     const uint16_t *dy_tile = dy + (n0 / kWgTile) * dy_tile_stride;
     const uint16_t *x_tile = x + (k0 / kWgTile) * x_tile_stride;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)&s_st[0][0];
@@ -220,8 +224,8 @@ __global__ __launch_bounds__(kWgThreads) void linear_wgrad_dma_kernel(
             const int64_t r = first + d_row;
             const uint32_t extra = (uint32_t)((r < R ? r : R - 1) - base_row);  // 0..3 rows below the base
             const uint32_t lds = lds0 + (uint32_t)(stage * kWdStageBytes + (8 * wave + 4 * q) * 256);
-            wd_dma16(dy_tile + base_row * dy_stride, (extra * (uint32_t)dy_stride + 8u * (uint32_t)d_piece) * 2u, lds);
-            wd_dma16(x_tile + base_row * x_stride, (extra * (uint32_t)x_stride + 8u * (uint32_t)d_piece) * 2u, lds + kWdRows * 256);
+            wd_dma16(dy_tile + base_row * dy_stride, extra * (uint32_t)dy_stride * 2u + dy_piece, lds);
+            wd_dma16(x_tile + base_row * x_stride, extra * (uint32_t)x_stride * 2u + x_piece, lds + kWdRows * 256);
         }
     };
     // rows of the last chunk that lie past the slice: the lanes that fetched them overwrite them with zeros
@@ -443,20 +447,28 @@ extern "C" int bnb_linear_wgrad_slices(int64_t R, int N, int K)
     return (int)s;
 }
 
-extern "C" int bnb_linear_wgrad_tiled_fwd(const void *dy, int64_t dy_row_stride, int64_t dy_tile_stride, const void *x,
-                                          int64_t x_row_stride, int64_t x_tile_stride, float *partials, int slices, float *dw,
-                                          int accumulate, int64_t R, int N, int K, void *stream)
+extern "C" int bnb_linear_wgrad_tiled_fwd(const void *dy, int64_t dy_row_stride, int64_t dy_tile_stride, int64_t dy_block_stride,
+                                          const void *x, int64_t x_row_stride, int64_t x_tile_stride, int64_t x_block_stride,
+                                          float *partials, int slices, float *dw, int accumulate, int64_t R, int N, int K,
+                                          void *stream)
 {
     using namespace bnb;
+    constexpr int kBlock = 32;
+    // a lane reaches its piece of a row, up to three blocks on, by a 32-bit byte offset
+    if (dy_block_stride < kBlock || x_block_stride < kBlock) return BNB_ERR_BAD_SHAPE;
+    if (dy_block_stride > BNB_WGRAD_MAX_BLOCK_STRIDE || x_block_stride > BNB_WGRAD_MAX_BLOCK_STRIDE) return BNB_ERR_UNSUPPORTED;
     if (R < 0 || N < 1 || K < 1 || slices < 1) return BNB_ERR_BAD_SHAPE;
     if (N % kWgTile != 0 || K % kWgTile != 0 || slices > 65535) return BNB_ERR_UNSUPPORTED;
     if (!dw || !partials || (R > 0 && (!dy || !x))) return BNB_ERR_NULL_POINTER;
-    // row-major operands hold all their columns in a row; tile-by-tile ones 128 per row
-    if (dy_row_stride < (dy_tile_stride == kWgTile ? N : kWgTile) || x_row_stride < (x_tile_stride == kWgTile ? K : kWgTile) ||
+    // row-major operands hold all their columns in a row; tile-by-tile ones 128 per row, block-by-block ones 32
+    const auto row_needs = [](int64_t tile_stride, int64_t block_stride, int columns) {
+        return block_stride != kBlock ? kBlock : tile_stride == kWgTile ? columns : kWgTile;
+    };
+    if (dy_row_stride < row_needs(dy_tile_stride, dy_block_stride, N) || x_row_stride < row_needs(x_tile_stride, x_block_stride, K) ||
         dy_tile_stride < kWgTile || x_tile_stride < kWgTile)
         return BNB_ERR_BAD_SHAPE;
     if ((R > 0 && (!aligned16(dy) || !aligned16(x))) || !aligned16(partials) || !aligned16(dw) || dy_row_stride % 8 != 0 ||
-        x_row_stride % 8 != 0 || dy_tile_stride % 8 != 0 || x_tile_stride % 8 != 0)
+        x_row_stride % 8 != 0 || dy_tile_stride % 8 != 0 || x_tile_stride % 8 != 0 || dy_block_stride % 8 != 0 || x_block_stride % 8 != 0)
         return BNB_ERR_MISALIGNED;
     hipStream_t s = (hipStream_t)stream;
     const int64_t rows_per_slice = ((R + slices - 1) / slices + kWgRows - 1) / kWgRows * kWgRows;
@@ -465,11 +477,12 @@ extern "C" int bnb_linear_wgrad_tiled_fwd(const void *dy, int64_t dy_row_stride,
     if (wgrad_dma())
         hipLaunchKernelGGL(linear_wgrad_dma_kernel, dim3((unsigned)groups), dim3(kWgThreads), 0, s, (const uint16_t *)dy,
                            dy_row_stride, (const uint16_t *)x, x_row_stride, partials, R, N, K,
-                           rows_per_slice > 0 ? rows_per_slice : kWgRows, slices, dy_tile_stride, x_tile_stride);
+                           rows_per_slice > 0 ? rows_per_slice : kWgRows, slices, dy_tile_stride, x_tile_stride, dy_block_stride,
+                           x_block_stride);
     else
         hipLaunchKernelGGL(linear_wgrad_kernel, dim3((unsigned)groups), dim3(kWgThreads), 0, s, (const uint16_t *)dy, dy_row_stride,
                            (const uint16_t *)x, x_row_stride, partials, R, N, K, rows_per_slice > 0 ? rows_per_slice : kWgRows, slices,
-                           dy_tile_stride, x_tile_stride);
+                           dy_tile_stride, x_tile_stride, dy_block_stride, x_block_stride);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     return launch_sum_slices(partials, dw, (int64_t)N * K, slices, accumulate, s);
@@ -479,6 +492,6 @@ extern "C" int bnb_linear_wgrad_fwd(const void *dy, int64_t dy_row_stride, const
                                     float *partials, int slices, float *dw, int accumulate, int64_t R, int N, int K,
                                     void *stream)
 {
-    return bnb_linear_wgrad_tiled_fwd(dy, dy_row_stride, bnb::kWgTile, x, x_row_stride, bnb::kWgTile, partials, slices, dw,
+    return bnb_linear_wgrad_tiled_fwd(dy, dy_row_stride, bnb::kWgTile, 32, x, x_row_stride, bnb::kWgTile, 32, partials, slices, dw,
                                       accumulate, R, N, K, stream);
 }

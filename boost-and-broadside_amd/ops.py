@@ -801,25 +801,31 @@ def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, out: torch.Tensor | None = N
 
 
 def _linear_wgrad_tiled(dy_tiles: torch.Tensor, x_tiles: torch.Tensor, R: int) -> torch.Tensor:
-    """``dW = dy^T x`` over the first R rows of operands stored tile by tile: ``dy_tiles`` (N/128, >= R, 128) and
-    ``x_tiles`` (K/128, >= R, 128) contiguous bfloat16 (a plain (>= R, 128) matrix is one tile).  Returns (N, K) float32."""
+    """``dW = dy^T x`` over the first R rows of operands stored tile by tile, ``dy_tiles`` (N/128, >= R, 128) and
+    ``x_tiles`` (K/128, >= R, 128) contiguous bfloat16 (a plain (>= R, 128) matrix is one tile), or block by block
+    (N/32, >= R, 32).  Returns (N, K) float32."""
     if dy_tiles.dim() == 2:
         dy_tiles = dy_tiles.unsqueeze(0)
     if x_tiles.dim() == 2:
         x_tiles = x_tiles.unsqueeze(0)
     for t, name in ((dy_tiles, "dy_tiles"), (x_tiles, "x_tiles")):
         _need_device(t, name)
-        if t.dtype != torch.bfloat16 or not t.is_contiguous() or t.dim() != 3 or t.shape[2] != 128 or t.shape[1] < R:
-            raise ValueError(f"{name} must be a contiguous bfloat16 (tiles, >= {R}, 128) tensor")
-    N, K = 128 * dy_tiles.shape[0], 128 * x_tiles.shape[0]
+        if (t.dtype != torch.bfloat16 or not t.is_contiguous() or t.dim() != 3 or t.shape[1] < R
+                or not (t.shape[2] == 128 or t.shape[2] == 32 and t.shape[0] % 4 == 0)):
+            raise ValueError(f"{name} must be a contiguous bfloat16 (tiles, >= {R}, 128) or (blocks, >= {R}, 32) tensor")
+    N, K = (t.shape[0] * t.shape[2] for t in (dy_tiles, x_tiles))
+
+    def strides(t):  # of rows, tiles and blocks
+        rows = max(t.shape[1], 1)
+        return (128, rows * 128, 32) if t.shape[2] == 128 else (32, rows * 128, rows * 32)
+
     out = torch.empty((N, K), dtype=torch.float32, device=dy_tiles.device)
     lib = _native.load()
     slices = int(lib.bnb_linear_wgrad_slices(R, N, K))
     partials = torch.empty((slices, N, K), dtype=torch.float32, device=dy_tiles.device)
     with _on_device(dy_tiles.device):
-        rc = lib.bnb_linear_wgrad_tiled_fwd(dy_tiles.data_ptr(), 128, max(dy_tiles.shape[1], 1) * 128, x_tiles.data_ptr(), 128,
-                                            max(x_tiles.shape[1], 1) * 128, partials.data_ptr(), slices, out.data_ptr(), 0, R, N, K,
-                                            _stream())
+        rc = lib.bnb_linear_wgrad_tiled_fwd(dy_tiles.data_ptr(), *strides(dy_tiles), x_tiles.data_ptr(), *strides(x_tiles),
+                                            partials.data_ptr(), slices, out.data_ptr(), 0, R, N, K, _stream())
     _native.check(rc, "bnb_linear_wgrad_tiled_fwd")
     return out
 
@@ -2190,14 +2196,18 @@ def pack_ffn_bwd_weights(gate_w: torch.Tensor, up_w: torch.Tensor, down_w: torch
     return torch.cat([x.reshape(16, -1) for x in (s0, s1, s2, s3, s4)], dim=1).contiguous()
 
 
-def ffn_bwd(n: torch.Tensor, dy: torch.Tensor, weights_packed: torch.Tensor):
+_FFN_BLOCK_ROWS = (1 << 28) // 32  # BNB_WGRAD_MAX_BLOCK_STRIDE: rows up to which the weight-gradient kernel reaches a tile's blocks
+
+
+def ffn_bwd(n: torch.Tensor, dy: torch.Tensor, weights_packed: torch.Tensor, *, by_blocks: bool = False):
     """Backward of ``y = down(gelu(gate(n)) * up(n))`` with the gate/up activations recomputed on chip.
 
     n (R, 128) bfloat16 contiguous, dy (R, 128) float32 or bfloat16, ``weights_packed`` from
     ``pack_ffn_bwd_weights``.  Returns ``(dn, dgu, h, dy_bf16)``: dn (R, 128) bfloat16; ``dgu`` (8, Rp, 128) and
     ``h`` (4, Rp, 128) bfloat16, the tile-by-tile operands of the weight gradients (see ``ffn_weight_grads``;
     Rp is R rounded up to a multiple of 256, rows past R are don't-cares); dy rounded to bfloat16 (dy itself
-    when it already is)."""
+    when it already is).  ``by_blocks``: ``dgu`` (32, Rp, 32), the 16 blocks of gate before those of up, and ``h`` (16, Rp, 32),
+    which leave in longer runs."""
     D = FFN_WIDTH
     _need_device(n, "n")
     _need_device(dy, "dy")
@@ -2213,14 +2223,15 @@ def ffn_bwd(n: torch.Tensor, dy: torch.Tensor, weights_packed: torch.Tensor):
     Rp = (R + 255) // 256 * 256
     dev = n.device
     dn = torch.empty((Rp, D), dtype=torch.bfloat16, device=dev)
-    dgu = torch.empty((8, Rp, 128), dtype=torch.bfloat16, device=dev)
-    h = torch.empty((4, Rp, 128), dtype=torch.bfloat16, device=dev)
+    wide, unit = (4, 32) if by_blocks else (1, 128)
+    dgu = torch.empty((8 * wide, Rp, unit), dtype=torch.bfloat16, device=dev)
+    h = torch.empty((4 * wide, Rp, unit), dtype=torch.bfloat16, device=dev)
     dy_lp = torch.empty((Rp, D), dtype=torch.bfloat16, device=dev) if dy.dtype == torch.float32 else None
     if R:
         with _on_device(dev):
             rc = _native.load().bnb_ffn_bwd(n.data_ptr(), dy.data_ptr(), _code(dy, "dy"), dy.stride(0), weights_packed.data_ptr(),
                                             dn.data_ptr(), dgu.data_ptr(), h.data_ptr(),
-                                            None if dy_lp is None else dy_lp.data_ptr(), R, Rp, D, FFN_HIDDEN, _stream())
+                                            None if dy_lp is None else dy_lp.data_ptr(), R, Rp, int(by_blocks), D, FFN_HIDDEN, _stream())
         _native.check(rc, "bnb_ffn_bwd")
     return dn[:R], dgu, h, (dy if dy_lp is None else dy_lp[:R])
 
@@ -2228,6 +2239,9 @@ def ffn_bwd(n: torch.Tensor, dy: torch.Tensor, weights_packed: torch.Tensor):
 def ffn_weight_grads(n: torch.Tensor, dgu: torch.Tensor, h: torch.Tensor, dy_bf16: torch.Tensor):
     """``(d gate_proj.weight, d up_proj.weight, d down_proj.weight)`` (float32) from ``ffn_bwd``'s operands."""
     R = n.shape[0]
+    if dgu.shape[2] == 32:  # by blocks: gate and up one after the other, in the units' own order
+        d_gate, d_up = _linear_wgrad_tiled(dgu, n, R).view(2, FFN_HIDDEN, FFN_WIDTH).unbind()
+        return d_gate, d_up, _linear_wgrad_tiled(dy_bf16, h, R)
     dw = _linear_wgrad_tiled(dgu, n, R).view(8, 2, 2, 32, FFN_WIDTH)  # [pair][chunk in pair][gate, up][unit][channel]
     d_gate = dw[:, :, 0].reshape(FFN_HIDDEN, FFN_WIDTH)
     d_up = dw[:, :, 1].reshape(FFN_HIDDEN, FFN_WIDTH)
@@ -2290,7 +2304,7 @@ class _FfnTailTrain(torch.autograd.Function):
         if dout2.dtype != torch.float32:
             dout2 = dout2.float()
         dout2 = dout2.contiguous()
-        dn, dgu, h, dy_lp = ffn_bwd(n, dout2, packed_bwd)
+        dn, dgu, h, dy_lp = ffn_bwd(n, dout2, packed_bwd, by_blocks=n.shape[0] + 255 < _FFN_BLOCK_ROWS)
         need_w = ctx.needs_input_grad[4] or ctx.needs_input_grad[5] or ctx.needs_input_grad[6]
         d_gate = d_up = d_down = None
         if need_w:

@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define BNB_ABI_VERSION 34
+#define BNB_ABI_VERSION 35
 
 /* element types of activation buffers */
 #define BNB_F32 0
@@ -293,11 +293,15 @@ int bnb_linear_wgrad_fwd(const void *dy, int64_t dy_row_stride, const void *x, i
 /*
  * The same with operands that may be stored tile by tile: the 128 columns 128j .. 128j+127 of dy
  * start dy_tile_stride elements after those of tile j-1 (128 = plain row-major rows; R * 128 with
- * dy_row_stride 128 = a (N/128, R, 128) array), likewise x.  bnb_ffn_bwd writes such operands.
+ * dy_row_stride 128 = a (N/128, R, 128) array), likewise x.  Within a tile 32 columns start dy_block_stride elements
+ * after the 32 before (32 = in a row; with R * 32, a tile stride of R * 128 and a row stride of 32: a (N/32, R, 32) array),
+ * at most BNB_WGRAD_MAX_BLOCK_STRIDE (else BNB_ERR_UNSUPPORTED).  bnb_ffn_bwd writes such operands.
  */
-int bnb_linear_wgrad_tiled_fwd(const void *dy, int64_t dy_row_stride, int64_t dy_tile_stride, const void *x,
-                               int64_t x_row_stride, int64_t x_tile_stride, float *partials, int slices, float *dw,
-                               int accumulate, int64_t R, int N, int K, void *stream);
+#define BNB_WGRAD_MAX_BLOCK_STRIDE (1ll << 28)
+int bnb_linear_wgrad_tiled_fwd(const void *dy, int64_t dy_row_stride, int64_t dy_tile_stride, int64_t dy_block_stride,
+                               const void *x, int64_t x_row_stride, int64_t x_tile_stride, int64_t x_block_stride,
+                               float *partials, int slices, float *dw, int accumulate, int64_t R, int N, int K,
+                               void *stream);
 
 /*
  * Bias gradient of a Linear layer:  out[n] (+)= sum_r x[r][n], fp32 sums of bf16 or fp32 rows.
@@ -875,17 +879,21 @@ int bnb_ffn_fused_proj_train_fwd(const float *x, int64_t x_row_stride, const voi
  *   out_rows  rows that every result has room for: a multiple of 256, >= R.  The kernel stores whole
  *        work-groups of 256 rows without a bounds test (rows R .. out_rows-1 receive don't-care values)
  *   dn   (out_rows, 128) bf16 contiguous: gradient of n in rows 0 .. R-1
+ *   by_blocks 1:
+ *   dgu  (32, out_rows, 32) bf16: dg of hidden units 32c .. 32c+31 in block c, du in block 16 + c
+ *   h    (16, out_rows, 32) bf16
+ *   by_blocks 0:
  *   dgu  (8, out_rows, 128) bf16: tile p holds, for hidden chunks 2p and 2p+1 (32 units each),
  *        [dg chunk 2p | du chunk 2p | dg chunk 2p+1 | du chunk 2p+1]
  *   h    (4, out_rows, 128) bf16: tile q holds hidden units 128q .. 128q+127
- *        (both are operands for bnb_linear_wgrad_tiled_fwd with tile stride out_rows * 128: dW(gate,up) =
- *        dgu^T n in dgu's column order, dWd = dy^T h)
+ *        (all are operands for bnb_linear_wgrad_tiled_fwd with tile stride out_rows * 128, by blocks with block stride
+ *        out_rows * 32: dW(gate,up) = dgu^T n in dgu's column order, dWd = dy^T h)
  *   dy_bf16  optional (out_rows, 128) bf16 contiguous: dy rounded to bf16, when dy is fp32 (the other operand of dWd)
  * Requirements: D == 128, hidden == 512 (else BNB_ERR_UNSUPPORTED), 16-byte aligned pointers.
  */
 int bnb_ffn_bwd(const void *n, const void *dy, int dy_dtype, int64_t dy_row_stride, const void *weights_packed,
-                void *dn, void *dgu, void *h, void *dy_bf16, int64_t R, int64_t out_rows, int D, int hidden,
-                void *stream);
+                void *dn, void *dgu, void *h, void *dy_bf16, int64_t R, int64_t out_rows, int by_blocks, int D,
+                int hidden, void *stream);
 
 /*
  * bnb_ffn_fused_fwd with the sublayer's output projection folded in: the tensor added to x

@@ -1119,6 +1119,30 @@ def test_ffn_bwd_matches_autograd_of_the_oracle(R, dy_dtype):
     assert torch.equal(again[0], dn) and torch.equal(again[1][:, :R], dgu[:, :R]) and torch.equal(again[2][:, :R], h[:, :R])
 
 
+@pytest.mark.parametrize("R,dy_dtype", [(1, torch.float32), (31, torch.bfloat16), (255, torch.float32), (257, torch.bfloat16), (20001, torch.float32)])
+@pytest.mark.parametrize("path", ["auto", "staged"])
+def test_ffn_bwd_by_blocks_holds_what_the_tiles_hold(R, dy_dtype, path):
+    """The two layouts of the weight-gradient operands: the same numbers and, every result a sum over the rows in the same order,
+    the same weight gradients bit for bit, on both weight-gradient kernels."""
+    from boost_and_broadside_amd import _native
+    _, _, _, p = _ffn_case(R + 5, R)
+    g = torch.Generator().manual_seed(R)
+    n, dy = torch.randn(R, 128, generator=g).bfloat16().to(DEV), torch.randn(R, 128, generator=g).to(DEV, dy_dtype)
+    pk = ops.pack_ffn_bwd_weights(*(p[k].to(DEV) for k in ("f.gate_proj.weight", "f.up_proj.weight", "f.down_proj.weight")))
+    dn, dgu, h, lp = ops.ffn_bwd(n, dy, pk)
+    dn_b, dgu_b, h_b, lp_b = ops.ffn_bwd(n, dy, pk, by_blocks=True)
+    assert torch.equal(dn, dn_b) and torch.equal(lp, lp_b)
+    t = dgu[:, :R].permute(1, 0, 2).reshape(R, 16, 2, 32).permute(2, 1, 0, 3).reshape(32, R, 32)
+    assert torch.equal(dgu_b[:, :R], t) and torch.equal(h_b[:, :R], h[:, :R].permute(1, 0, 2).reshape(R, 16, 32).permute(1, 0, 2))
+    lib = _native.load()
+    assert lib.bnb_linear_wgrad_path({"auto": 0, "staged": 1}[path]) == 0
+    try:
+        for a, b in zip(ops.ffn_weight_grads(n, dgu, h, lp), ops.ffn_weight_grads(n, dgu_b, h_b, lp_b)):
+            assert torch.equal(a, b) and b.is_contiguous()
+    finally:
+        lib.bnb_linear_wgrad_path(0)
+
+
 def test_ffn_bwd_at_update_size_on_sampled_rows():
     # the update's row count at 4v4 (128 steps x 256 environments x 12 tokens): six rounds of resident work-groups
     R = 128 * 256 * 12

@@ -332,9 +332,63 @@ __global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict
     }
 }
 
+// The same for few elements under many slices (a norm's weight gradient: 128 elements, 1,280 slices), where work-groups of 64
+// elements leave the sums to one or two CUs, each a long chain of loads: 16 elements (4 lanes x 4 floats) a work-group, 256 lane
+// groups that add every 256th slice, then 16 sums of 16 groups, then those, all in a fixed order.
+// 128 elements x 1,280 slices 8.9 -> 4.7 us, 1,024 x 2,048 13.4 -> 6.7 us.
+constexpr int kSsGroups = 256;
+
+__global__ __launch_bounds__(4 * kSsGroups) void sum_slices_few_kernel(const float *__restrict__ partials, float *__restrict__ dw,
+                                                                       int64_t elems, int slices, int accumulate)
+{
+    __shared__ f32x4 s_sum[kSsGroups][4], s_part[16][4];
+    const int q = threadIdx.x & 3, g = threadIdx.x >> 2;
+    const int64_t i = ((int64_t)blockIdx.x * 4 + q) * 4;  // elems is a multiple of 64
+    f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+    int k = g;
+    for (; k + 3 * kSsGroups < slices; k += 4 * kSsGroups) {
+        f32x4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const f32x4 *>(partials + (int64_t)(k + kSsGroups * u) * elems + i);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s.x += v[u].x, s.y += v[u].y, s.z += v[u].z, s.w += v[u].w;
+    }
+    for (; k < slices; k += kSsGroups) {
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(partials + (int64_t)k * elems + i);
+        s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
+    }
+    s_sum[g][q] = s;
+    __syncthreads();
+    auto add16 = [&](const f32x4 (*from)[4]) {
+        f32x4 t = from[0][q];
+#pragma unroll
+        for (int u = 1; u < 16; ++u) {
+            const f32x4 v = from[u][q];
+            t.x += v.x, t.y += v.y, t.z += v.z, t.w += v.w;
+        }
+        return t;
+    };
+    if (g < 16) s_part[g][q] = add16(s_sum + 16 * g);
+    __syncthreads();
+    if (g == 0) {
+        f32x4 t = add16(s_part);
+        if (accumulate) {
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(dw + i);
+            t.x += v.x, t.y += v.y, t.z += v.z, t.w += v.w;
+        }
+        *reinterpret_cast<f32x4 *>(dw + i) = t;
+    }
+}
+
 int launch_sum_slices(const float *partials, float *out, int64_t elems, int slices, int accumulate, hipStream_t stream)
 {
     if (elems <= 0 || elems % 64 != 0 || slices < 0) return BNB_ERR_BAD_SHAPE;
+    // below 4,096 elements the wide form has fewer than 64 work-groups for 256 CUs
+    if (elems < 4096 && slices >= kSsGroups) {
+        hipLaunchKernelGGL(sum_slices_few_kernel, dim3((unsigned)(elems / 16)), dim3(4 * kSsGroups), 0, stream, partials, out, elems,
+                           slices, accumulate);
+        return (int)hipGetLastError();
+    }
     hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)(elems / 64)), dim3(256), 0, stream, partials, out, elems, slices,
                        accumulate);
     return (int)hipGetLastError();

@@ -1119,6 +1119,26 @@ def test_ffn_bwd_matches_autograd_of_the_oracle(R, dy_dtype):
     assert torch.equal(again[0], dn) and torch.equal(again[1][:, :R], dgu[:, :R]) and torch.equal(again[2][:, :R], h[:, :R])
 
 
+@pytest.mark.parametrize("D", [64, 128, 512])
+@pytest.mark.parametrize("blocks", [1, 255, 256, 257, 1023, 1024, 1025, 1280])
+def test_norm_weight_gradient_sums_every_partial_row(D, blocks):
+    """One partial row a work-group, on both sides of every count at which the kernels that add them change over."""
+    R = blocks * (2048 // D) - (blocks > 1)  # 2048 / D rows a work-group, the last one short of a row
+    g = torch.Generator().manual_seed(blocks + D)
+    x, dy, w = torch.randn(R, D, generator=g), torch.randn(R, D, generator=g), torch.randn(D, generator=g)
+    assert _norm_blocks(R, D) == blocks
+    _, dw = ops.rmsnorm_bwd(x.to(DEV), dy.to(DEV), w.to(DEV))
+    terms = dy.double() * x.double() * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + torch.finfo(torch.float32).eps)
+    # a term carries the rounding of rstd and two products, a sum passes through at most 2048 / D + 37 additions in float32
+    assert ((dw.cpu().double() - terms.sum(0)).abs() <= 75 * 2.0 ** -24 * terms.abs().sum(0)).all()
+
+
+def _norm_blocks(R, D):
+    from boost_and_broadside_amd import _native
+
+    return int(_native.load().bnb_rmsnorm_bwd_blocks(R, D))
+
+
 @pytest.mark.parametrize("R,dy_dtype", [(1, torch.float32), (31, torch.bfloat16), (255, torch.float32), (257, torch.bfloat16), (20001, torch.float32)])
 @pytest.mark.parametrize("path", ["auto", "staged"])
 def test_ffn_bwd_by_blocks_holds_what_the_tiles_hold(R, dy_dtype, path):

@@ -2143,9 +2143,10 @@ class EagerTrunkStepper:
 
 
 # tokens per step below which a captured step beats plain launches, with the default trunk of 2 blocks x (2 attention +
-# 1 temporal sublayer) and bullets: the launches of a step take the host ~0.6 ms (float32 0.78 ms), a captured step copies its inputs.
-# us a step, captured / plain.  float32: 7,920 tokens 558 / 778, 9,960 705 / 775, 10,240 (160 a battle) 815 / 801, 12,288 750 / 775,
-# 16,320 866 / 832.  bfloat16: 40,000 479 .. 558 / 590, 50,400 539 / 590, 64,000 735 / 674, 93,696 924 / 860.
+# 1 temporal sublayer) and bullets: the launches of a step take the host ~0.6 ms (float32 0.7 ms), a captured step copies its inputs.
+# us a step, captured / plain.  float32: 7,920 tokens 370 / 696, 10,080 548 / 695, 12,240 582 / 701, 16,320 678 / 702; 10,240 (160 a
+# battle) 683 / 691, 12,160 781 / 750: the line is where every fleet size gains.  bfloat16 (separate kernels): 40,000 479 .. 558 / 590,
+# 50,400 539 / 590, 64,000 735 / 674, 93,696 924 / 860.
 GRAPH_BELOW_TOKENS = {torch.float32: 10_000, torch.bfloat16: 40_000}
 
 

@@ -2240,8 +2240,8 @@ def ffn_weight_grads(n: torch.Tensor, dgu: torch.Tensor, h: torch.Tensor, dy_bf1
     """``(d gate_proj.weight, d up_proj.weight, d down_proj.weight)`` (float32) from ``ffn_bwd``'s operands."""
     R = n.shape[0]
     if dgu.shape[2] == 32:  # by blocks: gate and up one after the other, in the units' own order
-        d_gate, d_up = _linear_wgrad_tiled(dgu, n, R).view(2, FFN_HIDDEN, FFN_WIDTH).unbind()
-        return d_gate, d_up, _linear_wgrad_tiled(dy_bf16, h, R)
+        dw = _linear_wgrad_tiled(dgu, n, R)
+        return dw[:FFN_HIDDEN], dw[FFN_HIDDEN:], _linear_wgrad_tiled(dy_bf16, h, R)
     dw = _linear_wgrad_tiled(dgu, n, R).view(8, 2, 2, 32, FFN_WIDTH)  # [pair][chunk in pair][gate, up][unit][channel]
     d_gate = dw[:, :, 0].reshape(FFN_HIDDEN, FFN_WIDTH)
     d_up = dw[:, :, 1].reshape(FFN_HIDDEN, FFN_WIDTH)

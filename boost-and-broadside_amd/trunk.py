@@ -44,6 +44,7 @@ import collections
 import contextlib
 import copy
 import math
+import operator
 import warnings
 import weakref
 from dataclasses import dataclass
@@ -1562,25 +1563,54 @@ class _LiveRows:
         self.rows, self.chained = rows, chained
 
 
-class _LayoutWatch:
-    """Whether a module still consists of the same submodules and parameters, unwritten, without forward hooks and with its
-    derived weights valid (``invalidate_weight_caches``).  Keeps those weights alive."""
+class _WholeStep:
+    """The trunk's step as ``ops.trunk_step`` takes it (``table``, ``bullet_eps``) and everything that was laid out in it: the
+    submodules, the parameters with their addresses and write counts, the derived weights, the constants.
 
-    def __init__(self, module: nn.Module) -> None:
-        self.children = [(m._modules, name, child) for m in module.modules() for name, child in m._modules.items()]
-        self.params = [(m._parameters, name, p) for m in module.modules() for name, p in m._parameters.items()]
-        self.derived = [(m.__dict__, k, v) for m in module.modules() for k, v in m.__dict__.items()
-                        if k.startswith(_CACHE_PREFIX) and isinstance(v, _DerivedWeight)]
-        self.stamp = self._stamp()
+    The table holds addresses, so ``same`` (or ``weights_same``, for a user that follows the weights only) is asked before every launch.
+    ``aliases`` share a parameter's memory and its version counter: they keep what the table points to from being freed under it, and
+    are read in half the time of the parameter subclass."""
 
-    def _stamp(self) -> int:
-        return _weights_stamp([p for _, _, p in self.params if p is not None])
+    __slots__ = ("table", "bullet_eps", "tensors", "children", "slots", "params", "held", "aliases", "written", "derived", "constants",
+                 "values", "layers")
+
+    def __init__(self, trunk: nn.Module, layers: list, bullet_eps: float) -> None:
+        self.table, self.bullet_eps = ops.trunk_table(layers), bullet_eps
+        self.tensors = [t for entry in layers for t in entry.values() if isinstance(t, torch.Tensor)]
+        modules = list(trunk.modules())
+        self.children = [(m._modules, dict(m._modules)) for m in modules if m._modules]
+        self.slots = [(m._parameters, name) for m in modules for name in m._parameters]
+        self.params = [d[name] for d, name in self.slots]
+        used = {t.data_ptr() for t in self.tensors}
+        self.derived = [(m.__dict__, k, v) for m in modules for k, v in m.__dict__.items()
+                        if k.startswith(_CACHE_PREFIX) and isinstance(v, _DerivedWeight) and isinstance(v.value, torch.Tensor)
+                        and v.value.data_ptr() in used]
+        self.layers = [l for block in trunk.yemong_layers for l in (*block.spatial, *block.temporal)]
+        self.constants = [(m.__dict__, name) for m in modules for name in ("eps", "c", "n_heads", "reads_bullets") if name in m.__dict__]
+        self.values = self._values()
+        self.held = [p for p in self.params if p is not None]
+        self.aliases = [torch._C.TensorBase.detach(p) for p in self.held]
+        self.written = self._written()
+
+    def _values(self) -> list:
+        return [d.get(name) for d, name in self.constants]
+
+    def _written(self):
+        return (list(map(torch._C.TensorBase.data_ptr, self.held)), [a._version for a in self.aliases],
+                [getattr(p, "_bnb_touch", 0) for p in self.held])
+
+    def weights_same(self) -> bool:
+        """Whether the parameters that were laid out lie where they lay and hold what they held."""
+        return self._written() == self.written
 
     def same(self) -> bool:
-        return (all(d.get(name) is child and not child._forward_hooks and not child._forward_pre_hooks for d, name, child in self.children)
-                and all(d.get(name) is p for d, name, p in self.params)
+        """Whether a table laid out now would be this one: besides the weights the same submodules, parameters and constants, no forward
+        hooks, no derived weight invalidated."""
+        return (all(now == then for now, then in self.children)
+                and all(map(operator.is_, [d.get(name) for d, name in self.slots], self.params))
+                and not any(l._forward_hooks or l._forward_pre_hooks for l in self.layers)
                 and all(d.get(slot) is entry and entry.key is not None for d, slot, entry in self.derived)
-                and self._stamp() == self.stamp)
+                and self._values() == self.values and self.weights_same())
 
 
 class _SteppedShape:
@@ -1774,7 +1804,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
 
         A direct call lays the kernel's table out anew each time, so it is left to shapes that a program is known to step again
         and again: those of the steppers alive, whose results a direct call then also repeats bit for bit.  ``laid_out``: a
-        stepper's own table, ``(ops.trunk_table, eps of the bullet norm)``."""
+        stepper's own ``_WholeStep``."""
         B, NM, D = x.shape
         slots = bullets.shape[1] if bullets is not None and self.config.reads_bullets and bullets.dim() == 3 else 0
         if (B, NM, n_rec, slots) not in _stepped_shapes(self):
@@ -1797,10 +1827,10 @@ class YemongTrunk(_WeightCaches, nn.Module):
             found = self._whole_step_layers(B, NM, n_rec, slots, x.device)
             if found is None:
                 return None
-            laid_out = (ops.trunk_table(found[0]), found[1])
-        return ops.trunk_step(laid_out[0], whole(x), n_rec, whole(alive), state_in, state_out, reset=whole(reset),
+            laid_out = _WholeStep(self, *found)
+        return ops.trunk_step(laid_out.table, whole(x), n_rec, whole(alive), state_in, state_out, reset=whole(reset),
                               bullets=whole(bullets) if slots else None, in_flight=whole(in_flight) if slots else None,
-                              bullet_eps=laid_out[1], out_dtype=x.dtype)
+                              bullet_eps=laid_out.bullet_eps, out_dtype=x.dtype)
 
     def _bullet_kv_of_all_layers(self, bullets, rows):
         """``{id(layer): [K | V] rows}`` of every bullet-reading sublayer of the step from ONE pass over the bullets in
@@ -2097,7 +2127,7 @@ class EagerTrunkStepper:
         self.reads_bullets = bool(num_bullet_slots)
         self._sizes = (num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
         self._shape = _register_shape(trunk, *self._sizes)
-        self._whole = self._whole_watch = None
+        self._whole = None
         self.states = [trunk.initial_hidden(num_envs, num_recurrent, dev) for _ in range(2)]
         self.cur = 0
 
@@ -2130,12 +2160,11 @@ class EagerTrunkStepper:
         dev = self.states[0].device
         if self.autocast_dtype != torch.bfloat16 or not _HEAD_FUSION or self._sizes[1] > ops.TRUNK_TOKENS:
             return None
-        if self._whole is None or not self._whole_watch.same():
+        if self._whole is None or not self._whole.same():
             found = self.trunk._whole_step_layers(*self._sizes, dev)
-            self._whole = None
-            if found is None:
+            self._whole = None if found is None else _WholeStep(self.trunk, *found)
+            if self._whole is None:
                 return None
-            self._whole, self._whole_watch = (ops.trunk_table(found[0]), found[1]), _LayoutWatch(self.trunk)
         if tuple(tokens.shape[:2]) != self._sizes[:2]:
             return None
         return self.trunk._whole_step(tokens, alive_mask, self.states[self.cur], self.states[1 - self.cur], self._sizes[2], reset_mask,

@@ -271,3 +271,82 @@ def test_steppers_refuse_to_drop_the_bullets_of_a_bullet_reading_trunk():
     with pytest.raises(ValueError, match="no bullet-reading"):
         trunk_module._bullet_buffers(plain, 4, 80, "cpu", torch.float32)
     assert trunk_module._bullet_buffers(plain, 4, None, "cpu", torch.float32) == (None, None)
+
+
+@pytest.fixture
+def whole_steps(monkeypatch):
+    """The host side of the step as one kernel: the launch is replaced by a recorder of what the kernel would read.  Yields the
+    list of launches, each the fields of the table's layers."""
+    import types
+
+    from boost_and_broadside_amd import trunk as trunk_module
+
+    launches = []
+
+    def launch(table, x, n_rec, alive, state_in, state_out, *, out=None, out_dtype=torch.float32, bullet_eps=0.0, **inputs):
+        launches.append({"layers": [{name: getattr(entry, name) for name, _ in entry._fields_} for entry in table], "x": x.clone(),
+                         "alive": alive, "bullet_eps": bullet_eps, **inputs})
+        state_out.copy_(state_in)
+        return (torch.empty(x.shape, dtype=out_dtype) if out is None else out).copy_(x)
+
+    real = bnb.YemongTrunk._whole_step_layers
+    monkeypatch.setattr(bnb.YemongTrunk, "_whole_step_layers",
+                        lambda self, *sizes: real(self, *sizes[:4], types.SimpleNamespace(type="cuda")))
+    monkeypatch.setattr(trunk_module, "_projection_dtype", lambda: torch.bfloat16)
+    monkeypatch.setattr(ops, "trunk_step_pays", lambda *a: True)
+    monkeypatch.setattr(ops, "trunk_step", launch)
+    return launches
+
+
+def _stepped_trunk(seed=0, **cfg):
+    torch.manual_seed(seed)
+    return bnb.YemongTrunk(bnb.ModelConfig(**{**dict(d_model=128, n_heads=4, n_yemong_blocks=2, n_spatial_per_block=2,
+                                                     n_temporal_per_block=1, n_bullet_cross_per_block=0), **cfg})).eval()
+
+
+@pytest.mark.filterwarnings("ignore:CUDA is not available")
+@pytest.mark.parametrize("change", ["plain_data", "watched_data", "norm_eps", "decay_constant", "bullet_eps", "another_layer", "fewer_layers"])
+def test_an_uncaptured_stepper_lays_the_whole_step_out_anew_when_the_trunk_changed(whole_steps, change):
+    trunk = _stepped_trunk(n_bullet_cross_per_block=1)
+    B, N, M, slots = 3, 8, 4, 80
+    spatial, temporal = trunk.yemong_layers[0].spatial[0], trunk.yemong_layers[0].temporal[0]
+    if change == "plain_data":  # a replaced parameter is an ordinary one, whose ``.data`` counts nothing
+        spatial.norm2.weight = torch.nn.Parameter(torch.ones(128))
+        temporal.linear_out.weight = torch.nn.Parameter(temporal.linear_out.weight.detach().clone())
+    stepper = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, graph=False, num_bullet_slots=slots)
+    x, alive = torch.randn(B, N + M, 128), torch.ones(B, N + M, dtype=torch.bool)
+    bullets = torch.randn(B, slots, 128)
+    for _ in range(2):
+        stepper.step(x, alive, bullets=bullets)
+    assert len(whole_steps) == 2 and whole_steps[0]["layers"] == whole_steps[1]["layers"]  # nothing changed: the same table
+    if change in ("plain_data", "watched_data"):
+        for p in (spatial.norm2.weight, temporal.linear_out.weight):
+            p.data = 2.0 * p.detach()
+    elif change == "norm_eps":
+        spatial.norm1.eps, temporal.norm2.eps = 1e-3, 1e-2
+    elif change == "decay_constant":
+        temporal.rg_lru.c = 4.0
+    elif change == "bullet_eps":
+        for block in trunk.yemong_layers:
+            block.spatial[0].norm_bullet.eps = 1e-3
+    elif change == "another_layer":
+        trunk.yemong_layers[0].spatial.append(bnb.TransformerBlock(trunk.config))
+    else:
+        del trunk.yemong_layers[1].spatial[1]
+    stepper.step(x, alive, bullets=bullets)
+    layers = whole_steps[2]["layers"]
+    want = [l for block in trunk.yemong_layers for l in (*block.spatial, *block.temporal)]
+    assert len(layers) == len(want)
+    for entry, layer in zip(layers, want):
+        assert entry["norm1"] == layer.norm1.weight.data_ptr() and entry["norm2"] == layer.norm2.weight.data_ptr()
+        for name in ("eps1", "eps2"):
+            eps = getattr(layer, "norm" + name[-1]).eps
+            assert entry[name] == pytest.approx(torch.finfo(torch.float32).eps if eps is None else eps)
+        if entry["temporal"]:
+            assert entry["c"] == layer.rg_lru.c and entry["conv_weight"] == layer.conv.weight.data_ptr()
+        out = layer.linear_out if entry["temporal"] else layer.out_proj
+        packed = out.__dict__["_bnb_proj_pack"]
+        assert entry["proj"] == packed.value.data_ptr()
+        assert torch.equal(packed.value, ops.pack_proj_weights(out.weight.detach()))
+    bullet_eps = trunk.yemong_layers[0].spatial[0].norm_bullet.eps
+    assert whole_steps[2]["bullet_eps"] == pytest.approx(torch.finfo(torch.float32).eps if bullet_eps is None else bullet_eps)

@@ -1982,11 +1982,10 @@ class GraphedTrunk:
         self.graphs, self.outputs = [], []
         self._sizes = (num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
         self._shape = _register_shape(trunk, *self._sizes)
-        self._whole = self._whole_step_table()
+        self._whole = self._lay_out()
         if self._whole is not None:
             # one launch is all there is: it reads the caller's tensors, and there is nothing to capture
             self.outputs = [torch.empty_like(self.tokens) for _ in range(2)]
-            self._keep_weights()
             return
         side = torch.cuda.Stream(device=dev)
         side.wait_stream(torch.cuda.current_stream(dev))
@@ -2004,31 +2003,28 @@ class GraphedTrunk:
             self.outputs.append(out)
         for s in self.states:
             s.zero_()
-        self._keep_weights()
-
-    def _keep_weights(self) -> None:
-        # the derived weights the kernels read: held here so their memory outlives any cache
+        # the derived weights the captured kernels read: held here so their memory outlives any cache
         # invalidation on the module, and rebuilt in place when their sources change
-        self._derived = derived_weights(self.trunk)
-        self._params = list(self.trunk.parameters())
+        self._derived = derived_weights(trunk)
+        self._params = list(trunk.parameters())
         self._stamp = _weights_stamp(self._params)
 
-    def _whole_step_table(self):
-        """``(table, eps of the bullet norm)`` of the step as one kernel, or None where that does not apply."""
+    def _lay_out(self) -> _WholeStep | None:
+        """The step as one kernel, or None where that does not apply."""
         with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None), torch.no_grad():
             found = self.trunk._whole_step_layers(*self._sizes, self.tokens.device)
-        return None if found is None else (ops.trunk_table(found[0]), found[1])
+        return None if found is None else _WholeStep(self.trunk, *found)
+
+    def _lay_out_anew(self) -> None:
+        whole = self._lay_out()
+        if whole is None:
+            raise RuntimeError("the trunk's layers have changed their form: make a new stepper")
+        self._whole = whole
 
     def _step_whole(self, inputs):
         """The step as one kernel: an input that is as the kernel reads it is read in place, any other is copied first."""
-        if self._follow_weights():
-            # assigning ``.data`` moves a parameter: its address is looked up anew
-            whole = self._whole_step_table()
-            if whole is None:
-                raise RuntimeError("the trunk's layers have changed their form: make a new stepper")
-            self._whole = whole
-            self._derived = derived_weights(self.trunk)
-        table, bullet_eps = self._whole
+        if not self._whole.weights_same():
+            self._lay_out_anew()
         ready = {}
         for name, held, given in inputs:
             if given is held or (given is None and name in ("reset", "bullets", "in_flight")):
@@ -2042,25 +2038,29 @@ class GraphedTrunk:
             else:
                 held.copy_(given)
                 ready[name] = held
-        return ops.trunk_step(table, ready["x"], self._sizes[2], ready["alive"], self.states[self.cur], self.states[1 - self.cur],
-                              reset=ready["reset"], bullets=ready["bullets"], in_flight=ready["in_flight"], bullet_eps=bullet_eps,
+        return ops.trunk_step(self._whole.table, ready["x"], self._sizes[2], ready["alive"], self.states[self.cur], self.states[1 - self.cur],
+                              reset=ready["reset"], bullets=ready["bullets"], in_flight=ready["in_flight"], bullet_eps=self._whole.bullet_eps,
                               out=self.outputs[self.cur])
 
     def refresh_weights(self) -> None:
-        """Rebuild every derived weight copy the graphs read from the current parameters, in place."""
+        """Rebuild every derived weight copy the graphs read from the current parameters, in place.  Where the step is one
+        kernel, its table is laid out anew as well: it holds the addresses of the parameters themselves."""
+        if self._whole is not None:
+            for _, _, entry in self._whole.derived:
+                entry.key = None
+            self._lay_out_anew()
+            return
         for entry in self._derived:
             entry.refresh()
         self._stamp = _weights_stamp(self._params)
 
-    def _follow_weights(self) -> bool:
+    def _follow_weights(self) -> None:
         stamp = _weights_stamp(self._params)
-        if stamp == self._stamp:
-            return False
-        for entry in self._derived:
-            if entry.key != _cache_key(entry.tensors, entry.dtype):
-                entry.refresh()
-        self._stamp = stamp
-        return True
+        if stamp != self._stamp:
+            for entry in self._derived:
+                if entry.key != _cache_key(entry.tensors, entry.dtype):
+                    entry.refresh()
+            self._stamp = stamp
 
     def _run(self, src: int) -> torch.Tensor:
         with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None):

@@ -350,3 +350,34 @@ def test_an_uncaptured_stepper_lays_the_whole_step_out_anew_when_the_trunk_chang
         assert torch.equal(packed.value, ops.pack_proj_weights(out.weight.detach()))
     bullet_eps = trunk.yemong_layers[0].spatial[0].norm_bullet.eps
     assert whole_steps[2]["bullet_eps"] == pytest.approx(torch.finfo(torch.float32).eps if bullet_eps is None else bullet_eps)
+
+
+@pytest.mark.filterwarnings("ignore:CUDA is not available")
+@pytest.mark.parametrize("plain", [False, True])
+@pytest.mark.parametrize("refresh", [False, True])
+def test_a_captured_stepper_s_whole_step_follows_parameters_that_moved(whole_steps, plain, refresh):
+    """``.data = t`` moves a parameter; the table holds the addresses of norm and conv weights.  A write that nothing counts is
+    picked up by ``refresh_weights``."""
+    trunk = _stepped_trunk(1)
+    B, N, M = 3, 8, 4
+    layer, temporal = trunk.yemong_layers[0].spatial[1], trunk.yemong_layers[1].temporal[0]
+    if plain:
+        layer.norm2.weight, temporal.conv.weight = (torch.nn.Parameter(p.detach().clone()) for p in (layer.norm2.weight, temporal.conv.weight))
+        layer.qkv.weight = torch.nn.Parameter(layer.qkv.weight.detach().clone())
+    stepper = bnb.GraphedTrunk(trunk, B, N + M, N, autocast_dtype=torch.bfloat16)
+    x, alive = torch.randn(B, N + M, 128), torch.ones(B, N + M, dtype=torch.bool)
+    stepper.step(x, alive)
+    for p in (layer.norm2.weight, temporal.conv.weight, layer.qkv.weight):
+        p.data = 2.0 * p.detach()
+    if refresh:
+        torch._C.TensorBase.data.__get__(layer.ffn.down_proj.weight).mul_(3.0)
+        stepper.refresh_weights()
+    stepper.step(x, alive)
+    layers = whole_steps[-1]["layers"]
+    assert layers[1]["norm2"] == layer.norm2.weight.data_ptr() and layers[5]["conv_weight"] == temporal.conv.weight.data_ptr()
+    packed = layer.qkv.__dict__["_bnb_head_pack"].value
+    assert layers[1]["head"] == packed.data_ptr() and torch.equal(packed, ops.pack_head_weights(layer.qkv.weight.detach()))
+    if refresh:
+        ws = (layer.ffn.gate_proj.weight, layer.ffn.up_proj.weight, layer.ffn.down_proj.weight)
+        packed = layer.ffn.__dict__["_bnb_ffn_pack"].value
+        assert layers[1]["ffn"] == packed.data_ptr() and torch.equal(packed, ops.pack_ffn_weights(*(w.detach() for w in ws)))

@@ -52,6 +52,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+import torch.nn.modules.module as module_internals
 import torch.utils.checkpoint
 
 from . import _native, ops
@@ -1388,6 +1389,20 @@ class _SplitTokens(torch.autograd.Function):
         return torch.cat([d_first, d_rest], dim=2), None
 
 
+def _plain_call(layer: nn.Module, method: str) -> bool:
+    """Whether ``layer.forward`` (called as a module) or ``layer.step_tokens`` runs as written in this file, on the rows it is handed:
+    no hook that may change what goes in or comes out, no override.  Only between such sublayers may one tail kernel form what the
+    next sublayer starts with."""
+    if method == "forward" and (layer._forward_hooks or layer._forward_pre_hooks or module_internals._global_forward_hooks
+                                or module_internals._global_forward_pre_hooks):
+        return False
+    wrapped = layer._modules.get("_orig_mod")
+    if wrapped is not None:  # torch.compile's wrapper
+        return _plain_call(wrapped, method)
+    own = TransformerBlock.forward if method == "forward" else GriffinTemporalBlock.step_tokens
+    return getattr(type(layer), method, None) is own and method not in layer.__dict__
+
+
 class YemongBlock(_WeightCaches, nn.Module):
     """``n_spatial_per_block`` attention sublayers, then ``n_temporal_per_block`` recurrent ones."""
 
@@ -1438,10 +1453,10 @@ class YemongBlock(_WeightCaches, nn.Module):
         return x, torch.stack(new_h), torch.stack(new_cb)
 
     def first_head_spec(self, x, num_recurrent):
-        """``head_spec`` of this block's first sublayer for tokens like ``x`` (B, NM, D), or None."""
+        """``head_spec`` of this block's first sublayer for tokens like ``x`` (B, NM, D), or None when it forms its own head."""
         if len(self.spatial):
-            return self.spatial[0].head_spec(x)
-        if len(self.temporal):
+            return self.spatial[0].head_spec(x) if _plain_call(self.spatial[0], "forward") else None
+        if len(self.temporal) and _plain_call(self.temporal[0], "step_tokens"):
             return self.temporal[0].head_spec(x, num_recurrent, self.field_sub[0] if x.shape[1] > num_recurrent else None)
         return None
 
@@ -1467,13 +1482,16 @@ class YemongBlock(_WeightCaches, nn.Module):
         act = _projection_dtype()
         n_s, n_t = len(self.spatial), len(self.temporal)
 
-        def spec_of(k, x):  # head_spec of sublayer k of this block (spatial first), of the next block's first past the end
+        def spec_of(k, x):  # for sublayer k - 1: head_spec of sublayer k of this block (spatial first), of the next block's first past the end
+            if not plain[k - 1] or (k < n_s + n_t and not plain[k]):
+                return None
             if k < n_s:
                 return self.spatial[k].head_spec(x)
             if k < n_s + n_t:
                 return self.temporal[k - n_s].head_spec(x, n_rec, self.field_sub[k - n_s] if NM > n_rec else None)
             return after(x) if after is not None else None
 
+        plain = [_plain_call(l, "forward") for l in self.spatial] + [_plain_call(l, "step_tokens") for l in self.temporal]
         for k, layer in enumerate(self.spatial):
             nxt = spec_of(k + 1, x)
             out = layer(x, alive, bullets, bullet_mask, head=head, next_head=nxt)

@@ -1908,3 +1908,46 @@ def test_whole_step_of_an_uncaptured_stepper_follows_weights_hooks_and_invalidat
     handle.remove()
     step()
     assert stepper._whole is not None
+
+
+@pytest.mark.parametrize("amp", [False, True])
+@pytest.mark.parametrize("what", ["pre_hook", "hook", "forward", "step_tokens"])
+def test_sublayers_with_hooks_or_overrides_form_their_own_head(amp, what, monkeypatch):
+    """A forward pre-hook that changes a sublayer's rows reaches its projections, a forward hook sees and replaces a tensor, an
+    overridden method gets the rows it would have got: as with every sublayer forming its own norm + projection."""
+    from boost_and_broadside_amd import trunk as trunk_module
+
+    D, H, B, N, M = 128, 4, 5, 8, 4
+    trunk, _ = _rollout_trunk(171)
+    gen = torch.Generator().manual_seed(172)
+    x, alive = torch.randn(B, N + M, D, generator=gen).to(DEV), torch.ones(B, N + M, dtype=torch.bool, device=DEV)
+    state = torch.randn(2, B * N, 4 * D, generator=gen).to(DEV)
+
+    def step():
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+            return trunk(x, alive, state)[0]
+
+    before, seen = step(), []
+    first, second = trunk.yemong_layers
+    if what == "pre_hook":
+        second.spatial[0].register_forward_pre_hook(lambda m, args: (args[0] * torch.linspace(0.5, 1.5, D, device=DEV),) + args[1:])
+        first.spatial[1].register_forward_pre_hook(lambda m, args: (args[0] + 0.5,) + args[1:])
+    elif what == "hook":
+        for layer in (*first.spatial, *second.spatial):
+            layer.register_forward_hook(lambda m, args, out: (seen.append(type(out)), out * 1.25)[1])
+    elif what == "forward":
+        real = first.spatial[1].forward
+        first.spatial[1].forward = lambda rows, *args, **kw: real(rows + 0.5, *args, **kw)
+    else:
+        class Shifted(bnb.GriffinTemporalBlock):
+            def step_tokens(self, rows, *args, **kw):
+                return super().step_tokens(rows + 0.5, *args, **kw)
+
+        first.temporal[0].__class__ = Shifted
+    got = step()
+    with trunk_module.separate_heads():
+        want = step()
+    assert all(t is torch.Tensor for t in seen) and len(seen) == (8 if what == "hook" else 0)
+    tol = BF16_TOL if amp else 1e-5
+    assert max_rel(got.cpu(), want.cpu()) <= tol
+    assert max_rel(got.cpu(), before.cpu()) > 5 * tol

@@ -280,6 +280,8 @@ def invalidate_weight_caches(module: nn.Module, *, drop: bool = False) -> None:
     outside autograd.  ``p.data.copy_(...)`` itself is seen (``WatchedParameter``).  ``drop=True`` frees the
     cached tensors instead of keeping their memory for the rebuild."""
     for m in module.modules():
+        if drop:
+            m.__dict__.get("_whole_steps", {}).clear()
         for k in [k for k, v in m.__dict__.items() if k.startswith(_CACHE_PREFIX) and isinstance(v, _DerivedWeight)]:
             if drop:
                 del m.__dict__[k]
@@ -1389,17 +1391,16 @@ class _SplitTokens(torch.autograd.Function):
         return torch.cat([d_first, d_rest], dim=2), None
 
 
-def _plain_call(layer: nn.Module, method: str) -> bool:
-    """Whether ``layer.forward`` (called as a module) or ``layer.step_tokens`` runs as written in this file, on the rows it is handed:
-    no hook that may change what goes in or comes out, no override.  Only between such sublayers may one tail kernel form what the
-    next sublayer starts with."""
+def _plain_call(layer: nn.Module, own) -> bool:
+    """Whether calling the layer's method of ``own``'s name runs ``own``, a method of this file, on what it is handed: no override and,
+    where it is ``forward`` and the layer is called as a module, no hook that may change what goes in or comes out."""
+    method = own.__name__
     if method == "forward" and (layer._forward_hooks or layer._forward_pre_hooks or module_internals._global_forward_hooks
                                 or module_internals._global_forward_pre_hooks):
         return False
     wrapped = layer._modules.get("_orig_mod")
     if wrapped is not None:  # torch.compile's wrapper
-        return _plain_call(wrapped, method)
-    own = TransformerBlock.forward if method == "forward" else GriffinTemporalBlock.step_tokens
+        return _plain_call(wrapped, own)
     return getattr(type(layer), method, None) is own and method not in layer.__dict__
 
 
@@ -1455,8 +1456,8 @@ class YemongBlock(_WeightCaches, nn.Module):
     def first_head_spec(self, x, num_recurrent):
         """``head_spec`` of this block's first sublayer for tokens like ``x`` (B, NM, D), or None when it forms its own head."""
         if len(self.spatial):
-            return self.spatial[0].head_spec(x) if _plain_call(self.spatial[0], "forward") else None
-        if len(self.temporal) and _plain_call(self.temporal[0], "step_tokens"):
+            return self.spatial[0].head_spec(x) if _plain_call(self.spatial[0], TransformerBlock.forward) else None
+        if len(self.temporal) and _plain_call(self.temporal[0], GriffinTemporalBlock.step_tokens):
             return self.temporal[0].head_spec(x, num_recurrent, self.field_sub[0] if x.shape[1] > num_recurrent else None)
         return None
 
@@ -1491,7 +1492,9 @@ class YemongBlock(_WeightCaches, nn.Module):
                 return self.temporal[k - n_s].head_spec(x, n_rec, self.field_sub[k - n_s] if NM > n_rec else None)
             return after(x) if after is not None else None
 
-        plain = [_plain_call(l, "forward") for l in self.spatial] + [_plain_call(l, "step_tokens") for l in self.temporal]
+        # one tail kernel forms what the next sublayer starts with only between two that are called as written
+        plain = [_plain_call(l, TransformerBlock.forward) for l in self.spatial] + [
+            _plain_call(l, GriffinTemporalBlock.step_tokens) for l in self.temporal]
         for k, layer in enumerate(self.spatial):
             nxt = spec_of(k + 1, x)
             out = layer(x, alive, bullets, bullet_mask, head=head, next_head=nxt)
@@ -1581,6 +1584,13 @@ class _LiveRows:
         self.rows, self.chained = rows, chained
 
 
+def _whole_step_calls(trunk) -> list:
+    """The calls that a step of the trunk consists of: ``(module, method)``."""
+    return [call for block in trunk.yemong_layers
+            for call in [(block, YemongBlock.step_packed), (block, YemongBlock.first_head_spec)]
+            + [(l, TransformerBlock.forward) for l in block.spatial] + [(l, GriffinTemporalBlock.step_tokens) for l in block.temporal]]
+
+
 class _WholeStep:
     """The trunk's step as ``ops.trunk_step`` takes it (``table``, ``bullet_eps``) and everything that was laid out in it: the
     submodules, the parameters with their addresses and write counts, the derived weights, the constants.
@@ -1590,7 +1600,7 @@ class _WholeStep:
     are read in half the time of the parameter subclass."""
 
     __slots__ = ("table", "bullet_eps", "tensors", "children", "slots", "params", "held", "aliases", "written", "derived", "constants",
-                 "values", "layers")
+                 "values", "calls")
 
     def __init__(self, trunk: nn.Module, layers: list, bullet_eps: float) -> None:
         self.table, self.bullet_eps = ops.trunk_table(layers), bullet_eps
@@ -1603,7 +1613,7 @@ class _WholeStep:
         self.derived = [(m.__dict__, k, v) for m in modules for k, v in m.__dict__.items()
                         if k.startswith(_CACHE_PREFIX) and isinstance(v, _DerivedWeight) and isinstance(v.value, torch.Tensor)
                         and v.value.data_ptr() in used]
-        self.layers = [l for block in trunk.yemong_layers for l in (*block.spatial, *block.temporal)]
+        self.calls = _whole_step_calls(trunk)
         self.constants = [(m.__dict__, name) for m in modules for name in ("eps", "c", "n_heads", "reads_bullets") if name in m.__dict__]
         self.values = self._values()
         self.held = [p for p in self.params if p is not None]
@@ -1622,13 +1632,23 @@ class _WholeStep:
         return self._written() == self.written
 
     def same(self) -> bool:
-        """Whether a table laid out now would be this one: besides the weights the same submodules, parameters and constants, no forward
-        hooks, no derived weight invalidated."""
+        """Whether a table laid out now would be this one: besides the weights the same submodules, parameters and constants, no hooks or
+        overrides, no derived weight invalidated."""
         return (all(now == then for now, then in self.children)
                 and all(map(operator.is_, [d.get(name) for d, name in self.slots], self.params))
-                and not any(l._forward_hooks or l._forward_pre_hooks for l in self.layers)
+                and all(_plain_call(m, own) for m, own in self.calls)
                 and all(d.get(slot) is entry and entry.key is not None for d, slot, entry in self.derived)
                 and self._values() == self.values and self.weights_same())
+
+
+class _WholeSteps(dict):
+    """The ``_WholeStep``s that a trunk keeps, by (field tokens, bullets read).  They hold addresses: a copy of the trunk starts without."""
+
+    def __deepcopy__(self, memo):
+        return _WholeSteps()
+
+    def __reduce__(self):
+        return (_WholeSteps, ())
 
 
 class _SteppedShape:
@@ -1752,20 +1772,20 @@ class YemongTrunk(_WeightCaches, nn.Module):
         NM tokens, n_rec of them recurrent, with ``slots`` bullet slots (0: no read): small fleets under bfloat16 autocast,
         every layer in its standard form.  Else None."""
         blocks = list(self.yemong_layers)
+        calls = _whole_step_calls(self)
+        if not (all(_plain_call(m, own) for m, own in calls)
+                and all(type(l) is TransformerBlock for block in blocks for l in block.spatial)
+                and all(type(l) is GriffinTemporalBlock for block in blocks for l in block.temporal)):
+            return None
         readers = [l for block in blocks for l in block.spatial if l.reads_bullets] if slots else []
-        n_layers = sum(len(block.spatial) + len(block.temporal) for block in blocks)
-        if not (
-            _HEAD_FUSION and device.type == "cuda" and _projection_dtype() == torch.bfloat16
-            and ops.trunk_step_supported(B, NM, n_rec, self.config.d_model, self.config.n_heads, n_layers, slots if readers else 0)
-            and ops.trunk_step_pays(B, NM, bool(readers), device)
-        ):
+        if not self._whole_step_fits(B, NM, n_rec, slots, device, len(calls) - 2 * len(blocks), bool(readers)):
             return None
 
         def vector(t):
             return t is not None and t.dtype == torch.float32 and t.is_contiguous()
 
         def plain(layer, mlp, *linears):
-            return (not layer._forward_hooks and not layer._forward_pre_hooks and vector(layer.norm1.weight) and vector(layer.norm2.weight)
+            return (vector(layer.norm1.weight) and vector(layer.norm2.weight)
                     and all(l.bias is None for l in (*linears, mlp.gate_proj, mlp.up_proj, mlp.down_proj))
                     and tuple(mlp.gate_proj.weight.shape) == (ops.FFN_HIDDEN, ops.FFN_WIDTH))
 
@@ -1785,7 +1805,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
         table, slot, reader = [], 0, 0
         for block in blocks:
             for l in block.spatial:
-                if not (type(l) is TransformerBlock and plain(l, l.ffn, l.qkv, l.out_proj)):
+                if not plain(l, l.ffn, l.qkv, l.out_proj):
                     return None
                 w = l.qkv.weight
                 entry = shared(l, l.ffn, l.out_proj)
@@ -1797,7 +1817,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
             for j, l in enumerate(block.temporal):
                 rg = l.rg_lru
                 fold, ws = l._head_weights(NM, n_rec, block.field_sub[j] if NM > n_rec else None)
-                if not (type(l) is GriffinTemporalBlock and plain(l, l.gated_mlp, l.linear1, l.linear2, l.linear_out)
+                if not (plain(l, l.gated_mlp, l.linear1, l.linear2, l.linear_out)
                         and rg.linear_a.bias is not None and rg.linear_x.bias is not None and fold == (NM > n_rec)
                         and vector(l.conv.weight) and (l.conv.bias is None or vector(l.conv.bias)) and rg.log_lambda.dtype == torch.float32):
                     return None
@@ -1817,12 +1837,30 @@ class YemongTrunk(_WeightCaches, nn.Module):
                 table.append(entry)
         return table, (eps(readers[0].norm_bullet) if readers else 0.0)
 
-    def _whole_step(self, x, alive, state_in, state_out, n_rec, reset, bullets, in_flight, laid_out=None):
+    def _whole_step_fits(self, B, NM, n_rec, slots, device, n_layers, reads) -> bool:
+        """Whether the kernel of the whole step covers these sizes, under the autocast of the call, and is the faster one."""
+        return (_HEAD_FUSION and device.type == "cuda" and _projection_dtype() == torch.bfloat16
+                and ops.trunk_step_supported(B, NM, n_rec, self.config.d_model, self.config.n_heads, n_layers, slots if reads else 0)
+                and ops.trunk_step_pays(B, NM, reads, device))
+
+    def _whole_step_plan(self, B, NM, n_rec, slots, device) -> _WholeStep | None:
+        """The step as one kernel, or None where that does not apply.  Kept while the trunk stays as it is."""
+        kept, key = self.__dict__.setdefault("_whole_steps", _WholeSteps()), (NM > n_rec, slots > 0)
+        plan = kept.get(key)
+        if plan is not None and plan.children[0][0] is self._modules and plan.same():
+            return plan if self._whole_step_fits(B, NM, n_rec, slots, device, len(plan.table), key[1]) else None
+        found = self._whole_step_layers(B, NM, n_rec, slots, device)
+        kept.pop(key, None)
+        if found is None:
+            return None
+        plan = kept[key] = _WholeStep(self, *found)
+        return plan
+
+    def _whole_step(self, x, alive, state_in, state_out, n_rec, reset, bullets, in_flight):
         """The step as one kernel where a stepper for this shape exists and that applies, else None.
 
-        A direct call lays the kernel's table out anew each time, so it is left to shapes that a program is known to step again
-        and again: those of the steppers alive, whose results a direct call then also repeats bit for bit.  ``laid_out``: a
-        stepper's own ``_WholeStep``."""
+        Laying the kernel's table out costs as much as the separate launches, so a direct call takes it only at shapes that a program is
+        known to step again and again: those of the steppers alive, whose results a direct call then also repeats bit for bit."""
         B, NM, D = x.shape
         slots = bullets.shape[1] if bullets is not None and self.config.reads_bullets and bullets.dim() == 3 else 0
         if (B, NM, n_rec, slots) not in _stepped_shapes(self):
@@ -1841,14 +1879,12 @@ class YemongTrunk(_WeightCaches, nn.Module):
                 and all(t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (state_in, state_out))
                 and (not slots or (given(bullets, (B, slots, D), rows) and given(in_flight, (B, slots), flags)))):
             return None
-        if laid_out is None:
-            found = self._whole_step_layers(B, NM, n_rec, slots, x.device)
-            if found is None:
-                return None
-            laid_out = _WholeStep(self, *found)
-        return ops.trunk_step(laid_out.table, whole(x), n_rec, whole(alive), state_in, state_out, reset=whole(reset),
+        plan = self._whole_step_plan(B, NM, n_rec, slots, x.device)
+        if plan is None:
+            return None
+        return ops.trunk_step(plan.table, whole(x), n_rec, whole(alive), state_in, state_out, reset=whole(reset),
                               bullets=whole(bullets) if slots else None, in_flight=whole(in_flight) if slots else None,
-                              bullet_eps=laid_out.bullet_eps, out_dtype=x.dtype)
+                              bullet_eps=plan.bullet_eps, out_dtype=x.dtype)
 
     def _bullet_kv_of_all_layers(self, bullets, rows):
         """``{id(layer): [K | V] rows}`` of every bullet-reading sublayer of the step from ONE pass over the bullets in
@@ -1973,7 +2009,8 @@ class GraphedTrunk:
     (optimizer step, ``load_state_dict``, a write through ``.data``), rebuilds the derived copies whose
     sources changed into the same memory; ``refresh_weights()`` rebuilds all of them unconditionally.
     This object keeps those copies alive, so nothing the graphs read is ever returned to the allocator.
-    Replacing parameter tensors, moving or casting the module requires a new capture.
+    Replacing parameter tensors, moving or casting the module requires a new capture, and hooks and overridden methods are
+    those of the time of capture.
 
     Args:
         trunk: the module to capture.
@@ -2028,21 +2065,22 @@ class GraphedTrunk:
         self._stamp = _weights_stamp(self._params)
 
     def _lay_out(self) -> _WholeStep | None:
-        """The step as one kernel, or None where that does not apply."""
+        """The step as one kernel, or None where that is not what calling the trunk comes to."""
+        if not _plain_call(self.trunk, YemongTrunk.forward):
+            return None
         with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None), torch.no_grad():
-            found = self.trunk._whole_step_layers(*self._sizes, self.tokens.device)
-        return None if found is None else _WholeStep(self.trunk, *found)
-
-    def _lay_out_anew(self) -> None:
-        whole = self._lay_out()
-        if whole is None:
-            raise RuntimeError("the trunk's layers have changed their form: make a new stepper")
-        self._whole = whole
+            return self.trunk._whole_step_plan(*self._sizes, self.tokens.device)
 
     def _step_whole(self, inputs):
         """The step as one kernel: an input that is as the kernel reads it is read in place, any other is copied first."""
         if not self._whole.weights_same():
-            self._lay_out_anew()
+            whole = self._lay_out()
+            if whole is None:  # no longer a trunk for the kernel: the call itself
+                x, alive, reset, bullets, in_flight = (given for _, _, given in inputs)
+                with torch.autocast("cuda", dtype=self.autocast_dtype):
+                    out, _ = self.trunk(x, alive, self.states[self.cur], bullets, in_flight, reset_mask=reset, out_state=self.states[1 - self.cur])
+                return self.outputs[self.cur].copy_(out)
+            self._whole = whole
         ready = {}
         for name, held, given in inputs:
             if given is held or (given is None and name in ("reset", "bullets", "in_flight")):
@@ -2066,7 +2104,8 @@ class GraphedTrunk:
         if self._whole is not None:
             for _, _, entry in self._whole.derived:
                 entry.key = None
-            self._lay_out_anew()
+            self._whole.written = None  # out of date, also if the trunk cannot be laid out any more
+            self._whole = self._lay_out() or self._whole
             return
         for entry in self._derived:
             entry.refresh()
@@ -2145,7 +2184,6 @@ class EagerTrunkStepper:
         self.reads_bullets = bool(num_bullet_slots)
         self._sizes = (num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
         self._shape = _register_shape(trunk, *self._sizes)
-        self._whole = None
         self.states = [trunk.initial_hidden(num_envs, num_recurrent, dev) for _ in range(2)]
         self.cur = 0
 
@@ -2166,27 +2204,16 @@ class EagerTrunkStepper:
         if not self.reads_bullets and bullets is not None:
             raise ValueError("this stepper was made without bullet inputs")
         with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None):
-            out = self._step_whole(tokens, alive_mask, reset_mask, bullets, bullet_mask)
-            if out is None:
-                out, _ = self.trunk(tokens, alive_mask, self.states[self.cur], bullets, bullet_mask,
-                                    reset_mask=reset_mask, out_state=self.states[1 - self.cur])
+            out, new_state = self.trunk(tokens, alive_mask, self.states[self.cur], bullets, bullet_mask,
+                                        reset_mask=reset_mask, out_state=self.states[1 - self.cur])
         self.cur = 1 - self.cur
-        return out, self.states[self.cur]
+        return out, new_state
 
-    def _step_whole(self, tokens, alive_mask, reset_mask, bullets, bullet_mask):
-        """The step as one kernel where that applies, with its table kept while the trunk stays as it is; else None."""
-        dev = self.states[0].device
-        if self.autocast_dtype != torch.bfloat16 or not _HEAD_FUSION or self._sizes[1] > ops.TRUNK_TOKENS:
-            return None
-        if self._whole is None or not self._whole.same():
-            found = self.trunk._whole_step_layers(*self._sizes, dev)
-            self._whole = None if found is None else _WholeStep(self.trunk, *found)
-            if self._whole is None:
-                return None
-        if tuple(tokens.shape[:2]) != self._sizes[:2]:
-            return None
-        return self.trunk._whole_step(tokens, alive_mask, self.states[self.cur], self.states[1 - self.cur], self._sizes[2], reset_mask,
-                                      bullets, bullet_mask, laid_out=self._whole)
+    @property
+    def _whole(self) -> _WholeStep | None:
+        """The step as one kernel, or None where the trunk's own forward runs separate kernels."""
+        with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None):
+            return self.trunk._whole_step_plan(*self._sizes, self.states[0].device)
 
 
 # tokens per step below which a captured step beats plain launches, with the default trunk of 2 blocks x (2 attention +

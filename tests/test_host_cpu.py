@@ -289,9 +289,9 @@ def whole_steps(monkeypatch):
         state_out.copy_(state_in)
         return (torch.empty(x.shape, dtype=out_dtype) if out is None else out).copy_(x)
 
-    real = bnb.YemongTrunk._whole_step_layers
-    monkeypatch.setattr(bnb.YemongTrunk, "_whole_step_layers",
-                        lambda self, *sizes: real(self, *sizes[:4], types.SimpleNamespace(type="cuda")))
+    real = bnb.YemongTrunk._whole_step_fits
+    monkeypatch.setattr(bnb.YemongTrunk, "_whole_step_fits",
+                        lambda self, *sizes: real(self, *sizes[:4], types.SimpleNamespace(type="cuda"), *sizes[5:]))
     monkeypatch.setattr(trunk_module, "_projection_dtype", lambda: torch.bfloat16)
     monkeypatch.setattr(ops, "trunk_step_pays", lambda *a: True)
     monkeypatch.setattr(ops, "trunk_step", launch)
@@ -381,3 +381,26 @@ def test_a_captured_stepper_s_whole_step_follows_parameters_that_moved(whole_ste
         ws = (layer.ffn.gate_proj.weight, layer.ffn.up_proj.weight, layer.ffn.down_proj.weight)
         packed = layer.ffn.__dict__["_bnb_ffn_pack"].value
         assert layers[1]["ffn"] == packed.data_ptr() and torch.equal(packed, ops.pack_ffn_weights(*(w.detach() for w in ws)))
+
+
+@pytest.mark.filterwarnings("ignore:CUDA is not available")
+def test_trunk_and_uncaptured_stepper_can_be_copied_after_a_whole_step(whole_steps):
+    """The table holds addresses: a copy lays out its own."""
+    import copy
+
+    B, N, M = 3, 8, 4
+    stepper = bnb.trunk_stepper(_stepped_trunk(2), B, N + M, N, autocast_dtype=torch.bfloat16, graph=False)
+    x, alive = torch.randn(B, N + M, 128), torch.ones(B, N + M, dtype=torch.bool)
+    stepper.step(x, alive)
+    stepper.load_state(torch.randn_like(stepper.state))
+    other = copy.deepcopy(stepper)
+    assert other.trunk is not stepper.trunk and torch.equal(other.state, stepper.state)
+    with torch.no_grad():
+        other.trunk.yemong_layers[0].spatial[0].out_proj.weight.mul_(2.0)
+    plan = other._whole
+    mine = stepper._whole
+    assert plan is not None and plan is not mine and mine.same()
+    for entry, layer in ((plan.table[0], other.trunk.yemong_layers[0].spatial[0]), (mine.table[0], stepper.trunk.yemong_layers[0].spatial[0])):
+        packed = layer.out_proj.__dict__["_bnb_proj_pack"].value
+        assert entry.norm1 == layer.norm1.weight.data_ptr() and entry.proj == packed.data_ptr()
+        assert torch.equal(packed, ops.pack_proj_weights(layer.out_proj.weight.detach()))

@@ -1951,3 +1951,102 @@ def test_sublayers_with_hooks_or_overrides_form_their_own_head(amp, what, monkey
     tol = BF16_TOL if amp else 1e-5
     assert max_rel(got.cpu(), want.cpu()) <= tol
     assert max_rel(got.cpu(), before.cpu()) > 5 * tol
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("what", ["hook", "pre_hook", "subclass", "instance", "block"])
+def test_steppers_run_the_trunk_s_hooks_and_overrides_at_every_size(graph, what):
+    """What a call of the trunk does beyond its own forward happens at every step, also where that forward is one kernel: against the
+    same trunk called directly on separate kernels."""
+    D, B, N, M = 128, 6, 8, 4
+
+    def made():
+        trunk, _ = _rollout_trunk(181)
+        calls = []
+
+        def scaled(self, tokens, *args, **kw):
+            calls.append("forward")
+            out, state = bnb.YemongTrunk.forward(self, tokens, *args, **kw)
+            return out * 1.25, state
+
+        if what == "hook":
+            trunk.register_forward_hook(lambda m, args, out: (calls.append("hook"), (out[0] * 1.25, out[1]))[1])
+        elif what == "pre_hook":
+            trunk.register_forward_pre_hook(lambda m, args: (calls.append("pre"), (args[0] + 0.5,) + args[1:])[1])
+        elif what == "subclass":
+            trunk.__class__ = type("Scaled", (bnb.YemongTrunk,), {"forward": scaled})
+        elif what == "instance":
+            trunk.forward = scaled.__get__(trunk)
+        else:
+            def shifted(self, x, *args, **kw):
+                calls.append("block")
+                return bnb.YemongBlock.step_packed(self, x + 0.5, *args, **kw)
+
+            trunk.yemong_layers[0].__class__ = type("Shifted", (bnb.YemongBlock,), {"step_packed": shifted})
+        return trunk, calls
+
+    gen = torch.Generator().manual_seed(182)
+    plain, _ = _rollout_trunk(181)
+    direct, _ = made()
+    trunk, calls = made()
+    stepper = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, graph=graph)
+    alive = torch.ones(B, N + M, dtype=torch.bool, device=DEV)
+    state = torch.randn(stepper.state.shape, generator=gen).to(DEV)
+    stepper.load_state(state)
+    for t in range(3):
+        x = torch.randn(B, N + M, D, generator=gen).to(DEV)
+        calls.clear()
+        out, new_state = stepper.step(x, alive)
+        assert graph or len(calls) == 1
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            want, want_state = direct(x, alive, state)
+            other, _ = plain(x, alive, state)
+        assert max_rel(out.cpu(), want.cpu()) <= BF16_TOL and max_rel(new_state.cpu(), want_state.cpu()) <= BF16_TOL, t
+        assert max_rel(out.cpu(), other.cpu()) > 5 * BF16_TOL, t
+        stepper.load_state(want_state)
+        state = want_state
+
+
+def test_an_uncaptured_stepper_follows_a_hook_registered_between_steps():
+    B, N, M = 6, 8, 4
+    trunk, _ = _rollout_trunk(183)
+    stepper = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, graph=False)
+    x, alive = torch.randn(B, N + M, 128, device=DEV), torch.ones(B, N + M, dtype=torch.bool, device=DEV)
+    first = stepper.step(x, alive)[0].clone()
+    seen = []
+    handles = [trunk.register_forward_hook(lambda *a: seen.append("trunk")),
+               torch.nn.modules.module.register_module_forward_hook(lambda m, *a: seen.append(type(m).__name__))]
+    try:
+        stepper.load_state(torch.zeros_like(stepper.state))
+        again = stepper.step(x, alive)[0].clone()
+    finally:
+        for h in handles:
+            h.remove()
+    assert seen.count("trunk") == 1 and seen.count("TransformerBlock") == 4 and seen.count("YemongTrunk") == 1
+    assert max_rel(again.cpu(), first.cpu()) <= BF16_TOL
+    stepper.load_state(torch.zeros_like(stepper.state))
+    assert torch.equal(stepper.step(x, alive)[0], first)
+
+
+def test_a_captured_stepper_whose_trunk_left_the_kernel_s_form_calls_the_trunk():
+    B, N, M = 6, 8, 4
+    trunk, _ = _rollout_trunk(185)
+    stepper = bnb.GraphedTrunk(trunk, B, N + M, N, autocast_dtype=torch.bfloat16)
+    assert stepper._whole is not None
+    gen = torch.Generator().manual_seed(186)
+    x, alive = torch.randn(B, N + M, 128, generator=gen).to(DEV), torch.ones(B, N + M, dtype=torch.bool, device=DEV)
+    done = (torch.rand(B, generator=gen) < 0.5).to(DEV)
+    state = torch.randn(stepper.state.shape, generator=gen).to(DEV)
+    layer = trunk.yemong_layers[0].spatial[0]
+    handle = layer.register_forward_hook(lambda m, args, out: out * 1.5)
+    with torch.no_grad():
+        layer.qkv.weight.mul_(1.5)
+    for hooked in (True, True, False):
+        if not hooked:
+            handle.remove()
+        stepper.load_state(state)
+        out, new_state = stepper.step(x, alive, done)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            want, want_state = trunk(x, alive, state, reset_mask=done)
+        assert out.data_ptr() in [o.data_ptr() for o in stepper.outputs] and new_state is stepper.state
+        assert torch.equal(out, want) and torch.equal(new_state, want_state), hooked

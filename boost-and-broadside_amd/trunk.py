@@ -46,7 +46,6 @@ import copy
 import math
 import operator
 import warnings
-import weakref
 from dataclasses import dataclass
 
 import torch
@@ -1651,24 +1650,6 @@ class _WholeSteps(dict):
         return (_WholeSteps, ())
 
 
-class _SteppedShape:
-    """Held by every stepper of one shape over one trunk."""
-
-    __slots__ = ("__weakref__",)
-
-
-_STEPPED = weakref.WeakKeyDictionary()  # trunk -> {(environments, tokens, recurrent tokens, bullet slots): _SteppedShape} of its steppers
-
-
-def _stepped_shapes(trunk):
-    return _STEPPED.get(trunk, ())
-
-
-def _register_shape(trunk, *shape) -> _SteppedShape:
-    shapes = _STEPPED.setdefault(trunk, weakref.WeakValueDictionary())
-    return shapes.setdefault(shape, _SteppedShape())
-
-
 class YemongTrunk(_WeightCaches, nn.Module):
     """The recurrent trunk: ``forward(tokens, alive_mask, recurrent_state) -> (hidden, new_state)``.
 
@@ -1837,6 +1818,12 @@ class YemongTrunk(_WeightCaches, nn.Module):
                 table.append(entry)
         return table, (eps(readers[0].norm_bullet) if readers else 0.0)
 
+    def _stepped_at(self, B, NM, n_rec, slots) -> None:
+        """From here on this trunk steps B environments of NM tokens, n_rec of them recurrent, with ``slots`` bullet slots as one kernel
+        under bfloat16 autocast, where that applies: said by a stepper when it is made.  A direct call of these sizes then gives
+        that stepper's bits, for as long as the trunk lives; a call of other sizes runs separate kernels, a bfloat16 rounding apart."""
+        self.__dict__.setdefault("_stepped_sizes", set()).add((B, NM, n_rec, slots))
+
     def _whole_step_fits(self, B, NM, n_rec, slots, device, n_layers, reads) -> bool:
         """Whether the kernel of the whole step covers these sizes, under the autocast of the call, and is the faster one."""
         return (_HEAD_FUSION and device.type == "cuda" and _projection_dtype() == torch.bfloat16
@@ -1857,13 +1844,10 @@ class YemongTrunk(_WeightCaches, nn.Module):
         return plan
 
     def _whole_step(self, x, alive, state_in, state_out, n_rec, reset, bullets, in_flight):
-        """The step as one kernel where a stepper for this shape exists and that applies, else None.
-
-        Laying the kernel's table out costs as much as the separate launches, so a direct call takes it only at shapes that a program is
-        known to step again and again: those of the steppers alive, whose results a direct call then also repeats bit for bit."""
+        """The step as one kernel at the sizes that a stepper has been made for (``_stepped_at``) and where that applies, else None."""
         B, NM, D = x.shape
         slots = bullets.shape[1] if bullets is not None and self.config.reads_bullets and bullets.dim() == 3 else 0
-        if (B, NM, n_rec, slots) not in _stepped_shapes(self):
+        if (B, NM, n_rec, slots) not in self.__dict__.get("_stepped_sizes", ()):
             return None
 
         def given(t, shape, dtypes):
@@ -2036,7 +2020,8 @@ class GraphedTrunk:
         self.cur = 0  # index of the buffer holding the current state
         self.graphs, self.outputs = [], []
         self._sizes = (num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
-        self._shape = _register_shape(trunk, *self._sizes)
+        if autocast_dtype == torch.bfloat16:
+            trunk._stepped_at(*self._sizes)
         self._whole = self._lay_out()
         if self._whole is not None:
             # one launch is all there is: it reads the caller's tensors, and there is nothing to capture
@@ -2183,7 +2168,8 @@ class EagerTrunkStepper:
             raise ValueError("this trunk has no bullet-reading sublayer")
         self.reads_bullets = bool(num_bullet_slots)
         self._sizes = (num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
-        self._shape = _register_shape(trunk, *self._sizes)
+        if autocast_dtype == torch.bfloat16:
+            trunk._stepped_at(*self._sizes)
         self.states = [trunk.initial_hidden(num_envs, num_recurrent, dev) for _ in range(2)]
         self.cur = 0
 

@@ -404,3 +404,37 @@ def test_trunk_and_uncaptured_stepper_can_be_copied_after_a_whole_step(whole_ste
         packed = layer.out_proj.__dict__["_bnb_proj_pack"].value
         assert entry.norm1 == layer.norm1.weight.data_ptr() and entry.proj == packed.data_ptr()
         assert torch.equal(packed, ops.pack_proj_weights(layer.out_proj.weight.detach()))
+
+
+@pytest.mark.filterwarnings("ignore:CUDA is not available")
+def test_what_a_direct_call_runs_does_not_hang_on_the_lifetime_of_other_objects(whole_steps, monkeypatch):
+    """A stepper settles for its trunk how steps of its sizes run under its autocast: not for another trunk, not for float32, and not
+    only until it is collected."""
+    import gc
+
+    def step_packed(self, x, *args, after=None, **kw):
+        separate.append(self)
+        return (x, None) if after is not None else x
+
+    separate = []
+    monkeypatch.setattr(bnb.YemongBlock, "step_packed", step_packed)
+    trunk, other = _stepped_trunk(3), _stepped_trunk(4)
+    B, N, M = 3, 8, 4
+    x, alive, state = torch.randn(B, N + M, 128), torch.ones(B, N + M, dtype=torch.bool), trunk.initial_hidden(B, N, "cpu")
+
+    def runs(t):
+        whole_steps.clear(), separate.clear()
+        t(x, alive, state)
+        assert bool(whole_steps) != bool(separate)
+        return "one" if whole_steps else "separate"
+
+    assert runs(trunk) == "separate"
+    in_float32 = bnb.trunk_stepper(trunk, B, N + M, N, graph=False)
+    assert runs(trunk) == "separate" and in_float32.state is not None
+    stepper = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, graph=False)
+    assert runs(trunk) == "one" and runs(other) == "separate"
+    stepper.step(x, alive)
+    del stepper
+    gc.collect()
+    assert runs(trunk) == "one" and runs(other) == "separate"
+    assert not trunk.state_dict().keys() ^ other.state_dict().keys()

@@ -1640,6 +1640,14 @@ class _WholeStep:
                 and self._values() == self.values and self.weights_same())
 
 
+_ROWS = (torch.float32, torch.bfloat16)
+
+
+def _read_in_place(t: torch.Tensor, dtypes: tuple) -> bool:
+    """Whether ``ops.trunk_step`` reads ``t`` where it lies: dense, its values as stored (no pending negation), rows on 16-byte pieces."""
+    return t.dtype in dtypes and t.is_contiguous() and not t.is_neg() and (dtypes is _FLAGS or t.data_ptr() % 16 == 0)
+
+
 class _WholeSteps(dict):
     """The ``_WholeStep``s that a trunk keeps, by (field tokens, bullets read).  They hold addresses: a copy of the trunk starts without."""
 
@@ -1850,24 +1858,21 @@ class YemongTrunk(_WeightCaches, nn.Module):
         if (B, NM, n_rec, slots) not in self.__dict__.get("_stepped_sizes", ()):
             return None
 
-        def given(t, shape, dtypes):
-            return t is None or (isinstance(t, torch.Tensor) and tuple(t.shape) == shape and t.dtype in dtypes and t.device == x.device)
-
-        def whole(t):  # in place where t is dense and on a 16-byte piece
-            if t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0):
-                return t
-            return t.clone(memory_format=torch.contiguous_format)
-
-        rows, flags = (torch.float32, torch.bfloat16), (torch.bool, torch.uint8)
-        if not (given(x, (B, NM, D), rows) and given(alive, (B, NM), flags) and given(reset, (B,), flags)
-                and all(t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (state_in, state_out))
-                and (not slots or (given(bullets, (B, slots, D), rows) and given(in_flight, (B, slots), flags)))):
+        rows, flags = (B, NM, D), (B, NM)
+        inputs = [(x, rows, _ROWS), (alive, flags, _FLAGS), (reset, (B,), _FLAGS)]
+        if slots:
+            inputs += [(bullets, (B, slots, D), _ROWS), (in_flight, (B, slots), _FLAGS)]
+        if not (all(t.device == x.device and _read_in_place(t, (torch.float32,)) for t in (state_in, state_out))
+                and all(t is None or (isinstance(t, torch.Tensor) and t.shape == shape and t.dtype in dtypes and t.device == x.device)
+                        for t, shape, dtypes in inputs)):
             return None
         plan = self._whole_step_plan(B, NM, n_rec, slots, x.device)
         if plan is None:
             return None
-        return ops.trunk_step(plan.table, whole(x), n_rec, whole(alive), state_in, state_out, reset=whole(reset),
-                              bullets=whole(bullets) if slots else None, in_flight=whole(in_flight) if slots else None,
+        x, alive, reset, *read = (t if t is None or _read_in_place(t, dtypes) else t.clone(memory_format=torch.contiguous_format)
+                                  for t, _, dtypes in inputs)
+        bullets, in_flight = read if read else (None, None)
+        return ops.trunk_step(plan.table, x, n_rec, alive, state_in, state_out, reset=reset, bullets=bullets, in_flight=in_flight,
                               bullet_eps=plan.bullet_eps, out_dtype=x.dtype)
 
     def _bullet_kv_of_all_layers(self, bullets, rows):
@@ -2071,10 +2076,8 @@ class GraphedTrunk:
             if given is held or (given is None and name in ("reset", "bullets", "in_flight")):
                 ready[name] = given
                 continue
-            rows = held.dtype == torch.float32 or name == "bullets"
-            if (isinstance(given, torch.Tensor) and given.shape == held.shape and given.device == held.device and given.is_contiguous()
-                    and (given.dtype in (torch.float32, torch.bfloat16) and given.data_ptr() % 16 == 0 if rows else given.dtype in _FLAGS)
-                    and not given.is_neg()):
+            if (isinstance(given, torch.Tensor) and given.shape == held.shape and given.device == held.device
+                    and _read_in_place(given, _ROWS if name in ("x", "bullets") else _FLAGS)):
                 ready[name] = given
             else:
                 held.copy_(given)

@@ -2050,3 +2050,46 @@ def test_a_captured_stepper_whose_trunk_left_the_kernel_s_form_calls_the_trunk()
             want, want_state = trunk(x, alive, state, reset_mask=done)
         assert out.data_ptr() in [o.data_ptr() for o in stepper.outputs] and new_state is stepper.state
         assert torch.equal(out, want) and torch.equal(new_state, want_state), hooked
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("form", ["transposed", "offset", "negated", "uint8", "no_masks", "bfloat16"])
+def test_whole_steps_read_inputs_in_every_form_like_the_dense_ones(graph, form):
+    """Inputs that the kernel cannot read where they lie are copied first, masks may be bytes or absent; 130 slots an environment, every one
+    live without a mask: the bullets of a work-group in several pieces."""
+    D, H, B, N, M, K = 128, 4, 3, 13, 3, 10
+    trunk = bnb.YemongTrunk(_cfg(D, H, 2, 2, 1, bullets=1)).eval()
+    trunk.load_state_dict(trunk_params(191, D, 2, 2, 1), strict=False)
+    trunk.to(DEV)
+    gen = torch.Generator().manual_seed(192)
+    stepper = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, graph=graph, num_bullet_slots=N * K)
+    assert stepper._whole is not None
+    state = torch.randn(stepper.state.shape, generator=gen).to(DEV)
+    dense = {"tokens": torch.randn(B, N + M, D, generator=gen), "alive_mask": torch.rand(B, N + M, generator=gen) < 0.7,
+             "reset_mask": torch.tensor([False, True, False]), "bullets": torch.randn(B, N * K, D, generator=gen),
+             "bullet_mask": torch.rand(B, N * K, generator=gen) < 0.5}
+    dense = {name: t.to(DEV) for name, t in dense.items()}
+    given = dict(dense)
+    floats = ("tokens", "bullets")
+    if form == "transposed":
+        given.update({name: dense[name].transpose(0, 1).contiguous().transpose(0, 1) for name in dense if name != "reset_mask"})
+        given["reset_mask"] = dense["reset_mask"].repeat_interleave(2)[::2]
+    elif form == "offset":
+        for name, t in dense.items():
+            given[name] = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view(t.shape).copy_(t)
+    elif form == "negated":
+        given.update({name: torch._neg_view(-dense[name]) for name in floats})
+    elif form == "uint8":
+        given.update({name: 3 * t.to(torch.uint8) for name, t in dense.items() if name not in floats})
+    elif form == "no_masks":
+        given.update(reset_mask=None, bullet_mask=None)
+        dense["reset_mask"], dense["bullet_mask"] = torch.zeros_like(dense["reset_mask"]), torch.ones_like(dense["bullet_mask"])
+    else:
+        given.update({name: dense[name].bfloat16() for name in floats})
+        dense.update({name: given[name].float() for name in floats})
+    results = []
+    for inputs in (given, dense):
+        stepper.load_state(state)
+        results.append([t.clone() for t in stepper.step(**inputs)])
+    (out, new_state), (want, want_state) = results
+    assert torch.equal(out, want.to(out.dtype)) and torch.equal(new_state, want_state)

@@ -22,10 +22,9 @@ import torch
 from . import _native
 
 _DTYPE_CODE = {torch.float32: _native.F32, torch.bfloat16: _native.BF16}
-class _autocast_off:
-    """``torch.autocast("cuda", enabled=False)`` around calls that state their dtypes themselves: only the flag, and only where
-    autocast is on (the general context costs 5 us a use; a pass of the update enters sixty)."""
 
+
+class _AutocastFlagOff:
     __slots__ = ("was_on",)
 
     def __enter__(self):
@@ -37,6 +36,13 @@ class _autocast_off:
         if self.was_on:
             torch.set_autocast_enabled("cuda", True)
         return False
+
+
+def _autocast_off():
+    """``torch.autocast("cuda", enabled=False)`` around calls that state their dtypes themselves: only the flag, and only where
+    autocast is on (the general context costs 5 us a use; a pass of the update enters sixty).  The tracer of torch.compile knows the
+    general context and not the flag."""
+    return torch.autocast("cuda", enabled=False) if torch.compiler.is_compiling() else _AutocastFlagOff()
 
 
 def _outside_autocast(backward):

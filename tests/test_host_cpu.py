@@ -438,3 +438,28 @@ def test_what_a_direct_call_runs_does_not_hang_on_the_lifetime_of_other_objects(
     gc.collect()
     assert runs(trunk) == "one" and runs(other) == "separate"
     assert not trunk.state_dict().keys() ^ other.state_dict().keys()
+
+
+def test_leaving_autocast_around_a_call_is_traced_by_torch_compile():
+    """Under autocast a compiled function that uses it is one graph, and runs with autocast off inside and on again behind it."""
+    from torch._dynamo.testing import CompileCounter
+
+    def inside(x):
+        with ops._autocast_off():
+            return torch.sin(x) + 1.0, torch.is_autocast_enabled("cuda")
+
+    counter = CompileCounter()
+    torch._dynamo.reset()
+    before = torch.is_autocast_enabled("cuda")
+    torch.set_autocast_enabled("cuda", True)
+    try:
+        for fn in (inside, torch.compile(inside, backend=counter, fullgraph=True)):
+            out, on = fn(torch.zeros(3))
+            assert torch.equal(out, torch.ones(3)) and on is False and torch.is_autocast_enabled("cuda")
+            with pytest.raises(ZeroDivisionError), ops._autocast_off():
+                1 // 0
+            assert torch.is_autocast_enabled("cuda")
+    finally:
+        torch.set_autocast_enabled("cuda", before)
+        torch._dynamo.reset()
+    assert counter.frame_count == 1

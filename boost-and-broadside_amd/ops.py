@@ -2363,7 +2363,7 @@ def _rows(t: torch.Tensor, D: int) -> torch.Tensor:
     """``t`` (..., D) as (R, D) rows at one pitch that the kernels read, copied only where it has none."""
     if not _uniform_rows(t, D):
         return t.reshape(-1, D).contiguous()
-    return t if t.dim() == 2 else t.view(-1, D)
+    return t if t.dim() == 2 and t.shape[0] > 1 else t.view(-1, D)  # (the view gives a single row a pitch, whatever its stride says)
 
 
 def _uniform_rows(t: torch.Tensor, D: int) -> bool:

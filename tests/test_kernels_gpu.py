@@ -3338,3 +3338,22 @@ def test_compact_rows_hints_are_checked_on_request(monkeypatch):
     with pytest.raises(ValueError, match="do not fit the mask"):
         ops.CompactRows(mask, total=total - 1, max_count=most)
     ops.CompactRows(mask, total=total, max_count=most)
+
+
+def test_a_single_row_of_any_stride_is_read_as_a_row():
+    """A column of a wider tensor turned into one row carries the column's stride, which says nothing about a row's pitch."""
+    g = torch.Generator().manual_seed(7)
+
+    def column(dtype):
+        return torch.randn(128, 1, generator=g).to(DEV, dtype).t()
+
+    x, dy = column(torch.float32), column(torch.float32)
+    assert x.stride() == (1, 1) and x.is_contiguous()
+    w = torch.randn(64, 128, generator=g).to(DEV)
+    packed, nw = ops.pack_linear_f32(w), torch.randn(128, generator=g).to(DEV)
+    assert torch.equal(ops.linear_f32(x, packed), ops.linear_f32(x.view(-1, 128), packed))
+    for got, want in zip(ops.rmsnorm_bwd(x, dy, nw), ops.rmsnorm_bwd(x.view(-1, 128), dy.view(-1, 128), nw)):
+        assert torch.equal(got, want)
+    a, b = column(torch.bfloat16), column(torch.bfloat16)
+    assert torch.equal(ops.linear_wgrad(a, b), ops.linear_wgrad(a.view(-1, 128), b.view(-1, 128)))
+    assert torch.equal(ops.linear_wgrad(a, b), a.float().t() @ b.float())

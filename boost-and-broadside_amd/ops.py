@@ -3035,6 +3035,13 @@ def trunk_step(table, x, n_rec, alive, state_in, state_out, *, reset=None, bulle
             raise ValueError(f"{name} must be a contiguous {shape} tensor of {dtypes} on {x.device}")
     if sum(entry.temporal for entry in table) > slots:
         raise ValueError("more recurrent sublayers than slots of the state")
+    return launch_trunk_step(table, x, n_rec, alive, state_in, state_out, out, reset, bullets, in_flight, bullet_eps)
+
+
+def launch_trunk_step(table, x, n_rec, alive, state_in, state_out, out, reset, bullets, in_flight, bullet_eps) -> torch.Tensor:
+    """``trunk_step`` for a caller that has asked all of its questions itself."""
+    B, NM, D = x.shape
+    NB = 0 if bullets is None else bullets.shape[1]
     ptr = [None if t is None else t.data_ptr() for t in (alive, reset, bullets, in_flight)]
     with _on_device(x.device):
         rc = _native.load().bnb_trunk_step_fwd(

@@ -1563,6 +1563,8 @@ def _byte_range(t: torch.Tensor) -> tuple[int, int]:
     """[first, last) byte addresses a (possibly strided) tensor can touch."""
     if t.numel() == 0:
         return (0, 0)
+    if t.is_contiguous():
+        return t.data_ptr(), t.data_ptr() + t.nbytes
     span = sum((n - 1) * abs(st) for n, st in zip(t.shape, t.stride())) + 1
     return t.data_ptr(), t.data_ptr() + span * t.element_size()
 
@@ -1598,33 +1600,40 @@ class _WholeStep:
     ``aliases`` share a parameter's memory and its version counter: they keep what the table points to from being freed under it, and
     are read in half the time of the parameter subclass."""
 
-    __slots__ = ("table", "bullet_eps", "tensors", "children", "slots", "params", "held", "aliases", "written", "derived", "constants",
-                 "values", "calls")
+    __slots__ = ("table", "bullet_eps", "recurrent", "tensors", "children", "slots", "params", "held", "watched", "aliases", "written", "derived", "constants",
+                 "values", "types", "overrides", "hooks")
 
     def __init__(self, trunk: nn.Module, layers: list, bullet_eps: float) -> None:
         self.table, self.bullet_eps = ops.trunk_table(layers), bullet_eps
+        self.recurrent = sum(entry.temporal for entry in self.table)  # slots of the state that the kernel writes
         self.tensors = [t for entry in layers for t in entry.values() if isinstance(t, torch.Tensor)]
         modules = list(trunk.modules())
         self.children = [(m._modules, dict(m._modules)) for m in modules if m._modules]
-        self.slots = [(m._parameters, name) for m in modules for name in m._parameters]
-        self.params = [d[name] for d, name in self.slots]
+        self.slots = [(m._parameters.get, name) for m in modules for name in m._parameters]
+        self.params = [get(name) for get, name in self.slots]
         used = {t.data_ptr() for t in self.tensors}
-        self.derived = [(m.__dict__, k, v) for m in modules for k, v in m.__dict__.items()
+        self.derived = [(m.__dict__.get, k, v) for m in modules for k, v in m.__dict__.items()
                         if k.startswith(_CACHE_PREFIX) and isinstance(v, _DerivedWeight) and isinstance(v.value, torch.Tensor)
                         and v.value.data_ptr() in used]
-        self.calls = _whole_step_calls(trunk)
-        self.constants = [(m.__dict__, name) for m in modules for name in ("eps", "c", "n_heads", "reads_bullets") if name in m.__dict__]
+        calls = _whole_step_calls(trunk)
+        self.types = [(m, type(m)) for m, _ in calls]
+        self.overrides = [(m.__dict__, own.__name__) for m, own in calls]
+        hooked = [m for m, own in calls if own.__name__ == "forward"]
+        self.hooks = [hooks for m in hooked for hooks in (m._forward_hooks, m._forward_pre_hooks)]
+        self.hooks += [module_internals._global_forward_hooks, module_internals._global_forward_pre_hooks]
+        self.constants = [(m.__dict__.get, name) for m in modules for name in ("eps", "c", "n_heads", "reads_bullets") if name in m.__dict__]
         self.values = self._values()
         self.held = [p for p in self.params if p is not None]
+        self.watched = [p for p in self.held if isinstance(p, WatchedParameter)]
         self.aliases = [torch._C.TensorBase.detach(p) for p in self.held]
         self.written = self._written()
 
     def _values(self) -> list:
-        return [d.get(name) for d, name in self.constants]
+        return [get(name) for get, name in self.constants]
 
     def _written(self):
         return (list(map(torch._C.TensorBase.data_ptr, self.held)), [a._version for a in self.aliases],
-                [getattr(p, "_bnb_touch", 0) for p in self.held])
+                [getattr(p, "_bnb_touch", 0) for p in self.watched])
 
     def weights_same(self) -> bool:
         """Whether the parameters that were laid out lie where they lay and hold what they held."""
@@ -1633,19 +1642,22 @@ class _WholeStep:
     def same(self) -> bool:
         """Whether a table laid out now would be this one: besides the weights the same submodules, parameters and constants, no hooks or
         overrides, no derived weight invalidated."""
-        return (all(now == then for now, then in self.children)
-                and all(map(operator.is_, [d.get(name) for d, name in self.slots], self.params))
-                and all(_plain_call(m, own) for m, own in self.calls)
-                and all(d.get(slot) is entry and entry.key is not None for d, slot, entry in self.derived)
+        return (all([now == then for now, then in self.children])
+                and all(map(operator.is_, [get(name) for get, name in self.slots], self.params))
+                and not any(self.hooks) and all([m.__class__ is kind for m, kind in self.types])
+                and not any([name in d for d, name in self.overrides])
+                and all([get(slot) is entry and entry.key is not None for get, slot, entry in self.derived])
                 and self._values() == self.values and self.weights_same())
 
 
+_KERNEL_DEVICE = "cuda"
 _ROWS = (torch.float32, torch.bfloat16)
 
 
 def _read_in_place(t: torch.Tensor, dtypes: tuple) -> bool:
-    """Whether ``ops.trunk_step`` reads ``t`` where it lies: dense, its values as stored (no pending negation), rows on 16-byte pieces."""
-    return t.dtype in dtypes and t.is_contiguous() and not t.is_neg() and (dtypes is _FLAGS or t.data_ptr() % 16 == 0)
+    """Whether ``ops.trunk_step`` reads ``t``, of one of ``dtypes``, where it lies: dense, its values as stored (no pending negation),
+    rows on 16-byte pieces."""
+    return t.is_contiguous() and not t.is_neg() and (dtypes is _FLAGS or t.data_ptr() % 16 == 0)
 
 
 class _WholeSteps(dict):
@@ -1756,10 +1768,9 @@ class YemongTrunk(_WeightCaches, nn.Module):
 
         return _cached_cast(self, "_bnb_bullet_kv_pack", ws, torch.bfloat16, folded)
 
-    def _whole_step_layers(self, B, NM, n_rec, slots, device):
-        """``(layers of ops.trunk_table, eps of the bullet norm)`` where the whole step runs as one kernel for B environments of
-        NM tokens, n_rec of them recurrent, with ``slots`` bullet slots (0: no read): small fleets under bfloat16 autocast,
-        every layer in its standard form.  Else None."""
+    def _whole_step_layers(self, NM, n_rec, slots):
+        """``(layers of ops.trunk_table, eps of the bullet norm)`` of the step as one kernel under bfloat16 autocast for NM tokens, n_rec
+        of them recurrent, and ``slots`` bullet slots (0: no read), where every layer has its standard form.  Else None."""
         blocks = list(self.yemong_layers)
         calls = _whole_step_calls(self)
         if not (all(_plain_call(m, own) for m, own in calls)
@@ -1767,7 +1778,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
                 and all(type(l) is GriffinTemporalBlock for block in blocks for l in block.temporal)):
             return None
         readers = [l for block in blocks for l in block.spatial if l.reads_bullets] if slots else []
-        if not self._whole_step_fits(B, NM, n_rec, slots, device, len(calls) - 2 * len(blocks), bool(readers)):
+        if self.config.d_model != ops.FFN_WIDTH or not 0 < len(calls) - 2 * len(blocks) <= _native.TRUNK_MAX_LAYERS:
             return None
 
         def vector(t):
@@ -1826,54 +1837,53 @@ class YemongTrunk(_WeightCaches, nn.Module):
                 table.append(entry)
         return table, (eps(readers[0].norm_bullet) if readers else 0.0)
 
-    def _stepped_at(self, B, NM, n_rec, slots) -> None:
+    def _stepped_at(self, B, NM, n_rec, slots, device) -> None:
         """From here on this trunk steps B environments of NM tokens, n_rec of them recurrent, with ``slots`` bullet slots as one kernel
-        under bfloat16 autocast, where that applies: said by a stepper when it is made.  A direct call of these sizes then gives
-        that stepper's bits, for as long as the trunk lives; a call of other sizes runs separate kernels, a bfloat16 rounding apart."""
-        self.__dict__.setdefault("_stepped_sizes", set()).add((B, NM, n_rec, slots))
+        under bfloat16 autocast, where that kernel covers these sizes and is the faster one: said by a stepper when it is made.  A
+        direct call of these sizes then gives that stepper's bits, for as long as the trunk lives; a call of other sizes runs separate
+        kernels, a bfloat16 rounding apart."""
+        if (ops.trunk_step_supported(B, NM, n_rec, self.config.d_model, self.config.n_heads, 1, slots) and device.type == _KERNEL_DEVICE
+                and ops.trunk_step_pays(B, NM, slots > 0, device)):
+            self.__dict__.setdefault("_stepped_sizes", set()).add((B, NM, n_rec, slots))
 
-    def _whole_step_fits(self, B, NM, n_rec, slots, device, n_layers, reads) -> bool:
-        """Whether the kernel of the whole step covers these sizes, under the autocast of the call, and is the faster one."""
-        return (_HEAD_FUSION and device.type == "cuda" and _projection_dtype() == torch.bfloat16
-                and ops.trunk_step_supported(B, NM, n_rec, self.config.d_model, self.config.n_heads, n_layers, slots if reads else 0)
-                and ops.trunk_step_pays(B, NM, reads, device))
-
-    def _whole_step_plan(self, B, NM, n_rec, slots, device) -> _WholeStep | None:
-        """The step as one kernel, or None where that does not apply.  Kept while the trunk stays as it is."""
+    def _whole_step_plan(self, B, NM, n_rec, slots) -> _WholeStep | None:
+        """The step as one kernel at the sizes that a stepper was made for (``_stepped_at``), or None where that does not apply.  Kept
+        while the trunk stays as it is."""
+        if not ((B, NM, n_rec, slots) in self.__dict__.get("_stepped_sizes", ()) and _HEAD_FUSION and _projection_dtype() == torch.bfloat16):
+            return None
         kept, key = self.__dict__.setdefault("_whole_steps", _WholeSteps()), (NM > n_rec, slots > 0)
         plan = kept.get(key)
-        if plan is not None and plan.children[0][0] is self._modules and plan.same():
-            return plan if self._whole_step_fits(B, NM, n_rec, slots, device, len(plan.table), key[1]) else None
-        found = self._whole_step_layers(B, NM, n_rec, slots, device)
-        kept.pop(key, None)
-        if found is None:
-            return None
-        plan = kept[key] = _WholeStep(self, *found)
+        if plan is None or plan.children[0][0] is not self._modules or not plan.same():
+            kept.pop(key, None)
+            found = self._whole_step_layers(NM, n_rec, slots)
+            if found is None:
+                return None
+            plan = kept[key] = _WholeStep(self, *found)
         return plan
 
     def _whole_step(self, x, alive, state_in, state_out, n_rec, reset, bullets, in_flight):
-        """The step as one kernel at the sizes that a stepper has been made for (``_stepped_at``) and where that applies, else None."""
+        """The step as one kernel, or None where ``_whole_step_plan`` has none or the inputs are not what the kernel takes."""
         B, NM, D = x.shape
         slots = bullets.shape[1] if bullets is not None and self.config.reads_bullets and bullets.dim() == 3 else 0
-        if (B, NM, n_rec, slots) not in self.__dict__.get("_stepped_sizes", ()):
-            return None
-
-        rows, flags = (B, NM, D), (B, NM)
-        inputs = [(x, rows, _ROWS), (alive, flags, _FLAGS), (reset, (B,), _FLAGS)]
-        if slots:
-            inputs += [(bullets, (B, slots, D), _ROWS), (in_flight, (B, slots), _FLAGS)]
-        if not (all(t.device == x.device and _read_in_place(t, (torch.float32,)) for t in (state_in, state_out))
-                and all(t is None or (isinstance(t, torch.Tensor) and t.shape == shape and t.dtype in dtypes and t.device == x.device)
-                        for t, shape, dtypes in inputs)):
-            return None
-        plan = self._whole_step_plan(B, NM, n_rec, slots, x.device)
+        plan = self._whole_step_plan(B, NM, n_rec, slots) if D == ops.FFN_WIDTH else None
         if plan is None:
             return None
-        x, alive, reset, *read = (t if t is None or _read_in_place(t, dtypes) else t.clone(memory_format=torch.contiguous_format)
-                                  for t, _, dtypes in inputs)
-        bullets, in_flight = read if read else (None, None)
-        return ops.trunk_step(plan.table, x, n_rec, alive, state_in, state_out, reset=reset, bullets=bullets, in_flight=in_flight,
-                              bullet_eps=plan.bullet_eps, out_dtype=x.dtype)
+        device, ready = x.device, []
+        for t, shape, dtypes in ((state_in, state_in.shape, (torch.float32,)), (state_out, state_in.shape, (torch.float32,)), (x, (B, NM, D), _ROWS),
+                                 (alive, (B, NM), _FLAGS), (reset, (B,), _FLAGS), (bullets if slots else None, (B, slots, D), _ROWS),
+                                 (in_flight if slots else None, (B, slots), _FLAGS)):
+            if t is not None and not (isinstance(t, torch.Tensor) and t.dtype in dtypes and t.shape == shape and t.device == device):
+                return None
+            ready.append(t)
+            if t is not None and not _read_in_place(t, dtypes):
+                if t is state_in or t is state_out:
+                    return None
+                ready[-1] = t.clone(memory_format=torch.contiguous_format)
+        if plan.recurrent > state_in.shape[0]:
+            return None
+        state_in, state_out, x, alive, reset, bullets, in_flight = ready
+        return ops.launch_trunk_step(plan.table, x, n_rec, alive, state_in, state_out, torch.empty_like(x), reset, bullets, in_flight,
+                                     plan.bullet_eps)
 
     def _bullet_kv_of_all_layers(self, bullets, rows):
         """``{id(layer): [K | V] rows}`` of every bullet-reading sublayer of the step from ONE pass over the bullets in
@@ -2026,7 +2036,7 @@ class GraphedTrunk:
         self.graphs, self.outputs = [], []
         self._sizes = (num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
         if autocast_dtype == torch.bfloat16:
-            trunk._stepped_at(*self._sizes)
+            trunk._stepped_at(*self._sizes, dev)
         self._whole = self._lay_out()
         if self._whole is not None:
             # one launch is all there is: it reads the caller's tensors, and there is nothing to capture
@@ -2059,7 +2069,8 @@ class GraphedTrunk:
         if not _plain_call(self.trunk, YemongTrunk.forward):
             return None
         with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None), torch.no_grad():
-            return self.trunk._whole_step_plan(*self._sizes, self.tokens.device)
+            plan = self.trunk._whole_step_plan(*self._sizes)
+        return plan if plan is not None and plan.recurrent <= self.states[0].shape[0] else None
 
     def _step_whole(self, inputs):
         """The step as one kernel: an input that is as the kernel reads it is read in place, any other is copied first."""
@@ -2077,14 +2088,14 @@ class GraphedTrunk:
                 ready[name] = given
                 continue
             if (isinstance(given, torch.Tensor) and given.shape == held.shape and given.device == held.device
-                    and _read_in_place(given, _ROWS if name in ("x", "bullets") else _FLAGS)):
+                    and given.dtype in (dtypes := _ROWS if name in ("x", "bullets") else _FLAGS) and _read_in_place(given, dtypes)):
                 ready[name] = given
             else:
                 held.copy_(given)
                 ready[name] = held
-        return ops.trunk_step(self._whole.table, ready["x"], self._sizes[2], ready["alive"], self.states[self.cur], self.states[1 - self.cur],
-                              reset=ready["reset"], bullets=ready["bullets"], in_flight=ready["in_flight"], bullet_eps=self._whole.bullet_eps,
-                              out=self.outputs[self.cur])
+        return ops.launch_trunk_step(self._whole.table, ready["x"], self._sizes[2], ready["alive"], self.states[self.cur],
+                                     self.states[1 - self.cur], self.outputs[self.cur], ready["reset"], ready["bullets"], ready["in_flight"],
+                                     self._whole.bullet_eps)
 
     def refresh_weights(self) -> None:
         """Rebuild every derived weight copy the graphs read from the current parameters, in place.  Where the step is one
@@ -2172,7 +2183,7 @@ class EagerTrunkStepper:
         self.reads_bullets = bool(num_bullet_slots)
         self._sizes = (num_envs, num_tokens, num_recurrent, num_bullet_slots or 0)
         if autocast_dtype == torch.bfloat16:
-            trunk._stepped_at(*self._sizes)
+            trunk._stepped_at(*self._sizes, dev)
         self.states = [trunk.initial_hidden(num_envs, num_recurrent, dev) for _ in range(2)]
         self.cur = 0
 
@@ -2202,7 +2213,7 @@ class EagerTrunkStepper:
     def _whole(self) -> _WholeStep | None:
         """The step as one kernel, or None where the trunk's own forward runs separate kernels."""
         with torch.autocast("cuda", dtype=self.autocast_dtype or torch.bfloat16, enabled=self.autocast_dtype is not None):
-            return self.trunk._whole_step_plan(*self._sizes, self.states[0].device)
+            return self.trunk._whole_step_plan(*self._sizes)
 
 
 # tokens per step below which a captured step beats plain launches, with the default trunk of 2 blocks x (2 attention +

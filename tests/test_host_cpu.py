@@ -277,24 +277,20 @@ def test_steppers_refuse_to_drop_the_bullets_of_a_bullet_reading_trunk():
 def whole_steps(monkeypatch):
     """The host side of the step as one kernel: the launch is replaced by a recorder of what the kernel would read.  Yields the
     list of launches, each the fields of the table's layers."""
-    import types
-
     from boost_and_broadside_amd import trunk as trunk_module
 
     launches = []
 
-    def launch(table, x, n_rec, alive, state_in, state_out, *, out=None, out_dtype=torch.float32, bullet_eps=0.0, **inputs):
-        launches.append({"layers": [{name: getattr(entry, name) for name, _ in entry._fields_} for entry in table], "x": x.clone(),
-                         "alive": alive, "bullet_eps": bullet_eps, **inputs})
+    def launch(table, x, n_rec, alive, state_in, state_out, out, reset, bullets, in_flight, bullet_eps):
+        launches.append({"layers": [{name: getattr(entry, name) for name, _ in entry._fields_} for entry in table],
+                         "bullet_eps": bullet_eps})
         state_out.copy_(state_in)
-        return (torch.empty(x.shape, dtype=out_dtype) if out is None else out).copy_(x)
+        return out.copy_(x)
 
-    real = bnb.YemongTrunk._whole_step_fits
-    monkeypatch.setattr(bnb.YemongTrunk, "_whole_step_fits",
-                        lambda self, *sizes: real(self, *sizes[:4], types.SimpleNamespace(type="cuda"), *sizes[5:]))
+    monkeypatch.setattr(trunk_module, "_KERNEL_DEVICE", "cpu")
     monkeypatch.setattr(trunk_module, "_projection_dtype", lambda: torch.bfloat16)
     monkeypatch.setattr(ops, "trunk_step_pays", lambda *a: True)
-    monkeypatch.setattr(ops, "trunk_step", launch)
+    monkeypatch.setattr(ops, "launch_trunk_step", launch)
     return launches
 
 

@@ -1600,13 +1600,14 @@ class _WholeStep:
     ``aliases`` share a parameter's memory and its version counter: they keep what the table points to from being freed under it, and
     are read in half the time of the parameter subclass."""
 
-    __slots__ = ("table", "bullet_eps", "recurrent", "tensors", "children", "slots", "params", "held", "watched", "aliases", "written", "derived", "constants",
+    __slots__ = ("table", "bullet_eps", "recurrent", "device", "tensors", "children", "slots", "params", "held", "watched", "aliases", "written", "derived", "constants",
                  "values", "types", "overrides", "hooks")
 
     def __init__(self, trunk: nn.Module, layers: list, bullet_eps: float) -> None:
         self.table, self.bullet_eps = ops.trunk_table(layers), bullet_eps
         self.recurrent = sum(entry.temporal for entry in self.table)  # slots of the state that the kernel writes
         self.tensors = [t for entry in layers for t in entry.values() if isinstance(t, torch.Tensor)]
+        self.device = self.tensors[0].device
         modules = list(trunk.modules())
         self.children = [(m._modules, dict(m._modules)) for m in modules if m._modules]
         self.slots = [(m._parameters.get, name) for m in modules for name in m._parameters]
@@ -1781,13 +1782,18 @@ class YemongTrunk(_WeightCaches, nn.Module):
         if self.config.d_model != ops.FFN_WIDTH or not 0 < len(calls) - 2 * len(blocks) <= _native.TRUNK_MAX_LAYERS:
             return None
 
-        def vector(t):
-            return t is not None and t.dtype == torch.float32 and t.is_contiguous()
+        D, hidden = ops.FFN_WIDTH, ops.FFN_HIDDEN
+
+        def shaped(t, *shape):
+            return t is not None and tuple(t.shape) == shape
+
+        def vector(t, *shape):  # read by the kernel as it is
+            return shaped(t, *(shape or (D,))) and t.dtype == torch.float32 and t.is_contiguous()
 
         def plain(layer, mlp, *linears):
             return (vector(layer.norm1.weight) and vector(layer.norm2.weight)
-                    and all(l.bias is None for l in (*linears, mlp.gate_proj, mlp.up_proj, mlp.down_proj))
-                    and tuple(mlp.gate_proj.weight.shape) == (ops.FFN_HIDDEN, ops.FFN_WIDTH))
+                    and all(l.bias is None and shaped(l.weight, *shape) for l, *shape in (
+                        *linears, (mlp.gate_proj, hidden, D), (mlp.up_proj, hidden, D), (mlp.down_proj, D, hidden))))
 
         def eps(norm):
             return ops._F32_EPS if norm.eps is None else norm.eps
@@ -1798,14 +1804,16 @@ class YemongTrunk(_WeightCaches, nn.Module):
                     "ffn": mlp.packed_weights(), "norm1": layer.norm1.weight, "norm2": layer.norm2.weight, "eps1": eps(layer.norm1),
                     "eps2": eps(layer.norm2)}
 
-        if any(l.kv_bullet.bias is not None or not vector(l.norm_bullet.weight) or l.norm_bullet.eps != readers[0].norm_bullet.eps
-               for l in readers):
+        if len({p.device for p in self.parameters()}) != 1:
+            return None
+        if any(l.kv_bullet.bias is not None or not shaped(l.kv_bullet.weight, 2 * D, D) or not vector(l.norm_bullet.weight)
+               or l.norm_bullet.eps != readers[0].norm_bullet.eps for l in readers):
             return None
         kv = self._folded_bullet_pack(readers) if readers else None
         table, slot, reader = [], 0, 0
         for block in blocks:
             for l in block.spatial:
-                if not plain(l, l.ffn, l.qkv, l.out_proj):
+                if not (plain(l, l.ffn, (l.qkv, 3 * D, D), (l.out_proj, D, D)) and l.n_heads == self.config.n_heads):
                     return None
                 w = l.qkv.weight
                 entry = shared(l, l.ffn, l.out_proj)
@@ -1817,9 +1825,11 @@ class YemongTrunk(_WeightCaches, nn.Module):
             for j, l in enumerate(block.temporal):
                 rg = l.rg_lru
                 fold, ws = l._head_weights(NM, n_rec, block.field_sub[j] if NM > n_rec else None)
-                if not (plain(l, l.gated_mlp, l.linear1, l.linear2, l.linear_out)
-                        and rg.linear_a.bias is not None and rg.linear_x.bias is not None and fold == (NM > n_rec)
-                        and vector(l.conv.weight) and (l.conv.bias is None or vector(l.conv.bias)) and rg.log_lambda.dtype == torch.float32):
+                if not (plain(l, l.gated_mlp, *((linear, D, D) for linear in (l.linear1, l.linear2, l.linear_out))) and fold == (NM > n_rec)
+                        and all(shaped(w, D, D) for w in (*ws, rg.linear_a.weight, rg.linear_x.weight))
+                        and shaped(rg.linear_a.bias, D) and shaped(rg.linear_x.bias, D) and vector(l.conv.weight, D, 1, CONV_KERNEL)
+                        and (l.conv.bias is None or vector(l.conv.bias)) and shaped(rg.log_lambda, D)
+                        and rg.log_lambda.dtype == torch.float32):
                     return None
                 gw, gb = (rg.linear_a.weight, rg.linear_x.weight), (rg.linear_a.bias, rg.linear_x.bias)
                 entry = shared(l, l.gated_mlp, l.linear_out)
@@ -1866,9 +1876,9 @@ class YemongTrunk(_WeightCaches, nn.Module):
         B, NM, D = x.shape
         slots = bullets.shape[1] if bullets is not None and self.config.reads_bullets and bullets.dim() == 3 else 0
         plan = self._whole_step_plan(B, NM, n_rec, slots) if D == ops.FFN_WIDTH else None
-        if plan is None:
-            return None
         device, ready = x.device, []
+        if plan is None or plan.device != device:
+            return None
         for t, shape, dtypes in ((state_in, state_in.shape, (torch.float32,)), (state_out, state_in.shape, (torch.float32,)), (x, (B, NM, D), _ROWS),
                                  (alive, (B, NM), _FLAGS), (reset, (B,), _FLAGS), (bullets if slots else None, (B, slots, D), _ROWS),
                                  (in_flight if slots else None, (B, slots), _FLAGS)):

@@ -459,3 +459,35 @@ def test_leaving_autocast_around_a_call_is_traced_by_torch_compile():
         torch.set_autocast_enabled("cuda", before)
         torch._dynamo.reset()
     assert counter.frame_count == 1
+
+
+@pytest.mark.filterwarnings("ignore:CUDA is not available")
+@pytest.mark.parametrize("where", ["norm1", "norm2", "qkv", "out_proj", "up_proj", "down_proj", "kv_bullet", "norm_bullet", "n_heads",
+                                   "linear1", "linear_out", "linear_a", "linear_a.bias", "conv.weight", "conv.bias", "log_lambda", "field_sub"])
+def test_a_layer_of_another_shape_is_not_laid_out_for_the_whole_step(whole_steps, where):
+    """The kernel reads every weight at the sizes of the standard layer."""
+    trunk = _stepped_trunk(5, n_bullet_cross_per_block=1)
+    stepper = bnb.trunk_stepper(trunk, 3, 12, 8, autocast_dtype=torch.bfloat16, graph=False, num_bullet_slots=80)
+    assert stepper._whole is not None
+    block = trunk.yemong_layers[1]
+    spatial, temporal = block.spatial[0], block.temporal[0]
+
+    def smaller(p):
+        return torch.nn.Parameter(p.detach()[:64].clone())
+
+    if where == "n_heads":
+        spatial.n_heads = 8
+    elif where in ("norm1", "norm2", "qkv", "out_proj", "kv_bullet", "norm_bullet"):
+        getattr(spatial, where).weight = smaller(getattr(spatial, where).weight)
+    elif where in ("up_proj", "down_proj"):
+        getattr(spatial.ffn, where).weight = smaller(getattr(spatial.ffn, where).weight)
+    elif where in ("linear1", "linear_out"):
+        getattr(temporal, where).weight = smaller(getattr(temporal, where).weight)
+    elif where == "field_sub":
+        block.field_sub[0].weight = smaller(block.field_sub[0].weight)
+    else:
+        owner, name = {"linear_a": (temporal.rg_lru.linear_a, "weight"), "linear_a.bias": (temporal.rg_lru.linear_a, "bias"),
+                       "conv.weight": (temporal.conv, "weight"), "conv.bias": (temporal.conv, "bias"),
+                       "log_lambda": (temporal.rg_lru, "log_lambda")}[where]
+        setattr(owner, name, smaller(getattr(owner, name)))
+    assert stepper._whole is None

@@ -2093,3 +2093,46 @@ def test_whole_steps_read_inputs_in_every_form_like_the_dense_ones(graph, form):
         results.append([t.clone() for t in stepper.step(**inputs)])
     (out, new_state), (want, want_state) = results
     assert torch.equal(out, want.to(out.dtype)) and torch.equal(new_state, want_state)
+
+
+@pytest.mark.parametrize("B,N,M,slots", [(5, 33, 0, 0), (3, 40, 4, 80), (24, 80, 4, 160)])
+def test_captured_bfloat16_steps_beyond_the_whole_step_kernel_replay_like_the_direct_call(B, N, M, slots):
+    """Battles of more than 32 tokens step as a captured graph of separate kernels: every replay gives the direct call's bits, with eager
+    work and synchronisations in between, the tails hand their projections over, and the replays follow the weights."""
+    from boost_and_broadside_amd import trunk as trunk_module
+
+    D, H = 128, 4
+    p = trunk_params(201 + N, D, 2, 2, 1)
+    trunk = bnb.YemongTrunk(_cfg(D, H, 2, 2, 1, bullets=int(slots > 0))).eval()
+    trunk.load_state_dict(p, strict=False)
+    trunk.to(DEV)
+    graphed = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, num_bullet_slots=slots if slots else None)
+    assert isinstance(graphed, bnb.GraphedTrunk) and len(graphed.graphs) == 2 and graphed._whole is None
+    gen = torch.Generator().manual_seed(202)
+    state = trunk.initial_hidden(B, N, DEV)
+    layer = trunk.yemong_layers[1].spatial[1]
+    for t in range(8):
+        x = torch.randn(B, N + M, D, generator=gen).to(DEV)
+        alive = (torch.rand(B, N + M, generator=gen) < 0.8).to(DEV)
+        done = (torch.rand(B, generator=gen) < 0.3).to(DEV) if t % 3 else None
+        bullets = torch.randn(B, slots, D, generator=gen).to(DEV) if slots else None
+        mask = (torch.rand(B, slots, generator=gen) < (2.0 if t == 5 else 0.3)).to(DEV) if slots else None
+        if t == 3:
+            with torch.no_grad():
+                layer.ffn.up_proj.weight.mul_(1.5)
+        elif t == 4:
+            layer.qkv.weight.data.mul_(0.5)
+        elif t == 6:
+            torch._C.TensorBase.data.__get__(layer.out_proj.weight).mul_(2.0)  # nothing counts this write
+            trunk.invalidate_weight_caches()
+            graphed.refresh_weights()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            want, want_state = trunk(x, alive, state, bullets, mask, reset_mask=done)
+            with trunk_module.separate_heads():
+                apart, _ = trunk(x, alive, state, bullets, mask, reset_mask=done)
+        if t % 2:
+            torch.cuda.synchronize()
+        out, new_state = graphed.step(x, alive, done, bullets, None if t == 5 else mask)  # without a mask: every slot holds a bullet
+        assert torch.equal(out, want) and torch.equal(new_state, want_state), t
+        assert max_rel(out.cpu(), apart.cpu()) <= BF16_TOL, t
+        state = want_state

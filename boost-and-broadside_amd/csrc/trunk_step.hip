@@ -3,8 +3,11 @@
 // Environments do not see each other, so a work-group takes the environments that fit 32 token rows through every sublayer
 // (reference: models/yemong/griffin.py:376-417 over models/yemong/attention.py:89-169 and griffin.py:269-317) and only tokens,
 // masks, bullets in flight and the recurrent state come from memory.  Step for step it computes what the separate kernels do
-// (norm_linear, sdpa_*, ffn_*, temporal_step), with their rounding points; the residual stream stays in registers, eight
-// channels a thread, and what one wave hands the next goes through LDS:
+// (norm_linear, sdpa_*, ffn_*, temporal_step), with their rounding points but two: the separate kernels round the merged heads, add the
+// read to them and round again, here each of the two is rounded once and the projection adds them (WAVES = 8) or their float32 sum
+// is rounded once (WAVES = 4); and a single reader's bullet norm weight is folded into its K and V weights like those of several.  The two forms also add the halves of a contraction in another order, so they agree to a bfloat16
+// rounding, not bit for bit.  The residual stream stays in registers, eight channels a thread, and what one wave hands the next goes
+// through LDS:
 //
 //   norm           16 lanes a row, bf16 rows into LDS
 //   attention      waves 0..3 one head of the self-attention each, waves 4..7 one head of the bullet read each.  Q, K and V of a
@@ -17,18 +20,20 @@
 //   gated MLP      gate / up: 64 hidden units a wave; down: four channel blocks x two halves of the hidden units
 //
 // What bounds it: every weight of the trunk passes through every work-group once, 0.5 to 0.6 MB a sublayer at the 64 bytes a
-// clock that a CU takes from its L2 (22 us of the 64 for two blocks of three sublayers; 27 us with all 256 CUs at it), and the
-// phases of a sublayer hang on one another over six to eight barriers.  So requests are dealt between matrix products and
+// clock that a CU takes from its L2 (22 us of the 61 for two blocks of three sublayers; 27 us with all 256 CUs at it), and the
+// phases of a sublayer hang on one another over six to eight barriers: matrix cores and vector ALU of a SIMD are busy for 86,000 of
+// 153,000 cycles.  So requests are dealt between matrix products and
 // activations (a burst of them stalls the wave that issues it), norm weights are asked for before operands (loads come back in
 // order), the barriers wait for LDS traffic only, and nothing may spill: a reload would wait for every operand under way.  In the
 // order in which that was found, 16 environments of 12 tokens: 93, 82, 66, 64 us; the separate kernels, 19 launches, 121 us.
-// 512 environments of 8 tokens 70 us (146).
+// 512 environments of 8 tokens 66 us (143).
 //
 // Two forms.  WAVES = 8 (one work-group a CU): heads and read, and the halves of a contraction, on different waves.  WAVES = 4 (two
 // work-groups a CU, where there are more than CUs): a wave does both one after the other and has twice the rows in the row
-// mapping; the first operands are requested where they are used, the neighbour's arithmetic covers the wait.  Its 0.2 us a
-// work-group of 24 rows is nearly all issue (matrix products, activations): 512 environments of 23 tokens 113 us (243), a rollout of 7808 x 12
-// 798 us (880), 51 us for every 32 rows of a CU against 62 us with eight waves.
+// mapping; the first operands are requested where they are used, the neighbour's arithmetic covers the wait.  A wave issues
+// 28,000 cycles of matrix products and 52,000 of vector instructions for its tile, which a SIMD does not overlap: busy for 72 % of the
+// time.  512 environments of 23 tokens 113 us (243), a rollout of 7808 x 12 760 us in a running loop (880), 50 us for every 32 rows of a
+// CU against 62 us with eight waves; 900 us in the first dozen launches after an idle spell, until the clock is up.
 
 #include "common.h"
 #include "ffn_math.h"
@@ -792,7 +797,7 @@ extern "C" int bnb_trunk_step_fwd(const bnb_trunk_layer *layers, int n_layers, c
     const int envs = kTkRows / NM;
     // Up to one work-group a CU: eight waves, the shortest way through a sublayer.  More: four waves and half the LDS, so that two
     // work-groups share a CU and one's arithmetic covers the other's waits; 512 work-groups 112 us against 133, 3904 work-groups
-    // 798 against 1000, where both SIMD slots issue nearly all the time.
+    // 760 against 1000.
     const int64_t groups = (B + envs - 1) / envs;
     if (groups <= cu_count())
         hipLaunchKernelGGL(trunk_step_kernel<8>, dim3((unsigned)groups), dim3(8 * kWave), 0, (hipStream_t)stream, a);

@@ -560,7 +560,8 @@ class _SdpaReadTrain(torch.autograd.Function):
 
 def sdpa_read_train(qkv: torch.Tensor, alive: torch.Tensor | None, kv_rows: torch.Tensor, rows: "CompactRows", n_heads: int) -> torch.Tensor:
     """``sdpa_train(qkv, alive) + sdpa_cross_rows_train(qkv, kv_rows, rows)`` (bfloat16, a non-empty list, where both cover the
-    shapes): the gradient of the queries is summed in float32 and written once."""
+    shapes).  The read's part of the queries' gradient is added in float32 to the bfloat16 gradient that the self-attention's backward
+    wrote, and the sum rounded: one rounding less than a read's gradient of its own, rounded before it is added."""
     total = rows.total_host()
     if kv_rows.shape[0] != total or total == 0:
         raise ValueError(f"kv_rows must hold the {total} listed rows, at least one")
@@ -2988,12 +2989,14 @@ def trunk_step_supported(B: int, NM: int, n_rec: int, D: int, n_heads: int, n_la
 def trunk_step_pays(B: int, NM: int, reads: bool, device) -> bool:
     """Whether the whole step as one kernel is faster than the separate kernels.
 
-    Up to one work-group of 32 rows (whole environments) a CU it takes about 65 us with the default trunk, behind that 15 us and
-    0.2 us a work-group of 256 CUs; the separate kernels about 95 us and 8.2 us for every thousand rows.  Without bullets 0.175 us
-    and 6.4 us.  us, one kernel / separate: 16 environments of 12 tokens 64 / 121,
-    512 of 8 71 / 146, 1024 of 12 (512 work-groups) 112 / 232, 1024 of 23 (1024) 214 / 343, 4096 of 12 (2048) 428 / 515, 7808 of 12
-    (3904) 798 / 880, 4096 of 23 (4096) 849 / 919, 8192 of 20 (8192, 20 of 32 rows filled) 1525 / 1347; without bullets 4955 of 9 (1652)
-    319 / 490, 5579 of 11 (2790) 499 / 490."""
+    Up to one work-group of 32 rows (whole environments) a CU it takes about 65 us with the default trunk, behind that up to 15 us and
+    0.2 us a work-group of 256 CUs; the separate kernels from 95 us and 8.2 us for every thousand rows.  Without bullets 0.175 us
+    and 6.4 us.  us, one kernel / separate: 16 environments of 12 tokens 62 / 122,
+    512 of 8 70 / 143, 1024 of 12 (512 work-groups) 115 / 233, 1024 of 23 (1024) 214 / 366, 4096 of 12 (2048) 405 / 617, 7808 of 12
+    (3904) 769 / 880, 4096 of 23 (4096) 806 / 916, 8192 of 20 (8192, 20 of 32 rows filled) 1544 / 1443, 6000 of 17 (6000) 1153 / 1066;
+    without bullets 4955 of 9 (1652) 328 / 509, 5579 of 11 (2790) 508 / 511, 3000 of 17 (3000) 538 / 507.  The line lies on the
+    separate kernels' side of what is measured: it leaves 4096 of 20 (779 / 838), 8192 of 11 (807 / 922) and 8000 of 23
+    (1565 / 1622) to them."""
     groups = -(-B // (TRUNK_TOKENS // NM))
     cus = torch.cuda.get_device_properties(device).multi_processor_count
     a_group, a_row = (0.2, 0.0082) if reads else (0.175, 0.0064)

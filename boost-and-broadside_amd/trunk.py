@@ -1592,6 +1592,11 @@ def _whole_step_calls(trunk) -> list:
             + [(l, TransformerBlock.forward) for l in block.spatial] + [(l, GriffinTemporalBlock.step_tokens) for l in block.temporal]]
 
 
+# where the layers cache the derived weights that the whole step reads
+_WHOLE_STEP_SLOTS = frozenset({"_bnb_proj_pack", "_bnb_head_pack", "_bnb_ffn_pack", "_bnb_l12_head_pack", "_bnb_l12f_head_pack", "_bnb_gate_pack",
+                               "_bnb_gate_bias", "_bnb_log2_sigmoid", "_bnb_bullet_kv_pack"})
+
+
 class _WholeStep:
     """The trunk's step as ``ops.trunk_step`` takes it (``table``, ``bullet_eps``) and everything that was laid out in it: the
     submodules, the parameters with their addresses and write counts, the derived weights, the constants.
@@ -1600,8 +1605,8 @@ class _WholeStep:
     ``aliases`` share a parameter's memory and its version counter: they keep what the table points to from being freed under it, and
     are read in half the time of the parameter subclass."""
 
-    __slots__ = ("table", "bullet_eps", "recurrent", "device", "tensors", "children", "slots", "params", "held", "watched", "aliases", "written", "derived", "constants",
-                 "values", "types", "overrides", "hooks")
+    __slots__ = ("table", "bullet_eps", "recurrent", "device", "tensors", "children", "slots", "params", "held", "watched", "aliases",
+                 "written", "derived", "constants", "values", "types", "overrides", "hooks")
 
     def __init__(self, trunk: nn.Module, layers: list, bullet_eps: float) -> None:
         self.table, self.bullet_eps = ops.trunk_table(layers), bullet_eps
@@ -1610,12 +1615,11 @@ class _WholeStep:
         self.device = self.tensors[0].device
         modules = list(trunk.modules())
         self.children = [(m._modules, dict(m._modules)) for m in modules if m._modules]
-        self.slots = [(m._parameters.get, name) for m in modules for name in m._parameters]
+        self.slots = [(parameters.get, name) for parameters in [m._parameters for m in modules] for name in parameters]
         self.params = [get(name) for get, name in self.slots]
         used = {t.data_ptr() for t in self.tensors}
-        self.derived = [(m.__dict__.get, k, v) for m in modules for k, v in m.__dict__.items()
-                        if k.startswith(_CACHE_PREFIX) and isinstance(v, _DerivedWeight) and isinstance(v.value, torch.Tensor)
-                        and v.value.data_ptr() in used]
+        self.derived = [(m.__dict__.get, k, m.__dict__[k]) for m in modules for k in _WHOLE_STEP_SLOTS.intersection(m.__dict__)
+                        if m.__dict__[k].value.data_ptr() in used]
         calls = _whole_step_calls(trunk)
         self.types = [(m, type(m)) for m, _ in calls]
         self.overrides = [(m.__dict__, own.__name__) for m, own in calls]
@@ -1625,7 +1629,7 @@ class _WholeStep:
         self.constants = [(m.__dict__.get, name) for m in modules for name in ("eps", "c", "n_heads", "reads_bullets") if name in m.__dict__]
         self.values = self._values()
         self.held = [p for p in self.params if p is not None]
-        self.watched = [p for p in self.held if isinstance(p, WatchedParameter)]
+        self.watched = [p for p in self.held if type(p) is WatchedParameter]
         self.aliases = [torch._C.TensorBase.detach(p) for p in self.held]
         self.written = self._written()
 
@@ -1785,7 +1789,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
         D, hidden = ops.FFN_WIDTH, ops.FFN_HIDDEN
 
         def shaped(t, *shape):
-            return t is not None and tuple(t.shape) == shape
+            return t is not None and t.shape == shape
 
         def vector(t, *shape):  # read by the kernel as it is
             return shaped(t, *(shape or (D,))) and t.dtype == torch.float32 and t.is_contiguous()
@@ -1804,8 +1808,6 @@ class YemongTrunk(_WeightCaches, nn.Module):
                     "ffn": mlp.packed_weights(), "norm1": layer.norm1.weight, "norm2": layer.norm2.weight, "eps1": eps(layer.norm1),
                     "eps2": eps(layer.norm2)}
 
-        if len({p.device for p in self.parameters()}) != 1:
-            return None
         if any(l.kv_bullet.bias is not None or not shaped(l.kv_bullet.weight, 2 * D, D) or not vector(l.norm_bullet.weight)
                or l.norm_bullet.eps != readers[0].norm_bullet.eps for l in readers):
             return None
@@ -1866,7 +1868,7 @@ class YemongTrunk(_WeightCaches, nn.Module):
         if plan is None or plan.children[0][0] is not self._modules or not plan.same():
             kept.pop(key, None)
             found = self._whole_step_layers(NM, n_rec, slots)
-            if found is None:
+            if found is None or len({t.device for entry in found[0] for t in entry.values() if isinstance(t, torch.Tensor)}) != 1:
                 return None
             plan = kept[key] = _WholeStep(self, *found)
         return plan

@@ -491,3 +491,22 @@ def test_a_layer_of_another_shape_is_not_laid_out_for_the_whole_step(whole_steps
                        "log_lambda": (temporal.rg_lru, "log_lambda")}[where]
         setattr(owner, name, smaller(getattr(owner, name)))
     assert stepper._whole is None
+
+
+@pytest.mark.filterwarnings("ignore:CUDA is not available")
+@pytest.mark.parametrize("fields", [0, 4])
+def test_a_whole_step_watches_every_derived_weight_it_reads(whole_steps, fields):
+    """Invalidating the caches lays the table out anew, whichever of its tensors is meant."""
+    trunk = _stepped_trunk(6, n_bullet_cross_per_block=1)
+    stepper = bnb.trunk_stepper(trunk, 3, 8 + fields, 8, autocast_dtype=torch.bfloat16, graph=False, num_bullet_slots=80)
+    plan = stepper._whole
+    held = {p.data_ptr() for p in trunk.parameters()}
+    read = {t.untyped_storage().data_ptr() for t in plan.tensors if t.data_ptr() not in held}
+    assert {entry.value.data_ptr() for _, _, entry in plan.derived} == read and len(read) == 25
+    for _, _, entry in plan.derived:
+        key, entry.key = entry.key, None
+        assert not plan.same()
+        entry.key = key
+    assert plan.same() and stepper._whole is plan
+    trunk.invalidate_weight_caches()
+    assert stepper._whole is not plan

@@ -2136,3 +2136,46 @@ def test_captured_bfloat16_steps_beyond_the_whole_step_kernel_replay_like_the_di
         assert torch.equal(out, want) and torch.equal(new_state, want_state), t
         assert max_rel(out.cpu(), apart.cpu()) <= BF16_TOL, t
         state = want_state
+
+
+def test_a_compiled_policy_steps_its_trunk_as_one_kernel_and_follows_weights_and_hooks():
+    """Where a stepper has settled the sizes, a traced call must ask the same questions before every launch as the eager one."""
+    import torch._dynamo
+
+    trunk, _ = _rollout_trunk(211)
+    B, N, M = 6, 8, 4
+    gen = torch.Generator().manual_seed(212)
+    x, alive = torch.randn(B, N + M, 128, generator=gen).to(DEV), torch.ones(B, N + M, dtype=torch.bool, device=DEV)
+    state = torch.randn(2, B * N, 512, generator=gen).to(DEV)
+    head = torch.nn.Linear(128, 6).to(DEV)
+    stepper = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, graph=False)
+    assert stepper._whole is not None
+
+    def policy(x, alive, state):
+        hidden, new_state = trunk(x * 1.0, alive, state)
+        return head(hidden), new_state
+
+    torch._dynamo.reset()
+    compiled = torch.compile(policy, backend="aot_eager")
+    layer, seen, handle = trunk.yemong_layers[0].spatial[0], [], None
+    try:
+        for change in ("none", "none", "in_place", "data", "eps", "hook", "unhook"):
+            if change == "in_place":
+                with torch.no_grad():
+                    layer.qkv.weight.mul_(1.5)
+            elif change == "data":
+                layer.norm2.weight.data = 1.5 * layer.norm2.weight.detach()
+            elif change == "eps":
+                layer.norm1.eps = 0.5
+            elif change == "hook":
+                handle = layer.register_forward_hook(lambda m, args, out: out * 1.25)
+            elif change == "unhook":
+                handle.remove()
+            with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+                want, got = policy(x, alive, state), compiled(x, alive, state)
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), change
+            seen.append(want[0])
+    finally:
+        torch._dynamo.reset()
+    assert torch.equal(seen[0], seen[1]) and torch.equal(seen[4], seen[6])
+    assert all(not torch.equal(a, b) for a, b in zip(seen[1:], seen[2:]))

@@ -2179,3 +2179,29 @@ def test_a_compiled_policy_steps_its_trunk_as_one_kernel_and_follows_weights_and
         torch._dynamo.reset()
     assert torch.equal(seen[0], seen[1]) and torch.equal(seen[4], seen[6])
     assert all(not torch.equal(a, b) for a, b in zip(seen[1:], seen[2:]))
+
+
+def test_the_whole_step_op_asks_for_what_its_kernel_reads_and_gives_the_stepper_s_bits():
+    from boost_and_broadside_amd import ops
+
+    D, B, N, M = 128, 5, 8, 4
+    trunk, _ = _rollout_trunk(221)
+    stepper = bnb.trunk_stepper(trunk, B, N + M, N, autocast_dtype=torch.bfloat16, graph=False)
+    plan = stepper._whole
+    gen = torch.Generator().manual_seed(222)
+    x, alive = torch.randn(B, N + M, D, generator=gen).to(DEV), (torch.rand(B, N + M, generator=gen) < 0.7).to(DEV)
+    state = torch.randn(stepper.state.shape, generator=gen).to(DEV)
+    new_state = torch.empty_like(state)
+    out = ops.trunk_step(plan.table, x, N, alive, state, new_state, bullet_eps=plan.bullet_eps)
+    stepper.load_state(state)
+    want, want_state = stepper.step(x, alive)
+    assert torch.equal(out, want) and torch.equal(new_state, want_state)
+    good = {"x": x, "alive": alive, "state_in": state, "state_out": new_state}
+    for name, bad in (("x", x.half()), ("x", x.transpose(0, 1).contiguous().transpose(0, 1)), ("alive", alive.float()), ("alive", alive[:, 1:]),
+                      ("state_in", state[:, 1:]), ("state_out", new_state[:1])):
+        with pytest.raises(ValueError):
+            ops.trunk_step(plan.table, n_rec=N, **{**good, name: bad})
+    with pytest.raises(ValueError, match="recurrent sublayers"):
+        ops.trunk_step(plan.table, x, N, alive, state[:1].contiguous(), new_state[:1].contiguous())
+    with pytest.raises(RuntimeError):
+        ops.trunk_step(plan.table, x[..., :64].contiguous(), N, alive, state, new_state)
